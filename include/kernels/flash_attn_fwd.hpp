@@ -32,7 +32,7 @@
 //     is only moved when a block exceeds it by more than 2^8 ("lazy rescaling": a stale maximum is
 //     harmless, p <= 2^8 stays far inside f16 / f32 range and the final division cancels it), which
 //     makes the rescale of the output accumulators a rare, wave-uniform branch.
-// M % (32 * kWaves) == 0 and N % kBN == 0 are required (checked by the host launcher).
+// M % 32 == 0 and N % kBN == 0 are required (checked by the host launcher).
 #pragma once
 
 #include "config.hpp"
@@ -74,12 +74,19 @@ namespace detail {
 DEVICE float exchange32(float v) { return __shfl_xor(v, 32, 64); }
 /// 2^x as one v_exp_f32 (no range fix-ups: arguments here are <= 8 and results below 2^-126 may flush to 0).
 DEVICE float exp2_raw(float x) { return __builtin_amdgcn_exp2f(x); }
+/// Head (or other unit with its own keys) and query block of this workgroup in a grid of q_blocks * units. Workgroup ids
+/// congruent modulo 8 land on the same XCD and share its L2: each XCD takes a run of consecutive (unit, query block)
+/// pairs, so the query blocks of a unit meet in one L2 (but for the few units a boundary between XCDs cuts) and every XCD
+/// gets the same number of workgroups whatever the number of units.
+DEVICE void xcd_head_block(int q_blocks, int units, int& unit, int& q_block) {
+    const int total = q_blocks * units, q = total / 8, r = total % 8, xcd = blockIdx.x & 7;
+    const int lin = xcd * q + min(xcd, r) + int(blockIdx.x >> 3);
+    unit = lin / q_blocks;
+    q_block = lin - unit * q_blocks;
+}
 }  // namespace detail
 
-/// grid = (M / kBM) * batch workgroups (1-D), block = Traits::kThreads, dynamic LDS = Traits::kLdsBytes.
-/// Workgroup ids that are congruent modulo 8 land on the same XCD (and share its L2): when the batch
-/// count is a multiple of 8 the query blocks of one (batch, head) item all get such ids, so its K and V
-/// are fetched from HBM once instead of once per XCD.
+/// grid = ceil(M / kBM) * batch workgroups (1-D), block = Traits::kThreads, dynamic LDS = Traits::kLdsBytes.
 template <typename Traits>
 __global__ void __launch_bounds__(Traits::kThreads)
     flash_attention_fwd(const __half* __restrict__ Q, const __half* __restrict__ K, const __half* __restrict__ V,
@@ -95,18 +102,13 @@ __global__ void __launch_bounds__(Traits::kThreads)
     const int q32 = lane & 31;  // query (column of Sᵀ / Oᵀ) owned by this lane
     const int h = lane >> 5;    // lane half
 
-    const int q_blocks = M / Traits::kBM;
+    const int q_blocks = (M + Traits::kBM - 1) / Traits::kBM;
     int head_i, q_block;
-    if (batch % 8 == 0) {
-        const int xcd = blockIdx.x & 7, rest = blockIdx.x >> 3;
-        q_block = rest % q_blocks;
-        head_i = (rest / q_blocks) * 8 + xcd;
-    } else {
-        q_block = blockIdx.x % q_blocks;
-        head_i = blockIdx.x / q_blocks;
-    }
+    detail::xcd_head_block(q_blocks, batch, head_i, q_block);
     const size_t head = head_i;
-    const int m0 = q_block * Traits::kBM + wave * 32;
+    // a wavefront of the last block whose 32 queries lie beyond M works on the last ones that exist and stores nothing
+    const bool valid = q_block * Traits::kBM + wave * 32 < M;
+    const int m0 = valid ? q_block * Traits::kBM + wave * 32 : M - 32;
     const __half* Qh = Q + (head * M + m0) * kD;
     const __half* Kh = K + head * size_t(N) * kD;
     const __half* Vh = V + head * size_t(N) * kD;
@@ -330,6 +332,7 @@ __global__ void __launch_bounds__(Traits::kThreads)
         }
     }
     __builtin_amdgcn_s_waitcnt(0xc07f);
+    if (!valid) return;
     constexpr int kLanesPerRow = kRowBytes / 16;
     constexpr int kRowsPerIter = kWaveSize / kLanesPerRow;
     const int rr = lane / kLanesPerRow, cc = lane % kLanesPerRow;
@@ -369,18 +372,13 @@ __global__ void __launch_bounds__(Traits::kThreads)
     const int q32 = lane & 31;  // query (column of Sᵀ / Oᵀ) owned by this lane
     const int h = lane >> 5;    // lane half
 
-    const int q_blocks = M / Traits::kBM;
+    const int q_blocks = (M + Traits::kBM - 1) / Traits::kBM;
     int head_i, q_block;
-    if (batch % 8 == 0) {
-        const int xcd = blockIdx.x & 7, rest = blockIdx.x >> 3;
-        q_block = rest % q_blocks;
-        head_i = (rest / q_blocks) * 8 + xcd;
-    } else {
-        q_block = blockIdx.x % q_blocks;
-        head_i = blockIdx.x / q_blocks;
-    }
+    detail::xcd_head_block(q_blocks, batch, head_i, q_block);
     const size_t head = head_i;
-    const int m0 = q_block * Traits::kBM + wave * 32;
+    // a wavefront of the last block whose 32 queries lie beyond M works on the last ones that exist and stores nothing
+    const bool valid = q_block * Traits::kBM + wave * 32 < M;
+    const int m0 = valid ? q_block * Traits::kBM + wave * 32 : M - 32;
     const __half* Qh = Q + (head * M + m0) * kD;
     const __half* Kh = K + head * size_t(N) * kD;
     const __half* Vh = V + head * size_t(N) * kD;
@@ -595,6 +593,7 @@ __global__ void __launch_bounds__(Traits::kThreads)
         }
     }
     __builtin_amdgcn_s_waitcnt(0xc07f);
+    if (!valid) return;
     constexpr int kLanesPerRow = kRowBytes / 16;
     constexpr int kRowsPerIter = kWaveSize / kLanesPerRow;
     const int rr = lane / kLanesPerRow, cc = lane % kLanesPerRow;

@@ -754,8 +754,10 @@ int launch_fa_fwd(const __half* Q, const __half* K, const __half* V, __half* O, 
                   hipStream_t stream) {
     using Traits = FlashFwdTraits<kD, kWaves, 64>;
     auto kernel = kFused ? &flash_attention_fwd_fused<Traits> : &flash_attention_fwd<Traits>;
-    return launch(kernel, dim3((M / Traits::kBM) * batch), dim3(Traits::kThreads), Traits::kLdsBytes, stream, Q, K, V,
-                  O, batch, M, N, scale);
+    const long grid = (long)((M + Traits::kBM - 1) / Traits::kBM) * batch;
+    if (grid > INT_MAX) return fail(TCU_ERR_UNSUPPORTED_SHAPE, "attention: too many query blocks for one launch");
+    return launch(kernel, dim3(unsigned(grid)), dim3(Traits::kThreads), Traits::kLdsBytes, stream, Q, K, V, O, batch, M, N,
+                  scale);
 }
 
 template <bool kVColMajor>
@@ -823,12 +825,36 @@ int fa_w64_k32_dispatch(const __half* Q, const __half* K, const __half* V, __hal
                                        : launch_fa_w64_k32<128, true>(Q, K, V, O, batch, M, N, scale, stream);
 }
 
+/// How many wavefronts (of 32 queries) a workgroup of the 8-wavefront kernels has, and what the launch costs relative to
+/// one round of 2-wavefront workgroups. More wavefronts share a block of keys (at head size 128 a CU holds one workgroup
+/// whatever its size: 96 KiB of LDS; at 64 up to three, which share the CU: 0.6, 0.75, 0.95 of a round for each further
+/// one), fewer leave less idle behind M. Queries beyond M cost their wavefronts' idle time only.
+/// Measured, us with 2, 4, 8 wavefronts (the largest that divides M was taken before): 200 x 192 x 512 at head size 128:
+/// 44.5, 33.5, 21.8; 100 x 448^2: 39.8, 29.7, 19.1; 40 x 832 x 960: 70.2, 50.3, 29.7; 96 x 576^2 at head size 64: 26.7,
+/// 18.4, 26.6; 300 x 64 x 512 at 128: 31.2, 33.2, 37.8; 36 x 448^2 at 128: 14.4, 14.8, 16.4.
+struct AttnWavesPlan {
+    int waves;
+    double rounds;
+};
+AttnWavesPlan attn_waves_plan(int batch, int M, int D) {
+    AttnWavesPlan plan{8, 1e30};
+    for (const auto& [waves, one, more] : {std::tuple{2, 1.0, 0.6}, std::tuple{4, 1.05, 0.75}, std::tuple{8, 1.15, 0.95}}) {
+        const long groups = (long)batch * ((M + 32 * waves - 1) / (32 * waves));
+        const long per_cu = (groups + 255) / 256;
+        const double rounds = one * (1.0 + double(per_cu - 1) * (D == 128 ? 1.0 : more));
+        if (rounds < plan.rounds) plan = {waves, rounds};
+    }
+    return plan;
+}
+
 template <int kD, bool kFused>
 int fa_fwd_by_rows(const __half* Q, const __half* K, const __half* V, __half* O, int batch, int M, int N, float scale,
                    hipStream_t stream) {
-    if (M % 256 == 0) return launch_fa_fwd<kD, 8, kFused>(Q, K, V, O, batch, M, N, scale, stream);
-    if (M % 128 == 0) return launch_fa_fwd<kD, 4, kFused>(Q, K, V, O, batch, M, N, scale, stream);
-    return launch_fa_fwd<kD, 2, kFused>(Q, K, V, O, batch, M, N, scale, stream);
+    switch (attn_waves_plan(batch, M, kD).waves) {
+        case 8: return launch_fa_fwd<kD, 8, kFused>(Q, K, V, O, batch, M, N, scale, stream);
+        case 4: return launch_fa_fwd<kD, 4, kFused>(Q, K, V, O, batch, M, N, scale, stream);
+        default: return launch_fa_fwd<kD, 2, kFused>(Q, K, V, O, batch, M, N, scale, stream);
+    }
 }
 
 int fa_dispatch(const __half* Q, const __half* K, const __half* V, __half* O, int batch, int M, int N, int Kd, int P,
