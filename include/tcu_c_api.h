@@ -95,8 +95,9 @@ typedef enum {
 
 /* Which attention kernel to run (tcu_flash_attn_fwd_f16_algo). For a row-major V, AUTO picks WAVE64_K32 with at least 256
  * whole blocks of 256 queries and N >= 320 (192 with N >= 1024), at head size 128 also WAVE64 with 128 to 191 such blocks
- * and N >= 1024, and MFMA32_FUSED otherwise; for a column-major V (head size 128) AUTO picks WAVE64_K32 under the same conditions and
- * WAVE64 otherwise (it takes every M % 64 == 0 and N % 64 == 0). */
+ * and N >= 1024, and otherwise KEYS or MFMA32_FUSED, whichever a cost model expects to be the shorter; for a column-major V
+ * (head size 128) AUTO picks WAVE64_K32 under the same conditions and KEYS or WAVE64 otherwise (both take every
+ * M % 64 == 0 and N % 64 == 0). */
 typedef enum {
     TCU_ATTN_AUTO = 0,
     TCU_ATTN_TILE_LIBRARY = 1, /* composed from the 16x16 tile primitives, like the reference kernel */
@@ -113,7 +114,7 @@ typedef enum {
                                   ahead with SharedToRegPieces / SharedToRegTrPieces); compile-time sequence lengths:
                                   (M, N) in {(2048, 2048), (512, 1024), (256, 640), (256, 320)}, head size 128, row-major
                                   V; results identical to WAVE64 bit for bit */
-    TCU_ATTN_WAVE64_K32 = 6    /* the WAVE64 design on v_mfma_f32_16x16x32_f16 (tile-library functors; twice the matrix
+    TCU_ATTN_WAVE64_K32 = 6,   /* the WAVE64 design on v_mfma_f32_16x16x32_f16 (tile-library functors; twice the matrix
                                   instructions, each contracting 32 indices: the chip sustains a higher clock on them),
                                   launched as one workgroup per CU that takes its blocks of 256 queries one after the
                                   other and fetches the next one's first operands under the last steps of the current;
@@ -121,6 +122,10 @@ typedef enum {
                                   (wavefronts of a head's last block whose 64 queries lie beyond M idle), N % 64 == 0,
                                   N >= 320; results equal to WAVE64 (MFMA32_FUSED at head size 64) up to the
                                   summation order inside a matrix instruction */
+    TCU_ATTN_KEYS = 8          /* a workgroup per 64 queries whose 4 wavefronts split the keys (and, through a workspace,
+                                  several workgroups per 64 queries: tcu_flash_attn_fwd_f16_ws): for launches with few
+                                  query blocks; M % 64 == 0, N % 64 == 0, head size 128 with either V layout or 64 with a
+                                  row-major V; results equal to the others up to rounding and the order of the sums */
 } tcu_attn_algo;
 
 /* Which LSTM step kernel to run (tcu_lstm_f16_algo). AUTO picks STREAMING where it is instantiated, else
@@ -202,6 +207,18 @@ int tcu_flash_attn_fwd_f16(const void* Q, const void* K, const void* V, void* O,
 /* tcu_flash_attn_fwd_f16 with an explicit kernel choice (tcu_attn_algo); same arguments otherwise. */
 int tcu_flash_attn_fwd_f16_algo(const void* Q, const void* K, const void* V, void* O, int batch, int M, int N,
                                 int Kdim, int P, float scale, int v_layout, int algo, void* stream);
+
+/*
+ * tcu_flash_attn_fwd_f16 for calls with few query blocks and many keys (a short block of new queries against a long
+ * cache), where one workgroup per 64 queries leaves most of the chip idle: the keys are split over several workgroups,
+ * their f32 partial outputs go to `workspace`, and a second kernel adds them. tcu_flash_attn_workspace_bytes(...) is the
+ * workspace this takes, or 0 when the keys are not split: then, and when `workspace` is NULL, the call is
+ * tcu_flash_attn_fwd_f16. The workspace (16-byte aligned device memory) is the caller's and free to reuse once the work
+ * enqueued here has run. Results differ from the unsplit ones by rounding and the order of the f32 sums only.
+ */
+unsigned long long tcu_flash_attn_workspace_bytes(int batch, int M, int N, int Kdim, int P, int v_layout);
+int tcu_flash_attn_fwd_f16_ws(const void* Q, const void* K, const void* V, void* O, int batch, int M, int N, int Kdim, int P,
+                              float scale, int v_layout, void* workspace, unsigned long long workspace_bytes, void* stream);
 
 /*
  * Fused LSTM layer over T steps. x [T, B, I] f16; W [4H, I+H] f16 row-major, gate rows in the

@@ -40,3 +40,76 @@ def test_query_counts_that_are_not_whole_blocks(tcu, oracle, device, batch, M, N
     print(f"attention partial blocks b{batch} {M}x{N} D{D} {algo}", flush=True)
     _run(tcu, oracle, device, lambda q, k, v, o: tcu.flash_attention(q, k, v, out=o, algo=algo), batch, M, N, D,
          (0, batch // 2, batch - 1))
+
+
+@pytest.mark.parametrize("v_layout", ["row", "col"])
+@pytest.mark.parametrize("batch,M,N,D", [(1, 64, 64, 128), (1, 64, 128, 128), (3, 192, 320, 128), (2, 128, 576, 128),
+                                         (5, 64, 1024, 128), (1, 64, 64, 64), (3, 192, 320, 64), (9, 128, 832, 64)])
+def test_wavefronts_split_the_keys(tcu, oracle, device, batch, M, N, D, v_layout):
+    """The key-splitting kernel by name: 1 to 8 blocks of 32 keys per wavefront (even and odd counts take different ways
+    out of its unrolled loop), wavefronts with no block at all (64 keys) and with one less than the others, head counts
+    that are not multiples of 8; both V layouts at head size 128."""
+    if v_layout == "col" and D != 128:
+        pytest.skip("a column-major V is instantiated for head size 128")
+    print(f"attention keys b{batch} {M}x{N} D{D} V {v_layout}", flush=True)
+
+    def call(q, k, v, o):
+        if v_layout == "row":
+            tcu.flash_attention(q, k, v, out=o, algo="keys")
+        else:
+            tcu.flash_attention_fwd(q.flatten(), k.flatten(), v.transpose(1, 2).contiguous().flatten(), o.view(-1), M, N, D, D,
+                                    scale=1.0 / math.sqrt(D), batch=batch, algo="keys")
+
+    _run(tcu, oracle, device, call, batch, M, N, D, range(batch))
+
+
+@pytest.mark.parametrize("batch,M,N,D,v_layout", [(1, 64, 8192, 128, "row"), (1, 64, 8192, 128, "col"), (32, 64, 4096, 128, "row"),
+                                                  (3, 192, 2112, 128, "row"), (2, 64, 4096, 64, "row")])
+def test_workgroups_split_the_keys_through_a_workspace(tcu, oracle, device, batch, M, N, D, v_layout):
+    """Few queries against many keys: AUTO splits the keys over workgroups when it has a workspace (one of the caller's,
+    whose bytes past the stated size stay untouched, or one it takes itself) and gives the same result without one, up to
+    rounding; splits of unequal length (66 blocks of 32 keys)."""
+    import torch
+
+    code = tcu.TCU_V_ROW_MAJOR if v_layout == "row" else tcu.TCU_V_COL_MAJOR
+    need = tcu.attention_workspace_bytes(batch, M, N, D, D, code)
+    print(f"attention split keys b{batch} {M}x{N} D{D} V {v_layout}: {need} bytes", flush=True)
+    assert need > 0 and need % (batch * M * (D + 2) * 4) == 0
+    ws = torch.full((need + 256,), 0x5A, dtype=torch.uint8, device=device)
+
+    def call(workspace):
+        def go(q, k, v, o):
+            if v_layout == "row":
+                tcu.flash_attention(q, k, v, out=o, workspace=workspace)
+            else:
+                tcu.flash_attention_fwd(q.flatten(), k.flatten(), v.transpose(1, 2).contiguous().flatten(), o.view(-1), M, N, D,
+                                        D, scale=1.0 / math.sqrt(D), batch=batch, workspace=workspace)
+        return go
+
+    q, k, v, out = _run(tcu, oracle, device, call(ws), batch, M, N, D, {0, batch - 1})
+    assert bool((ws[need:] == 0x5A).all())
+    own, unsplit = torch.empty_like(out), torch.empty_like(out)
+    call(None)(q, k, v, own)
+    call(False)(q, k, v, unsplit)
+    torch.cuda.synchronize()
+    assert torch.equal(own, out)
+    assert float((unsplit.float() - out.float()).abs().max()) <= 2 * ABS_TOL
+
+
+@pytest.mark.parametrize("N,splits", [(512, 1), (4096, 4)])
+def test_keys_kernel_moves_its_maxima(tcu, oracle, device, N, splits):
+    """Keys whose norm grows along the sequence and large queries: the maxima move in many blocks, and the splits of the
+    keys differ in theirs by far. Logits reach 30 here, where rounding the scaled queries to f16 alone costs
+    30 * 2^-11 * 5 / 2 = 4e-2 at most."""
+    import torch
+
+    batch, M, D = 2, 64, 128
+    q = (oracle.fill_normal(batch * M * D, 41).reshape(batch, M, D).astype(np.float32) * 2).astype(np.float16)
+    k = oracle.fill_normal(batch * N * D, 42).reshape(batch, N, D).astype(np.float32)
+    k = (k * np.linspace(0.2, 3.0, N, dtype=np.float32)[None, :, None]).astype(np.float16)
+    v = oracle.fill_normal(batch * N * D, 43).reshape(batch, N, D)
+    assert (tcu.attention_workspace_bytes(batch, M, N, D, D) > 0) == (splits > 1)
+    dq, dk, dv = (torch.from_numpy(np.ascontiguousarray(a)).to(device) for a in (q, k, v))
+    out = tcu.flash_attention(dq, dk, dv) if splits > 1 else tcu.flash_attention(dq, dk, dv, algo="keys")
+    torch.cuda.synchronize()
+    assert oracle.max_abs_err(out.float().cpu().numpy(), oracle.attention(q, k, v, 1.0 / math.sqrt(D))) <= 4e-2

@@ -18,7 +18,7 @@ import torch
 
 __all__ = [
     "TcuError", "library_path", "lib", "last_error", "gemm", "gemm_workspace_bytes", "b2b_gemm", "flash_attention_fwd",
-    "flash_attention", "TiledFlashAttention", "lstm", "lstm_workspace_bytes", "lstm_persistent_workspace_bytes", "lstm_persistent_status", "scatter_nd", "GEMM_ALGOS", "ATTN_ALGOS", "LSTM_ALGOS", "B2B_ALGOS",
+    "flash_attention", "attention_workspace_bytes", "TiledFlashAttention", "lstm", "lstm_workspace_bytes", "lstm_persistent_workspace_bytes", "lstm_persistent_status", "scatter_nd", "GEMM_ALGOS", "ATTN_ALGOS", "LSTM_ALGOS", "B2B_ALGOS",
     "SCATTER_MODES",
 ]
 
@@ -40,7 +40,7 @@ GEMM_ALGOS = {"auto": 0, "global_reg": 1, "all_mem": 2, "pipelined": 3, "wave128
 TCU_V_COL_MAJOR = 0
 TCU_V_ROW_MAJOR = 1
 
-ATTN_ALGOS = {"auto": 0, "tile_library": 1, "mfma32": 2, "mfma32_fused": 3, "wave64": 4, "tile_wave64": 5, "wave64_k32": 6}
+ATTN_ALGOS = {"auto": 0, "tile_library": 1, "mfma32": 2, "mfma32_fused": 3, "wave64": 4, "tile_wave64": 5, "wave64_k32": 6, "keys": 8}
 LSTM_ALGOS = {"auto": 0, "tile_library": 1, "streaming": 2, "ragged": 3}
 B2B_ALGOS = {"auto": 0, "tile_library": 1, "resident": 2, "rows": 3, "tile_resident": 4}
 SCATTER_MODES = {"assign": 0, "add": 1}
@@ -60,6 +60,9 @@ _SIGNATURES = {
                                                                                            ctypes.c_void_p]),
     "tcu_flash_attn_fwd_f16_algo": (ctypes.c_int, [ctypes.c_void_p] * 4 + [ctypes.c_int] * 5 + [ctypes.c_float, ctypes.c_int,
                                                                                                 ctypes.c_int, ctypes.c_void_p]),
+    "tcu_flash_attn_workspace_bytes": (ctypes.c_ulonglong, [ctypes.c_int] * 6),
+    "tcu_flash_attn_fwd_f16_ws": (ctypes.c_int, [ctypes.c_void_p] * 4 + [ctypes.c_int] * 5 + [ctypes.c_float, ctypes.c_int, ctypes.c_void_p,
+                                                                                              ctypes.c_ulonglong, ctypes.c_void_p]),
     "tcu_lstm_f16": (ctypes.c_int, [ctypes.c_void_p] * 7 + [ctypes.c_int] * 4 + [ctypes.c_void_p]),
     "tcu_lstm_f16_algo": (ctypes.c_int, [ctypes.c_void_p] * 7 + [ctypes.c_int] * 5 + [ctypes.c_void_p]),
     "tcu_lstm_workspace_bytes": (ctypes.c_ulonglong, [ctypes.c_int] * 4),
@@ -210,11 +213,31 @@ def b2b_gemm(a: torch.Tensor, b_t: torch.Tensor, c_t: torch.Tensor, out: torch.T
 
 
 # ------------------------------------------------------------------------------ attention
+def _attention_with_workspace(ptrs: tuple[int, ...], batch: int, m: int, n: int, k: int, p: int, scale: float, v_layout: int,
+                              algo: str, workspace: torch.Tensor | None, device: torch.device) -> None:
+    if workspace is None:
+        need = attention_workspace_bytes(batch, m, n, k, p, v_layout)
+        if need > 0:
+            workspace = torch.empty(need, dtype=torch.uint8, device=device)
+    elif algo != "auto":
+        raise ValueError("a workspace goes with algo='auto'")
+    elif not workspace.is_cuda or not workspace.is_contiguous():
+        raise ValueError("workspace must be a contiguous device tensor")
+    ws, size = (0, 0) if workspace is None else (workspace.data_ptr(), workspace.numel() * workspace.element_size())
+    _check(lib().tcu_flash_attn_fwd_f16_ws(*ptrs, batch, m, n, k, p, scale, v_layout, ws, size, _stream()))
+
+
+def attention_workspace_bytes(batch: int, m: int, n: int, k: int, p: int, v_layout: int = TCU_V_ROW_MAJOR) -> int:
+    """Device bytes an attention call uses to split its keys over workgroups; 0 when they are not split."""
+    return int(lib().tcu_flash_attn_workspace_bytes(batch, m, n, k, p, v_layout))
+
+
 def flash_attention_fwd(Q: torch.Tensor, K: torch.Tensor, V: torch.Tensor, O: torch.Tensor, m: int, n: int, k: int,
-                        p: int, scale: float = 1.0, batch: int = 1, algo: str = "auto") -> None:
+                        p: int, scale: float = 1.0, batch: int = 1, algo: str = "auto",
+                        workspace: torch.Tensor | None | bool = None) -> None:
     """Same call shape as the reference's ``pytiledcuda.flash_attention_fwd`` (flattened fp16
     device tensors; K as [n, k], V as [p, n]; O written in place; ``scale`` defaults to the
-    reference's 1; ``algo`` picks a kernel, as in ``flash_attention``).  Unsupported shapes raise
+    reference's 1; ``algo`` picks a kernel and ``workspace`` is as in ``flash_attention``).  Unsupported shapes raise
     ``RuntimeError`` like the reference op."""
     if min(m, n, k, p, batch) <= 0:
         raise ValueError("m, n, k, p and batch must be positive")
@@ -222,15 +245,21 @@ def flash_attention_fwd(Q: torch.Tensor, K: torch.Tensor, V: torch.Tensor, O: to
                           ("O", O, batch * m * p)):
         if t.numel() != want:
             raise ValueError(f"{name} must hold batch*rows*cols = {want} elements, got {t.numel()}")
-    _check(lib().tcu_flash_attn_fwd_f16_algo(_dev_ptr(Q, torch.float16, "Q"), _dev_ptr(K, torch.float16, "K"),
-                                             _dev_ptr(V, torch.float16, "V"), _dev_ptr(O, torch.float16, "O"), batch, m,
-                                             n, k, p, float(scale), TCU_V_COL_MAJOR, ATTN_ALGOS[algo], _stream()))
+    ptrs = (_dev_ptr(Q, torch.float16, "Q"), _dev_ptr(K, torch.float16, "K"), _dev_ptr(V, torch.float16, "V"),
+            _dev_ptr(O, torch.float16, "O"))
+    if workspace is not False and (workspace is not None or (algo == "auto" and n > 512)):  # fewer keys are never split
+        _attention_with_workspace(ptrs, batch, m, n, k, p, float(scale), TCU_V_COL_MAJOR, algo, workspace, Q.device)
+        return
+    _check(lib().tcu_flash_attn_fwd_f16_algo(*ptrs, batch, m, n, k, p, float(scale), TCU_V_COL_MAJOR, ATTN_ALGOS[algo], _stream()))
 
 
 def flash_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scale: float | None = None,
-                    out: torch.Tensor | None = None, algo: str = "auto") -> torch.Tensor:
+                    out: torch.Tensor | None = None, algo: str = "auto",
+                    workspace: torch.Tensor | None | bool = None) -> torch.Tensor:
     """softmax(scale · q kᵀ) v for [..., S, D] tensors in the usual layout (V row-major [S, D]).
-    ``scale`` defaults to 1/sqrt(D)."""
+    ``scale`` defaults to 1/sqrt(D). With ``algo="auto"`` a call with few queries and many keys splits the keys over
+    workgroups through ``workspace`` (a contiguous device tensor of at least ``attention_workspace_bytes(...)`` bytes) or,
+    when none is given, through one taken from torch's caching allocator for the call; ``workspace=False`` never splits."""
     if q.dim() < 2 or k.dim() < 2 or v.dim() < 2:
         raise ValueError("q, k and v must be [..., S, D]")
     *lead, M, D = q.shape
@@ -249,10 +278,12 @@ def flash_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scale: fl
         out = torch.empty(*lead, M, P, dtype=torch.float16, device=q.device)
     elif tuple(out.shape) != (*lead, M, P):
         raise ValueError(f"out must be {(*lead, M, P)}, got {tuple(out.shape)}")
-    _check(lib().tcu_flash_attn_fwd_f16_algo(_dev_ptr(q, torch.float16, "q"), _dev_ptr(k, torch.float16, "k"),
-                                             _dev_ptr(v, torch.float16, "v"), _dev_ptr(out, torch.float16, "out"),
-                                             batch, M, N, D, P, float(scale), TCU_V_ROW_MAJOR, ATTN_ALGOS[algo],
-                                             _stream()))
+    ptrs = (_dev_ptr(q, torch.float16, "q"), _dev_ptr(k, torch.float16, "k"), _dev_ptr(v, torch.float16, "v"),
+            _dev_ptr(out, torch.float16, "out"))
+    if workspace is not False and (workspace is not None or (algo == "auto" and N > 512)):  # fewer keys are never split
+        _attention_with_workspace(ptrs, batch, M, N, D, P, float(scale), TCU_V_ROW_MAJOR, algo, workspace, q.device)
+        return out
+    _check(lib().tcu_flash_attn_fwd_f16_algo(*ptrs, batch, M, N, D, P, float(scale), TCU_V_ROW_MAJOR, ATTN_ALGOS[algo], _stream()))
     return out
 
 

@@ -6,6 +6,7 @@
 
 #include "kernels/b2b_gemm_fwd.hpp"
 #include "kernels/flash_attn_fwd.hpp"
+#include "kernels/flash_attn_keys.hpp"
 #include "kernels/flash_attn_tile_w64.hpp"
 #include "kernels/flash_attn_w64_k32.hpp"
 #include "kernels/flash_attn_w64.hpp"
@@ -827,22 +828,25 @@ int fa_w64_k32_dispatch(const __half* Q, const __half* K, const __half* V, __hal
 
 /// How many wavefronts (of 32 queries) a workgroup of the 8-wavefront kernels has, and what the launch costs relative to
 /// one round of 2-wavefront workgroups. More wavefronts share a block of keys (at head size 128 a CU holds one workgroup
-/// whatever its size: 96 KiB of LDS; at 64 up to three, which share the CU: 0.6, 0.75, 0.95 of a round for each further
-/// one), fewer leave less idle behind M. Queries beyond M cost their wavefronts' idle time only.
+/// whatever its size: 96 KiB of LDS; at 64 up to three of 2 or 4 wavefronts share one, the second for half a round, the
+/// third for 0.7), fewer leave less idle behind M. Queries beyond M cost their wavefronts' idle time only.
 /// Measured, us with 2, 4, 8 wavefronts (the largest that divides M was taken before): 200 x 192 x 512 at head size 128:
 /// 44.5, 33.5, 21.8; 100 x 448^2: 39.8, 29.7, 19.1; 40 x 832 x 960: 70.2, 50.3, 29.7; 96 x 576^2 at head size 64: 26.7,
 /// 18.4, 26.6; 300 x 64 x 512 at 128: 31.2, 33.2, 37.8; 36 x 448^2 at 128: 14.4, 14.8, 16.4.
 struct AttnWavesPlan {
     int waves;
     double rounds;
+    long groups;
 };
 AttnWavesPlan attn_waves_plan(int batch, int M, int D) {
-    AttnWavesPlan plan{8, 1e30};
-    for (const auto& [waves, one, more] : {std::tuple{2, 1.0, 0.6}, std::tuple{4, 1.05, 0.75}, std::tuple{8, 1.15, 0.95}}) {
+    AttnWavesPlan plan{8, 1e30, 0};
+    for (const auto& [waves, one, second, rise] :
+         {std::tuple{2, 1.0, 0.55, 0.1}, std::tuple{4, 1.05, 0.45, 0.23}, std::tuple{8, 1.15, 1.15, 0.0}}) {
         const long groups = (long)batch * ((M + 32 * waves - 1) / (32 * waves));
         const long per_cu = (groups + 255) / 256;
-        const double rounds = one * (1.0 + double(per_cu - 1) * (D == 128 ? 1.0 : more));
-        if (rounds < plan.rounds) plan = {waves, rounds};
+        const double more = double(per_cu - 1);
+        const double rounds = one * (1.0 + (D == 128 ? more : more * second + more * (more - 1.0) / 2.0 * rise));
+        if (rounds < plan.rounds) plan = {waves, rounds, groups};
     }
     return plan;
 }
@@ -857,18 +861,121 @@ int fa_fwd_by_rows(const __half* Q, const __half* K, const __half* V, __half* O,
     }
 }
 
+template <int kD, bool kVColMajor>
+int launch_fa_keys(const __half* Q, const __half* K, const __half* V, __half* O, float* part, int batch, int M, int N,
+                   int splits, float scale, hipStream_t stream) {
+    using Traits = FlashKeysTraits<kD, kVColMajor>;
+    const long grid = (long)batch * splits * (M / Traits::kBM);
+    if (grid > INT_MAX || N >= (1 << 24)) return fail(TCU_ERR_UNSUPPORTED_SHAPE, "attention: too many query blocks or keys for one launch");
+    int rc = launch(&flash_attention_keys<Traits>, dim3(unsigned(grid)), dim3(Traits::kThreads), Traits::kLdsBytes, stream, Q,
+                    K, V, O, part, batch, M, N, splits, scale);
+    if (rc != TCU_OK || splits == 1) return rc;
+    const size_t rows = size_t(batch) * M;
+    auto combine = splits <= 4 ? &flash_attention_combine<kD, 4> : splits <= 8 ? &flash_attention_combine<kD, 8> : &flash_attention_combine<kD, 16>;
+    return launch(combine, dim3(unsigned((rows * kD / 4 + 255) / 256)), dim3(256), 0, stream, static_cast<const float*>(part), O,
+                  rows, splits);
+}
+
+int fa_keys_dispatch(const __half* Q, const __half* K, const __half* V, __half* O, float* part, int batch, int M, int N, int Kd,
+                     int splits, float scale, int v_layout, hipStream_t stream) {
+    if (Kd == 128 && v_layout == TCU_V_ROW_MAJOR)
+        return launch_fa_keys<128, false>(Q, K, V, O, part, batch, M, N, splits, scale, stream);
+    if (Kd == 128) return launch_fa_keys<128, true>(Q, K, V, O, part, batch, M, N, splits, scale, stream);
+    if (Kd == 64 && v_layout == TCU_V_ROW_MAJOR)
+        return launch_fa_keys<64, false>(Q, K, V, O, part, batch, M, N, splits, scale, stream);
+    return fail(TCU_ERR_UNSUPPORTED_SHAPE, "the key-splitting attention kernel is instantiated for head size 128, and for head "
+                                           "size 64 with a row-major V");
+}
+
+/// Expected time (us) of the key-splitting kernel with `splits` workgroups per 64 queries: rounds of 256 (head size 128) or
+/// 512 workgroups (64: two per CU), a fixed part for the queries, the first keys and the merge, and per block of 4 x 32 keys
+/// 0.95 us (0.62 at head size 64) plus what the memory adds as more workgroups read keys of their own (M / 64 of them share
+/// theirs): 2.3 us with 256 of them, 6.8 TB/s; no less than the L2s take for a full chip (1.05, 1.15 us); with splits the
+/// partial outputs written, read and one launch more. Fitted to 14 shapes at both head sizes with keys and values not in
+/// any cache (32 x 64 x 8192 at 128 with 1, 2, 4, 8, 16 workgroups: 83, 52, 34, 31, 37 us; 64 x 64 x 4096: 50, 35, 32, 37;
+/// 8 x 64 x 8192: 77, 46, 29, 21, 18).
+double attn_keys_us(int batch, int M, int N, int D, int splits) {
+    const long groups = (long)batch * (M / 64) * splits, cap = D == 128 ? 256 : 512;
+    const double blocks = double(N) / (128.0 * splits);
+    double us = D == 128 ? 1.5 : 1.3;
+    for (long left = groups; left > 0; left -= cap) {
+        const double at_once = double(std::min(left, cap)), own = at_once * 64.0 / M, fill = at_once / cap;
+        us += D == 128 ? 5.0 + blocks * std::max(0.95 + 0.0052 * own, 1.05 * fill)
+                       : 3.5 + 1.6 * std::max(0.0, 2.0 * fill - 1.0) + blocks * std::max(0.62 + 0.0035 * own, 1.15 * fill);
+    }
+    return us + (splits == 1 ? 0.0 : 2.4 + (D == 128 ? 0.011 : 0.006) * groups);
+}
+
+/// Expected time (us) of the kernels with 64 queries per wavefront in blocks of 256 (the 16x16x32 one, and the 32x32x16 one
+/// where AUTO runs it), one block per CU at a time, and of the 32-queries-per-wavefront kernel. The time per key rises by a
+/// fifth from a few busy CUs to all of them (the chip is power-limited). Within 10 % of the measured times.
+double attn_w64_us(int batch, int M, int N, int D) {
+    const long items = (long)batch * ((M + 255) / 256), rounds = (items + 255) / 256;
+    const double fill = double(items) / (256.0 * rounds);
+    return 1.3 + rounds * (D == 128 ? 6.0 + N * (0.02 + 0.005 * fill) : 4.0 + N * (0.0135 + 0.0043 * fill));
+}
+double attn_fused_us(int batch, int M, int N, int D) {
+    const AttnWavesPlan plan = attn_waves_plan(batch, M, D);
+    const double fill = std::min(1.0, plan.groups / 256.0);
+    return D == 128 ? 1.3 + plan.rounds * (3.2 + N * (0.0205 + 0.0055 * fill)) : 1.0 + plan.rounds * (2.2 + N * (0.0138 + 0.002 * fill));
+}
+
+/// Whether AUTO's choice among the kernels that give wavefronts their own queries is the 16x16x32 one: from 256 whole blocks of
+/// 256 queries on (192 with N >= 1024), unless a last round of few blocks makes it longer than the 32-queries-per-wavefront
+/// kernel (22 x 2944^2 at head size 64, 264 blocks: 99.8 against 76.3 us; a column-major V has no such alternative).
+bool attn_k32_is_the_choice(int batch, int M, int N, int D, int v_layout) {
+    const long blocks = (long)batch * (M / 256);
+    if (N < 320 || !(blocks >= 256 || (blocks >= 192 && N >= 1024))) return false;
+    return v_layout == TCU_V_COL_MAJOR || attn_w64_us(batch, M, N, D) <= 1.05 * attn_fused_us(batch, M, N, D);
+}
+
+/// Whether it is the 32x32x16 kernel with 64 queries per wavefront (row-major V).
+bool attn_w64_is_the_choice(int batch, int M, int N, int D) {
+    const long blocks = (long)batch * (M / 256);
+    return D == 128 && N >= 1024 && blocks >= 128 && blocks < 192;
+}
+
+/// Expected time of that choice.
+double attn_blocks_us(int batch, int M, int N, int D, int v_layout) {
+    if (v_layout == TCU_V_COL_MAJOR || attn_k32_is_the_choice(batch, M, N, D, v_layout) || attn_w64_is_the_choice(batch, M, N, D))
+        return attn_w64_us(batch, M, N, D);
+    return attn_fused_us(batch, M, N, D);
+}
+
+/// How many workgroups per 64 queries split the keys in the shortest plan of the key-splitting kernel (at most
+/// max_splits <= 16; every wavefront gets a block, one workgroup per CU at most: 32 x 64 x 8192 at head size 64 with 8, 12,
+/// 16: 20.8, 24.9, 24.2 us), or 0 where the other kernels are expected to be as fast. A split has to promise 2.5 us more,
+/// which the second launch and the workspace cost the host.
+int attn_keys_plan(int batch, int M, int N, int D, int v_layout, int max_splits) {
+    if ((D != 128 && !(D == 64 && v_layout == TCU_V_ROW_MAJOR)) || N >= (1 << 24)) return 0;
+    const long groups = (long)batch * (M / 64);
+    if (groups > 4096) return 0;
+    double best_us = attn_blocks_us(batch, M, N, D, v_layout);
+    int best = 0;
+    for (int s : {1, 2, 3, 4, 6, 8, 12, 16}) {
+        if (s > max_splits || (s > 1 && (s * groups > 256 || N < 128 * s))) break;
+        const double us = attn_keys_us(batch, M, N, D, s) + (s > 1 ? 2.5 : 0.0);
+        if (us < best_us) {
+            best_us = us;
+            best = s;
+        }
+    }
+    return best;
+}
+
 int fa_dispatch(const __half* Q, const __half* K, const __half* V, __half* O, int batch, int M, int N, int Kd, int P,
-                float scale, int v_layout, int algo, hipStream_t stream) {
+                float scale, int v_layout, int algo, hipStream_t stream, float* part = nullptr, int splits = 1) {
     using W41 = tl::RowMajor<4, 1>;
     if (Kd != P) return fail(TCU_ERR_UNSUPPORTED_SHAPE, "attention needs the query and value head sizes equal");
     if (M % 64 != 0 || N % 64 != 0) return fail(TCU_ERR_UNSUPPORTED_SHAPE, "attention needs M % 64 == 0 and N % 64 == 0");
     if (algo != TCU_ATTN_AUTO && algo != TCU_ATTN_TILE_LIBRARY && algo != TCU_ATTN_MFMA32 &&
         algo != TCU_ATTN_MFMA32_FUSED && algo != TCU_ATTN_WAVE64 && algo != TCU_ATTN_TILE_WAVE64 &&
-        algo != TCU_ATTN_WAVE64_K32)
+        algo != TCU_ATTN_WAVE64_K32 && algo != TCU_ATTN_KEYS)
         return fail(TCU_ERR_INVALID_ARGUMENT, "unknown attention algo");
     if (v_layout != TCU_V_ROW_MAJOR && v_layout != TCU_V_COL_MAJOR) return fail(TCU_ERR_INVALID_ARGUMENT, "unknown v_layout");
     if (algo == TCU_ATTN_TILE_WAVE64) return fa_tile_w64_dispatch(Q, K, V, O, batch, M, N, Kd, scale, v_layout, stream);
     if (algo == TCU_ATTN_WAVE64_K32) return fa_w64_k32_dispatch(Q, K, V, O, batch, M, N, Kd, scale, v_layout, stream);
+    if (algo == TCU_ATTN_KEYS) return fa_keys_dispatch(Q, K, V, O, part, batch, M, N, Kd, splits, scale, v_layout, stream);
     if (algo == TCU_ATTN_WAVE64) {
         if (Kd != 128)
             return fail(TCU_ERR_UNSUPPORTED_SHAPE, "the one-wavefront-per-SIMD attention kernel is instantiated for head size 128");
@@ -877,16 +984,17 @@ int fa_dispatch(const __half* Q, const __half* K, const __half* V, __half* O, in
     }
     if (v_layout == TCU_V_ROW_MAJOR && algo != TCU_ATTN_TILE_LIBRARY) {
         if (Kd != 128 && Kd != 64) return fail(TCU_ERR_UNSUPPORTED_SHAPE, "attention is instantiated for head sizes 64 and 128");
-        // Enough query blocks to fill the chip: the kernels with 64 queries per wavefront. From one block of 256 queries
-        // per CU on (counting a sequence's whole blocks; M is any multiple of 64) the chip runs at its power limit, where
+        // Few query blocks: the wavefronts split the keys. Enough to fill the chip: the kernels with 64 queries per wavefront.
+        // From one block of 256 queries per CU on the chip runs at its power limit, where
         // the 16x16x32 instruction wins, at every sequence length that kernel takes (256 x 512 x 512 x 128: 45.6 against
         // 57.9 us for the 8-wavefront kernel, 1024 x 320 x 320: 117.7 against 203); a half-empty chip runs at full clock,
         // where the 32x32x16 kernel's fewer issue cycles do (long sequences, head size 128: 16 x 2048^2 45.7 against 48.8
         // us; with 192 blocks the 16x16x32 kernel is ahead again, 52.6 against 55.5).
-        const long blocks = (long)batch * (M / 256);
-        if (algo == TCU_ATTN_AUTO && N >= 320 && (blocks >= 256 || (blocks >= 192 && N >= 1024)))
+        if (algo == TCU_ATTN_AUTO && attn_keys_plan(batch, M, N, Kd, v_layout, 1) == 1)
+            return fa_keys_dispatch(Q, K, V, O, nullptr, batch, M, N, Kd, 1, scale, v_layout, stream);
+        if (algo == TCU_ATTN_AUTO && attn_k32_is_the_choice(batch, M, N, Kd, v_layout))
             return fa_w64_k32_dispatch(Q, K, V, O, batch, M, N, Kd, scale, v_layout, stream);
-        if (algo == TCU_ATTN_AUTO && Kd == 128 && N >= 1024 && blocks >= 128)
+        if (algo == TCU_ATTN_AUTO && attn_w64_is_the_choice(batch, M, N, Kd))
             return launch_fa_w64<false>(Q, K, V, O, batch, M, N, scale, stream);
         if (algo == TCU_ATTN_MFMA32)
             return Kd == 128 ? fa_fwd_by_rows<128, false>(Q, K, V, O, batch, M, N, scale, stream)
@@ -906,9 +1014,10 @@ int fa_dispatch(const __half* Q, const __half* K, const __half* V, __half* O, in
     // column-major V (the reference op's convention), any N % 64 == 0
     if (Kd != 128) return fail(TCU_ERR_UNSUPPORTED_SHAPE, "column-major V is instantiated for head size 128");
     if (algo == TCU_ATTN_AUTO) {
-        // enough query blocks to fill the chip: the 16x16x32 kernel, as for a row-major V
-        const long blocks = (long)batch * (M / 256);
-        if (N >= 320 && (blocks >= 256 || (blocks >= 192 && N >= 1024)))
+        // as for a row-major V
+        if (attn_keys_plan(batch, M, N, Kd, v_layout, 1) == 1)
+            return fa_keys_dispatch(Q, K, V, O, nullptr, batch, M, N, Kd, 1, scale, v_layout, stream);
+        if (attn_k32_is_the_choice(batch, M, N, Kd, v_layout))
             return fa_w64_k32_dispatch(Q, K, V, O, batch, M, N, Kd, scale, v_layout, stream);
         return launch_fa_w64<true>(Q, K, V, O, batch, M, N, scale, stream);
     }
@@ -1102,6 +1211,29 @@ int tcu_flash_attn_fwd_f16_algo(const void* Q, const void* K, const void* V, voi
 int tcu_flash_attn_fwd_f16(const void* Q, const void* K, const void* V, void* O, int batch, int M, int N, int Kdim,
                            int P, float scale, int v_layout, void* stream) {
     return tcu_flash_attn_fwd_f16_algo(Q, K, V, O, batch, M, N, Kdim, P, scale, v_layout, TCU_ATTN_AUTO, stream);
+}
+
+unsigned long long tcu_flash_attn_workspace_bytes(int batch, int M, int N, int Kdim, int P, int v_layout) {
+    if (!positive({batch, M, N, Kdim, P}) || Kdim != P || M % 64 != 0 || N % 64 != 0) return 0;
+    if (v_layout != TCU_V_ROW_MAJOR && v_layout != TCU_V_COL_MAJOR) return 0;
+    const int splits = attn_keys_plan(batch, M, N, Kdim, v_layout, 16);
+    return splits > 1 ? (unsigned long long)splits * batch * M * (Kdim + 2) * sizeof(float) : 0;
+}
+
+int tcu_flash_attn_fwd_f16_ws(const void* Q, const void* K, const void* V, void* O, int batch, int M, int N, int Kdim, int P,
+                              float scale, int v_layout, void* workspace, unsigned long long workspace_bytes, void* stream) {
+    const unsigned long long need = tcu_flash_attn_workspace_bytes(batch, M, N, Kdim, P, v_layout);
+    if (need == 0 || !workspace)
+        return tcu_flash_attn_fwd_f16_algo(Q, K, V, O, batch, M, N, Kdim, P, scale, v_layout, TCU_ATTN_AUTO, stream);
+    if (!Q || !K || !V || !O) return fail(TCU_ERR_INVALID_ARGUMENT, "tcu_flash_attn_fwd_f16_ws: null pointer");
+    if (!aligned16({Q, K, V, O, workspace}))
+        return fail(TCU_ERR_INVALID_ARGUMENT, "tcu_flash_attn_fwd_f16_ws: operands must be 16-byte aligned");
+    if (workspace_bytes < need)
+        return fail(TCU_ERR_INVALID_ARGUMENT, "tcu_flash_attn_fwd_f16_ws: workspace smaller than tcu_flash_attn_workspace_bytes()");
+    return fa_dispatch(static_cast<const __half*>(Q), static_cast<const __half*>(K), static_cast<const __half*>(V),
+                       static_cast<__half*>(O), batch, M, N, Kdim, P, scale, v_layout, TCU_ATTN_KEYS,
+                       static_cast<hipStream_t>(stream), static_cast<float*>(workspace),
+                       attn_keys_plan(batch, M, N, Kdim, v_layout, 16));
 }
 
 int tcu_lstm_f16(const void* x, const void* W, const void* bias, const void* h0, const void* c0, void* h_all,

@@ -73,8 +73,13 @@ void flash_attention_fwd(const at::Tensor& Q, const at::Tensor& K, const at::Ten
     TORCH_CHECK(V.numel() == p * n, "V must hold p * n elements");
     TORCH_CHECK(O.numel() == m * p, "O must hold m * p elements");
     c10::hip::HIPGuardMasqueradingAsCUDA guard(Q.device());
-    check_status(tcu_flash_attn_fwd_f16(Q.data_ptr(), K.data_ptr(), V.data_ptr(), O.data_ptr(), 1, int(m), int(n), int(k),
-                                        int(p), 1.0f, TCU_V_COL_MAJOR, current_stream(Q)),
+    // many keys: split over workgroups through a block from torch's caching allocator, as in gemm
+    const unsigned long long need = tcu_flash_attn_workspace_bytes(1, int(m), int(n), int(k), int(p), TCU_V_COL_MAJOR);
+    at::Tensor ws;
+    if (need > 0) ws = at::empty({static_cast<int64_t>(need)}, Q.options().dtype(at::kByte));
+    check_status(tcu_flash_attn_fwd_f16_ws(Q.data_ptr(), K.data_ptr(), V.data_ptr(), O.data_ptr(), 1, int(m), int(n), int(k),
+                                           int(p), 1.0f, TCU_V_COL_MAJOR, need > 0 ? ws.data_ptr() : nullptr, need,
+                                           current_stream(Q)),
                  "flash_attention_fwd");
 }
 
