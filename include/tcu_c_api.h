@@ -128,15 +128,15 @@ typedef enum {
                                   row-major V; results equal to the others up to rounding and the order of the sums */
 } tcu_attn_algo;
 
-/* Which LSTM step kernel to run (tcu_lstm_f16_algo). AUTO picks STREAMING where it is instantiated, else
- * TILE_LIBRARY, else RAGGED: every B, I, H in multiples of 16 is accepted. */
+/* Which LSTM step kernel to run (tcu_lstm_f16_algo). Every B, I, H in multiples of 16 is accepted: AUTO runs a step kernel
+ * of its own whose wavefronts split the columns (kernels/lstm_direct.hpp) unless W or an activation exceeds 4 GiB, then
+ * STREAMING, TILE_LIBRARY or RAGGED, the first that takes the shape. */
 typedef enum {
     TCU_LSTM_AUTO = 0,
     TCU_LSTM_TILE_LIBRARY = 1, /* composed from the 16x16 tile primitives, single LDS stage; (I, H) in {(1024,1024),
                                   (128,128), (64,128)}, B % 64 == 0 */
     TCU_LSTM_STREAMING = 2,    /* 32x32x16 MFMA, multi-stage direct-to-LDS ring, k split over two wavefront groups;
-                                  I % 128 == 0, H % 128 == 0, B % 64 == 0 (sizes are kernel arguments, except the
-                                  (1024, 1024) instantiation, which has them as constants) */
+                                  I % 128 == 0, H % 128 == 0, B % 64 == 0 */
     TCU_LSTM_RAGGED = 3        /* run-time B, I, H in multiples of 16: MFMA operand tiles filled from global memory */
 } tcu_lstm_algo;
 
@@ -226,9 +226,7 @@ int tcu_flash_attn_fwd_f16_ws(const void* Q, const void* K, const void* V, void*
  * c0 [B, H] f32 or NULL (zeros); h_all [T, B, H] f16 receives every h_t; c_out [B, H] f32
  * receives c_T (it is also the running cell state, so it must not alias c0 unless c0 == c_out).
  * One kernel per step (gate GEMM fused with the cell update). B, I and H must be multiples of 16 (whole tiles) and
- * T * B fit in 31 bits. With B % 64 == 0 the streaming kernel takes every I and H in multiples of 128, and the
- * tile-library kernel is instantiated for (I, H) = (1024,1024), (128,128), (64,128); AUTO takes the streaming kernel
- * where it applies, else the tile-library one, else the run-time-shape kernel (TCU_LSTM_RAGGED), which takes every shape.
+ * T * B fit in 31 bits.
  * The reference snapshot has no LSTM entry (Makefile:3 names a test only).
  */
 int tcu_lstm_f16(const void* x, const void* W, const void* bias, const void* h0, const void* c0, void* h_all,

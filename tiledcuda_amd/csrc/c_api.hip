@@ -14,6 +14,7 @@
 #include "kernels/gemm_ragged.hpp"
 #include "kernels/gemm_w128.hpp"
 #include "kernels/gemm_w128k.hpp"
+#include "kernels/lstm_direct.hpp"
 #include "kernels/lstm_fwd.hpp"
 #include "kernels/lstm_ragged.hpp"
 #include "kernels/lstm_recurrent.hpp"
@@ -1052,16 +1053,85 @@ int launch_lstm(const __half* x, const __half* W, const __half* bias, const __ha
     return TCU_OK;
 }
 
-/// kI == kH == 0: the run-time-shape instantiation of the streaming kernel (I, H any multiples of 128).
-template <int kI, int kH>
-int launch_lstm_hoisted(const __half* x, const __half* W, const __half* bias, const __half* h0, const float* c0,
-                        __half* h_all, float* c_out, int T, int B, int I, int H, float* pre, hipStream_t stream) {
-    using Traits = LstmFwdTraits<kI, kH>;
+/// The step kernel for any B, I, H in multiples of 16 addresses its operands with 32-bit byte offsets.
+bool lstm_direct_takes(int B, int I, int H) {
+    return B % 16 == 0 && I % 16 == 0 && H % 16 == 0 && 8.0 * H * (double(I) + H) < 4294967296.0 &&
+           2.0 * B * std::max(I, H) < 4294967296.0;
+}
+
+/// Tile of that kernel (16-row tiles of weights x of the batch) for a step over `columns` columns: rounds of one workgroup per
+/// CU, each as long as its rows take to arrive (95 KB per us and CU) plus 0.1 us per 16 x 16 tile for the sums of the eight
+/// wavefronts. Measured, us per step with 1x1, 2x1, 2x2, 4x1, 4x2, 4x4 tiles: B 80, I 336, H 656: 6.5, 6.1, 4.5, 4.6, 5.2, 6.9;
+/// 16, 1024, 1024: 3.9, 4.4, 4.9, 5.4, 6.1, 7.9; 64, 1024, 1024: 8.8, 8.2, 5.7, 5.8, 6.7, 8.9; 240, 368, 592: 12.1, 12.8,
+/// 10.0, 8.5, 9.0, 7.4; 256, 1024, 1024: 28, 28, 18, 18, 14, 9.7.
+struct LstmTilePlan {
+    int ut, rt;
+    double us;
+};
+LstmTilePlan lstm_direct_plan(int B, int H, int columns) {
+    LstmTilePlan plan{1, 1, 1e30};
+    for (const auto& [ut, rt] : {std::pair{1, 1}, std::pair{1, 2}, std::pair{2, 1}, std::pair{2, 2}, std::pair{4, 1},
+                                 std::pair{4, 2}, std::pair{4, 4}}) {
+        const long groups = (long)((H + 4 * ut - 1) / (4 * ut)) * ((B + 16 * rt - 1) / (16 * rt));
+        const double us = double((groups + 255) / 256) * (0.1 * ut * rt + 32.0 * (ut + rt) * columns / 95e3);
+        if (us < plan.us) plan = {ut, rt, us};
+    }
+    return plan;
+}
+
+template <int kUT, int kRT, bool kHoisted>
+int launch_lstm_direct_tiles(const __half* x, const __half* W, const __half* bias, const __half* h0, const float* c0,
+                             __half* h_all, float* c_out, int T, int B, int I, int H, const float* pre, hipStream_t stream) {
+    using Traits = LstmDirectTraits<kUT, kRT>;
+    const long grid = (long)((H + Traits::kUnits - 1) / Traits::kUnits) * ((B + Traits::kRows - 1) / Traits::kRows);
+    if (grid > INT_MAX) return fail(TCU_ERR_UNSUPPORTED_SHAPE, "tcu_lstm_f16: too many tiles for one launch");
+    for (int t = 0; t < T; ++t) {
+        const __half* h_in = t == 0 ? h0 : h_all + size_t(t - 1) * B * H;
+        const float* c_in = t == 0 ? c0 : c_out;
+        int rc = launch(&lstm_cell_direct<Traits, kHoisted>, dim3(unsigned(grid)), dim3(Traits::kThreads), Traits::kLdsBytes,
+                        stream, x + size_t(t) * B * I, h_in, W, bias, c_in, c_out, h_all + size_t(t) * B * H, B,
+                        pre ? pre + size_t(t) * B * 4 * H : nullptr, I, H);
+        if (rc != TCU_OK) return lstm_step_failed(rc, t, T);
+    }
+    return TCU_OK;
+}
+
+template <bool kHoisted>
+int launch_lstm_direct(const __half* x, const __half* W, const __half* bias, const __half* h0, const float* c0, __half* h_all,
+                       float* c_out, int T, int B, int I, int H, const float* pre, hipStream_t stream) {
+    const LstmTilePlan plan = lstm_direct_plan(B, H, kHoisted ? H : I + H);
+    auto go = [&](auto ut, auto rt) {
+        return launch_lstm_direct_tiles<decltype(ut)::value, decltype(rt)::value, kHoisted>(x, W, bias, h0, c0, h_all, c_out, T,
+                                                                                           B, I, H, pre, stream);
+    };
+    using one = std::integral_constant<int, 1>;
+    using two = std::integral_constant<int, 2>;
+    using four = std::integral_constant<int, 4>;
+    if (plan.ut == 1) return plan.rt == 1 ? go(one{}, one{}) : go(one{}, two{});
+    if (plan.ut == 2) return plan.rt == 1 ? go(two{}, one{}) : go(two{}, two{});
+    return plan.rt == 1 ? go(four{}, one{}) : plan.rt == 2 ? go(four{}, two{}) : go(four{}, four{});
+}
+
+int launch_lstm_hoisted(const __half* x, const __half* W, const __half* bias, const __half* h0, const float* c0, __half* h_all,
+                        float* c_out, int T, int B, int I, int H, float* pre, hipStream_t stream) {
     // pre[T * B, 4H] = x[T * B, I] . W[:, :I]^T: the stored [4H, I] operand is the first I columns of W's rows
     const long rows = long(T) * B;
     if (rows > INT_MAX) return fail(TCU_ERR_UNSUPPORTED_SHAPE, "tcu_lstm_f16_ws: T * B exceeds the 32-bit row count");
-    int rc = gemm_w128_dispatch<float>(x, W, pre, int(rows), 4 * H, I, stream, I, I + H);
+    // with few rows the 128 x 128 tiles of the K-splitting kernel (T * B 1024, I and H 1024: 13 against 22 us)
+    const long tiles128 = ((rows + 127) / 128) * ((4l * H + 127) / 128), tiles256 = ((rows + 255) / 256) * ((4l * H + 255) / 256);
+    const double us128 = double((tiles128 + 255) / 256) * (5.0 + 0.95 * (I / 128));
+    int rc;
+    if (us128 < gemm_w128_us(tiles256, I) && (long)(I + H) * 256 < (1l << 32)) {
+        using Tk = GemmW128kTraits;
+        auto kernel = rows % Tk::kBM == 0 ? &gemm_w128k<float, false, Tk> : &gemm_w128k<float, true, Tk>;
+        rc = launch(kernel, dim3(unsigned(tiles128)), dim3(Tk::kThreads), Tk::kLdsBytes, stream, x, W, pre, int(rows), 4 * H, I, I,
+                    I + H, 4 * H);
+    } else {
+        rc = gemm_w128_dispatch<float>(x, W, pre, int(rows), 4 * H, I, stream, I, I + H);
+    }
     if (rc != TCU_OK) return rc;
+    if (lstm_direct_takes(B, I, H)) return launch_lstm_direct<true>(x, W, bias, h0, c0, h_all, c_out, T, B, I, H, pre, stream);
+    using Traits = LstmFwdTraits<0, 0>;
     auto kernel = &lstm_cell_fwd<Traits, true>;
     const int grid = (B / Traits::kTM) * (H / Traits::kTH);
     for (int t = 0; t < T; ++t) {
@@ -1093,11 +1163,9 @@ int launch_lstm_ragged(const __half* x, const __half* W, const __half* bias, con
     return TCU_OK;
 }
 
-/// kI == kH == 0: the run-time-shape instantiation (I, H any multiples of 128).
-template <int kI, int kH>
-int launch_lstm_fwd(const __half* x, const __half* W, const __half* bias, const __half* h0, const float* c0,
-                    __half* h_all, float* c_out, int T, int B, int I, int H, hipStream_t stream) {
-    using Traits = LstmFwdTraits<kI, kH>;
+int launch_lstm_fwd(const __half* x, const __half* W, const __half* bias, const __half* h0, const float* c0, __half* h_all,
+                    float* c_out, int T, int B, int I, int H, hipStream_t stream) {
+    using Traits = LstmFwdTraits<0, 0>;
     auto kernel = &lstm_cell_fwd<Traits>;
     const int grid = (B / Traits::kTM) * (H / Traits::kTH);
     for (int t = 0; t < T; ++t) {
@@ -1259,12 +1327,13 @@ int tcu_lstm_f16_algo(const void* x, const void* W, const void* bias, const void
     if (B % 16 != 0 || I % 16 != 0 || H % 16 != 0)
         return fail(TCU_ERR_UNSUPPORTED_SHAPE, "tcu_lstm_f16: shapes are whole 16 x 16 tiles: B, I and H must be multiples of 16");
     if (algo == TCU_LSTM_RAGGED) return launch_lstm_ragged(xp, wp, bp, h0p, c0p, hp, cp, T, B, I, H, s);
+    // every shape whose operands 32-bit offsets reach (gigabytes of weights do not fit): per step 4.5 us against 16.6 for the
+    // kernel below it at B 80, I 336, H 656, 9.7 against 12.0 for the streaming one at 256, 1024, 1024
+    if (algo == TCU_LSTM_AUTO && lstm_direct_takes(B, I, H))
+        return launch_lstm_direct<false>(xp, wp, bp, h0p, c0p, hp, cp, T, B, I, H, nullptr, s);
     const bool b64 = B % 64 == 0;
-    if (algo != TCU_LSTM_TILE_LIBRARY && b64 && I % 128 == 0 && H % 128 == 0) {
-        // the benchmark shape with its sizes as constants; every other shape with the sizes as kernel arguments
-        if (I == 1024 && H == 1024) return launch_lstm_fwd<1024, 1024>(xp, wp, bp, h0p, c0p, hp, cp, T, B, I, H, s);
-        return launch_lstm_fwd<0, 0>(xp, wp, bp, h0p, c0p, hp, cp, T, B, I, H, s);
-    }
+    if (algo != TCU_LSTM_TILE_LIBRARY && b64 && I % 128 == 0 && H % 128 == 0)
+        return launch_lstm_fwd(xp, wp, bp, h0p, c0p, hp, cp, T, B, I, H, s);
     if (algo == TCU_LSTM_STREAMING)
         return fail(TCU_ERR_UNSUPPORTED_SHAPE, "the streaming LSTM kernel needs I % 128 == 0, H % 128 == 0 and B % 64 == 0");
     if (b64) {
@@ -1309,8 +1378,7 @@ int tcu_lstm_f16_ws(const void* x, const void* W, const void* bias, const void* 
     auto hp = static_cast<__half*>(h_all);
     auto cp = static_cast<float*>(c_out);
     auto pre = static_cast<float*>(workspace);
-    if (I == 1024 && H == 1024) return launch_lstm_hoisted<1024, 1024>(xp, wp, bp, h0p, c0p, hp, cp, T, B, I, H, pre, s);
-    return launch_lstm_hoisted<0, 0>(xp, wp, bp, h0p, c0p, hp, cp, T, B, I, H, pre, s);
+    return launch_lstm_hoisted(xp, wp, bp, h0p, c0p, hp, cp, T, B, I, H, pre, s);
 }
 
 unsigned long long tcu_lstm_persistent_workspace_bytes(int T, int B, int I, int H) {
