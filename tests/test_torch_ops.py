@@ -162,6 +162,43 @@ def test_scatter_nd_add_with_duplicates_and_skipped_rows(tcu, oracle, device):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [np.float32, np.float16])
+@pytest.mark.parametrize("width", [1, 2, 3, 17, 64, 511, 512, 1023, 1024, 1025, 4096])
+@pytest.mark.parametrize("offset", [0, 1])
+def test_scatter_nd_add_words(tcu, oracle, device, dtype, width, offset):
+    """Add mode over slices around the 512 words (1024 f16 elements) that a workgroup takes, and slices and bases that do not start on whole words
+    (f16). Distinct rows of values over the type's range, subnormals among them: one addition per element, so the result is
+    the rounded sum bit for bit. Duplicate rows hold small integers (exact in any order)."""
+    rng = np.random.default_rng(width)
+    rows, n = 37, 23
+    tiny = np.finfo(dtype).smallest_subnormal
+    data = (rng.standard_normal((rows, width)) * np.exp2(rng.integers(-20, 10, size=(rows, width)))).astype(dtype)
+    upd = (rng.standard_normal((n, width)) * np.exp2(rng.integers(-20, 10, size=(n, width)))).astype(dtype)
+    data[:, ::3] = rng.integers(-40, 40, size=data[:, ::3].shape).astype(dtype) * tiny
+    upd[:, ::2] = rng.integers(-40, 40, size=upd[:, ::2].shape).astype(dtype) * tiny
+    idx = rng.permutation(rows)[:n].reshape(n, 1).astype(np.int64)
+
+    def on_device(a):
+        whole = torch.zeros(a.size + offset, dtype=torch.from_numpy(a).dtype, device=device)
+        whole[offset:] = torch.from_numpy(a).to(device).flatten()
+        return whole, whole[offset:].view(a.shape)
+
+    whole, d = on_device(data)
+    tcu.scatter_nd(d, torch.from_numpy(idx).to(device), on_device(upd)[1], mode="add")
+    assert np.array_equal(d.cpu().numpy(), oracle.scatter_nd(data, idx, upd, mode="add"))
+    assert not whole[:offset].any()
+
+    data = rng.integers(-8, 8, size=(5, 4, width)).astype(dtype)
+    upd = rng.integers(-2, 3, size=(60, width)).astype(dtype)
+    idx = np.stack([rng.integers(-1, 5, size=60), rng.integers(0, 4, size=60)], 1).astype(np.int64)
+    _, d = on_device(data)
+    skipped = torch.zeros(1, dtype=torch.int32, device=device)
+    tcu.scatter_nd(d, torch.from_numpy(idx).to(device), on_device(upd)[1], mode="add", skipped_rows=skipped)
+    assert np.array_equal(d.cpu().numpy(), oracle.scatter_nd(data, idx, upd, mode="add"))
+    assert int(skipped.item()) == int((idx[:, 0] < 0).sum())
+
+
+@pytest.mark.gpu
 def test_scatter_nd_large_round_trip(tcu, device):
     """Full-size property check: scattering the rows of X to a random permutation and gathering them back is the
     identity (64 Mi elements, 256 MiB each way)."""

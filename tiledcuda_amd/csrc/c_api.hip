@@ -142,6 +142,20 @@ int scratch_address(void** out) {
     return TCU_OK;
 }
 
+// ---------------------------------------------------------------------------- scatter_nd
+/// Whether p is ordinary (coarse-grained) memory of the current device. Packed f16 atomics are carried out in its L2s; on
+/// host, managed, fine-grained and other devices' memory, which a caller may hand over as well, they need not be.
+bool plain_device_memory(const void* p) {
+    hipPointerAttribute_t attr{};
+    if (hipPointerGetAttributes(&attr, p) != hipSuccess) {
+        (void)hipGetLastError();  // a caller that checks its own launches later must not find this one's error
+        return false;
+    }
+    int device = -1;
+    return attr.type == hipMemoryTypeDevice && !attr.isManaged && attr.allocationFlags == 0 &&
+           hipGetDevice(&device) == hipSuccess && attr.device == device;
+}
+
 // ---------------------------------------------------------------------------- GEMM
 template <typename OutType, int kM, int kN, int kK, int kTM, int kTN, int kChunkK, typename WarpLayout>
 int launch_simple_gemm(const __half* A, const __half* B, OutType* C, hipStream_t stream) {
@@ -1501,6 +1515,14 @@ int tcu_scatter_nd(void* data, const void* updates, const void* indices, const l
     auto s = static_cast<hipStream_t>(stream);
     auto idx = static_cast<const int64_t*>(indices);
     auto bad = static_cast<unsigned int*>(skipped_rows);
+    // f16 additions: a word of two elements at a time (see the kernel for both sides measured)
+    if (dtype == TCU_DTYPE_F16 && mode == TCU_SCATTER_ADD && plain_device_memory(data)) {
+        const bool whole = shape.slice % 2 == 0 && reinterpret_cast<uintptr_t>(data) % 4 == 0 && reinterpret_cast<uintptr_t>(updates) % 4 == 0;
+        const int64_t blocks = (n * scatter_pair_words(whole, shape.slice) + kScatterPairsBlock - 1) / kScatterPairsBlock;
+        return launch(whole ? &scatter_nd_add_pairs<true> : &scatter_nd_add_pairs<false>,
+                      dim3(static_cast<unsigned>(std::min<int64_t>(blocks, 1 << 22))), dim3(256), 0, s, static_cast<__half*>(data),
+                      static_cast<const __half*>(updates), idx, shape, bad);
+    }
     const size_t elem = dtype == TCU_DTYPE_F32 ? 4 : 2;
     const int vec = int(16 / elem);
     const bool vec_ok = mode == TCU_SCATTER_ASSIGN && shape.slice % vec == 0 &&
