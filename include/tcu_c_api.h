@@ -33,7 +33,8 @@ typedef enum { TCU_DTYPE_F32 = 0, TCU_DTYPE_F16 = 1 } tcu_dtype;
  * disjoint parts of C, bit for bit the result of one launch) when M or N lie a little above such multiples and that
  * saves a round of workgroups; WAVE128 on the leading rows or columns that fill whole rounds of 256 workgroups plus a
  * kernel with smaller tiles (WAVE128_KSPLIT, WAVE128_NARROW or PIPELINED) on the rest of C when the last round would be
- * far from full (2560 x 8192: 320 tiles); WAVE128_KSPLIT and WAVE128_NARROW as described below; else PIPELINED; RAGGED for problems below 64 x 64. Every shape made of whole 16 x 16
+ * far from full (2560 x 8192: 320 tiles); WAVE128_KSPLIT and WAVE128_NARROW as described below; DIRECT for products with few output tiles, where a cost model
+ * expects it to be the shorter launch; else PIPELINED. Every shape made of whole 16 x 16
  * BaseTiles (M, N, K multiples of 16), the granularity of the reference's tile types, is accepted. */
 typedef enum {
     TCU_GEMM_AUTO = 0,
@@ -63,6 +64,10 @@ typedef enum {
                                 1552 x 1552 x 4096); K a multiple of 128,
                                 M and N multiples of 16 (edge tiles: rows clamped, stores guarded); the sum over K is
                                 taken in four interleaved parts (differs from the other kernels by f32 rounding) */
+    TCU_GEMM_DIRECT = 11,    /* tiles of 16 to 64 x 16 to 64 by a cost model, 8 wavefronts that split K and bring their own
+                                chunks to LDS without barriers: for products with few output tiles (32 x 4096 x 4096,
+                                256 x 256 x 8192); M, N, K multiples of 16; the sum over K is taken in eight interleaved
+                                parts (differs from the other kernels by f32 rounding) */
     TCU_GEMM_WAVE128_NARROW = 9 /* the WAVE128 kernel with 256 x 128 workgroup tiles (a wavefront owns 128 x 64; three stages): for
                                 products between the two above - too few 256 x 256 tiles to fill the GPU, too many
                                 128 x 128 tiles for one round of WAVE128_KSPLIT (2048 x 2560 x 4096, 4096 x 2048 x 8192,
@@ -167,11 +172,14 @@ int tcu_gemm_f16(const void* A, const void* B, void* C, int M, int N, int K, int
  * this takes, or 0 when the product is not split (more than 128 tiles of 256 x 256, M or N not multiples of 16,
  * less than 512 of K per range, or the unsplit kernel expected to be as fast): then, and when `workspace` is NULL,
  * the call is tcu_gemm_f16 with TCU_GEMM_AUTO. The workspace (16-byte aligned device
- * memory) is the caller's and free to reuse once the work enqueued here has run. Results differ from the unsplit
+ * memory) is the caller's and free to reuse once the work enqueued here has run. Where TCU_GEMM_DIRECT is expected to be
+ * faster than the split (short M or N) the call runs that kernel and leaves the workspace alone; tcu_gemm_uses_workspace()
+ * is 0 there, so that a caller that would allocate one need not. Results differ from the unsplit
  * product by the order of the f32 summation only. No counterpart in the reference, whose GEMM examples fix one
  * workgroup per output tile (examples/cpp/01_gemm/02_gemm_all_mem/main.cu:54-72).
  */
 unsigned long long tcu_gemm_workspace_bytes(int M, int N, int K);
+int tcu_gemm_uses_workspace(int M, int N, int K);
 int tcu_gemm_f16_ws(const void* A, const void* B, void* C, int M, int N, int K, int out_dtype, void* workspace,
                     unsigned long long workspace_bytes, void* stream);
 

@@ -1,0 +1,45 @@
+"""The GEMM kernel whose wavefronts split K without barriers (algo "direct", AUTO's choice for few output tiles), at the sizes
+where its tiles, its chunks of K and its rings end. Against the oracle; relative tolerance of the layer's other tests (1e-3 of
+a result rounded to f16)."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+REL_TOL = 1e-3
+
+
+@pytest.mark.parametrize("M,N,K", [(16, 16, 16), (16, 16, 64), (16, 48, 80), (48, 16, 496), (32, 4080, 512), (16, 4096, 528),  # 1 wide
+                                   (16, 64, 4096), (32, 2064, 2096), (48, 4112, 1040), (64, 4096, 1552),  # rings of 2 to 4 chunks
+                                   (112, 4096, 576), (4112, 48, 592), (272, 400, 1088), (528, 1040, 608), (256, 4096, 1072),
+                                   (2064, 48, 304), (16, 8208, 48), (208, 464, 1008)])
+@pytest.mark.parametrize("out_dtype", ["f32", "f16"])
+def test_gemm_direct(tcu, oracle, device, M, N, K, out_dtype):
+    import torch
+
+    print(f"gemm direct {M}x{N}x{K} {out_dtype}", flush=True)
+    dt = torch.float32 if out_dtype == "f32" else torch.float16
+    A = oracle.fill_uniform(M * K, 31 + M).reshape(M, K)
+    Bt = oracle.fill_uniform(N * K, 37 + N).reshape(N, K)
+    # rows beyond the operands hold NaN: a product that took one in would show it
+    a = torch.full((M + 64, K), float("nan"), dtype=torch.float16, device=device)
+    b = torch.full((N + 64, K), float("nan"), dtype=torch.float16, device=device)
+    a[:M], b[:N] = torch.from_numpy(A).to(device), torch.from_numpy(Bt).to(device)
+    guard = torch.full((M + 2, N), -7.0, dtype=dt, device=device)
+    tcu.gemm(a[:M], b[:N], out=guard[1:M + 1], algo="direct")
+    torch.cuda.synchronize()
+    assert oracle.max_rel_err(guard[1:M + 1].float().cpu().numpy(), oracle.gemm(A, Bt)) <= REL_TOL
+    assert torch.all(guard[0] == -7.0) and torch.all(guard[M + 1] == -7.0)
+
+
+def test_gemm_direct_leaves_the_workspace(tcu, device):
+    """A short product that could be split: AUTO runs this kernel, with or without a workspace, which stays untouched."""
+    import torch
+
+    M, N, K = 256, 256, 8192
+    a = torch.randn(M, K, device=device).half()
+    b = torch.randn(N, K, device=device).half()
+    assert not tcu.lib().tcu_gemm_uses_workspace(M, N, K)
+    ws = torch.full((tcu.gemm_workspace_bytes(M, N, K),), 0xFF, dtype=torch.uint8, device=device)
+    want = tcu.gemm(a, b, algo="direct")
+    assert torch.equal(tcu.gemm(a, b, workspace=ws), want) and torch.equal(tcu.gemm(a, b), want)
+    assert bool((ws == 0xFF).all())

@@ -35,7 +35,8 @@ TCU_ERR_NO_DEVICE = -4
 TCU_DTYPE_F32 = 0
 TCU_DTYPE_F16 = 1
 
-GEMM_ALGOS = {"auto": 0, "global_reg": 1, "all_mem": 2, "pipelined": 3, "wave128": 4, "tile_pipelined": 5, "ragged": 6, "tile_wave128": 7, "wave128_ksplit": 8, "wave128_narrow": 9}
+GEMM_ALGOS = {"auto": 0, "global_reg": 1, "all_mem": 2, "pipelined": 3, "wave128": 4, "tile_pipelined": 5, "ragged": 6, "tile_wave128": 7, "wave128_ksplit": 8, "wave128_narrow": 9,
+              "direct": 11}
 
 TCU_V_COL_MAJOR = 0
 TCU_V_ROW_MAJOR = 1
@@ -52,6 +53,7 @@ _SIGNATURES = {
     "tcu_device_count": (ctypes.c_int, []),
     "tcu_gemm_f16": (ctypes.c_int, [ctypes.c_void_p] * 3 + [ctypes.c_int] * 5 + [ctypes.c_void_p]),
     "tcu_gemm_workspace_bytes": (ctypes.c_ulonglong, [ctypes.c_int] * 3),
+    "tcu_gemm_uses_workspace": (ctypes.c_int, [ctypes.c_int] * 3),
     "tcu_gemm_f16_ws": (ctypes.c_int, [ctypes.c_void_p] * 3 + [ctypes.c_int] * 4 + [ctypes.c_void_p, ctypes.c_ulonglong,
                                                                                   ctypes.c_void_p]),
     "tcu_b2b_gemm_f16": (ctypes.c_int, [ctypes.c_void_p] * 4 + [ctypes.c_int] * 6 + [ctypes.c_void_p]),
@@ -149,7 +151,7 @@ def gemm(a: torch.Tensor, b_t: torch.Tensor, out: torch.Tensor | None = None,
     """C[M, N] = A[M, K] · B with B column-major, i.e. ``b_t`` is the [N, K] array (``a @ b_t.T``).
 
     Mirrors the reference's GEMM examples (A row-major, B column-major, f32 accumulate). With ``algo="auto"`` a
-    product with few output tiles and a long K is split over K (``tcu_gemm_f16_ws``) through ``workspace`` (a contiguous
+    product with few output tiles and a long K may be split over K (``tcu_gemm_f16_ws``) through ``workspace`` (a contiguous
     device tensor of at least ``gemm_workspace_bytes(M, N, K)`` bytes), or, when none is given, through one taken from
     torch's caching allocator for the call; ``workspace=False`` never splits (use it, or a workspace of your own, when
     the call is being captured into a HIP graph: an allocation has no place in a captured stream).
@@ -163,9 +165,8 @@ def gemm(a: torch.Tensor, b_t: torch.Tensor, out: torch.Tensor | None = None,
     elif tuple(out.shape) != (M, N):
         raise ValueError("out has the wrong shape")
     if workspace is None and algo == "auto" and a.is_cuda:
-        need = gemm_workspace_bytes(M, N, K)
-        if need > 0:
-            workspace = torch.empty(need, dtype=torch.uint8, device=a.device)
+        if lib().tcu_gemm_uses_workspace(M, N, K):
+            workspace = torch.empty(gemm_workspace_bytes(M, N, K), dtype=torch.uint8, device=a.device)
     if workspace is False:
         workspace = None
     if workspace is not None:
@@ -184,7 +185,7 @@ def gemm(a: torch.Tensor, b_t: torch.Tensor, out: torch.Tensor | None = None,
 
 
 def gemm_workspace_bytes(M: int, N: int, K: int) -> int:
-    """Device bytes ``gemm(..., workspace=...)`` uses for a split over K; 0 when the product is not split."""
+    """Device bytes ``gemm(..., workspace=...)`` needs for a split over K; 0 when the product is never split."""
     return int(lib().tcu_gemm_workspace_bytes(M, N, K))
 
 

@@ -10,6 +10,7 @@
 #include "kernels/flash_attn_tile_w64.hpp"
 #include "kernels/flash_attn_w64_k32.hpp"
 #include "kernels/flash_attn_w64.hpp"
+#include "kernels/gemm_direct.hpp"
 #include "kernels/gemm_pipelined.hpp"
 #include "kernels/gemm_ragged.hpp"
 #include "kernels/gemm_w128.hpp"
@@ -496,26 +497,32 @@ int gemm_rounds_and_rest(const __half* A, const __half* B, OutType* C, int M, in
 struct GemmSplitPlan {
     int splits;
     bool tiles128;
+    double us;
 };
+
+/// Expected time of the unsplit launch on few output tiles, apart from the kernel of gemm_direct_plan().
+double gemm_unsplit_us(int M, int N, int K) {
+    double us = pipelined_plan(M, N, K).us;
+    if (gemm_w128k_is_the_choice(M, N, K)) us = std::min(us, gemm_w128k_us(M, N, K));
+    if (gemm_narrow_is_the_choice(M, N, K)) us = std::min(us, gemm_narrow_us(M, N, K));
+    const long tiles = (long)((M + 255) / 256) * ((N + 255) / 256);
+    return tiles > 128 ? std::min(us, gemm_w128_us(tiles, (K + 63) / 64 * 64)) : us;
+}
 
 GemmSplitPlan gemm_split_plan(int M, int N, int K) {
     using T = GemmW128Traits;
-    GemmSplitPlan plan{1, false};
+    GemmSplitPlan plan{1, false, 0.0};
     if (M % 16 != 0 || N % 16 != 0 || K % T::kBK != 0) return plan;
     const bool whole256 = M % T::kBM == 0 && N % T::kBN == 0;  // the 256 x 256 form splits whole tiles only
     const long tiles = (long)((M + T::kBM - 1) / T::kBM) * ((N + T::kBN - 1) / T::kBN);
     const long tiles128 = (long)((M + 127) / 128) * ((N + 127) / 128);  // (the 128 x 128 form has edge tiles)
     if (tiles > 128) return plan;
-    double unsplit_us = pipelined_plan(M, N, K).us;
-    // the kernels AUTO would run instead of the pipelined one
-    if (gemm_w128k_is_the_choice(M, N, K)) unsplit_us = std::min(unsplit_us, gemm_w128k_us(M, N, K));
-    if (gemm_narrow_is_the_choice(M, N, K)) unsplit_us = std::min(unsplit_us, gemm_narrow_us(M, N, K));
-    double best_us = 0.95 * unsplit_us;
+    double best_us = 0.95 * gemm_unsplit_us(M, N, K);
     const double plane_us = 2.0 * double(M) * N * 4 / 5.3e6;  // a plane of partial products written and read once
     for (int s = 2; whole256 && s * tiles <= 256 && K % (s * T::kBK) == 0 && K / s >= 512; s *= 2) {
         const double us = 10.0 + 1.4 * (K / s / T::kBK) + s * plane_us;
         if (us < best_us) {
-            plan = {s, false};
+            plan = {s, false, us};
             best_us = us;
         }
     }
@@ -528,7 +535,7 @@ GemmSplitPlan gemm_split_plan(int M, int N, int K) {
             const double per_tile = 0.62 + 0.33 * (groups > 128 ? double(groups - 128) / 128.0 : 0.0);
             const double us = 8.0 + per_tile * (K / s / 128) + s * plane_us;
             if (us < best_us) {
-                plan = {s, true};
+                plan = {s, true, us};
                 best_us = us;
             }
         }
@@ -537,6 +544,66 @@ GemmSplitPlan gemm_split_plan(int M, int N, int K) {
 }
 
 int gemm_split_count(int M, int N, int K) { return gemm_split_plan(M, N, K).splits; }
+
+/// The tile of the kernel whose 8 wavefronts split K without barriers, and what its launch is expected to cost: 2.4 us + rounds
+/// of one workgroup per CU, each as long as its rows take to arrive (95 KB per us and CU) plus 0.1 us per 16 x 16 tile for
+/// the sums of the wavefronts, + 0.4 of the time operands and result take at 5.2 TB/s; no less than that whole time. Within 15 %
+/// of the measured times from half a round of workgroups on (with fewer, a CU receives up to 147 KB per us).
+struct GemmDirectPlan {
+    int ut, rt;
+    double us;
+};
+GemmDirectPlan gemm_direct_plan(int M, int N, int K) {
+    GemmDirectPlan plan{0, 0, 1e30};
+    if (M % 16 != 0 || N % 16 != 0 || K % 16 != 0 || K >= (1 << 24)) return plan;
+    const double once_us = 2.0 * (double(K) * (double(M) + N) + double(M) * N) / 5.2e6;
+    for (const auto& [ut, rt] : {std::pair{1, 1}, std::pair{1, 2}, std::pair{2, 1}, std::pair{2, 2}, std::pair{1, 4},
+                                 std::pair{4, 1}, std::pair{2, 4}, std::pair{4, 2}, std::pair{4, 4}}) {
+        const long groups = (long)((M + 16 * rt - 1) / (16 * rt)) * ((N + 16 * ut - 1) / (16 * ut));
+        if (groups > INT_MAX) continue;
+        const double cu_us = double((groups + 255) / 256) * (0.1 * ut * rt + 32.0 * (ut + rt) * K / 95e3);
+        const double us = 2.4 + std::max(cu_us + 0.4 * once_us, once_us);
+        if (us < plan.us) plan = {ut, rt, us};
+    }
+    return plan;
+}
+
+/// Whether AUTO runs that kernel rather than another one in a single launch: us, others -> this kernel, 32 x 1024 x 1024:
+/// 6.8 -> 2.8; 208 x 464 x 1008: 7.5 -> 3.6; 512^3: 4.4 -> 3.3; 512 x 1024 x 1024: 6.4 -> 5.0; 256 x 4096 x 4096: 21.1 -> 19.5;
+/// 1024^3 stays: 6.9 against 7.2.
+bool gemm_direct_is_the_choice(int M, int N, int K) { return gemm_direct_plan(M, N, K).us < gemm_unsplit_us(M, N, K); }
+
+/// ... and whether rather than a split over K through a workspace, which takes up to 6 us more than gemm_split_plan() expects
+/// when it does not find its operands and planes in the L2s: 32 x 4096 x 4096: 18.1 -> 10.5, 256 x 256 x 8192: 18.1 -> 8.9,
+/// 512 x 512 x 8192: 19.4 -> 14.2; 1024 x 1024 x 8192: 29.3 -> 28.3.
+bool gemm_split_is_the_choice(int M, int N, int K) {
+    const GemmSplitPlan plan = gemm_split_plan(M, N, K);
+    return plan.splits > 1 && plan.us + 4.0 <= gemm_direct_plan(M, N, K).us;
+}
+
+template <typename OutType>
+int gemm_direct_dispatch(const __half* A, const __half* B, OutType* C, int M, int N, int K, hipStream_t stream) {
+    if (M % 16 != 0 || N % 16 != 0 || K % 16 != 0)
+        return fail(TCU_ERR_UNSUPPORTED_SHAPE, "GEMM shapes are whole 16 x 16 tiles: M, N and K must be multiples of 16");
+    const GemmDirectPlan plan = gemm_direct_plan(M, N, K);
+    if (plan.ut == 0) return fail(TCU_ERR_UNSUPPORTED_SHAPE, "the barrier-free GEMM addresses a tile's rows with 32-bit offsets: K < 2^24");
+    auto go = [&](auto traits) {
+        using T = decltype(traits);
+        const long grid = (long)((M + T::kBM - 1) / T::kBM) * ((N + T::kBN - 1) / T::kBN);
+        return launch(&gemm_direct<T, OutType>, dim3(unsigned(grid)), dim3(T::kThreads), T::kLdsBytes, stream, A, B, C, M, N, K);
+    };
+    switch (10 * plan.ut + plan.rt) {
+        case 11: return go(GemmDirectTraits<1, 1>{});
+        case 12: return go(GemmDirectTraits<1, 2>{});
+        case 21: return go(GemmDirectTraits<2, 1>{});
+        case 22: return go(GemmDirectTraits<2, 2>{});
+        case 14: return go(GemmDirectTraits<1, 4>{});
+        case 41: return go(GemmDirectTraits<4, 1>{});
+        case 24: return go(GemmDirectTraits<2, 4>{});
+        case 42: return go(GemmDirectTraits<4, 2>{});
+        default: return go(GemmDirectTraits<4, 4>{});
+    }
+}
 
 template <typename OutType>
 int gemm_splitk(const __half* A, const __half* B, OutType* C, int M, int N, int K, GemmSplitPlan plan, float* partial,
@@ -589,7 +656,11 @@ int gemm_dispatch(const __half* A, const __half* B, OutType* C, int M, int N, in
             return gemm_w128k_dispatch<OutType>(A, B, C, M, N, K, stream);
         case TCU_GEMM_WAVE128_NARROW:
             return gemm_w128_narrow_dispatch<OutType>(A, B, C, M, N, K, stream);
+        case TCU_GEMM_DIRECT:
+            return gemm_direct_dispatch<OutType>(A, B, C, M, N, K, stream);
         case TCU_GEMM_AUTO:
+            // few output tiles: the kernel that splits K over wavefronts without barriers
+            if (gemm_direct_is_the_choice(M, N, K)) return gemm_direct_dispatch<OutType>(A, B, C, M, N, K, stream);
             // where the 256 x 256 tile is the choice anyway, the one-wavefront-per-SIMD kernel is the faster one
             if (M % 256 == 0 && N % 256 == 0 && K % 64 == 0 && (long)(M / 256) * (N / 256) > 128 &&
                 (long)K * 512 < (1l << 32)) {
@@ -622,8 +693,6 @@ int gemm_dispatch(const __half* A, const __half* B, OutType* C, int M, int N, in
                     return gemm_rounds_and_rest<OutType>(A, B, C, M, N, K, rounds, stream);
                 if (edge_us < pipelined_us) return gemm_w128_dispatch<OutType>(A, B, C, M, N, K, stream);
             }
-            // tiny problems: the kernel that takes its operand tiles straight from global memory has the shorter start
-            if ((long)M * N < 64 * 64) return gemm_ragged_dispatch<OutType>(A, B, C, M, N, K, stream);
             [[fallthrough]];
         case TCU_GEMM_PIPELINED:
             return gemm_pipelined_dispatch<OutType>(A, B, C, M, N, K, stream);
@@ -1242,6 +1311,10 @@ unsigned long long tcu_gemm_workspace_bytes(int M, int N, int K) {
     return splits > 1 ? (unsigned long long)splits * M * N * sizeof(float) : 0;
 }
 
+int tcu_gemm_uses_workspace(int M, int N, int K) {
+    return M > 0 && N > 0 && K > 0 && gemm_split_is_the_choice(M, N, K) ? 1 : 0;
+}
+
 int tcu_gemm_f16_ws(const void* A, const void* B, void* C, int M, int N, int K, int out_dtype, void* workspace,
                     unsigned long long workspace_bytes, void* stream) {
     const unsigned long long need = (M > 0 && N > 0 && K > 0) ? tcu_gemm_workspace_bytes(M, N, K) : 0;
@@ -1250,6 +1323,7 @@ int tcu_gemm_f16_ws(const void* A, const void* B, void* C, int M, int N, int K, 
     if (!aligned16({A, B, C, workspace})) return fail(TCU_ERR_INVALID_ARGUMENT, "tcu_gemm_f16_ws: operands must be 16-byte aligned");
     if (workspace_bytes < need)
         return fail(TCU_ERR_INVALID_ARGUMENT, "tcu_gemm_f16_ws: workspace smaller than tcu_gemm_workspace_bytes()");
+    if (!gemm_split_is_the_choice(M, N, K)) return tcu_gemm_f16(A, B, C, M, N, K, out_dtype, TCU_GEMM_AUTO, stream);
     auto a = static_cast<const __half*>(A), b = static_cast<const __half*>(B);
     auto s = static_cast<hipStream_t>(stream);
     auto ws = static_cast<float*>(workspace);
