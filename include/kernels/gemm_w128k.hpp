@@ -21,8 +21,11 @@
 //   * Accumulators in AGPRs through inline assembly, scalar-base addressing, XCD-aware tile order: as in gemm_w128.
 // The sum over K is taken in four interleaved parts, so results differ from the other kernels by f32 rounding.
 // The tile is 128 x 128 or 128 x 96 (GemmW128kTraitsN: the numbers above are those of the wider one).
-// K % 128 == 0; M % 128 == 0 and N a multiple of the tile width, or with kEdges any M, N in multiples of 16: the grid
-// then covers ceil(M / 128) x ceil(N / width) tiles, rows beyond the edge are loaded from the last valid row (their products are
+// K % 128 == 0, or with kTail any multiple of 16: in the last tile of K the 16-byte pieces beyond a row are fetched from the
+// row's first piece in that tile instead, and every wavefront zeroes its fragments there before it multiplies them, in a
+// branch at the top of the phase (a mask applied in every phase cost 0.1 us in each). 2000 x 2000 x 2064: 42.5 us on the 64 x 64
+// tiles that took it before, 25.9 here; 2064 x 1040 x 1072: 15.6 -> 14.5 (128 x 96).
+// M % 128 == 0 and N a multiple of the tile width, or with kEdges any M, N in multiples of 16: the grid then covers ceil(M / 128) x ceil(N / width) tiles, rows beyond the edge are loaded from the last valid row (their products are
 // computed and dropped) and the stores are guarded per 16 x 16 block (checked by the launcher).
 #pragma once
 
@@ -59,7 +62,8 @@ using GemmW128kTraits = GemmW128kTraitsN<8>;
 /// consecutive rows of A, of the stored [N, K] array and of C. kEdges: grid.x = ceil(M / 128) * ceil(N / kBN). With
 /// splits > 1 workgroup row z multiplies the K-range [z K, (z + 1) K) of wider operands (lda, ldb >= splits * K) and
 /// writes plane z of C ([splits, M, N]: partial sums for splitk_reduce).
-template <typename OutType, bool kEdges = false, typename T = GemmW128kTraits>
+/// kTail (with one range of K only): K is any multiple of 16.
+template <typename OutType, bool kEdges = false, typename T = GemmW128kTraits, bool kTail = false>
 __global__ void __launch_bounds__(T::kThreads)
     gemm_w128k(const __half* __restrict__ A, const __half* __restrict__ Bt, OutType* __restrict__ C, int M, int N, int K,
                int lda, int ldb, int ldc) {
@@ -100,6 +104,23 @@ __global__ void __launch_bounds__(T::kThreads)
                                               (q < 8 ? wave * T::kLoads + q : wave * T::kLoadsB + (q - 8)) * 1024);
     };
     auto load_src = [&](int kt, int q) -> const __half* { return (q < 8 ? a_base : b_base) + kt * T::kBK; };
+    const int ktiles = kTail ? (K + T::kBK - 1) / T::kBK : K / T::kBK;
+    // kTail: how far back a lane's piece of the last tile has to come from to lie inside its row; the swizzle of a row
+    // repeats every 16 rows, which are four load instructions
+    const int last_pieces = kTail ? (K - (ktiles - 1) * T::kBK) / 8 : 16;  // of 16 in the last tile
+    unsigned int back_a[4], back_b[4];
+    if constexpr (kTail) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int pa = lchk ^ (((wave * T::kLoads + q) * 4 + lrow) & 15), pb = lchk ^ (((wave * T::kLoadsB + q) * 4 + lrow) & 15);
+            back_a[q] = pa < last_pieces ? 0 : 16 * pa;
+            back_b[q] = pb < last_pieces ? 0 : 16 * pb;
+        }
+    }
+    auto load_off = [&](int kt, int q) -> unsigned int {
+        if constexpr (!kTail) return voff[q];
+        else return voff[q] - (kt == ktiles - 1 ? q < 8 ? back_a[q & 3] : back_b[(q - 8) & 3] : 0u);
+    };
 
     // ---- LDS -> registers: fragment r (r < 8: A rows 16 r .., else B rows 16 (r - 8) ..); lane l holds row l % 16,
     // k = 32 wave + 8 (l / 16) .. + 7 of the tile = logical chunk 4 wave + l / 16 of its row. The 16 rows a 16-lane
@@ -116,14 +137,13 @@ __global__ void __launch_bounds__(T::kThreads)
     };
 
     f16x8 fx[T::kFrags], fy[T::kFrags];  // fragments of the tile being multiplied / of the next one: [0..7] A, [8..] B
-    const int ktiles = K / T::kBK;
     auto clamped = [&](int kt) { return kt < ktiles ? kt : ktiles - 1; };
     // prologue: A0 B0 A1 B1 A2 fill the ring
 #pragma unroll
     for (int u = 0; u < T::kSlots; ++u) {
 #pragma unroll
         for (int q = (u & 1) ? 8 : 0; q < ((u & 1) ? kNumLoads : 8); ++q)
-            detail::load_lds_16B_sbase(voff[q], load_src(clamped(u >> 1), q), load_dst(u * T::kSlotBytes, q));
+            detail::load_lds_16B_sbase(load_off(clamped(u >> 1), q), load_src(clamped(u >> 1), q), load_dst(u * T::kSlotBytes, q));
     }
     // the accumulators are pinned to the AGPR half row group by row group
     auto pin_row = [](f32x4 (&row)[kNT]) {
@@ -164,6 +184,19 @@ __global__ void __launch_bounds__(T::kThreads)
         // tile kt + 1 has landed (behind its B part: the A part of tile kt + 2) and this wavefront's reads of tile kt's
         // slots (issued during the previous phase) have returned; then everyone's
         detail::lds_barrier<8>();
+        if (kTail && kt == ktiles - 1) {
+            // (the fragments were requested in the previous phase and have returned: the barrier waited for them)
+            const unsigned int keep = 4 * wave + fquad >= last_pieces ? 0u : ~0u;
+#pragma unroll
+            for (int r = 0; r < T::kFrags; ++r) {
+                u32x4 bits = __builtin_bit_cast(u32x4, cur[r]);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) bits[e] &= keep;
+                cur[r] = __builtin_bit_cast(f16x8, bits);
+                asm volatile("" : "+v"(cur[r]));
+            }
+            asm volatile("s_nop 4");  // the matrix instructions below are assembly: the compiler adds no wait states for them
+        }
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
 #pragma unroll
@@ -174,7 +207,7 @@ __global__ void __launch_bounds__(T::kThreads)
                 const int s = 2 * i + (n >> 2);  // load slot of the phase: B of tile kt + 2 first, then A of tile kt + 3
                 if ((n & 3) == 1 && s < kNumLoads) {
                     const int q = s < T::kLoadsB ? 8 + s : s - T::kLoadsB;
-                    detail::mfma_16x16x32_agpr_then_load(acc[i][j], cur[8 + j], cur[i], voff[q],
+                    detail::mfma_16x16x32_agpr_then_load(acc[i][j], cur[8 + j], cur[i], load_off(q < 8 ? kt_a : kt_b, q),
                                                          load_src(q < 8 ? kt_a : kt_b, q), load_dst(q < 8 ? load_a : load_b, q));
                 } else {
                     detail::mfma_16x16x32_agpr(acc[i][j], cur[8 + j], cur[i]);

@@ -61,7 +61,7 @@ typedef enum {
     TCU_GEMM_WAVE128_KSPLIT = 8, /* 128 x 128 tile (128 x 96 where that fills the GPU better) on 4 wavefronts (one per SIMD)
                                 that each own the whole tile over a quarter of every 128-wide step of K, partial tiles
                                 added through LDS: for products with too few 256 x 256 tiles to fill the GPU (2048^3,
-                                1552 x 1552 x 4096); K a multiple of 128,
+                                1552 x 1552 x 4096); K a multiple of 128 (AUTO runs it with a tail in K, any multiple of 16, too),
                                 M and N multiples of 16 (edge tiles: rows clamped, stores guarded); the sum over K is
                                 taken in four interleaved parts (differs from the other kernels by f32 rounding) */
     TCU_GEMM_DIRECT = 11,    /* tiles of 16 to 64 x 16 to 64 by a cost model, 8 wavefronts that split K and bring their own

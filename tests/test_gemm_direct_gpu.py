@@ -43,3 +43,28 @@ def test_gemm_direct_leaves_the_workspace(tcu, device):
     want = tcu.gemm(a, b, algo="direct")
     assert torch.equal(tcu.gemm(a, b, workspace=ws), want) and torch.equal(tcu.gemm(a, b), want)
     assert bool((ws == 0xFF).all())
+
+
+@pytest.mark.parametrize("M,N,K", [(2048, 2048, 1040), (1808, 1808, 1552), (2064, 1040, 1072), (1552, 1552, 1600),
+                                   (1536, 1536, 1648), (1296, 1296, 4112), (1040, 1040, 8304), (1936, 1984, 1136)])
+@pytest.mark.parametrize("out_dtype", ["f32", "f16"])
+def test_gemm_tail_of_the_k_splitting_kernel(tcu, oracle, device, M, N, K, out_dtype):
+    """AUTO's choice for one round of 128 x 128 (or 128 x 96) tiles where K is not a multiple of 128: tails of 16 to 112 columns, odd
+    and even numbers of steps, whole and edge tiles; what lies behind the operands' last rows is NaN."""
+    import torch
+
+    print(f"gemm k tail {M}x{N}x{K} {out_dtype}", flush=True)
+    dt = torch.float32 if out_dtype == "f32" else torch.float16
+    A = oracle.fill_uniform(M * K, 31 + M).reshape(M, K)
+    Bt = oracle.fill_uniform(N * K, 37 + N).reshape(N, K)
+    a = torch.full((M + 16, K), float("nan"), dtype=torch.float16, device=device)
+    b = torch.full((N + 16, K), float("nan"), dtype=torch.float16, device=device)
+    a[:M], b[:N] = torch.from_numpy(A).to(device), torch.from_numpy(Bt).to(device)
+    guard = torch.full((M + 2, N), -7.0, dtype=dt, device=device)
+    tcu.gemm(a[:M], b[:N], out=guard[1:M + 1])
+    torch.cuda.synchronize()
+    rows = sorted(set(list(range(0, 32)) + list(range(M - 32, M))))
+    assert oracle.max_rel_err(guard[1:M + 1].float().cpu().numpy()[rows], oracle.gemm(A[rows], Bt)) <= REL_TOL
+    want = tcu.gemm(a[:M], b[:N], out_dtype=torch.float32, algo="pipelined").cpu().numpy()
+    assert oracle.max_rel_err(guard[1:M + 1].float().cpu().numpy(), want) <= REL_TOL
+    assert torch.all(guard[0] == -7.0) and torch.all(guard[M + 1] == -7.0)

@@ -289,12 +289,11 @@ template <typename OutType, typename T>
 int launch_gemm_w128k(const __half* A, const __half* B, OutType* C, int M, int N, int K, hipStream_t stream, int ldc) {
     const long grid = (long)((M + T::kBM - 1) / T::kBM) * ((N + T::kBN - 1) / T::kBN);
     if (grid > INT_MAX) return fail(TCU_ERR_UNSUPPORTED_SHAPE, "GEMM: too many tiles for one launch");
-    if (M % T::kBM == 0 && N % T::kBN == 0)
-        return launch(&gemm_w128k<OutType, false, T>, dim3(unsigned(grid)), dim3(T::kThreads), T::kLdsBytes, stream, A, B, C,
-                      M, N, K, K, K, ldc);
-    // edge tiles: rows beyond M or N loaded from the last valid row, stores guarded per 16 x 16 block
-    return launch(&gemm_w128k<OutType, true, T>, dim3(unsigned(grid)), dim3(T::kThreads), T::kLdsBytes, stream, A, B, C, M,
-                  N, K, K, K, ldc);
+    // edge tiles: rows beyond M or N loaded from the last valid row, stores guarded per 16 x 16 block; with a tail in K also
+    // where M and N are whole tiles
+    const bool whole = M % T::kBM == 0 && N % T::kBN == 0;
+    auto kernel = K % T::kBK != 0 ? &gemm_w128k<OutType, true, T, true> : whole ? &gemm_w128k<OutType, false, T> : &gemm_w128k<OutType, true, T>;
+    return launch(kernel, dim3(unsigned(grid)), dim3(T::kThreads), T::kLdsBytes, stream, A, B, C, M, N, K, K, K, ldc);
 }
 
 template <typename OutType>
@@ -302,9 +301,8 @@ int gemm_w128k_dispatch(const __half* A, const __half* B, OutType* C, int M, int
                         int ldc = 0) {
     using T = GemmW128kTraits;
     if (ldc == 0) ldc = N;
-    if (M % 16 != 0 || N % 16 != 0 || K % T::kBK != 0)
-        return fail(TCU_ERR_UNSUPPORTED_SHAPE, "the K-splitting one-wavefront-per-SIMD GEMM needs M and N in multiples of 16 "
-                                               "and K in multiples of 128");
+    if (M % 16 != 0 || N % 16 != 0 || K % 16 != 0)
+        return fail(TCU_ERR_UNSUPPORTED_SHAPE, "the K-splitting one-wavefront-per-SIMD GEMM needs M, N and K in multiples of 16");
     if ((long)K * 2 * T::kBM >= (1l << 32))
         return fail(TCU_ERR_UNSUPPORTED_SHAPE, "the K-splitting GEMM addresses a 128-row panel with 32-bit offsets");
     // All workgroups run at once (one per CU), so the launch takes as long as one tile: when 128 x 128 tiles would
@@ -390,9 +388,12 @@ int gemm_main_and_strips(const __half* A, const __half* B, OutType* C, int M, in
 /// Whether AUTO sends an unsplit product to the kernel whose wavefronts split K: about one 128 x 128 tile per CU and a
 /// long enough K (2048^3: 21.9 against 26.8 us for the LDS-bound 64 x 64-per-wavefront tilings, 1536 x 1536 x 4096: 26.6
 /// against 38.5 us, 2048 x 2048 x 1536: 19.8 against 22.6 us); with a short K its reduction through LDS costs more than
-/// it saves.
+/// it saves. A K that is not a multiple of 128 costs the last step in full; the kernels it would go to instead lose as much
+/// (1808 x 1808 x 1040: 20.8 -> 15.8 us, 2064 x 1040 x 1072: 15.6 -> 14.5, 1552 x 1552 x 1600: 18.4 -> 15.7, 2048 x 2048 x 4112:
+/// 74.0 -> 39.3, 1040 x 1040 x 8208: 67.4 -> 50.2), but for a short K in multiples of 64 (2000 x 2000 x 1088: 16.0 against 16.4).
 bool gemm_w128k_is_the_choice(int M, int N, int K) {
-    if (M % 16 != 0 || N % 16 != 0 || K % 128 != 0 || K < 1024 || (long)K * 256 >= (1l << 32)) return false;
+    if (M % 16 != 0 || N % 16 != 0 || K % 16 != 0 || K < 1024 || (long)K * 256 >= (1l << 32)) return false;
+    if (K % 128 == 64 && K < 1536) return false;
     const long tiles = (long)((M + 127) / 128) * ((N + 127) / 128);
     // the fewer tiles, the longer K has to be (1408 x 1280 x 4096, 110 tiles: 24.7 against 26.1 us; 1536 x 1280 x 2048, 120:
     // 15.6 against 14.2; 1792^2 x 1024, 196: 11.8 against 13.2; 1536^2 x 1024, 144: 10.3 against 10.0)
@@ -420,7 +421,7 @@ bool gemm_narrow_is_the_choice(int M, int N, int K) {
 double gemm_w128k_us(int M, int N, int K) {
     const long rows = (M + 127) / 128;
     const long tiles128 = rows * ((N + 127) / 128), tiles96 = rows * ((N + 95) / 96);
-    return 5.0 + (tiles128 <= 192 && tiles96 <= 256 ? 0.75 : 0.95) * (K / 128);
+    return 5.0 + (tiles128 <= 192 && tiles96 <= 256 ? 0.75 : 0.95) * ((K + 127) / 128);
 }
 
 double gemm_narrow_us(int M, int N, int K) {
@@ -500,10 +501,11 @@ struct GemmSplitPlan {
     double us;
 };
 
-/// Expected time of the unsplit launch on few output tiles, apart from the kernel of gemm_direct_plan().
-double gemm_unsplit_us(int M, int N, int K) {
+/// Expected time of the unsplit launch on few output tiles, apart from the kernel of gemm_direct_plan() and, without `tail`,
+/// from the K-splitting kernel where K is not a multiple of its step.
+double gemm_unsplit_us(int M, int N, int K, bool tail = true) {
     double us = pipelined_plan(M, N, K).us;
-    if (gemm_w128k_is_the_choice(M, N, K)) us = std::min(us, gemm_w128k_us(M, N, K));
+    if (gemm_w128k_is_the_choice(M, N, K) && (tail || K % 128 == 0)) us = std::min(us, gemm_w128k_us(M, N, K));
     if (gemm_narrow_is_the_choice(M, N, K)) us = std::min(us, gemm_narrow_us(M, N, K));
     const long tiles = (long)((M + 255) / 256) * ((N + 255) / 256);
     return tiles > 128 ? std::min(us, gemm_w128_us(tiles, (K + 63) / 64 * 64)) : us;
@@ -517,7 +519,7 @@ GemmSplitPlan gemm_split_plan(int M, int N, int K) {
     const long tiles = (long)((M + T::kBM - 1) / T::kBM) * ((N + T::kBN - 1) / T::kBN);
     const long tiles128 = (long)((M + 127) / 128) * ((N + 127) / 128);  // (the 128 x 128 form has edge tiles)
     if (tiles > 128) return plan;
-    double best_us = 0.95 * gemm_unsplit_us(M, N, K);
+    double best_us = 0.95 * gemm_unsplit_us(M, N, K, false);  // (the workspace a caller is told is that of this plan)
     const double plane_us = 2.0 * double(M) * N * 4 / 5.3e6;  // a plane of partial products written and read once
     for (int s = 2; whole256 && s * tiles <= 256 && K % (s * T::kBK) == 0 && K / s >= 512; s *= 2) {
         const double us = 10.0 + 1.4 * (K / s / T::kBK) + s * plane_us;
@@ -578,7 +580,7 @@ bool gemm_direct_is_the_choice(int M, int N, int K) { return gemm_direct_plan(M,
 /// 512 x 512 x 8192: 19.4 -> 14.2; 1024 x 1024 x 8192: 29.3 -> 28.3.
 bool gemm_split_is_the_choice(int M, int N, int K) {
     const GemmSplitPlan plan = gemm_split_plan(M, N, K);
-    return plan.splits > 1 && plan.us + 4.0 <= gemm_direct_plan(M, N, K).us;
+    return plan.splits > 1 && plan.us + 4.0 <= gemm_direct_plan(M, N, K).us && plan.us < gemm_unsplit_us(M, N, K);
 }
 
 template <typename OutType>
@@ -653,6 +655,7 @@ int gemm_dispatch(const __half* A, const __half* B, OutType* C, int M, int N, in
         case TCU_GEMM_TILE_WAVE128:
             return gemm_tile_w128_dispatch<OutType>(A, B, C, M, N, K, stream);
         case TCU_GEMM_WAVE128_KSPLIT:
+            if (K % 128 != 0) return fail(TCU_ERR_UNSUPPORTED_SHAPE, "the K-splitting one-wavefront-per-SIMD GEMM needs K in multiples of 128");
             return gemm_w128k_dispatch<OutType>(A, B, C, M, N, K, stream);
         case TCU_GEMM_WAVE128_NARROW:
             return gemm_w128_narrow_dispatch<OutType>(A, B, C, M, N, K, stream);
