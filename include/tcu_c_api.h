@@ -75,8 +75,9 @@ typedef enum {
                                 K % 64 == 0; results identical to WAVE128 and PIPELINED bit for bit */
 } tcu_gemm_algo;
 
-/* Which back-to-back GEMM kernel to run (tcu_b2b_gemm_f16_algo). AUTO picks ROWS for many rows, else RESIDENT, where
- * they apply; TILE_RESIDENT for K = P = 64 with N in {128, 256}; else TILE_LIBRARY. */
+/* Which back-to-back GEMM kernel to run (tcu_b2b_gemm_f16_algo). AUTO picks ROWS for many rows at N = 256; for longer N
+ * (K = P = 128, multiples of 256) a kernel that streams B and C once past 128 or 256 rows per workgroup, where its expected time
+ * is below RESIDENT's; else RESIDENT, where it applies; TILE_RESIDENT for K = P = 64 with N in {128, 256}; else TILE_LIBRARY. */
 typedef enum {
     TCU_B2B_AUTO = 0,
     TCU_B2B_TILE_LIBRARY = 1, /* composed from the 16x16 tile primitives, the reference kernel's structure */

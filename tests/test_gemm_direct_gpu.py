@@ -68,3 +68,25 @@ def test_gemm_tail_of_the_k_splitting_kernel(tcu, oracle, device, M, N, K, out_d
     want = tcu.gemm(a[:M], b[:N], out_dtype=torch.float32, algo="pipelined").cpu().numpy()
     assert oracle.max_rel_err(guard[1:M + 1].float().cpu().numpy(), want) <= REL_TOL
     assert torch.all(guard[0] == -7.0) and torch.all(guard[M + 1] == -7.0)
+
+
+@pytest.mark.parametrize("M,N,batch", [(32, 512, 520), (96, 1024, 260), (2080, 768, 16), (65536, 512, 1), (1600, 1024, 16), (288, 2048, 150)])
+@pytest.mark.parametrize("out_dtype", ["f32", "f16"])
+def test_b2b_streamed_weights(tcu, device, M, N, batch, out_dtype):
+    """AUTO's choice for long N and many rows: workgroups of 128 and 256 rows of which the last is partial, 8 to 32 blocks of
+    columns, many and few items. Against the kernel with 32 rows per workgroup, which the oracle's tests cover: the same f16
+    intermediate up to the order of its f32 sums (an ulp of f16, 2^-11, in few elements), then f32 sums of N terms; a tenth of
+    that for the whole."""
+    import torch
+
+    print(f"b2b stream {M}x{N} batch {batch} {out_dtype}", flush=True)
+    dt = torch.float32 if out_dtype == "f32" else torch.float16
+    gen = torch.Generator(device=device)
+    gen.manual_seed(M + N)
+    normal = lambda *shape: torch.randn(*shape, generator=gen, device=device).mul_(0.1).half()
+    a, b, c = normal(batch, M, 128), normal(batch, N, 128), normal(batch, 128, N)
+    guard = torch.full((batch * M + 2, 128), -7.0, dtype=dt, device=device)
+    out = tcu.b2b_gemm(a, b, c, out=guard[1:-1].view(batch, M, 128))
+    want = tcu.b2b_gemm(a, b, c, out_dtype=dt, algo="resident").float()
+    assert ((out.float() - want).norm() / want.norm()).item() <= (5e-5 if dt == torch.float32 else 2.0 ** -12)
+    assert torch.all(guard[0] == -7.0) and torch.all(guard[-1] == -7.0)

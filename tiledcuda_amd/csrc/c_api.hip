@@ -5,6 +5,7 @@
 #include "tcu_c_api.h"
 
 #include "kernels/b2b_gemm_fwd.hpp"
+#include "kernels/b2b_gemm_stream.hpp"
 #include "kernels/flash_attn_fwd.hpp"
 #include "kernels/flash_attn_keys.hpp"
 #include "kernels/flash_attn_tile_w64.hpp"
@@ -742,6 +743,25 @@ int launch_b2b_tile_resident(const __half* A, const __half* B, const __half* C, 
                   Traits::kShmBytes, stream, A, B, C, D, M);
 }
 
+/// Wavefronts of the kernel that streams the weights past 32 rows per wavefront, or 0 where the one with 32 rows per workgroup
+/// is expected to be as fast (K = P = 128, N a multiple of 256). Both run rounds of one workgroup per CU; a round takes 1.85 us per
+/// 256 columns + 1.7 with 32 rows, per 64 columns 1.65 us + 5.5 with 256 rows (8 wavefronts), 1.3 us + 5 with 128 (4).
+int b2b_stream_waves(int M, int N, int batch) {
+    const auto rounds = [&](int rows) { return double(((long)((M + rows - 1) / rows) * batch + 255) / 256); };
+    const double resident = rounds(32) * (1.85 * (N / 256) + 1.7);
+    const double eight = rounds(256) * (1.65 * (N / 64) + 5.5), four = rounds(128) * (1.3 * (N / 64) + 5.0);
+    if (std::min(eight, four) >= 0.93 * resident || N >= (1 << 23)) return 0;
+    return eight <= four ? 8 : 4;
+}
+
+template <int kWaves, typename OutType>
+int launch_b2b_stream(const __half* A, const __half* B, const __half* C, OutType* D, int M, int N, int batch, hipStream_t stream) {
+    using T = B2bStreamTraits<kWaves, 2>;
+    const long grid = (long)((M + T::kTM - 1) / T::kTM) * batch;
+    if (grid > INT_MAX) return fail(TCU_ERR_UNSUPPORTED_SHAPE, "b2b GEMM: too many row blocks for one launch");
+    return launch(&b2b_gemm_stream<T, OutType>, dim3(unsigned(grid)), dim3(T::kThreads), T::kLdsBytes, stream, A, B, C, D, M, N, batch);
+}
+
 template <typename OutType>
 int b2b_dispatch(const __half* A, const __half* B, const __half* C, OutType* D, int M, int N, int K, int P, int batch,
                  int algo, hipStream_t stream) {
@@ -773,6 +793,12 @@ int b2b_dispatch(const __half* A, const __half* B, const __half* C, OutType* D, 
         }
         if (algo == TCU_B2B_ROWS)
             return fail(TCU_ERR_UNSUPPORTED_SHAPE, "the many-rows b2b kernel takes N = 256, K = P = 128 and M a multiple of 64");
+    }
+    // long N and many rows: the weights pass once for 128 or 256 rows
+    if (algo == TCU_B2B_AUTO && N % 256 == 0 && N > 256 && K == 128 && P == 128 && M % 32 == 0) {
+        const int waves = b2b_stream_waves(M, N, batch);
+        if (waves == 8) return launch_b2b_stream<8>(A, B, C, D, M, N, batch, stream);
+        if (waves == 4) return launch_b2b_stream<4>(A, B, C, D, M, N, batch, stream);
     }
     if (algo != TCU_B2B_TILE_LIBRARY) {
         if (N % 256 == 0 && K == 128 && P == 128 && M % 32 == 0)
