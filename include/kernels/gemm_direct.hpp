@@ -124,13 +124,17 @@ __global__ void __launch_bounds__(T::kThreads)
                     for (int r = 0; r < kRT; ++r) af[s][r] = f16x8{0, 0, 0, 0, 0, 0, 0, 0};
                 }
         }
+        // a chunk's sum is added to the total as a whole: the error of the sums stays that of short chains (256 x 256 x 8192: 1.1e-7; 2.1e-7
+        // with one chain per wavefront, as fast to within 2 %)
 #pragma unroll
-        for (int s = 0; s < 2; ++s)
+        for (int u = 0; u < kUT; ++u)
 #pragma unroll
-            for (int u = 0; u < kUT; ++u)
+            for (int r = 0; r < kRT; ++r) {
+                f32x4 part = __builtin_amdgcn_mfma_f32_16x16x32_f16(bf[0][u], af[0][r], f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+                part = __builtin_amdgcn_mfma_f32_16x16x32_f16(bf[1][u], af[1][r], part, 0, 0, 0);
 #pragma unroll
-                for (int r = 0; r < kRT; ++r)
-                    acc[u][r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(bf[s][u], af[s][r], acc[u][r], 0, 0, 0);
+                for (int e = 0; e < 4; ++e) acc[u][r][e] += part[e];
+            }
     }
 
     // ---- add the eight wavefronts' sums through LDS. A lane's accumulator holds columns 16 u + 4 (lane / 16) .. + 3 of row
