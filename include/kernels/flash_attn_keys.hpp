@@ -43,6 +43,9 @@ struct FlashKeysTraits {
     static constexpr int kRowBytes = 2 * kD;
     static constexpr int kTileBytes = kBN * kRowBytes;        // one K or V block
     static constexpr int kLoads = kTileBytes / 1024;          // 1 KiB direct-to-LDS instructions per block
+    // Per-lane offsets of these: at head size 64 an instruction fills 8 rows of 128 bytes and both swizzles repeat every 8
+    // rows, so one offset serves all of them (256 registers per lane are just enough there)
+    static constexpr int kOffsets = kD == 64 ? 1 : kLoads;
     static constexpr int kDSteps = kD / 16, kDTiles = kD / 32;
     static constexpr int kWaveBytes = 4 * kTileBytes;         // two K and two V slots
     static constexpr int kRingBytes = kWaves * kWaveBytes;
@@ -53,7 +56,7 @@ struct FlashKeysTraits {
     static constexpr int kLdsBytes = kFactorOffset + kWaves * kBM * 4;
     static constexpr int kGroupsPerCu = kD == 128 ? 1 : 2;
     static constexpr bool kAgprQ = kGroupsPerCu == 1;         // Q in AGPRs: 512 registers per lane (else 256, all VGPRs)
-    static_assert(kD == 128 || kD == 64, "head size 64 or 128");
+    static_assert(kD == 128 || (kD == 64 && !kVColMajor), "head size 64 or 128");
     static_assert(kQT * kDSteps == 2 * kLoads, "one load behind every matrix instruction of the scores");
 
     /// XOR on the 16-byte chunk index of K row `row` (rows of 256 or 128 bytes).
@@ -121,9 +124,9 @@ __global__ void __launch_bounds__(Traits::kThreads, Traits::kGroupsPerCu)
     auto v_slot = [](int s) { return (2 + s) * Traits::kTileBytes; };
 
     // ---- global -> LDS: per-lane byte offsets of a block's load instructions (the swizzles are applied here)
-    unsigned k_off[Traits::kLoads], v_off[Traits::kLoads];
+    unsigned k_off[Traits::kOffsets], v_off[Traits::kOffsets];
 #pragma unroll
-    for (int t = 0; t < Traits::kLoads; ++t) {
+    for (int t = 0; t < Traits::kOffsets; ++t) {
         const int row = t * (64 / kChunks) + lane / kChunks, chk = lane % kChunks;
         k_off[t] = row * kRowBytes + (chk ^ Traits::k_swz(row)) * 16;
         if constexpr (Traits::kVColMajor) {
@@ -133,16 +136,18 @@ __global__ void __launch_bounds__(Traits::kThreads, Traits::kGroupsPerCu)
             v_off[t] = row * kRowBytes + (chk ^ (Traits::v_swz(row) << 1)) * 16;
         }
     }
+    auto load_off = [](const unsigned (&off)[Traits::kOffsets], int t) { return off[t % Traits::kOffsets]; };
+    auto load_base = [](const __half* base, int t) { return Traits::kOffsets == 1 ? base + t * 512 : base; };
     auto issue_k = [&](int j) {
         const __half* base = Kh + size_t(b_first + wave + j * Traits::kWaves) * (Traits::kBN * kD);
 #pragma unroll
-        for (int t = 0; t < Traits::kLoads; ++t) detail::load_lds_16B_sbase(k_off[t], base, lds0 + k_slot(j & 1) + t * 1024);
+        for (int t = 0; t < Traits::kLoads; ++t) detail::load_lds_16B_sbase(load_off(k_off, t), load_base(base, t), lds0 + k_slot(j & 1) + t * 1024);
     };
     auto issue_v = [&](int j) {
         const size_t key = size_t(b_first + wave + j * Traits::kWaves) * Traits::kBN;
         const __half* base = Vh + (Traits::kVColMajor ? key : key * kD);
 #pragma unroll
-        for (int t = 0; t < Traits::kLoads; ++t) detail::load_lds_16B_sbase(v_off[t], base, lds0 + v_slot(j & 1) + t * 1024);
+        for (int t = 0; t < Traits::kLoads; ++t) detail::load_lds_16B_sbase(load_off(v_off, t), load_base(base, t), lds0 + v_slot(j & 1) + t * 1024);
     };
 
     f32x16 o_acc[kQT][Traits::kDTiles];
@@ -250,9 +255,37 @@ __global__ void __launch_bounds__(Traits::kThreads, Traits::kGroupsPerCu)
 #pragma unroll
             for (int e = 1; e < 16; ++e) mx = fmaxf(mx, s_a[t][e]);
             m_run[t] = fmaxf(mx, detail::exchange32(mx));
+        }
+        // Every score of block 0 may be -infinity (keys masked by an infinite feature; any of 4 * splits blocks of the sequence
+        // is some wavefront's block 0): then the exact maximum of this wavefront's first block with another score, its keys
+        // read once more, is where the query starts. A query without any starts at 0 and keeps a sum of 0.
+        if (__any(m_run[0] == -INFINITY || m_run[1] == -INFINITY)) {
+            for (int j = 1; j < nb; ++j) {
+                const __half* k_row = Kh + (size_t(b_first + wave + j * Traits::kWaves) * Traits::kBN + krow) * kD + 8 * h;
+#pragma unroll
+                for (int t = 0; t < kQT; ++t) {
+                    f32x16 sc;
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) sc[e] = 0.f;
+#pragma unroll
+                    for (int s = 0; s < Traits::kDSteps; ++s)
+                        sc = __builtin_amdgcn_mfma_f32_32x32x16_f16(*reinterpret_cast<const f16x8*>(k_row + 16 * s), qf[t][s], sc, 0, 0, 0);
+                    float mx = sc[0];
+#pragma unroll
+                    for (int e = 1; e < 16; ++e) mx = fmaxf(mx, sc[e]);
+                    mx = fmaxf(mx, detail::exchange32(mx));
+                    if (m_run[t] == -INFINITY) m_run[t] = mx;
+                }
+                if (!__any(m_run[0] == -INFINITY || m_run[1] == -INFINITY)) break;
+            }
+#pragma unroll
+            for (int t = 0; t < kQT; ++t)
+                if (m_run[t] == -INFINITY) m_run[t] = 0.f;
+        }
+#pragma unroll
+        for (int t = 0; t < kQT; ++t)
 #pragma unroll
             for (int e = 0; e < 16; ++e) s_a[t][e] -= m_run[t], m_init[t][e] = -m_run[t];
-        }
 
         constexpr float kLazy = 8.0f;  // a maximum moves only when a block exceeds it by 2^8 (p stays inside f16)
         // One block: the matrix instructions of the next block's scores (the first kQkSlots slots) and of this block's
@@ -296,10 +329,10 @@ __global__ void __launch_bounds__(Traits::kThreads, Traits::kGroupsPerCu)
                     // with K of block j + 2, then V of block j + 1 requested behind the instruction
                     constexpr bool kOfK = i < Traits::kLoads;
                     constexpr int l = kOfK ? i : i - Traits::kLoads;
-                    const unsigned off = kOfK ? k_off[l] : v_off[l];
+                    const unsigned off = load_off(kOfK ? k_off : v_off, l);
                     const unsigned dst = lds0 + (kOfK ? k_slot(j & 1) : v_slot((j + 1) & 1)) + l * 1024;
                     detail::mfma32_score_then_load<s == 0, Traits::kAgprQ>(s_nxt[t], kf[s % 3], qf[t][s], m_init[t], off,
-                                                                           kOfK ? k_base : v_base, dst);
+                                                                           load_base(kOfK ? k_base : v_base, l), dst);
                 } else {
                     constexpr int f = (i - kQkSlots) / kQT, t = i % kQT, s = f / Traits::kDTiles, dt = f % Traits::kDTiles;
                     constexpr int fn = f + 2;
@@ -372,7 +405,8 @@ __global__ void __launch_bounds__(Traits::kThreads, Traits::kGroupsPerCu)
 #pragma unroll
     for (int t = 0; t < kQT; ++t) {
         const float l = l_run[t] + detail::exchange32(l_run[t]);
-        if (h == 0) stat[wave * Traits::kBM + 32 * t + q32] = make_float2(m_run[t], l);
+        // (a sum of 0: no key, or none but masked ones; its weight below is 0)
+        if (h == 0) stat[wave * Traits::kBM + 32 * t + q32] = make_float2(l == 0.f ? -INFINITY : m_run[t], l);
         unsigned char* dst = ring + (32 * t + q32) * (kD * 4);
 #pragma unroll
         for (int dt = 0; dt < Traits::kDTiles; ++dt)
@@ -389,7 +423,7 @@ __global__ void __launch_bounds__(Traits::kThreads, Traits::kGroupsPerCu)
         const float2 ml = stat[w * Traits::kBM + q];
         float mm = fmaxf(ml.x, __shfl_xor(ml.x, 1, 4));
         mm = fmaxf(mm, __shfl_xor(mm, 2, 4));
-        float f = detail::exp2_raw(ml.x - mm);
+        float f = detail::exp2_raw(ml.x - (mm == -INFINITY ? 0.f : mm));
         float ll = ml.y * f;
         ll += __shfl_xor(ll, 1, 4);
         ll += __shfl_xor(ll, 2, 4);
@@ -439,11 +473,13 @@ __global__ void __launch_bounds__(256)
     float mm = ml[0].x;
 #pragma unroll
     for (int s = 1; s < kMax; ++s) mm = fmaxf(mm, ml[s].x);
+    if (mm == -INFINITY) mm = 0.f;
     float ll = 0.f;
     f32x4 sum = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int s = 0; s < kMax; ++s) {
-        const float f = s < splits ? detail::exp2_raw(ml[s].x - mm) : 0.f;
+        if (s >= splits) break;  // (not a weight of 0: a value may be infinite)
+        const float f = detail::exp2_raw(ml[s].x - mm);
         ll += ml[s].y * f;
         sum += v[s] * f;
     }

@@ -113,3 +113,74 @@ def test_keys_kernel_moves_its_maxima(tcu, oracle, device, N, splits):
     out = tcu.flash_attention(dq, dk, dv) if splits > 1 else tcu.flash_attention(dq, dk, dv, algo="keys")
     torch.cuda.synchronize()
     assert oracle.max_abs_err(out.float().cpu().numpy(), oracle.attention(q, k, v, 1.0 / math.sqrt(D))) <= 4e-2
+
+
+def _masked(oracle, batch, M, N, D, masked, level):
+    """N(0, 1) operands whose feature 0 masks keys: 1 in every query, -infinity in the masked keys and `level` in the others."""
+    q = oracle.fill_normal(batch * M * D, 51).reshape(batch, M, D)
+    k = oracle.fill_normal(batch * N * D, 52).reshape(batch, N, D)
+    v = oracle.fill_normal(batch * N * D, 53).reshape(batch, N, D)
+    q[..., 0] = 1.0
+    k[..., 0] = level
+    k[:, masked, 0] = -np.inf
+    return q, k, v
+
+
+@pytest.mark.parametrize("D,v_layout", [(128, "row"), (128, "col"), (64, "row")])
+@pytest.mark.parametrize("N,masked", [(512, slice(32, 64)), (512, slice(0, 128)), (512, slice(192, 512)), (512, slice(1, 512)),
+                                      (4096, slice(0, 1024)), (4096, slice(1024, 2048)), (4096, slice(1000, 4096)),
+                                      (4096, slice(0, 4032))])
+@pytest.mark.parametrize("level", [0.0, -600.0])
+def test_masked_keys(tcu, oracle, device, N, masked, D, v_layout, level):
+    """Scores of -infinity: over one wavefront's first block of 32 keys, over every wavefront's, over a whole split of the keys,
+    over their tail, over all but one. level = -600 puts the scores that are left near -53 (-75 at head size 64), far below a
+    maximum of 0, where 2^s itself is far below the least f16. By name and through AUTO with its workspace and without. The
+    tolerance is that of the other tests with N(0, 1) logits: the level adds the same rounded number to all scores of a row
+    (its product with q's rounded scale enters every score alike), and f32 scores of magnitude 110 in the log2 domain are
+    off by 110 * 2^-24 each: nothing beside f16's 2^-11."""
+    import torch
+
+    batch, M = 2, 64
+    q, k, v = _masked(oracle, batch, M, N, D, masked, level)
+    print(f"attention masked keys {N} {masked} D{D} V {v_layout} level {level}", flush=True)
+    dq, dk, dv = (torch.from_numpy(np.ascontiguousarray(a)).to(device) for a in (q, k, v))
+    ref = oracle.attention(q, k, v, 1.0 / math.sqrt(D))
+    assert np.isfinite(ref).all()
+    calls = [dict(algo="keys"), dict(workspace=False), dict()]
+    for kw in calls:
+        if v_layout == "row":
+            out = tcu.flash_attention(dq, dk, dv, **kw)
+        else:
+            out = torch.empty_like(dq)
+            tcu.flash_attention_fwd(dq.flatten(), dk.flatten(), dv.transpose(1, 2).contiguous().flatten(), out.view(-1), M, N, D, D,
+                                    scale=1.0 / math.sqrt(D), batch=batch, **kw)
+        torch.cuda.synchronize()
+        assert oracle.max_abs_err(out.float().cpu().numpy(), ref) <= ABS_TOL, kw
+
+
+@pytest.mark.parametrize("N", [64, 512, 4096])
+def test_all_keys_masked_stay_undefined(tcu, oracle, device, N):
+    """A row of nothing but -infinity has no softmax: NaN, as before the keys were split, in the masked head only."""
+    import torch
+
+    q, k, v = _masked(oracle, 2, 64, N, 128, slice(0, 0), 0.0)
+    k[1, :, 0] = -np.inf
+    out = tcu.flash_attention(*(torch.from_numpy(np.ascontiguousarray(a)).to(device) for a in (q, k, v)), algo="auto")
+    torch.cuda.synchronize()
+    assert bool(out[1].isnan().all()) and not bool(out[0].isnan().any())
+
+
+def test_infinite_value_keeps_its_sign(tcu, oracle, device):
+    """One infinite value, at a key with a weight of about 1/N: its column is infinite, not NaN, also where fewer workgroups
+    than the combining kernel has slots for split the keys."""
+    import torch
+
+    q, k, v = _masked(oracle, 3, 192, 2112, 128, slice(0, 0), 0.0)
+    v[:, 5, 7] = np.inf
+    dq, dk, dv = (torch.from_numpy(np.ascontiguousarray(a)).to(device) for a in (q, k, v))
+    need = tcu.attention_workspace_bytes(3, 192, 2112, 128, 128)
+    assert need // (3 * 192 * 130 * 4) == 12
+    out = tcu.flash_attention(dq, dk, dv)
+    torch.cuda.synchronize()
+    assert bool((out[..., 7] == float("inf")).all())
+    assert bool(out[..., :7].isfinite().all()) and bool(out[..., 8:].isfinite().all())
