@@ -255,6 +255,9 @@ int tcu_lstm_f16_algo(const void* x, const void* W, const void* bias, const void
  * tcu_lstm_f16_ws then fails with TCU_ERR_UNSUPPORTED_SHAPE. No counterpart in the reference (it has no LSTM).
  */
 unsigned long long tcu_lstm_workspace_bytes(int T, int B, int I, int H);
+/* 1 where tcu_lstm_f16_ws is expected to be faster than tcu_lstm_f16 (long inputs: I of 2048 and more at most sizes), else 0:
+ * the Python and torch entries take a workspace for it there. */
+int tcu_lstm_uses_workspace(int T, int B, int I, int H);
 int tcu_lstm_f16_ws(const void* x, const void* W, const void* bias, const void* h0, const void* c0, void* h_all,
                     void* c_out, int T, int B, int I, int H, void* workspace, unsigned long long workspace_bytes,
                     void* stream);

@@ -68,6 +68,7 @@ _SIGNATURES = {
     "tcu_lstm_f16": (ctypes.c_int, [ctypes.c_void_p] * 7 + [ctypes.c_int] * 4 + [ctypes.c_void_p]),
     "tcu_lstm_f16_algo": (ctypes.c_int, [ctypes.c_void_p] * 7 + [ctypes.c_int] * 5 + [ctypes.c_void_p]),
     "tcu_lstm_workspace_bytes": (ctypes.c_ulonglong, [ctypes.c_int] * 4),
+    "tcu_lstm_uses_workspace": (ctypes.c_int, [ctypes.c_int] * 4),
     "tcu_lstm_f16_ws": (ctypes.c_int, [ctypes.c_void_p] * 7 + [ctypes.c_int] * 4 + [ctypes.c_void_p, ctypes.c_ulonglong,
                                                                                      ctypes.c_void_p]),
     "tcu_lstm_persistent_workspace_bytes": (ctypes.c_ulonglong, [ctypes.c_int] * 4),
@@ -319,10 +320,11 @@ def lstm(x: torch.Tensor, W: torch.Tensor, bias: torch.Tensor, h0: torch.Tensor 
     """Fused LSTM layer. x [T, B, I] f16, W [4H, I+H] f16 (gate rows i,f,g,o), bias [4H] f16,
     h0 [B, H] f16 / c0 [B, H] f32 (None = zeros). Returns (h_all [T, B, H] f16, c_T [B, H] f32).
 
-    ``algo="auto"`` runs one fused kernel per step and needs no workspace. ``algo="hoisted"`` computes the input half of the
-    gates for all steps in one GEMM first (``tcu_lstm_f16_ws``); it needs ``lstm_workspace_bytes(T, B, I, H)`` bytes of device
-    memory, taken from ``workspace`` (any dtype) if given, else allocated here. ``out`` = (h_all, c_T) tensors to write into
-    instead of allocating them.
+    ``algo="hoisted"`` computes the input half of the gates for all steps in one GEMM first (``tcu_lstm_f16_ws``); it
+    needs ``lstm_workspace_bytes(T, B, I, H)`` bytes of device memory, taken from ``workspace`` (any dtype) if given,
+    else allocated here. ``algo="auto"`` takes that path where it applies and pays (long inputs) unless ``workspace=False`` (use
+    that, or a workspace of your own, under HIP graph capture: an allocation has no place in a captured stream), else one
+    fused kernel per step. ``out`` = (h_all, c_T) tensors to write into instead of allocating them.
 
     ``algo="persistent"`` runs the whole time loop in one weight-stationary launch after the same GEMM
     (``tcu_lstm_f16_persistent``: H in {256, 512, 768, 1024}, B <= 256 in multiples of 32; ``lstm_persistent_workspace_bytes``). Its
@@ -359,6 +361,8 @@ def lstm(x: torch.Tensor, W: torch.Tensor, bias: torch.Tensor, h0: torch.Tensor 
         if check:
             lstm_persistent_status(workspace)
         return h_all, c_out
+    if algo == "auto" and workspace is not False and x.is_cuda and lib().tcu_lstm_uses_workspace(T, B, I, H):
+        algo = "hoisted"  # a long input size: its half of the gates is cheaper as one GEMM over all steps
     if algo == "hoisted":
         need = lstm_workspace_bytes(T, B, I, H)
         if workspace is None or workspace is False:

@@ -1224,19 +1224,52 @@ int launch_lstm_direct(const __half* x, const __half* W, const __half* bias, con
     return plan.rt == 1 ? go(four{}, one{}) : plan.rt == 2 ? go(four{}, two{}) : go(four{}, four{});
 }
 
+/// The GEMM that computes the input half of the gates of all steps (rows = T * B): with few rows the 128 x 128 tiles of the
+/// K-splitting kernel (1024 rows, I and H 1024: 13 against 22 us), else the 256 x 256 ones (tiles128 = 0).
+struct LstmProjectionPlan {
+    long tiles128;
+    double us;
+};
+LstmProjectionPlan lstm_projection_plan(long rows, int I, int H) {
+    const long tiles128 = ((rows + 127) / 128) * ((4l * H + 127) / 128), tiles256 = ((rows + 255) / 256) * ((4l * H + 255) / 256);
+    const double us128 = double((tiles128 + 255) / 256) * (5.0 + 0.95 * (I / 128)), us256 = gemm_w128_us(tiles256, I);
+    if (us128 < us256 && (long)(I + H) * 256 < (1l << 32)) return {tiles128, us128};
+    return {0, us256};
+}
+
+/// Expected time of one launch of the step kernel. Beyond the rounds of lstm_direct_plan() it counts the operands that the
+/// 32 workgroups of an XCD bring into its L2 (0.7 us per MB and round): many rows of a large batch pass once per round.
+double lstm_step_us(int B, int H, int columns) {
+    const LstmTilePlan plan = lstm_direct_plan(B, H, columns);
+    const long row_blocks = (B + 16 * plan.rt - 1) / (16 * plan.rt), unit_blocks = (H + 4 * plan.ut - 1) / (4 * plan.ut);
+    const double mb = 32e-6 * columns * (std::min(32l, row_blocks) * plan.rt + (32 + row_blocks - 1) / row_blocks * plan.ut);
+    return 2.2 + double((row_blocks * unit_blocks + 255) / 256) * (0.12 * plan.ut * plan.rt + 2.2e-4 * (plan.ut + plan.rt) * columns + 0.7 * mb);
+}
+
+/// Whether AUTO computes the input half of the gates of all steps beforehand where the caller has a workspace for it: the
+/// projection runs at the rate of a GEMM (0.83 of its expected time and 3.5 us, with the pre-activations written and read
+/// 0.37 us per MB), and a step is left with H of its I + H columns. Both plans within 12 % of the measured times of most of
+/// 133 sizes; us, a fused kernel per step against this: T 8, B 64, I 8192, H 4096: 710, 364; 2048, 4096, 256: 378, 198; 1024, 4096,
+/// 512: 286, 197; T 16, B 256, I 4096, H 1024: 317, 237; 256, 2048, 1024: 210, 183; 256, 1024, 1024: 151, 157; T 8, B 512, I
+/// 512, H 1024: 118, 138. The chosen plan was at most 7 % longer than the other.
+bool lstm_projection_pays(int T, int B, int I, int H) {
+    if (tcu_lstm_workspace_bytes(T, B, I, H) == 0 || I < 512 || T < 4 || (long)T * B > INT_MAX) return false;
+    if (!lstm_direct_takes(B, I, H)) return true;  // (the streaming step kernel: half of its bytes are W[:, :I])
+    const double projection = 3.5 + 0.83 * lstm_projection_plan((long)T * B, I, H).us + 0.37 * 16e-6 * T * double(B) * H;
+    return 1.02 * (projection + T * lstm_step_us(B, H, H)) < T * lstm_step_us(B, H, I + H);
+}
+
 int launch_lstm_hoisted(const __half* x, const __half* W, const __half* bias, const __half* h0, const float* c0, __half* h_all,
                         float* c_out, int T, int B, int I, int H, float* pre, hipStream_t stream) {
     // pre[T * B, 4H] = x[T * B, I] . W[:, :I]^T: the stored [4H, I] operand is the first I columns of W's rows
     const long rows = long(T) * B;
     if (rows > INT_MAX) return fail(TCU_ERR_UNSUPPORTED_SHAPE, "tcu_lstm_f16_ws: T * B exceeds the 32-bit row count");
-    // with few rows the 128 x 128 tiles of the K-splitting kernel (T * B 1024, I and H 1024: 13 against 22 us)
-    const long tiles128 = ((rows + 127) / 128) * ((4l * H + 127) / 128), tiles256 = ((rows + 255) / 256) * ((4l * H + 255) / 256);
-    const double us128 = double((tiles128 + 255) / 256) * (5.0 + 0.95 * (I / 128));
+    const LstmProjectionPlan plan = lstm_projection_plan(rows, I, H);
     int rc;
-    if (us128 < gemm_w128_us(tiles256, I) && (long)(I + H) * 256 < (1l << 32)) {
+    if (plan.tiles128 > 0) {
         using Tk = GemmW128kTraits;
         auto kernel = rows % Tk::kBM == 0 ? &gemm_w128k<float, false, Tk> : &gemm_w128k<float, true, Tk>;
-        rc = launch(kernel, dim3(unsigned(tiles128)), dim3(Tk::kThreads), Tk::kLdsBytes, stream, x, W, pre, int(rows), 4 * H, I, I,
+        rc = launch(kernel, dim3(unsigned(plan.tiles128)), dim3(Tk::kThreads), Tk::kLdsBytes, stream, x, W, pre, int(rows), 4 * H, I, I,
                     I + H, 4 * H);
     } else {
         rc = gemm_w128_dispatch<float>(x, W, pre, int(rows), 4 * H, I, stream, I, I + H);
@@ -1473,6 +1506,8 @@ unsigned long long tcu_lstm_workspace_bytes(int T, int B, int I, int H) {
     if (!shape_ok || T <= 0 || B <= 0 || B % 64 != 0 || ((long)T * B) % 256 != 0) return 0;
     return (unsigned long long)T * B * 4 * H * sizeof(float);
 }
+
+int tcu_lstm_uses_workspace(int T, int B, int I, int H) { return lstm_projection_pays(T, B, I, H) ? 1 : 0; }
 
 int tcu_lstm_f16_ws(const void* x, const void* W, const void* bias, const void* h0, const void* c0, void* h_all,
                     void* c_out, int T, int B, int I, int H, void* workspace, unsigned long long workspace_bytes,
