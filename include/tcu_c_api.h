@@ -223,7 +223,8 @@ int tcu_flash_attn_fwd_f16_algo(const void* Q, const void* K, const void* V, voi
  * their f32 partial outputs go to `workspace`, and a second kernel adds them. tcu_flash_attn_workspace_bytes(...) is the
  * workspace this takes, or 0 when the keys are not split: then, and when `workspace` is NULL, the call is
  * tcu_flash_attn_fwd_f16. The workspace (16-byte aligned device memory) is the caller's and free to reuse once the work
- * enqueued here has run. Results differ from the unsplit ones by rounding and the order of the f32 sums only.
+ * enqueued here has run; a graph that captured the call uses it at every replay. Results differ from the unsplit ones by
+ * rounding and the order of the f32 sums only.
  */
 unsigned long long tcu_flash_attn_workspace_bytes(int batch, int M, int N, int Kdim, int P, int v_layout);
 int tcu_flash_attn_fwd_f16_ws(const void* Q, const void* K, const void* V, void* O, int batch, int M, int N, int Kdim, int P,

@@ -184,3 +184,45 @@ def test_infinite_value_keeps_its_sign(tcu, oracle, device):
     torch.cuda.synchronize()
     assert bool((out[..., 7] == float("inf")).all())
     assert bool(out[..., :7].isfinite().all()) and bool(out[..., 8:].isfinite().all())
+
+
+@pytest.mark.parametrize("entry", ["python", "torch_op"])
+def test_captured_calls_allocate_nothing(tcu, oracle, device, entry):
+    """A call that would split its keys through a workspace from the allocator takes none while it is captured (it runs unsplit);
+    a workspace of the caller's is used at every replay. Replays with eager work between them, each against the eager call."""
+    import torch
+
+    import tiledcuda_amd.torch_ops  # noqa: F401
+
+    M, N, D = 64, 8192, 128
+    q, k, v = (torch.from_numpy(oracle.fill_normal(rows * D, seed)).to(device) for rows, seed in ((M, 71), (N, 72), (N, 73)))
+    need = tcu.attention_workspace_bytes(1, M, N, D, D, tcu.TCU_V_COL_MAJOR)
+    assert need > 0
+    ws = torch.empty(need, dtype=torch.uint8, device=device)
+    own, plain = (torch.empty(M * D, dtype=torch.float16, device=device) for _ in range(2))
+
+    def call(out, workspace):
+        if entry == "python":
+            tcu.flash_attention_fwd(q, k, v, out, M, N, D, D, workspace=workspace)
+        else:
+            torch.ops.tiledcuda.flash_attention_fwd(q, k, v, out, M, N, D, D)
+
+    split, unsplit = torch.empty_like(own), torch.empty_like(own)
+    tcu.flash_attention_fwd(q, k, v, split, M, N, D, D)
+    tcu.flash_attention_fwd(q, k, v, unsplit, M, N, D, D, workspace=False)
+    call(own, None)
+    torch.cuda.synchronize()
+    assert torch.equal(own, split) and not torch.equal(split, unsplit)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        before = torch.cuda.memory_stats()["allocation.all.allocated"]
+        call(plain, None)
+        assert torch.cuda.memory_stats()["allocation.all.allocated"] == before
+        if entry == "python":
+            call(own, ws)
+    for _ in range(3):
+        own.zero_(), plain.zero_(), ws.fill_(0x5A)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(plain, unsplit)
+        assert entry != "python" or torch.equal(own, split)

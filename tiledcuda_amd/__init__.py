@@ -220,7 +220,9 @@ def _attention_with_workspace(ptrs: tuple[int, ...], batch: int, m: int, n: int,
                               algo: str, workspace: torch.Tensor | None, device: torch.device) -> None:
     if workspace is None:
         need = attention_workspace_bytes(batch, m, n, k, p, v_layout)
-        if need > 0:
+        # (nothing is allocated in a captured stream: outside torch's own graphs the graph would keep a block that goes back
+        # to the allocator)
+        if need > 0 and not torch.cuda.is_current_stream_capturing():
             workspace = torch.empty(need, dtype=torch.uint8, device=device)
     elif algo != "auto":
         raise ValueError("a workspace goes with algo='auto'")
@@ -262,7 +264,9 @@ def flash_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scale: fl
     """softmax(scale · q kᵀ) v for [..., S, D] tensors in the usual layout (V row-major [S, D]).
     ``scale`` defaults to 1/sqrt(D). With ``algo="auto"`` a call with few queries and many keys splits the keys over
     workgroups through ``workspace`` (a contiguous device tensor of at least ``attention_workspace_bytes(...)`` bytes) or,
-    when none is given, through one taken from torch's caching allocator for the call; ``workspace=False`` never splits."""
+    when none is given, through one taken from torch's caching allocator for the call; ``workspace=False`` never splits. A call
+    that is being captured into a HIP graph splits through a workspace of yours only (it has to live as long as the graph)
+    and without one runs unsplit: an allocation has no place in a captured stream."""
     if q.dim() < 2 or k.dim() < 2 or v.dim() < 2:
         raise ValueError("q, k and v must be [..., S, D]")
     *lead, M, D = q.shape

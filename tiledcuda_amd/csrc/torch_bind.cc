@@ -10,6 +10,7 @@
 #include <ATen/ATen.h>
 #include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
+#include <c10/hip/HIPGraphsC10Utils.h>
 #include <torch/library.h>
 
 #include <tuple>
@@ -73,8 +74,10 @@ void flash_attention_fwd(const at::Tensor& Q, const at::Tensor& K, const at::Ten
     TORCH_CHECK(V.numel() == p * n, "V must hold p * n elements");
     TORCH_CHECK(O.numel() == m * p, "O must hold m * p elements");
     c10::hip::HIPGuardMasqueradingAsCUDA guard(Q.device());
-    // many keys: split over workgroups through a block from torch's caching allocator, as in gemm
-    const unsigned long long need = tcu_flash_attn_workspace_bytes(1, int(m), int(n), int(k), int(p), TCU_V_COL_MAJOR);
+    // many keys: split over workgroups through a block from torch's caching allocator, as in gemm; not in a captured stream,
+    // where a graph that is not torch's own would keep a block that goes back to the allocator
+    unsigned long long need = tcu_flash_attn_workspace_bytes(1, int(m), int(n), int(k), int(p), TCU_V_COL_MAJOR);
+    if (need > 0 && c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None) need = 0;
     at::Tensor ws;
     if (need > 0) ws = at::empty({static_cast<int64_t>(need)}, Q.options().dtype(at::kByte));
     check_status(tcu_flash_attn_fwd_f16_ws(Q.data_ptr(), K.data_ptr(), V.data_ptr(), O.data_ptr(), 1, int(m), int(n), int(k),
