@@ -391,9 +391,12 @@ int gemm_main_and_strips(const __half* A, const __half* B, OutType* C, int M, in
 /// against 38.5 us, 2048 x 2048 x 1536: 19.8 against 22.6 us); with a short K its reduction through LDS costs more than
 /// it saves. A K that is not a multiple of 128 costs the last step in full; the kernels it would go to instead lose as much
 /// (1808 x 1808 x 1040: 20.8 -> 15.8 us, 2064 x 1040 x 1072: 15.6 -> 14.5, 1552 x 1552 x 1600: 18.4 -> 15.7, 2048 x 2048 x 4112:
-/// 74.0 -> 39.3, 1040 x 1040 x 8208: 67.4 -> 50.2), but for a short K in multiples of 64 (2000 x 2000 x 1088: 16.0 against 16.4).
+/// 74.0 -> 39.3, 1040 x 1040 x 8208: 67.4 -> 50.2, 176 x 7104 x 13104: 159 -> 115), but for a short K in multiples of 64 (2000 x
+/// 2000 x 1088: 16.0 against 16.4), and where half or more of a tile would lie beyond M or N (48 x 11968 x 12864: 102 us
+/// against 77, 15936 x 32 x 12816: 128 against 93, 64 x 13200 x 7856: 78 against 71).
 bool gemm_w128k_is_the_choice(int M, int N, int K) {
     if (M % 16 != 0 || N % 16 != 0 || K % 16 != 0 || K < 1024 || (long)K * 256 >= (1l << 32)) return false;
+    if (K % 128 != 0 && (M <= 64 || N <= 64)) return false;
     if (K % 128 == 64 && K < 1536) return false;
     const long tiles = (long)((M + 127) / 128) * ((N + 127) / 128);
     // the fewer tiles, the longer K has to be (1408 x 1280 x 4096, 110 tiles: 24.7 against 26.1 us; 1536 x 1280 x 2048, 120:
