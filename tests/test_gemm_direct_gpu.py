@@ -90,3 +90,23 @@ def test_b2b_streamed_weights(tcu, device, M, N, batch, out_dtype):
     want = tcu.b2b_gemm(a, b, c, out_dtype=dt, algo="resident").float()
     assert ((out.float() - want).norm() / want.norm()).item() <= (5e-5 if dt == torch.float32 else 2.0 ** -12)
     assert torch.all(guard[0] == -7.0) and torch.all(guard[-1] == -7.0)
+
+
+@pytest.mark.parametrize("M,N", [(16, 16), (48, 80)])
+def test_gemm_auto_takes_every_k(tcu, device, M, N):
+    """AUTO accepts a K beyond the 32-bit offsets of the tiled kernels where it has one that counts in 64 bits (outputs below
+    64 x 64): operands of zeros with a few small integers, some in the last columns, whose products are exact."""
+    import torch
+
+    K = (1 << 24) + 16
+    print(f"gemm {M}x{N}x{K}", flush=True)
+    gen = torch.Generator(device=device)
+    gen.manual_seed(M)
+    cols = torch.cat((torch.randint(K, (500,), generator=gen, device=device), torch.arange(K - 12, K, device=device))).unique()
+    a, b = (torch.zeros(rows, K, dtype=torch.float16, device=device) for rows in (M, N))
+    for t in (a, b):
+        t[:, cols] = torch.randint(-3, 4, (t.shape[0], cols.numel()), generator=gen, device=device).half()
+    want = a[:, cols].float() @ b[:, cols].float().t()
+    got = tcu.gemm(a, b, out_dtype=torch.float32)
+    torch.cuda.synchronize()
+    assert torch.equal(got, want) and bool(want.any())

@@ -667,8 +667,9 @@ int gemm_dispatch(const __half* A, const __half* B, OutType* C, int M, int N, in
             return gemm_direct_dispatch<OutType>(A, B, C, M, N, K, stream);
         case TCU_GEMM_AUTO:
             // one product of tiles or three: the kernel that takes its operand tiles straight from global memory has the
-            // shortest start (48 x 48 x 32: 2.1 us against 2.4; from K = 64 on the next one is as fast)
-            if ((long)M * N < 64 * 64 && K <= 48) return gemm_ragged_dispatch<OutType>(A, B, C, M, N, K, stream);
+            // shortest start (48 x 48 x 32: 2.1 us against 2.4; from K = 64 on the next one is as fast). It is also the one
+            // whose offsets have 64 bits: every K is accepted there, as it is without the other kernels
+            if ((long)M * N < 64 * 64 && (K <= 48 || K >= (1 << 24))) return gemm_ragged_dispatch<OutType>(A, B, C, M, N, K, stream);
             // few output tiles: the kernel that splits K over wavefronts without barriers
             if (gemm_direct_is_the_choice(M, N, K)) return gemm_direct_dispatch<OutType>(A, B, C, M, N, K, stream);
             // where the 256 x 256 tile is the choice anyway, the one-wavefront-per-SIMD kernel is the faster one
