@@ -553,7 +553,9 @@ int gemm_split_count(int M, int N, int K) { return gemm_split_plan(M, N, K).spli
 
 /// The tile of the kernel whose 8 wavefronts split K without barriers, and what its launch is expected to cost: 2.4 us + rounds
 /// of one workgroup per CU, each as long as its rows take to arrive (95 KB per us and CU) plus 0.1 us per 16 x 16 tile for
-/// the sums of the wavefronts, + 0.4 of the time operands and result take at 5.2 TB/s; no less than that whole time. Within 15 %
+/// the sums of the wavefronts, + 0.4 of the time operands and result take at 5.2 TB/s; no less than that whole time; 0.6 us for
+/// every round after the first, which a short K does not hide (384 x 448 x 128: three rounds of 1 x 1 tiles 4.5 us, one of 2 x 2
+/// 2.9; 3664 x 640 x 1472: three of 4 x 4 22.1, the pipelined kernel 19.8). Within 15 %
 /// of the measured times from half a round of workgroups on (with fewer, a CU receives up to 147 KB per us).
 struct GemmDirectPlan {
     int ut, rt;
@@ -568,7 +570,7 @@ GemmDirectPlan gemm_direct_plan(int M, int N, int K) {
         const long groups = (long)((M + 16 * rt - 1) / (16 * rt)) * ((N + 16 * ut - 1) / (16 * ut));
         if (groups > INT_MAX) continue;
         const double cu_us = double((groups + 255) / 256) * (0.1 * ut * rt + 32.0 * (ut + rt) * K / 95e3);
-        const double us = 2.4 + std::max(cu_us + 0.4 * once_us, once_us);
+        const double us = 2.4 + std::max(cu_us + 0.4 * once_us, once_us) + 0.6 * double((groups + 255) / 256 - 1);
         if (us < plan.us) plan = {ut, rt, us};
     }
     return plan;
