@@ -84,6 +84,12 @@ DEVICE void xcd_head_block(int q_blocks, int units, int& unit, int& q_block) {
     unit = lin / q_blocks;
     q_block = lin - unit * q_blocks;
 }
+/// The same for the kernels below: heads of one query block share nothing, and are neighbours in memory when taken in the
+/// order of the workgroups (308 heads of 64 x 64 at head size 128: 10.3 us in runs, 9.75 in this order).
+DEVICE void attn_head_block(int q_blocks, int batch, int& head, int& q_block) {
+    if (q_blocks == 1) head = blockIdx.x, q_block = 0;
+    else xcd_head_block(q_blocks, batch, head, q_block);
+}
 }  // namespace detail
 
 /// grid = ceil(M / kBM) * batch workgroups (1-D), block = Traits::kThreads, dynamic LDS = Traits::kLdsBytes.
@@ -104,7 +110,7 @@ __global__ void __launch_bounds__(Traits::kThreads)
 
     const int q_blocks = (M + Traits::kBM - 1) / Traits::kBM;
     int head_i, q_block;
-    detail::xcd_head_block(q_blocks, batch, head_i, q_block);
+    detail::attn_head_block(q_blocks, batch, head_i, q_block);
     const size_t head = head_i;
     // a wavefront of the last block whose 32 queries lie beyond M works on the last ones that exist and stores nothing
     const bool valid = q_block * Traits::kBM + wave * 32 < M;
@@ -374,7 +380,7 @@ __global__ void __launch_bounds__(Traits::kThreads)
 
     const int q_blocks = (M + Traits::kBM - 1) / Traits::kBM;
     int head_i, q_block;
-    detail::xcd_head_block(q_blocks, batch, head_i, q_block);
+    detail::attn_head_block(q_blocks, batch, head_i, q_block);
     const size_t head = head_i;
     // a wavefront of the last block whose 32 queries lie beyond M works on the last ones that exist and stores nothing
     const bool valid = q_block * Traits::kBM + wave * 32 < M;
