@@ -1030,7 +1030,8 @@ double attn_keys_us(int batch, int M, int N, int D, int splits) {
 
 /// Expected time (us) of the kernels with 64 queries per wavefront in blocks of 256 (the 16x16x32 one, and the 32x32x16 one
 /// where AUTO runs it), one block per CU at a time, and of the 32-queries-per-wavefront kernel. The time per key rises by a
-/// fifth from a few busy CUs to all of them (the chip is power-limited). Within 10 % of the measured times.
+/// fifth from a few busy CUs to all of them (the chip is power-limited). Workgroups of 2 wavefronts start sooner at head size 128
+/// (7 x 1600 x 128: 7.0 us, which the key-splitting kernel takes 7.7 for). Within 10 % of the measured times.
 double attn_w64_us(int batch, int M, int N, int D) {
     const long items = (long)batch * ((M + 255) / 256), rounds = (items + 255) / 256;
     const double fill = double(items) / (256.0 * rounds);
@@ -1039,7 +1040,7 @@ double attn_w64_us(int batch, int M, int N, int D) {
 double attn_fused_us(int batch, int M, int N, int D) {
     const AttnWavesPlan plan = attn_waves_plan(batch, M, D);
     const double fill = std::min(1.0, plan.groups / 256.0);
-    return D == 128 ? 1.3 + plan.rounds * (3.2 + N * (0.0205 + 0.0055 * fill)) : 1.0 + plan.rounds * (2.2 + N * (0.0138 + 0.002 * fill));
+    return D == 128 ? 1.3 + plan.rounds * ((plan.waves == 2 ? 2.6 : 3.2) + N * (0.0205 + 0.0055 * fill)) : 1.0 + plan.rounds * (2.2 + N * (0.0138 + 0.002 * fill));
 }
 
 /// Whether AUTO's choice among the kernels that give wavefronts their own queries is the 16x16x32 one: from 256 whole blocks of
