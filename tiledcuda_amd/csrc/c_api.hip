@@ -1048,11 +1048,12 @@ double attn_fused_us(int batch, int M, int N, int D) {
 
 /// Whether AUTO's choice among the kernels that give wavefronts their own queries is the 16x16x32 one: from 256 whole blocks of
 /// 256 queries on (192 with N >= 1024), unless a last round of few blocks makes it longer than the 32-queries-per-wavefront
-/// kernel (22 x 2944^2 at head size 64, 264 blocks: 99.8 against 76.3 us; a column-major V has no such alternative).
+/// kernel (22 x 2944^2 at head size 64, 264 blocks: 99.8 against 76.3 us; where the two are expected to be about as long it stays:
+/// 128 x 1024 x 448 at 64: 23.9 against 25.1; a column-major V has no such alternative).
 bool attn_k32_is_the_choice(int batch, int M, int N, int D, int v_layout) {
     const long blocks = (long)batch * (M / 256);
     if (N < 320 || !(blocks >= 256 || (blocks >= 192 && N >= 1024))) return false;
-    return v_layout == TCU_V_COL_MAJOR || attn_w64_us(batch, M, N, D) <= 1.05 * attn_fused_us(batch, M, N, D);
+    return v_layout == TCU_V_COL_MAJOR || attn_w64_us(batch, M, N, D) <= 1.15 * attn_fused_us(batch, M, N, D);
 }
 
 /// Whether it is the 32x32x16 kernel with 64 queries per wavefront (row-major V).
