@@ -478,12 +478,10 @@ __global__ void __launch_bounds__(256)
     f32x4 sum = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int s = 0; s < kMax; ++s) {
-        // (a slot without a split is left out, not weighted 0: a value may be infinite)
-        const bool in = s < splits;
-        const float f = detail::exp2_raw(ml[s].x - mm);
-        ll += in ? ml[s].y * f : 0.f;
+        const float f = s < splits ? detail::exp2_raw(ml[s].x - mm) : 0.f;
+        ll += ml[s].y * f;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) sum[e] += in ? v[s][e] * f : 0.f;
+        for (int e = 0; e < 4; ++e) sum[e] += (s < splits ? v[s][e] : 0.f) * f;  // (a value may be infinite)
     }
     const float inv = 1.f / ll;
     f16x4 o;

@@ -1015,9 +1015,9 @@ int fa_keys_dispatch(const __half* Q, const __half* K, const __half* V, __half* 
 /// theirs): 2.3 us with 256 of them, 6.8 TB/s; no less than the L2s take for a full chip (1.05, 1.15 us); with splits the
 /// partial outputs written, read and one launch more. Fitted to 14 shapes at both head sizes with keys and values not in
 /// any cache (32 x 64 x 8192 at 128 with 1, 2, 4, 8, 16 workgroups: 83, 52, 34, 31, 37 us; 64 x 64 x 4096: 50, 35, 32, 37;
-/// 8 x 64 x 8192: 77, 46, 29, 21, 18). The two or three workgroups of a head with M up to 192 do not stay together over a long
-/// sequence at head size 128: its keys come from beyond the L2s for each of them, at 9 TB/s (136 x 192 x 5952: 159 us where the
-/// sum gives 133; with blocks of 256 queries 142).
+/// 8 x 64 x 8192: 77, 46, 29, 21, 18). The three workgroups of a head of 192 queries (of which an XCD's 32 CUs hold ten heads and a
+/// part) do not stay together over a long sequence at head size 128: its keys come from beyond the L2s for each of them, at 9 TB/s
+/// (136 x 192 x 5952: 159 us where the sum gives 133; with blocks of 256 queries 142).
 double attn_keys_us(int batch, int M, int N, int D, int splits) {
     const long groups = (long)batch * (M / 64) * splits, cap = D == 128 ? 256 : 512;
     const double blocks = double(N) / (128.0 * splits);
@@ -1027,7 +1027,7 @@ double attn_keys_us(int batch, int M, int N, int D, int splits) {
         us += D == 128 ? 5.0 + blocks * std::max(0.95 + 0.0052 * own, 1.05 * fill)
                        : 3.5 + 1.6 * std::max(0.0, 2.0 * fill - 1.0) + blocks * std::max(0.62 + 0.0035 * own, 1.15 * fill);
     }
-    if (D == 128 && M <= 192 && splits == 1) us = std::max(us, 6.5 + double(groups) * N * 512.0 / 9e6);
+    if (D == 128 && M == 192 && splits == 1) us = std::max(us, 6.5 + double(groups) * N * 512.0 / 9e6);
     return us + (splits == 1 ? 0.0 : 2.4 + (D == 128 ? 0.011 : 0.006) * groups);
 }
 
@@ -1077,7 +1077,7 @@ int attn_keys_plan(int batch, int M, int N, int D, int v_layout, int max_splits)
     if ((D != 128 && !(D == 64 && v_layout == TCU_V_ROW_MAJOR)) || N >= (1 << 24)) return 0;
     const long groups = (long)batch * (M / 64);
     if (groups > 4096) return 0;
-    double best_us = attn_blocks_us(batch, M, N, D, v_layout);
+    double best_us = 1e30;
     int best = 0;
     for (int s : {1, 2, 3, 4, 6, 8, 12, 16}) {
         if (s > max_splits || (s > 1 && (s * groups > 256 || N < 128 * s))) break;
@@ -1087,7 +1087,10 @@ int attn_keys_plan(int batch, int M, int N, int D, int v_layout, int max_splits)
             best = s;
         }
     }
-    return best;
+    // the first keys of a few workgroups arrive 0.5 us sooner, those of a full chip 0.3 us later: beside the other kernels
+    // that counts (8 x 128 x 192 at 128: 7.5 against 7.9 us, 7 x 1600 x 128: 7.7 against 7.0)
+    if (D == 128 && best == 1) best_us += 0.8 * std::min(1.0, groups / 256.0) - 0.55;
+    return best_us < attn_blocks_us(batch, M, N, D, v_layout) ? best : 0;
 }
 
 int fa_dispatch(const __half* Q, const __half* K, const __half* V, __half* O, int batch, int M, int N, int Kd, int P,
