@@ -950,11 +950,13 @@ int fa_w64_k32_dispatch(const __half* Q, const __half* K, const __half* V, __hal
 
 /// How many wavefronts (of 32 queries) a workgroup of the 8-wavefront kernels has, and what the launch costs relative to
 /// one round of 2-wavefront workgroups. More wavefronts share a block of keys (at head size 128 a CU holds one workgroup
-/// whatever its size: 96 KiB of LDS; at 64 up to three of 2 or 4 wavefronts share one, the second for half a round, the
-/// third for 0.7), fewer leave less idle behind M. Queries beyond M cost their wavefronts' idle time only.
+/// whatever its size: 96 KiB of LDS; at 64 up to three of 2 or 4 wavefronts share one, and every workgroup per CU after the third
+/// costs as much as the next: fitted to 286 sizes of up to 30 per CU, 8 % deviation), fewer leave less idle behind M. Queries
+/// beyond M cost their wavefronts' idle time only; wavefronts that save no workgroup are not taken (489 heads of 64 x 64 at head
+/// size 64: 6.2 us with 2, 6.5 with 4).
 /// Measured, us with 2, 4, 8 wavefronts (the largest that divides M was taken before): 200 x 192 x 512 at head size 128:
 /// 44.5, 33.5, 21.8; 100 x 448^2: 39.8, 29.7, 19.1; 40 x 832 x 960: 70.2, 50.3, 29.7; 96 x 576^2 at head size 64: 26.7,
-/// 18.4, 26.6; 300 x 64 x 512 at 128: 31.2, 33.2, 37.8; 36 x 448^2 at 128: 14.4, 14.8, 16.4.
+/// 18.4, 26.6; 1848 x 320 x 64 at 64: 54.2, 48.2, 73.3; 300 x 64 x 512 at 128: 31.2, 33.2, 37.8; 36 x 448^2 at 128: 14.4, 14.8, 16.4.
 struct AttnWavesPlan {
     int waves;
     double rounds;
@@ -962,13 +964,18 @@ struct AttnWavesPlan {
 };
 AttnWavesPlan attn_waves_plan(int batch, int M, int D) {
     AttnWavesPlan plan{8, 1e30, 0};
-    for (const auto& [waves, one, second, rise] :
-         {std::tuple{2, 1.0, 0.55, 0.1}, std::tuple{4, 1.05, 0.45, 0.23}, std::tuple{8, 1.15, 1.15, 0.0}}) {
-        const long groups = (long)batch * ((M + 32 * waves - 1) / (32 * waves));
+    struct Cost {
+        int waves;
+        double round128;  // of one workgroup per CU, head size 128
+        double one, second, third, next;  // at head size 64, by the number of workgroups per CU
+    };
+    for (const Cost& c : {Cost{2, 1.0, 1.0, 0.36, 0.41, 0.43}, Cost{4, 1.05, 1.01, 0.43, 0.83, 0.60}, Cost{8, 1.15, 1.16, 1.3, 1.23, 1.40}}) {
+        const long groups = (long)batch * ((M + 32 * c.waves - 1) / (32 * c.waves));
+        if (groups == plan.groups) continue;
         const long per_cu = (groups + 255) / 256;
-        const double more = double(per_cu - 1);
-        const double rounds = one * (1.0 + (D == 128 ? more : more * second + more * (more - 1.0) / 2.0 * rise));
-        if (rounds < plan.rounds) plan = {waves, rounds, groups};
+        const double rounds = D == 128 ? c.round128 * double(per_cu)
+                                       : c.one + (per_cu > 1 ? c.second : 0.0) + (per_cu > 2 ? c.third + double(per_cu - 3) * c.next : 0.0);
+        if (rounds < plan.rounds) plan = {c.waves, rounds, groups};
     }
     return plan;
 }
