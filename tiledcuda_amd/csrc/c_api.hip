@@ -1031,8 +1031,11 @@ double attn_keys_us(int batch, int M, int N, int D, int splits) {
     double us = D == 128 ? 1.5 : 1.3;
     for (long left = groups; left > 0; left -= cap) {
         const double at_once = double(std::min(left, cap)), own = at_once * 64.0 / M, fill = at_once / cap;
-        us += D == 128 ? 5.0 + blocks * std::max(0.95 + 0.0052 * own, 1.05 * fill)
-                       : 3.5 + 1.6 * std::max(0.0, 2.0 * fill - 1.0) + blocks * std::max(0.62 + 0.0035 * own, 1.15 * fill);
+        const double round = D == 128 ? 5.0 + blocks * std::max(0.95 + 0.0052 * own, 1.05 * fill)
+                                      : 3.5 + 1.6 * std::max(0.0, 2.0 * fill - 1.0) + blocks * std::max(0.62 + 0.0035 * own, 1.15 * fill);
+        // (a last round behind full ones, two workgroups per CU: a few of them run beside the stragglers, many start late. Measured
+        // against the price of a round by itself 0.6 at fill 0.1 (24 x 1536 x 1728: 29.2 us), 1.25 at 0.6 (18 x 2880 x 1920: 40.9))
+        us += round * (D == 64 && left < cap && left < groups ? std::min(1.2, 0.5 + 1.1 * fill) : 1.0);
     }
     if (D == 128 && M == 192 && splits == 1) us = std::max(us, 6.5 + double(groups) * N * 512.0 / 9e6);
     return us + (splits == 1 ? 0.0 : 2.4 + (D == 128 ? 0.011 : 0.006) * groups);
@@ -1056,11 +1059,11 @@ double attn_fused_us(int batch, int M, int N, int D) {
 /// Whether AUTO's choice among the kernels that give wavefronts their own queries is the 16x16x32 one: from 256 whole blocks of
 /// 256 queries on (192 with N >= 1024), unless a last round of few blocks makes it longer than the 32-queries-per-wavefront
 /// kernel (22 x 2944^2 at head size 64, 264 blocks: 99.8 against 76.3 us; where the two are expected to be about as long it stays:
-/// 128 x 1024 x 448 at 64: 23.9 against 25.1; a column-major V has no such alternative).
+/// 128 x 1024 x 448 at 64: 23.9 against 25.1, 6 % apart in the model; 88 x 832 x 320 at 64: 18.9 against 16.5, 13 %; a column-major V has no such alternative).
 bool attn_k32_is_the_choice(int batch, int M, int N, int D, int v_layout) {
     const long blocks = (long)batch * (M / 256);
     if (N < 320 || !(blocks >= 256 || (blocks >= 192 && N >= 1024))) return false;
-    return v_layout == TCU_V_COL_MAJOR || attn_w64_us(batch, M, N, D) <= 1.15 * attn_fused_us(batch, M, N, D);
+    return v_layout == TCU_V_COL_MAJOR || attn_w64_us(batch, M, N, D) <= 1.08 * attn_fused_us(batch, M, N, D);
 }
 
 /// Whether it is the 32x32x16 kernel with 64 queries per wavefront (row-major V).
