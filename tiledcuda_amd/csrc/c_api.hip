@@ -948,34 +948,48 @@ int fa_w64_k32_dispatch(const __half* Q, const __half* K, const __half* V, __hal
                                        : launch_fa_w64_k32<128, true>(Q, K, V, O, batch, M, N, scale, stream);
 }
 
-/// How many wavefronts (of 32 queries) a workgroup of the 8-wavefront kernels has, and what the launch costs relative to
-/// one round of 2-wavefront workgroups. More wavefronts share a block of keys (at head size 128 a CU holds one workgroup
-/// whatever its size: 96 KiB of LDS; at 64 up to three of 2 or 4 wavefronts share one, and every workgroup per CU after the third
-/// costs as much as the next: fitted to 286 sizes of up to 30 per CU, 8 % deviation), fewer leave less idle behind M. Queries
-/// beyond M cost their wavefronts' idle time only; wavefronts that save no workgroup are not taken (489 heads of 64 x 64 at head
-/// size 64: 6.2 us with 2, 6.5 with 4).
+/// How many wavefronts (of 32 queries) a workgroup of the 8-wavefront kernels has, and what the launch is expected to take (us).
+/// More wavefronts share a block of keys (at head size 128 a CU holds one workgroup whatever its size: 96 KiB of LDS; at 64 up to
+/// three of 2 or 4 wavefronts share one, and every workgroup per CU after the third costs as much as the next: fitted to 286
+/// sizes of up to 30 per CU, 6 % deviation), fewer leave less idle behind M. Queries beyond M cost their wavefronts' idle time
+/// only; wavefronts that save no workgroup are not taken (489 heads of 64 x 64 at head size 64: 6.2 us with 2, 6.5 with 4), and there
+/// more than divide M have to promise 6 % (64 x 2688 x 128: 16.6 with 4, 18.4 with 8, 5 % ahead in the model). The time per key rises from a few busy CUs to all of them (the chip is power-limited); workgroups of 2 wavefronts start
+/// sooner at head size 128 (7 x 1600 x 128: 7.0 us, which the key-splitting kernel takes 7.7 for).
 /// Measured, us with 2, 4, 8 wavefronts (the largest that divides M was taken before): 200 x 192 x 512 at head size 128:
 /// 44.5, 33.5, 21.8; 100 x 448^2: 39.8, 29.7, 19.1; 40 x 832 x 960: 70.2, 50.3, 29.7; 96 x 576^2 at head size 64: 26.7,
 /// 18.4, 26.6; 1848 x 320 x 64 at 64: 54.2, 48.2, 73.3; 300 x 64 x 512 at 128: 31.2, 33.2, 37.8; 36 x 448^2 at 128: 14.4, 14.8, 16.4.
 struct AttnWavesPlan {
     int waves;
-    double rounds;
+    double us;
     long groups;
 };
-AttnWavesPlan attn_waves_plan(int batch, int M, int D) {
-    AttnWavesPlan plan{8, 1e30, 0};
+AttnWavesPlan attn_waves_plan(int batch, int M, int N, int D) {
     struct Cost {
         int waves;
-        double round128;  // of one workgroup per CU, head size 128
-        double one, second, third, next;  // at head size 64, by the number of workgroups per CU
+        double round128, start128;               // head size 128: rounds of one workgroup per CU
+        double one, second, third, next, start;  // head size 64, by the number of workgroups per CU
     };
-    for (const Cost& c : {Cost{2, 1.0, 1.0, 0.36, 0.41, 0.43}, Cost{4, 1.05, 1.01, 0.43, 0.83, 0.60}, Cost{8, 1.15, 1.16, 1.3, 1.23, 1.40}}) {
-        const long groups = (long)batch * ((M + 32 * c.waves - 1) / (32 * c.waves));
+    AttnWavesPlan plan{8, 1e30, 0};
+    double best = 1e30;
+    for (const Cost& c : {Cost{2, 1.0, 2.6, 1.0, 0.36, 0.41, 0.43, 2.1}, Cost{4, 1.05, 3.2, 0.985, 0.415, 0.808, 0.573, 2.45},
+                          Cost{8, 1.15, 3.2, 1.05, 1.13, 1.12, 1.11, 3.05}}) {
+        const long groups = (long)batch * ((M + 32 * c.waves - 1) / (32 * c.waves)), per_cu = (groups + 255) / 256;
         if (groups == plan.groups) continue;
-        const long per_cu = (groups + 255) / 256;
-        const double rounds = D == 128 ? c.round128 * double(per_cu)
-                                       : c.one + (per_cu > 1 ? c.second : 0.0) + (per_cu > 2 ? c.third + double(per_cu - 3) * c.next : 0.0);
-        if (rounds < plan.rounds) plan = {c.waves, rounds, groups};
+        const double fill = std::min(1.0, groups / 256.0);
+        double us, score;
+        if (D == 128) {
+            score = c.round128 * double(per_cu);
+            us = 1.3 + score * (c.start128 + N * (0.0205 + 0.0055 * fill));
+        } else {
+            const double rounds = c.one + (per_cu > 1 ? c.second : 0.0) + (per_cu > 2 ? c.third + double(per_cu - 3) * c.next : 0.0);
+            us = 1.0 + rounds * (c.start + N * (0.0138 + 0.002 * fill));
+            const int whole = M % 256 == 0 ? 8 : M % 128 == 0 ? 4 : 2;
+            score = c.waves > whole ? 1.06 * us : us;
+        }
+        if (score < best) {
+            best = score;
+            plan = {c.waves, us, groups};
+        }
     }
     return plan;
 }
@@ -983,7 +997,7 @@ AttnWavesPlan attn_waves_plan(int batch, int M, int D) {
 template <int kD, bool kFused>
 int fa_fwd_by_rows(const __half* Q, const __half* K, const __half* V, __half* O, int batch, int M, int N, float scale,
                    hipStream_t stream) {
-    switch (attn_waves_plan(batch, M, kD).waves) {
+    switch (attn_waves_plan(batch, M, N, kD).waves) {
         case 8: return launch_fa_fwd<kD, 8, kFused>(Q, K, V, O, batch, M, N, scale, stream);
         case 4: return launch_fa_fwd<kD, 4, kFused>(Q, K, V, O, batch, M, N, scale, stream);
         default: return launch_fa_fwd<kD, 2, kFused>(Q, K, V, O, batch, M, N, scale, stream);
@@ -1043,27 +1057,25 @@ double attn_keys_us(int batch, int M, int N, int D, int splits) {
 
 /// Expected time (us) of the kernels with 64 queries per wavefront in blocks of 256 (the 16x16x32 one, and the 32x32x16 one
 /// where AUTO runs it), one block per CU at a time, and of the 32-queries-per-wavefront kernel. The time per key rises by a
-/// fifth from a few busy CUs to all of them (the chip is power-limited). Workgroups of 2 wavefronts start sooner at head size 128
-/// (7 x 1600 x 128: 7.0 us, which the key-splitting kernel takes 7.7 for). Within 10 % of the measured times.
+/// fifth from a few busy CUs to all of them (the chip is power-limited). Within 10 % of the measured times.
 double attn_w64_us(int batch, int M, int N, int D) {
     const long items = (long)batch * ((M + 255) / 256), rounds = (items + 255) / 256;
     const double fill = double(items) / (256.0 * rounds);
     return 1.3 + rounds * (D == 128 ? 6.0 + N * (0.02 + 0.005 * fill) : 4.0 + N * (0.0135 + 0.0043 * fill));
 }
-double attn_fused_us(int batch, int M, int N, int D) {
-    const AttnWavesPlan plan = attn_waves_plan(batch, M, D);
-    const double fill = std::min(1.0, plan.groups / 256.0);
-    return D == 128 ? 1.3 + plan.rounds * ((plan.waves == 2 ? 2.6 : 3.2) + N * (0.0205 + 0.0055 * fill)) : 1.0 + plan.rounds * (2.2 + N * (0.0138 + 0.002 * fill));
-}
+double attn_fused_us(int batch, int M, int N, int D) { return attn_waves_plan(batch, M, N, D).us; }
 
 /// Whether AUTO's choice among the kernels that give wavefronts their own queries is the 16x16x32 one: from 256 whole blocks of
 /// 256 queries on (192 with N >= 1024), unless a last round of few blocks makes it longer than the 32-queries-per-wavefront
-/// kernel (22 x 2944^2 at head size 64, 264 blocks: 99.8 against 76.3 us; where the two are expected to be about as long it stays:
-/// 128 x 1024 x 448 at 64: 23.9 against 25.1, 6 % apart in the model; 88 x 832 x 320 at 64: 18.9 against 16.5, 13 %; a column-major V has no such alternative).
+/// kernel (22 x 2944^2 at head size 64, 264 blocks: 99.8 against 76.3 us; a column-major V has no such alternative). Where that one
+/// runs 8 wavefronts it has to promise 10 % (128 x 1024 x 448 at 64, 8 % ahead in the model: 24.2 against 23.0; 716 x 256 x 320: 31.5
+/// against 28.1), else 5 (144 x 512 x 448, 7 %: 20.5 against 22.7; 88 x 832 x 320, 12 %: 16.3 against 18.8).
 bool attn_k32_is_the_choice(int batch, int M, int N, int D, int v_layout) {
     const long blocks = (long)batch * (M / 256);
     if (N < 320 || !(blocks >= 256 || (blocks >= 192 && N >= 1024))) return false;
-    return v_layout == TCU_V_COL_MAJOR || attn_w64_us(batch, M, N, D) <= 1.08 * attn_fused_us(batch, M, N, D);
+    if (v_layout == TCU_V_COL_MAJOR) return true;
+    const AttnWavesPlan other = attn_waves_plan(batch, M, N, D);
+    return attn_w64_us(batch, M, N, D) <= (other.waves == 8 ? 1.1 : 1.05) * other.us;
 }
 
 /// Whether it is the 32x32x16 kernel with 64 queries per wavefront (row-major V).
