@@ -100,14 +100,16 @@ __global__ void __launch_bounds__(256)
     }
 }
 
-constexpr int kScatterPairsPieces = 2, kScatterPairsBlock = 256 * kScatterPairsPieces;
+/// Words a lane takes one after the other. One where slices start or stop inside a word: their compare-and-swap loops would
+/// follow each other (4096 rows of 3: 7.4 us with two, 5.1 with one; 16384 of 513: 26.5, 26.3).
+HOST_DEVICE constexpr int scatter_pair_pieces(bool whole) { return whole ? 2 : 1; }
 /// Aligned 32-bit words of `data` that a slice of f16 touches; with whole = false it may start or end inside a word.
 HOST_DEVICE int64_t scatter_pair_words(bool whole, int64_t slice) { return whole ? slice / 2 : slice / 2 + 1; }
 
 /// f16 add: one lane per aligned 32-bit word of `data`, both elements added by one global_atomic_pk_add_f16 (each half rounded
 /// to nearest even, subnormals kept: what the f32 addition and conversion of the compare-and-swap loop give); the ends of a
 /// slice that start or stop inside a word by that loop. kWhole: there are none (even slices, `data` and `updates` 4-byte
-/// aligned). A workgroup takes 512 consecutive words of the updates, so that the 64-bit division by the words of a slice is
+/// aligned). A workgroup takes 512 (or 256) consecutive words of the updates, so that the 64-bit division by the words of a slice is
 /// done once for all of them.
 /// What bounds it: the L2s carry out about one 32-bit atomic per clock and channel (f32 addition: 8.4 M words in 31 us). In
 /// the loop neighbouring lanes also contended for each word. 8192 rows of 1024 added into 32768: 300 -> 19 us, of
@@ -118,14 +120,15 @@ __global__ void __launch_bounds__(256)
     scatter_nd_add_pairs(__half* __restrict__ data, const __half* __restrict__ updates, const int64_t* __restrict__ indices,
                          const ScatterNdShape shape, unsigned int* __restrict__ bad_rows) {
     using detail::scatter_pair_t;
+    constexpr int kPieces = scatter_pair_pieces(kWhole), kBlock = 256 * kPieces;
     const int64_t words = scatter_pair_words(kWhole, shape.slice), total = shape.n * words;
-    for (int64_t g0 = int64_t(blockIdx.x) * kScatterPairsBlock; g0 < total; g0 += int64_t(gridDim.x) * kScatterPairsBlock) {
+    for (int64_t g0 = int64_t(blockIdx.x) * kBlock; g0 < total; g0 += int64_t(gridDim.x) * kBlock) {
         const int64_t row0 = g0 / words, rest0 = g0 - row0 * words;
-        int64_t dst[kScatterPairsPieces];                          // first element of the word
-        int lo[kScatterPairsPieces], hi[kScatterPairsPieces];      // its elements that belong to the slice: [lo, hi)
-        scatter_pair_t v[kScatterPairsPieces];
+        int64_t dst[kPieces];          // first element of the word
+        int lo[kPieces], hi[kPieces];  // its elements that belong to the slice: [lo, hi)
+        scatter_pair_t v[kPieces];
 #pragma unroll
-        for (int p = 0; p < kScatterPairsPieces; ++p) {
+        for (int p = 0; p < kPieces; ++p) {
             const int local = threadIdx.x + 256 * p;
             lo[p] = hi[p] = 0;
             if (g0 + local >= total) continue;
@@ -154,7 +157,7 @@ __global__ void __launch_bounds__(256)
             }
         }
 #pragma unroll
-        for (int p = 0; p < kScatterPairsPieces; ++p) {
+        for (int p = 0; p < kPieces; ++p) {
             if (lo[p] >= hi[p]) continue;
             if (kWhole || hi[p] - lo[p] == 2) detail::atomic_add_pair(data + dst[p], v[p]);
             else detail::atomic_add_elem(data + dst[p] + lo[p], __half(v[p][lo[p]]));
