@@ -64,6 +64,7 @@ typedef enum {
                                 1552 x 1552 x 4096); K a multiple of 128 (AUTO runs it with a tail in K, any multiple of 16, too),
                                 M and N multiples of 16 (edge tiles: rows clamped, stores guarded); the sum over K is
                                 taken in four interleaved parts (differs from the other kernels by f32 rounding) */
+    /* (10 is not assigned) */
     TCU_GEMM_DIRECT = 11,    /* tiles of 16 to 64 x 16 to 64 by a cost model, 8 wavefronts that split K and bring their own
                                 chunks to LDS without barriers: for products with few output tiles (32 x 4096 x 4096,
                                 256 x 256 x 8192); M, N, K multiples of 16; the sum over K is taken in eight interleaved
@@ -76,8 +77,7 @@ typedef enum {
 } tcu_gemm_algo;
 
 /* Which back-to-back GEMM kernel to run (tcu_b2b_gemm_f16_algo). AUTO picks ROWS for many rows at N = 256; for longer N
- * (K = P = 128, multiples of 256) a kernel that streams B and C once past 128 or 256 rows per workgroup, where its expected time
- * is below RESIDENT's; else RESIDENT, where it applies; TILE_RESIDENT for K = P = 64 with N in {128, 256}; else TILE_LIBRARY. */
+ * STREAM where its expected time is below RESIDENT's; else RESIDENT, where it applies; TILE_RESIDENT for K = P = 64 with N in {128, 256}; else TILE_LIBRARY. */
 typedef enum {
     TCU_B2B_AUTO = 0,
     TCU_B2B_TILE_LIBRARY = 1, /* composed from the 16x16 tile primitives, the reference kernel's structure */
@@ -87,6 +87,11 @@ typedef enum {
                                  16x16x32 operand tiles, the intermediate through a shared tile); compile-time sizes:
                                  K = P = 128 with N in {256, 1024, 2048} (results identical to RESIDENT bit for bit) and
                                  K = P = 64 with N in {128, 256}; M % 32 == 0 */
+    /* (5 is not assigned) */
+    TCU_B2B_STREAM = 6,       /* for longer N and many rows: blocks of 64 columns of B and C pass once through a ring in LDS for 128 or
+                                 256 rows per workgroup, every wavefront owning 32 of them (A fragments and the intermediate in
+                                 registers); K = P = 128, N % 256 == 0, N >= 512, M % 32 == 0; agrees with RESIDENT up to the
+                                 order of the f32 sums inside an MFMA */
     TCU_B2B_ROWS = 3          /* for many rows (AUTO from M x batch = 32768): N = 256, K = P = 128, M % 64 == 0; a
                                  workgroup keeps B and C in LDS and walks over blocks of 256 rows, every wavefront owning
                                  64 rows (A fragments from global memory, the intermediate stays in registers); agrees
@@ -128,6 +133,7 @@ typedef enum {
                                   (wavefronts of a head's last block whose 64 queries lie beyond M idle), N % 64 == 0,
                                   N >= 320; results equal to WAVE64 (MFMA32_FUSED at head size 64) up to the
                                   summation order inside a matrix instruction */
+    /* (7 is not assigned) */
     TCU_ATTN_KEYS = 8          /* a workgroup per 64 queries whose 4 wavefronts split the keys (and, through a workspace,
                                   several workgroups per 64 queries: tcu_flash_attn_fwd_f16_ws): for launches with few
                                   query blocks; M % 64 == 0, N % 64 == 0, head size 128 with either V layout or 64 with a

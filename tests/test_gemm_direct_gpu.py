@@ -73,8 +73,8 @@ def test_gemm_tail_of_the_k_splitting_kernel(tcu, oracle, device, M, N, K, out_d
 @pytest.mark.parametrize("M,N,batch", [(32, 512, 520), (96, 1024, 260), (2080, 768, 16), (65536, 512, 1), (1600, 1024, 16), (288, 2048, 150)])
 @pytest.mark.parametrize("out_dtype", ["f32", "f16"])
 def test_b2b_streamed_weights(tcu, device, M, N, batch, out_dtype):
-    """AUTO's choice for long N and many rows: workgroups of 128 and 256 rows of which the last is partial, 8 to 32 blocks of
-    columns, many and few items. Against the kernel with 32 rows per workgroup, which the oracle's tests cover: the same f16
+    """AUTO for long N (its choice is the streaming kernel with (2080, 768, 16), (65536, 512, 1) and (1600, 1024, 16), the resident
+    one with the others): 8 to 32 blocks of columns, many and few items. Against the kernel with 32 rows per workgroup: the same f16
     intermediate up to the order of its f32 sums (an ulp of f16, 2^-11, in few elements), then f32 sums of N terms; a tenth of
     that for the whole."""
     import torch
@@ -110,3 +110,78 @@ def test_gemm_auto_takes_every_k(tcu, device, M, N):
     got = tcu.gemm(a, b, out_dtype=torch.float32)
     torch.cuda.synchronize()
     assert torch.equal(got, want) and bool(want.any())
+
+
+@pytest.mark.parametrize("M,N,batch,auto", [(32, 512, 520, False), (96, 1024, 260, False), (288, 2048, 150, False), (32, 512, 1, False),
+                                            (160, 4096, 3, False), (2080, 768, 16, True), (65536, 512, 1, True), (1600, 1024, 16, True),
+                                            (8128, 2048, 5, True)])
+@pytest.mark.parametrize("out_dtype", ["f32", "f16"])
+def test_b2b_stream_by_name(tcu, oracle, device, M, N, batch, auto, out_dtype):
+    """The weight-streaming kernel by name with workgroups of 128 rows (the first five, and 1600 x 16) and of 256, most or part of which
+    lie beyond M, rings of 8 to 64 blocks; against the oracle on the first and last rows of the first and last item, in the
+    tolerance of the other kernels' tests, with guard rows around the output. `auto`: this is AUTO's choice, bit for bit."""
+    import torch
+
+    print(f"b2b stream by name {M}x{N} batch {batch} {out_dtype}", flush=True)
+    dt = torch.float32 if out_dtype == "f32" else torch.float16
+    gen = torch.Generator(device=device)
+    gen.manual_seed(M + N)
+    normal = lambda *shape: torch.randn(*shape, generator=gen, device=device).mul_(0.1).half()
+    a, b, c = normal(batch, M, 128), normal(batch, N, 128), normal(batch, 128, N)
+    guard = torch.full((batch * M + 2, 128), -7.0, dtype=dt, device=device)
+    out = tcu.b2b_gemm(a, b, c, out=guard[1:-1].view(batch, M, 128), algo="stream")
+    torch.cuda.synchronize()
+    rows, items = sorted({*range(min(M, 40)), *range(max(0, M - 40), M)}), sorted({0, batch - 1})
+    pick = lambda t: np.ascontiguousarray(t[items].cpu().numpy())
+    want = oracle.b2b_gemm(np.ascontiguousarray(pick(a)[:, rows]), pick(b), pick(c))
+    assert oracle.max_rel_err(out[items][:, rows].float().cpu().numpy(), want, eps=1.0) <= REL_TOL
+    assert torch.all(guard[0] == -7.0) and torch.all(guard[-1] == -7.0)
+    if auto:
+        assert torch.equal(out, tcu.b2b_gemm(a, b, c, out_dtype=dt))
+
+
+@pytest.mark.parametrize("M,N,K", [(48, 2064, 304), (112, 1040, 80), (80, 4112, 592), (208, 2064, 1040)])
+@pytest.mark.parametrize("out_dtype", ["f32", "f16"])
+def test_gemm_direct_wide_tiles(tcu, oracle, device, M, N, K, out_dtype):
+    """The tiles of 32 x 16 (first two) and 64 x 32, which the shapes of the first test do not select, with partial last tiles."""
+    test_gemm_direct(tcu, oracle, device, M, N, K, out_dtype)
+
+
+@pytest.mark.parametrize("M,N,K", [(384, 448, 128), (112, 1600, 144), (3664, 640, 1472), (48, 11968, 1296), (2064, 48, 8208)])
+@pytest.mark.parametrize("out_dtype", ["f32", "f16"])
+def test_gemm_auto_around_the_direct_kernel(tcu, oracle, device, M, N, K, out_dtype):
+    """AUTO where its choice lies close to another kernel's: short K, one more round of tiles, tails of K with most of a tile beyond
+    M or N. Against the oracle on the first and last rows, and everywhere against the kernel without LDS."""
+    import torch
+
+    print(f"gemm auto {M}x{N}x{K} {out_dtype}", flush=True)
+    dt = torch.float32 if out_dtype == "f32" else torch.float16
+    A = oracle.fill_uniform(M * K, 31 + M).reshape(M, K)
+    Bt = oracle.fill_uniform(N * K, 37 + N).reshape(N, K)
+    a, b = torch.from_numpy(A).to(device), torch.from_numpy(Bt).to(device)
+    got = tcu.gemm(a, b, out_dtype=dt).float().cpu().numpy()
+    rows = sorted({*range(24), *range(M - 24, M)})
+    assert oracle.max_rel_err(got[rows], oracle.gemm(A[rows], Bt)) <= REL_TOL
+    assert oracle.max_rel_err(got, tcu.gemm(a, b, out_dtype=torch.float32, algo="ragged").cpu().numpy()) <= REL_TOL
+
+
+@pytest.mark.parametrize("M,N,K,splits", [(224, 352, 16384, 16), (192, 384, 16384, 32), (16, 32, 32768, 64), (464, 592, 8192, 8)])
+@pytest.mark.parametrize("out_dtype", ["f32", "f16"])
+def test_gemm_split_k_in_many_ranges(tcu, oracle, device, M, N, K, splits, out_dtype):
+    """Products that are split over K into 8 to 64 ranges rather than sent to the kernel of this file: the workspace's bytes past
+    the stated size stay untouched, those before it do not; against the oracle on 32 rows and the unsplit call."""
+    import torch
+
+    print(f"gemm split-K {M}x{N}x{K} {splits} {out_dtype}", flush=True)
+    dt = torch.float32 if out_dtype == "f32" else torch.float16
+    need = tcu.gemm_workspace_bytes(M, N, K)
+    assert need == splits * M * N * 4 and tcu.lib().tcu_gemm_uses_workspace(M, N, K)
+    A = oracle.fill_uniform(M * K, 131 + M).reshape(M, K)
+    Bt = oracle.fill_uniform(N * K, 137 + N).reshape(N, K)
+    a, b = torch.from_numpy(A).to(device), torch.from_numpy(Bt).to(device)
+    ws = torch.full((need + 4096,), 0xFF, dtype=torch.uint8, device=device)
+    got = tcu.gemm(a, b, out_dtype=dt, workspace=ws).float().cpu().numpy()
+    assert bool((ws[need:] == 0xFF).all()) and not bool((ws[:need] == 0xFF).all())
+    rows = sorted({*range(min(M, 16)), *range(M - 16, M)})
+    assert oracle.max_rel_err(got[rows], oracle.gemm(A[rows], Bt)) <= REL_TOL
+    assert oracle.max_rel_err(got, tcu.gemm(a, b, out_dtype=torch.float32, workspace=False).cpu().numpy()) <= REL_TOL

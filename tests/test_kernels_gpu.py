@@ -101,7 +101,7 @@ def test_gemm_wave128_shapes(tcu, oracle, device, M, N, K, out_dtype):
 def test_gemm_ragged_shapes(tcu, oracle, device, M, N, K, out_dtype):
     """Every shape made of whole 16 x 16 BaseTiles (the granularity of the reference's tile types,
     include/types/register.hpp:108-112) runs: blocks that hang over the edge in M, in N and in both, a last k-step of
-    16, one tile, a thin N; through AUTO (which must route them to the run-time-shape kernel) and by name. The output is
+    16, one tile, a thin N; through AUTO and with the run-time-shape kernel by name. The output is
     surrounded by a guard band that must stay untouched."""
     import torch
 
@@ -130,9 +130,9 @@ def test_gemm_ragged_shapes(tcu, oracle, device, M, N, K, out_dtype):
 def test_gemm_split_k_with_workspace(tcu, oracle, device, M, N, K, splits, out_dtype):
     """tcu_gemm_f16_ws: few output tiles and a long K are split over K (f32 partial products in the caller's workspace,
     then a reduction) where that is expected to beat the unsplit launch - the partial products from the kernel with
-    128 x 128 tiles whose wavefronts split K once more (first four cases, 1024 x 1024 x 8192, and - with edge tiles - the
-    three shapes that are not whole tiles) or, where those tiles alone fill the chip, from
-    the one with 256 x 256 tiles (2048 x 2048 x 32768); against the oracle and against the unsplit kernel; the workspace size is splits * M * N * 4, bytes past it stay untouched; shapes that are not split (last six
+    128 x 128 tiles whose wavefronts split K once more (the next three cases, and - with edge tiles - 752 x 1808 and 528 x 512) or,
+    where those tiles alone fill the chip, from the one with 256 x 256 tiles (2048 x 2048 x 32768); 256 x 256, 272 x 400 and 1024 x
+    1024 x 8192 have a split of their own, but run the kernel whose wavefronts split K without barriers, which is faster still; against the oracle and against the unsplit kernel; the workspace size is splits * M * N * 4, bytes past it stay untouched; shapes that are not split (last six
     cases: among them 2048 x 2048 x 8192 and 1536 x 1536 x 4096, where the kernel whose wavefronts split K inside the
     workgroup is the faster plan) take the ordinary path and need no workspace."""
     import torch
@@ -162,9 +162,9 @@ def test_gemm_split_k_with_workspace(tcu, oracle, device, M, N, K, splits, out_d
                                    (1040, 528, 272), (2064, 1040, 1072), (256, 256, 48), (4096, 4096, 144), (144, 208, 16)])
 @pytest.mark.parametrize("out_dtype", ["f32", "f16"])
 def test_gemm_edge_tiles(tcu, oracle, device, M, N, K, out_dtype):
-    """M, N, K multiples of 16 but not all of 64: AUTO runs the pipelined kernel with edge tiles (rows beyond the edge
-    loaded from the last valid row, stores guarded, the pieces of the last k-tile beyond K zeroed in LDS) in all three
-    tile sizes, with k tails of 16, 32 and 48 and a single partial k-tile; against the oracle on sampled rows including
+    """M, N, K multiples of 16 but not all of 64: AUTO runs a kernel with edge tiles, with most of these shapes the pipelined one (the
+    smallest go to the kernel whose wavefronts split K without barriers, 2064 x 1040 x 1072 to the one with 128 x 96 tiles). Rows
+    beyond the edge are loaded from the last valid row, stores guarded, the pieces of the last k-tile beyond K zeroed; with k tails of 16, 32 and 48 and a single partial k-tile; against the oracle on sampled rows including
     the last ones, against the run-time-shape kernel everywhere, with guard bands around the output."""
     import torch
 
@@ -1260,8 +1260,8 @@ def test_lstm_hoisted_rejects_what_it_cannot_do(tcu, device):
 @pytest.mark.parametrize("T,B,I,H", [(3, 16, 16, 16), (2, 48, 80, 112), (4, 32, 256, 64), (2, 64, 144, 272), (1, 80, 1024, 48)])
 @pytest.mark.parametrize("with_state", [False, True])
 def test_lstm_any_shape_of_whole_tiles(tcu, oracle, device, T, B, I, H, with_state):
-    """Every B, I, H in multiples of 16 runs (the granularity of the tile types): AUTO routes shapes no tuned kernel is
-    instantiated for to the run-time-shape step kernel; k ranges that end in a half-filled 32-wide operand tile, hidden
+    """Every B, I, H in multiples of 16 runs (the granularity of the tile types), through AUTO and with the run-time-shape step
+    kernel by name; k ranges that end in a half-filled 32-wide operand tile, hidden
     sizes that leave wavefronts of the last workgroup without work, batches that are not multiples of 64."""
     import torch
 

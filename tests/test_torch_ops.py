@@ -245,3 +245,38 @@ def test_gemm_b2b_lstm_ops(ops, tcu, oracle, device):
     h_ref, c_ref = oracle.lstm(x, W, b)
     assert oracle.max_abs_err(h.float().cpu().numpy(), h_ref) <= 1e-2
     assert oracle.max_abs_err(c.cpu().numpy(), c_ref) <= 1e-2
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("width", [1, 2, 3, 64, 511])
+def test_scatter_nd_add_to_fine_grained_memory(tcu, oracle, device, width):
+    """f16 additions into device memory that is not coarse-grained take the compare-and-swap kernel whatever the slice (packed
+    atomics are only used where the L2s carry them out). Duplicate rows of small integers: exact in any order. The allocation
+    lives until the process ends."""
+    import ctypes
+
+    tcu.lib()
+    hip = ctypes.CDLL("libamdhip64.so")
+    rng = np.random.default_rng(width)
+    rows, n = 37, 200
+    data = rng.integers(-8, 8, size=(rows, width)).astype(np.float16)
+    upd = rng.integers(-2, 3, size=(n, width)).astype(np.float16)
+    idx = rng.integers(-1, rows, size=(n, 1)).astype(np.int64)
+    mem = ctypes.c_void_p()
+    assert hip.hipExtMallocWithFlags(ctypes.byref(mem), ctypes.c_size_t(data.nbytes + 256), ctypes.c_uint(1)) == 0  # fine-grained
+    guard = np.full(data.nbytes + 256, 0x5A, dtype=np.uint8)
+    guard[:data.nbytes] = np.frombuffer(data.tobytes(), dtype=np.uint8)
+    assert hip.hipMemcpy(mem, guard.ctypes.data_as(ctypes.c_void_p), ctypes.c_size_t(guard.nbytes), 1) == 0
+    dims = (ctypes.c_longlong * 2)(rows, width)
+    u, i = torch.from_numpy(upd).to(device), torch.from_numpy(idx).to(device)
+    skipped = torch.zeros(1, dtype=torch.int32, device=device)
+    torch.cuda.synchronize()
+    assert tcu.lib().tcu_scatter_nd(mem, u.data_ptr(), i.data_ptr(), dims, 2, n, 1, tcu.TCU_DTYPE_F16, tcu.SCATTER_MODES["add"],
+                                    skipped.data_ptr(), torch.cuda.current_stream().cuda_stream) == 0
+    torch.cuda.synchronize()
+    out = np.empty_like(guard)
+    assert hip.hipMemcpy(out.ctypes.data_as(ctypes.c_void_p), mem, ctypes.c_size_t(out.nbytes), 2) == 0
+    want = oracle.scatter_nd(data, idx, upd, mode="add")
+    assert np.array_equal(np.frombuffer(out[:data.nbytes].tobytes(), dtype=np.float16).reshape(rows, width), want)
+    assert (out[data.nbytes:] == 0x5A).all()
+    assert int(skipped.item()) == int((idx[:, 0] < 0).sum())

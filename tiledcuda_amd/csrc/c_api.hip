@@ -752,15 +752,18 @@ int launch_b2b_tile_resident(const __half* A, const __half* B, const __half* C, 
                   Traits::kShmBytes, stream, A, B, C, D, M);
 }
 
-/// Wavefronts of the kernel that streams the weights past 32 rows per wavefront, or 0 where the one with 32 rows per workgroup
-/// is expected to be as fast (K = P = 128, N a multiple of 256). Both run rounds of one workgroup per CU; a round takes 1.85 us per
+/// Wavefronts of the kernel that streams the weights past 32 rows per wavefront, and whether AUTO runs it rather than the one with 32
+/// rows per workgroup (K = P = 128, N a multiple of 256). Both run rounds of one workgroup per CU; a round takes 1.85 us per
 /// 256 columns + 1.7 with 32 rows, per 64 columns 1.65 us + 5.5 with 256 rows (8 wavefronts), 1.3 us + 5 with 128 (4).
-int b2b_stream_waves(int M, int N, int batch) {
+struct B2bStreamPlan {
+    int waves;
+    bool is_the_choice;
+};
+B2bStreamPlan b2b_stream_plan(int M, int N, int batch) {
     const auto rounds = [&](int rows) { return double(((long)((M + rows - 1) / rows) * batch + 255) / 256); };
     const double resident = rounds(32) * (1.85 * (N / 256) + 1.7);
     const double eight = rounds(256) * (1.65 * (N / 64) + 5.5), four = rounds(128) * (1.3 * (N / 64) + 5.0);
-    if (std::min(eight, four) >= 0.93 * resident || N >= (1 << 23)) return 0;
-    return eight <= four ? 8 : 4;
+    return {eight <= four ? 8 : 4, std::min(eight, four) < 0.93 * resident};
 }
 
 template <int kWaves, typename OutType>
@@ -775,7 +778,7 @@ template <typename OutType>
 int b2b_dispatch(const __half* A, const __half* B, const __half* C, OutType* D, int M, int N, int K, int P, int batch,
                  int algo, hipStream_t stream) {
     if (algo != TCU_B2B_AUTO && algo != TCU_B2B_TILE_LIBRARY && algo != TCU_B2B_RESIDENT && algo != TCU_B2B_ROWS &&
-        algo != TCU_B2B_TILE_RESIDENT)
+        algo != TCU_B2B_TILE_RESIDENT && algo != TCU_B2B_STREAM)
         return fail(TCU_ERR_INVALID_ARGUMENT, "tcu_b2b_gemm_f16: unknown algo");
     if (algo == TCU_B2B_TILE_RESIDENT) {
         // the LDS-resident kernel composed from tile-library functors: compile-time N, like every tile-API kernel
@@ -804,10 +807,15 @@ int b2b_dispatch(const __half* A, const __half* B, const __half* C, OutType* D, 
             return fail(TCU_ERR_UNSUPPORTED_SHAPE, "the many-rows b2b kernel takes N = 256, K = P = 128 and M a multiple of 64");
     }
     // long N and many rows: the weights pass once for 128 or 256 rows
-    if (algo == TCU_B2B_AUTO && N % 256 == 0 && N > 256 && K == 128 && P == 128 && M % 32 == 0) {
-        const int waves = b2b_stream_waves(M, N, batch);
-        if (waves == 8) return launch_b2b_stream<8>(A, B, C, D, M, N, batch, stream);
-        if (waves == 4) return launch_b2b_stream<4>(A, B, C, D, M, N, batch, stream);
+    if (algo == TCU_B2B_STREAM || algo == TCU_B2B_AUTO) {
+        if (N % 256 == 0 && N > 256 && N < (1 << 23) && K == 128 && P == 128 && M % 32 == 0) {
+            const B2bStreamPlan plan = b2b_stream_plan(M, N, batch);
+            if (algo == TCU_B2B_STREAM || plan.is_the_choice)
+                return plan.waves == 8 ? launch_b2b_stream<8>(A, B, C, D, M, N, batch, stream) : launch_b2b_stream<4>(A, B, C, D, M, N, batch, stream);
+        }
+        if (algo == TCU_B2B_STREAM)
+            return fail(TCU_ERR_UNSUPPORTED_SHAPE, "the weight-streaming b2b kernel takes K = P = 128, N a multiple of 256 from 512 to "
+                                                   "2^23 and M a multiple of 32");
     }
     if (algo != TCU_B2B_TILE_LIBRARY) {
         if (N % 256 == 0 && K == 128 && P == 128 && M % 32 == 0)
