@@ -175,7 +175,8 @@ __global__ void __launch_bounds__(T::kThreads)
     // Every phase is the same straight-line code: behind the last tile of K the fragment reads fetch stale data that
     // nobody uses and the loads fetch the last tile once more (clamped index) - cheaper than peeled copies of the
     // phase, whose control-flow merges made the compiler shuffle and spill accumulators between the assembly
-    // statements, where it knows of no wait states.
+    // statements, where it knows of no wait states. (kTail has a branch at the top of a phase: it writes fragments only, and the
+    // listing of these instantiations has neither spills nor accumulator moves in the loop.)
     auto tile = [&](int kt, f16x8 (&cur)[T::kFrags], f16x8 (&nxt)[T::kFrags]) {
         unsigned int read_a = frag_lane + slot_bytes(2 * kt + 2), read_b = frag_lane + slot_bytes(2 * kt + 3);  // tile kt + 1
         asm volatile("" : "+v"(read_a), "+v"(read_b));  // (these two sums, not one per fragment)

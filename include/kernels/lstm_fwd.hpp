@@ -30,10 +30,9 @@
 
 namespace tiledcuda::kernels {
 
-template <const int kI_, const int kH_, const int kStages_ = 5>
+template <const int kStages_ = 5>
 struct LstmFwdTraits {
-    static constexpr int kI = kI_, kH = kH_, kStages = kStages_;
-    static constexpr int kKK = kI + kH;
+    static constexpr int kStages = kStages_;
     static constexpr int kTM = 64;   // batch rows per workgroup
     static constexpr int kTH = 16;   // hidden units per workgroup (x 4 gates = 64 weight rows)
     static constexpr int kBK = 128;  // k-columns per stage: 256 contiguous bytes per row and request
@@ -45,10 +44,7 @@ struct LstmFwdTraits {
     static constexpr int kStageBytes = 2 * kTileBytes;             // 32 KiB
     static constexpr int kLoadsPerWave = 4;                        // 32 one-KiB instructions per stage / 8 wavefronts
     static constexpr int kLdsBytes = kStages * kStageBytes;
-    // kI == kH == 0: the sizes are kernel arguments (I % 128 == 0, H % 128 == 0, checked by the launcher)
-    static constexpr bool kRuntimeShape = kI == 0 && kH == 0;
-    static_assert(kI % kBK == 0 && kH % kBK == 0 && kH % kTH == 0);
-    static_assert((kH / kTH) % 8 == 0, "the workgroup map deals hidden tiles to the 8 XCDs");
+    static_assert(kBK / kTH % 8 == 0, "the workgroup map deals hidden tiles to the 8 XCDs");
     static_assert(kStages >= 2 && (kStages - 2) * kLoadsPerWave <= 63, "vmcnt is a 6-bit counter");
     static_assert(kLdsBytes <= kMaxLdsBytes);
 };
@@ -70,15 +66,14 @@ DEVICE void wait_vmcnt_lgkm0() {
 /// kHoisted: the input half of the gates, x_t · W[:, :I]ᵀ, was computed beforehand for the whole sequence (one large
 /// GEMM) and is passed as pre_t [B, 4H] f32; the step then streams only h_{t-1} and W[:, I:] (half the bytes) and x_t
 /// is not read.
-/// I, H: the sizes, used by LstmFwdTraits<0, 0> (any multiples of 128); the other instantiations have them as constants.
+/// I, H: any multiples of 128 (checked by the launcher).
 template <typename Traits, bool kHoisted = false>
 __global__ void __launch_bounds__(Traits::kThreads)
     lstm_cell_fwd(const __half* __restrict__ x_t, const __half* __restrict__ h_in, const __half* __restrict__ W,
                   const __half* __restrict__ bias, const float* c_in, float* c_out, __half* __restrict__ h_out,
                   int B, const float* __restrict__ pre_t, int I, int H) {
     constexpr int kBK = Traits::kBK;
-    const int kI = Traits::kRuntimeShape ? I : Traits::kI, kH = Traits::kRuntimeShape ? H : Traits::kH;
-    const int kKK = kI + kH;
+    const int KK = I + H;
     constexpr int S = Traits::kStages, L = Traits::kLoadsPerWave;
     extern __shared__ __align__(1024) unsigned char lds[];
 
@@ -101,8 +96,8 @@ __global__ void __launch_bounds__(Traits::kThreads)
     // 32 wn + 8 gate + jj is weight row gate * H + hid0 + 8 wn + jj. Wavefront w issues t = 4 w .. 4 w + 3.
     // Physical 16-byte chunk p of row r holds logical chunk p ^ (r % 16).
     const int lrow = lane >> 4, lchk = lane & 15;
-    const int k_begin = kHoisted ? kI : 0;
-    const int k_end = h_in ? kKK : kI;
+    const int k_begin = kHoisted ? I : 0;
+    const int k_end = h_in ? KK : I;
     const int ktiles = (k_end - k_begin) / kBK;
     auto issue_stage = [&](int stage, int kt) {
         const int k0 = k_begin + kt * kBK;
@@ -114,11 +109,11 @@ __global__ void __launch_bounds__(Traits::kThreads)
             const int chunk = lchk ^ (row & 15);
             const __half* src;
             if (t < 16) {
-                src = k0 < kI ? x_t + size_t(row0 + row) * kI + k0 + chunk * 8
-                              : h_in + size_t(row0 + row) * kH + (k0 - kI) + chunk * 8;
+                src = k0 < I ? x_t + size_t(row0 + row) * I + k0 + chunk * 8
+                              : h_in + size_t(row0 + row) * H + (k0 - I) + chunk * 8;
             } else {
-                const int wrow = ((row >> 3) & 3) * kH + hid0 + 8 * (row >> 5) + (row & 7);
-                src = W + size_t(wrow) * kKK + k0 + chunk * 8;
+                const int wrow = ((row >> 3) & 3) * H + hid0 + 8 * (row >> 5) + (row & 7);
+                src = W + size_t(wrow) * KK + k0 + chunk * 8;
             }
             detail::load_lds_16B_untracked(src, sbase + t * 1024);
         }
@@ -138,11 +133,11 @@ __global__ void __launch_bounds__(Traits::kThreads)
     f16x4 bias_v[4];
     f32x4 pre_v[4];
     if (group == 0) {
-        if (c_in) c_prev = *reinterpret_cast<const f32x4*>(c_in + size_t(b) * kH + hid);
+        if (c_in) c_prev = *reinterpret_cast<const f32x4*>(c_in + size_t(b) * H + hid);
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
-            bias_v[g] = *reinterpret_cast<const f16x4*>(bias + g * kH + hid);
-            if constexpr (kHoisted) pre_v[g] = *reinterpret_cast<const f32x4*>(pre_t + size_t(b) * (4 * kH) + g * kH + hid);
+            bias_v[g] = *reinterpret_cast<const f16x4*>(bias + g * H + hid);
+            if constexpr (kHoisted) pre_v[g] = *reinterpret_cast<const f32x4*>(pre_t + size_t(b) * (4 * H) + g * H + hid);
         }
     }
 
@@ -227,8 +222,8 @@ __global__ void __launch_bounds__(Traits::kThreads)
         c_new[e] = cn;
         h_new[e] = static_cast<_Float16>(detail::sigmoid_fast(go) * detail::tanh_fast(cn));
     }
-    *reinterpret_cast<f32x4*>(c_out + size_t(b) * kH + hid) = c_new;
-    *reinterpret_cast<f16x4*>(h_out + size_t(b) * kH + hid) = h_new;
+    *reinterpret_cast<f32x4*>(c_out + size_t(b) * H + hid) = c_new;
+    *reinterpret_cast<f16x4*>(h_out + size_t(b) * H + hid) = h_new;
 }
 
 }  // namespace tiledcuda::kernels

@@ -1323,7 +1323,7 @@ int launch_lstm_hoisted(const __half* x, const __half* W, const __half* bias, co
     }
     if (rc != TCU_OK) return rc;
     if (lstm_direct_takes(B, I, H)) return launch_lstm_direct<true>(x, W, bias, h0, c0, h_all, c_out, T, B, I, H, pre, stream);
-    using Traits = LstmFwdTraits<0, 0>;
+    using Traits = LstmFwdTraits<>;
     auto kernel = &lstm_cell_fwd<Traits, true>;
     const int grid = (B / Traits::kTM) * (H / Traits::kTH);
     for (int t = 0; t < T; ++t) {
@@ -1357,7 +1357,7 @@ int launch_lstm_ragged(const __half* x, const __half* W, const __half* bias, con
 
 int launch_lstm_fwd(const __half* x, const __half* W, const __half* bias, const __half* h0, const float* c0, __half* h_all,
                     float* c_out, int T, int B, int I, int H, hipStream_t stream) {
-    using Traits = LstmFwdTraits<0, 0>;
+    using Traits = LstmFwdTraits<>;
     auto kernel = &lstm_cell_fwd<Traits>;
     const int grid = (B / Traits::kTM) * (H / Traits::kTH);
     for (int t = 0; t < T; ++t) {
