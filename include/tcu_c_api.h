@@ -33,8 +33,9 @@ typedef enum { TCU_DTYPE_F32 = 0, TCU_DTYPE_F16 = 1 } tcu_dtype;
  * disjoint parts of C, bit for bit the result of one launch) when M or N lie a little above such multiples and that
  * saves a round of workgroups; WAVE128 on the leading rows or columns that fill whole rounds of 256 workgroups plus a
  * kernel with smaller tiles (WAVE128_KSPLIT, WAVE128_NARROW or PIPELINED) on the rest of C when the last round would be
- * far from full (2560 x 8192: 320 tiles); WAVE128_KSPLIT and WAVE128_NARROW as described below; DIRECT for products with few output tiles, where a cost model
- * expects it to be the shorter launch; else PIPELINED. Every shape made of whole 16 x 16
+ * far from full (2560 x 8192: 320 tiles); WAVE128_KSPLIT and WAVE128_NARROW as described below; DIRECT wherever a cost model
+ * expects it to be the shorter launch (few output tiles); RAGGED for outputs below 64 x 64 with K <= 48 or K >= 2^24; else
+ * PIPELINED. Every shape made of whole 16 x 16
  * BaseTiles (M, N, K multiples of 16), the granularity of the reference's tile types, is accepted. */
 typedef enum {
     TCU_GEMM_AUTO = 0,
@@ -61,7 +62,7 @@ typedef enum {
     TCU_GEMM_WAVE128_KSPLIT = 8, /* 128 x 128 tile (128 x 96 where that fills the GPU better) on 4 wavefronts (one per SIMD)
                                 that each own the whole tile over a quarter of every 128-wide step of K, partial tiles
                                 added through LDS: for products with too few 256 x 256 tiles to fill the GPU (2048^3,
-                                1552 x 1552 x 4096); K a multiple of 128 (AUTO runs it with a tail in K, any multiple of 16, too),
+                                1552 x 1552 x 4096); K a multiple of 128 (AUTO runs it with a tail in K, any multiple of 16, too, where M and N exceed 64),
                                 M and N multiples of 16 (edge tiles: rows clamped, stores guarded); the sum over K is
                                 taken in four interleaved parts (differs from the other kernels by f32 rounding) */
     /* (10 is not assigned) */
@@ -104,11 +105,11 @@ typedef enum {
     TCU_V_ROW_MAJOR = 1  /* V stored [N, P] per batch item: the usual [seq, head_dim] */
 } tcu_v_layout;
 
-/* Which attention kernel to run (tcu_flash_attn_fwd_f16_algo). For a row-major V, AUTO picks WAVE64_K32 with at least 256
- * whole blocks of 256 queries and N >= 320 (192 with N >= 1024), at head size 128 also WAVE64 with 128 to 191 such blocks
- * and N >= 1024, and otherwise KEYS or MFMA32_FUSED, whichever a cost model expects to be the shorter; for a column-major V
- * (head size 128) AUTO picks WAVE64_K32 under the same conditions and KEYS or WAVE64 otherwise (both take every
- * M % 64 == 0 and N % 64 == 0). */
+/* Which attention kernel to run (tcu_flash_attn_fwd_f16_algo). AUTO picks the kernel with the shortest expected time among KEYS
+ * and, for a row-major V, WAVE64_K32 (with at least 256 whole blocks of 256 queries and N >= 320, or 192 and N >= 1024, unless
+ * MFMA32_FUSED is expected to be clearly shorter), at head size 128 also WAVE64 (128 to 191 such blocks and N >= 1024), and
+ * MFMA32_FUSED otherwise; for a column-major V (head size 128) WAVE64_K32 under the same conditions and WAVE64 otherwise (it
+ * takes every M % 64 == 0 and N % 64 == 0). */
 typedef enum {
     TCU_ATTN_AUTO = 0,
     TCU_ATTN_TILE_LIBRARY = 1, /* composed from the 16x16 tile primitives, like the reference kernel */
