@@ -53,10 +53,10 @@ __global__ void __launch_bounds__(T::kThreads)
     // one column block together whatever M and N: 4096 x 256 x 8192 41.4 us, 2048 x 256 x 8192 40.0, 8192 x 64 x 4096 21.1; in
     // this order 25.9, 18.8, 13.7.)
     const int m_blocks = (M + T::kBM - 1) / T::kBM, n_blocks = (N + T::kBN - 1) / T::kBN;
-    int n_block, m_block;
-    if (M > N) detail::xcd_head_block(n_blocks, m_blocks, m_block, n_block);
-    else detail::xcd_head_block(m_blocks, n_blocks, n_block, m_block);
-    const int n0 = n_block * T::kBN, m0 = m_block * T::kBM;
+    const bool tall = M > N;
+    int larger, smaller;
+    detail::xcd_head_block(tall ? n_blocks : m_blocks, tall ? m_blocks : n_blocks, larger, smaller);
+    const int n0 = (tall ? smaller : larger) * T::kBN, m0 = (tall ? larger : smaller) * T::kBM;
     const __half* const b_rows = Bt + size_t(n0) * K;
     const __half* const a_rows = A + size_t(m0) * K;
 
