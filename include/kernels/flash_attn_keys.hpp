@@ -259,7 +259,7 @@ __global__ void __launch_bounds__(Traits::kThreads, Traits::kGroupsPerCu)
         // Every score of block 0 may be -infinity (keys masked by an infinite feature; any of 4 * splits blocks of the sequence
         // is some wavefront's block 0): then the exact maximum of this wavefront's first block with another score, its keys
         // read once more, is where the query starts. A query without any starts at 0 and keeps a sum of 0.
-        if (__any(m_run[0] == -INFINITY || m_run[1] == -INFINITY)) {
+        if (__builtin_expect(__any(m_run[0] == -INFINITY || m_run[1] == -INFINITY), 0)) {
             for (int j = 1; j < nb; ++j) {
                 const __half* k_row = Kh + (size_t(b_first + wave + j * Traits::kWaves) * Traits::kBN + krow) * kD + 8 * h;
 #pragma unroll
