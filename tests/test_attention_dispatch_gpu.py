@@ -226,3 +226,21 @@ def test_captured_calls_allocate_nothing(tcu, oracle, device, entry):
         torch.cuda.synchronize()
         assert torch.equal(plain, unsplit)
         assert entry != "python" or torch.equal(own, split)
+
+
+@pytest.mark.parametrize("batch,N,algo", [(85, 2368, "keys"), (88, 1600, "keys"), (88, 4160, "wave64"), (96, 2368, "wave64")])
+def test_192_queries_and_a_column_major_v(tcu, device, batch, N, algo):
+    """Three workgroups per head split the keys until they need a second round of any size; then AUTO takes blocks of 256
+    queries, one per head. Bit for bit the kernel by name, which the other differs from by the order of its sums."""
+    import torch
+
+    print(f"attention b{batch} 192x{N} D128 V col {algo}", flush=True)
+    gen = torch.Generator(device=device)
+    gen.manual_seed(N)
+    q, k, v = (torch.randn(batch * n * 128, generator=gen, device=device).half() for n in (192, N, N))
+    outs = {}
+    for name in ("auto", "keys", "wave64"):
+        outs[name] = torch.empty_like(q)
+        tcu.flash_attention_fwd(q, k, v, outs[name], 192, N, 128, 128, scale=128 ** -0.5, batch=batch, algo=name)
+    assert torch.equal(outs["auto"], outs[algo])
+    assert not torch.equal(outs["keys"], outs["wave64"])

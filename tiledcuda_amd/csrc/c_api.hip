@@ -1107,6 +1107,11 @@ int attn_keys_plan(int batch, int M, int N, int D, int v_layout, int max_splits)
     if ((D != 128 && !(D == 64 && v_layout == TCU_V_ROW_MAJOR)) || N >= (1 << 24)) return 0;
     const long groups = (long)batch * (M / 64);
     if (groups > 4096) return 0;
+    // 192 queries, a column-major V, more workgroups than CUs: blocks of 256 queries, whose fourth wavefront idles, need one round
+    // per 256 heads (us, key-splitting against blocks: 96 x 192 x 2368: 61.3, 53; 110 x 192 x 4096: 99, 85; 128 x 192 x 10240:
+    // 263, 210), unless the second round has a few workgroups only and not too many keys (88 x 192 x 1600: 34.4, 36.6; x 4096: 80,
+    // 84; x 10240: 230, 199)
+    if (D == 128 && M == 192 && v_layout == TCU_V_COL_MAJOR && (groups > 272 || (groups > 256 && N > 4096))) return 0;
     double best_us = 1e30;
     int best = 0;
     for (int s : {1, 2, 3, 4, 6, 8, 12, 16}) {
