@@ -1225,7 +1225,10 @@ bool lstm_direct_takes(int B, int I, int H) {
 
 /// Tile of that kernel (16-row tiles of weights x of the batch) for a step over `columns` columns: rounds of one workgroup per
 /// CU, each as long as its rows take to arrive (95 KB per us and CU) plus 0.1 us per 16 x 16 tile for the sums of the eight
-/// wavefronts. Measured, us per step with 1x1, 2x1, 2x2, 4x1, 4x2, 4x4 tiles: B 80, I 336, H 656: 6.5, 6.1, 4.5, 4.6, 5.2, 6.9;
+/// wavefronts and 0.8 us whatever the tile, without which a short sum got many rounds of small tiles (66 sizes with all seven
+/// tiles: on average 0.7 % from the best of them, 3.8 before; 1x1, 2x2, 4x4: 768 x 256 and 256 columns, as with a projection:
+/// 14.1, 8.1, 6.0; 384 x 128, 128: 5.8, 4.1, 5.5; 1568 x 176, 400 columns: 16.4, 11.9, 9.2, 4x1 8.5). Measured, us per step with
+/// 1x1, 2x1, 2x2, 4x1, 4x2, 4x4 tiles: B 80, I 336, H 656: 6.5, 6.1, 4.5, 4.6, 5.2, 6.9;
 /// 16, 1024, 1024: 3.9, 4.4, 4.9, 5.4, 6.1, 7.9; 64, 1024, 1024: 8.8, 8.2, 5.7, 5.8, 6.7, 8.9; 240, 368, 592: 12.1, 12.8,
 /// 10.0, 8.5, 9.0, 7.4; 256, 1024, 1024: 28, 28, 18, 18, 14, 9.7.
 struct LstmTilePlan {
@@ -1237,7 +1240,7 @@ LstmTilePlan lstm_direct_plan(int B, int H, int columns) {
     for (const auto& [ut, rt] : {std::pair{1, 1}, std::pair{1, 2}, std::pair{2, 1}, std::pair{2, 2}, std::pair{4, 1},
                                  std::pair{4, 2}, std::pair{4, 4}}) {
         const long groups = (long)((H + 4 * ut - 1) / (4 * ut)) * ((B + 16 * rt - 1) / (16 * rt));
-        const double us = double((groups + 255) / 256) * (0.1 * ut * rt + 32.0 * (ut + rt) * columns / 95e3);
+        const double us = double((groups + 255) / 256) * (0.8 + 0.1 * ut * rt + 32.0 * (ut + rt) * columns / 95e3);
         if (us < plan.us) plan = {ut, rt, us};
     }
     return plan;
@@ -1303,7 +1306,8 @@ double lstm_step_us(int B, int H, int columns) {
 /// 0.37 us per MB), and a step is left with H of its I + H columns. Both plans within 12 % of the measured times of most of
 /// 133 sizes; us, a fused kernel per step against this: T 8, B 64, I 8192, H 4096: 710, 364; 2048, 4096, 256: 378, 198; 1024, 4096,
 /// 512: 286, 197; T 16, B 256, I 4096, H 1024: 317, 237; 256, 2048, 1024: 210, 183; 256, 1024, 1024: 151, 157; T 8, B 512, I
-/// 512, H 1024: 118, 138. The chosen plan was at most 7 % longer than the other.
+/// 512, H 1024: 118, 138. Of 115 more sizes the chosen plan is within 3 % of the shorter for 108, at most 14 % above it
+/// (T 4, B 1472, I 1280, H 128: 41, 36).
 bool lstm_projection_pays(int T, int B, int I, int H) {
     if (tcu_lstm_workspace_bytes(T, B, I, H) == 0 || I < 512 || T < 4 || (long)T * B > INT_MAX) return false;
     if (!lstm_direct_takes(B, I, H)) return true;  // (the streaming step kernel: half of its bytes are W[:, :I])
