@@ -244,3 +244,22 @@ def test_192_queries_and_a_column_major_v(tcu, device, batch, N, algo):
         tcu.flash_attention_fwd(q, k, v, outs[name], 192, N, 128, 128, scale=128 ** -0.5, batch=batch, algo=name)
     assert torch.equal(outs["auto"], outs[algo])
     assert not torch.equal(outs["keys"], outs["wave64"])
+
+
+def _auto_is(tcu, device, batch, M, N, algo):
+    import torch
+
+    print(f"attention auto b{batch} {M}x{N} D64 {algo}", flush=True)
+    gen = torch.Generator(device=device)
+    gen.manual_seed(M)
+    q, k, v = (torch.randn(batch, n, 64, generator=gen, device=device).half() for n in (M, N, N))
+    named = {name: tcu.flash_attention(q, k, v, algo=name) for name in ("keys", "mfma32_fused", "wave64_k32")}
+    got = tcu.flash_attention(q, k, v)
+    assert [name for name, out in named.items() if torch.equal(got, out)] == [algo]
+
+
+@pytest.mark.parametrize("batch,M,N,algo", [(84, 576, 2688, "keys"), (104, 448, 2560, "keys"), (62, 640, 704, "mfma32_fused")])
+def test_blocks_partly_beyond_the_queries_against_split_keys(tcu, device, batch, M, N, algo):
+    """One block of 256 queries per CU, the last of a head partly empty: AUTO counts what that costs when it looks at the
+    key-splitting kernel. Bit for bit the kernel by name."""
+    _auto_is(tcu, device, batch, M, N, algo)

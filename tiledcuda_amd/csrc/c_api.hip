@@ -970,6 +970,7 @@ struct AttnWavesPlan {
     int waves;
     double us;
     long groups;
+    double partial_us;  // head size 64: with the 6 % of blocks partly beyond M, which measure 2 to 8 % above us
 };
 AttnWavesPlan attn_waves_plan(int batch, int M, int N, int D) {
     struct Cost {
@@ -1071,7 +1072,8 @@ double attn_w64_us(int batch, int M, int N, int D) {
     const double fill = double(items) / (256.0 * rounds);
     return 1.3 + rounds * (D == 128 ? 6.0 + N * (0.02 + 0.005 * fill) : 4.0 + N * (0.0135 + 0.0043 * fill));
 }
-double attn_fused_us(int batch, int M, int N, int D) { return attn_waves_plan(batch, M, N, D).us; }
+/// (with blocks partly beyond M dearer: 104 x 448 x 2560 at head size 64: 44.8 us, the key-splitting kernel 38.8; 84 x 576 x 2688: 54, 43)
+double attn_fused_us(int batch, int M, int N, int D) { return attn_waves_plan(batch, M, N, D).partial_us; }
 
 /// Whether AUTO's choice among the kernels that give wavefronts their own queries is the 16x16x32 one: from 256 whole blocks of
 /// 256 queries on (192 with N >= 1024), unless a last round of few blocks makes it longer than the 32-queries-per-wavefront
