@@ -263,3 +263,10 @@ def test_blocks_partly_beyond_the_queries_against_split_keys(tcu, device, batch,
     """One block of 256 queries per CU, the last of a head partly empty: AUTO counts what that costs when it looks at the
     key-splitting kernel. Bit for bit the kernel by name."""
     _auto_is(tcu, device, batch, M, N, algo)
+
+
+@pytest.mark.parametrize("batch,M,N,algo", [(142, 3392, 448, "wave64_k32"), (134, 1856, 384, "mfma32_fused")])
+def test_many_rounds_of_query_blocks(tcu, device, batch, M, N, algo):
+    """More than three rounds of blocks of 256 queries that are not whole: AUTO runs the 16x16x32 kernel unless its estimate is
+    far behind. Bit for bit the kernel by name."""
+    _auto_is(tcu, device, batch, M, N, algo)

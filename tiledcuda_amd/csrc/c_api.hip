@@ -978,7 +978,7 @@ AttnWavesPlan attn_waves_plan(int batch, int M, int N, int D) {
         double round128, start128;               // head size 128: rounds of one workgroup per CU
         double one, second, third, next, start;  // head size 64, by the number of workgroups per CU
     };
-    AttnWavesPlan plan{8, 1e30, 0};
+    AttnWavesPlan plan{8, 1e30, 0, 1e30};
     double best = 1e30;
     for (const Cost& c : {Cost{2, 1.0, 2.6, 1.0, 0.36, 0.41, 0.43, 2.1}, Cost{4, 1.05, 3.2, 0.985, 0.415, 0.808, 0.573, 2.45},
                           Cost{8, 1.15, 3.2, 1.05, 1.13, 1.12, 1.11, 3.05}}) {
@@ -997,7 +997,7 @@ AttnWavesPlan attn_waves_plan(int batch, int M, int N, int D) {
         }
         if (score < best) {
             best = score;
-            plan = {c.waves, us, groups};
+            plan = {c.waves, us, groups, D == 128 ? us : score};
         }
     }
     return plan;
@@ -1079,13 +1079,18 @@ double attn_fused_us(int batch, int M, int N, int D) { return attn_waves_plan(ba
 /// 256 queries on (192 with N >= 1024), unless a last round of few blocks makes it longer than the 32-queries-per-wavefront
 /// kernel (22 x 2944^2 at head size 64, 264 blocks: 99.8 against 76.3 us; a column-major V has no such alternative). Where that one
 /// runs 8 wavefronts it has to promise 10 % (128 x 1024 x 448 at 64, 8 % ahead in the model: 24.2 against 23.0; 716 x 256 x 320: 31.5
-/// against 28.1), else 5 (144 x 512 x 448, 7 %: 20.5 against 22.7; 88 x 832 x 320, 12 %: 16.3 against 18.8).
+/// against 28.1), else 5 (144 x 512 x 448, 7 %: 20.5 against 22.7; 88 x 832 x 320, 12 %: 16.3 against 18.8). More than three rounds of
+/// blocks at 64 run at the power limit, where this kernel's fewer instructions count for more than its estimate says: there it may be
+/// 18 % behind (509 x 3264 x 576, 6 %: 322 against 367 us; 458 x 576 x 1152, 23 %: 129, 129; 94 x 3456 x 320, 22 %: 49, 44; with 5 %
+/// as below three rounds 39 such sizes were up to 19 % above the shorter of the two, so 1 %).
 bool attn_k32_is_the_choice(int batch, int M, int N, int D, int v_layout) {
     const long blocks = (long)batch * (M / 256);
     if (N < 320 || !(blocks >= 256 || (blocks >= 192 && N >= 1024))) return false;
     if (v_layout == TCU_V_COL_MAJOR) return true;
     const AttnWavesPlan other = attn_waves_plan(batch, M, N, D);
-    return attn_w64_us(batch, M, N, D) <= (other.waves == 8 ? 1.1 : 1.05) * other.us;
+    const long items = (long)batch * ((M + 255) / 256);
+    const double margin = other.waves == 8 ? 1.1 : D == 64 && items > 3 * 256 ? 1.18 : 1.05;
+    return attn_w64_us(batch, M, N, D) <= margin * other.us;
 }
 
 /// Whether it is the 32x32x16 kernel with 64 queries per wavefront (row-major V).
