@@ -365,7 +365,7 @@ def lstm(x: torch.Tensor, W: torch.Tensor, bias: torch.Tensor, h0: torch.Tensor 
         if check:
             lstm_persistent_status(workspace)
         return h_all, c_out
-    # (T < 4 or I < 512 never uses one: 0.15 us a call for not asking)
+    # (T < 4 or I < 512 never uses one; asking costs 0.5 us)
     if algo == "auto" and T >= 4 and I >= 512 and workspace is not False and x.is_cuda and lib().tcu_lstm_uses_workspace(T, B, I, H):
         algo = "hoisted"  # a long input size: its half of the gates is cheaper as one GEMM over all steps
     if algo == "hoisted":
