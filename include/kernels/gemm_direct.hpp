@@ -38,16 +38,20 @@ struct GemmDirectTraits {
     static_assert(kLdsBytes <= kMaxLdsBytes);
 };
 
-/// grid = ceil(N / kBN) * ceil(M / kBM), block = 512, dynamic LDS = T::kLdsBytes. M, N, K multiples of 16, K < 2^24 (32-bit
-/// byte offsets inside a tile's rows).
+/// grid = ceil(N / kBN) * ceil(M / kBM), block = 512, dynamic LDS = T::kLdsBytes. M, N, K multiples of 16, K and ldb (the
+/// distance of B's stored rows, in elements) < 2^24 (32-bit byte offsets inside a tile's rows). zero_words / zero_count: device
+/// words that the first workgroup sets to zero on the side (null / 0: none).
 template <typename T, typename OutType>
 __global__ void __launch_bounds__(T::kThreads)
-    gemm_direct(const __half* __restrict__ A, const __half* __restrict__ Bt, OutType* __restrict__ C, int M, int N, int K) {
+    gemm_direct(const __half* __restrict__ A, const __half* __restrict__ Bt, OutType* __restrict__ C, int M, int N, int K, int ldb,
+                unsigned int* __restrict__ zero_words, int zero_count) {
     constexpr int kUT = T::kUT, kRT = T::kRT, kRing = T::kRing, kBK = T::kBK, kWaves = T::kWaves;
     extern __shared__ __align__(1024) unsigned char lds[];
     const int lane = lane_id();
     const int wave = __builtin_amdgcn_readfirstlane(wave_id());
     const int line = lane & 15, group = lane >> 4;
+    if (zero_count > 0 && blockIdx.x == 0)
+        for (int i = threadIdx.x; i < zero_count; i += T::kThreads) zero_words[i] = 0u;
 
     // The blocks that share rows of the larger operand run on one XCD: these rows come to one L2 only. (With the row blocks of
     // one column block together whatever M and N: 4096 x 256 x 8192 41.4 us, 2048 x 256 x 8192 40.0, 8192 x 64 x 4096 21.1; in
@@ -57,7 +61,7 @@ __global__ void __launch_bounds__(T::kThreads)
     int larger, smaller;
     detail::xcd_head_block(tall ? n_blocks : m_blocks, tall ? m_blocks : n_blocks, larger, smaller);
     const int n0 = (tall ? smaller : larger) * T::kBN, m0 = (tall ? larger : smaller) * T::kBM;
-    const __half* const b_rows = Bt + size_t(n0) * K;
+    const __half* const b_rows = Bt + size_t(n0) * ldb;
     const __half* const a_rows = A + size_t(m0) * K;
 
     // ---- global -> LDS: instruction q of a chunk fills 8 rows of 128 bytes, those of B before those of A (rows beyond the
@@ -65,7 +69,7 @@ __global__ void __launch_bounds__(T::kThreads)
     const int lrow = lane >> 3;
     unsigned b_off[2 * kUT], a_off[2 * kRT];
 #pragma unroll
-    for (int q = 0; q < 2 * kUT; ++q) b_off[q] = min(8 * q + lrow, N - 1 - n0) * (2u * K);
+    for (int q = 0; q < 2 * kUT; ++q) b_off[q] = min(8 * q + lrow, N - 1 - n0) * (2u * ldb);
 #pragma unroll
     for (int q = 0; q < 2 * kRT; ++q) a_off[q] = min(8 * q + lrow, M - 1 - m0) * (2u * K);
     unsigned piece[2];  // for even and odd instructions

@@ -177,11 +177,12 @@ HOST_DEVICE void xcd_tile_coords(int bid, int tiles_m, int tiles_n, int& tile_m,
 /// ceil(N / kBN) tiles, rows beyond the edge are loaded from the last valid row (their products are computed and
 /// dropped) and the stores are guarded; the loop runs over ceil(K / kBK) tiles, and in the last one every lane loads
 /// the 16-byte pieces that lie beyond K from the start of its row instead and, once they have landed, overwrites them
-/// in LDS with zeros. ldc: elements between consecutive rows of C (N for a dense C).
+/// in LDS with zeros. ldb, ldc: elements between consecutive stored rows of B (K for a dense B) and rows of C (N for a dense
+/// C). zero_words / zero_count: device words that the first workgroup sets to zero on the side (null / 0: none).
 template <typename Traits, typename OutType, bool kEdges = false>
 __global__ void __launch_bounds__(Traits::kThreads)
     gemm_pipelined(const __half* __restrict__ A, const __half* __restrict__ Bt, OutType* __restrict__ C, int M, int N,
-                   int K, int ldc) {
+                   int K, int ldb, int ldc, unsigned int* __restrict__ zero_words, int zero_count) {
     constexpr int kBM = Traits::kBM, kBN = Traits::kBN, kBK = Traits::kBK;
     constexpr int kMT = Traits::kMT, kNT = Traits::kNT, kKS = Traits::kKS;
 
@@ -191,6 +192,8 @@ __global__ void __launch_bounds__(Traits::kThreads)
     const int wave = __builtin_amdgcn_readfirstlane(wave_id());
     const int wave_m = wave / Traits::kWN;
     const int wave_n = wave % Traits::kWN;
+    if (zero_count > 0 && blockIdx.x == 0)
+        for (int i = threadIdx.x; i < zero_count; i += Traits::kThreads) zero_words[i] = 0u;
 
     int tile_m, tile_n;
     detail::xcd_tile_coords(blockIdx.x, kEdges ? (M + kBM - 1) / kBM : M / kBM, kEdges ? (N + kBN - 1) / kBN : N / kBN,
@@ -206,7 +209,7 @@ __global__ void __launch_bounds__(Traits::kThreads)
     const int lchk = lane & 7;   // physical 16-byte chunk
     // Each load's source is a wave-uniform base (the tile's first row at the k-tile, in scalar registers) plus a byte
     // offset per lane that is fixed for the whole kernel: one 32-bit register per load instruction. Offsets stay below
-    // kBM * K * 2 bytes, so K up to 2^23 / (kBM / 256) fits.
+    // kBM * K * 2 bytes, so K (and ldb) up to 2^23 / (kBM / 256) fits.
     auto row_chunk = [&](int loads_per_wave, int j) {
         const int row = (wave * loads_per_wave + j) * Traits::kRowsPerLoad + lrow;
         return lchk ^ ((row >> 1) & 7);
@@ -220,14 +223,14 @@ __global__ void __launch_bounds__(Traits::kThreads)
 #pragma unroll
     for (int j = 0; j < Traits::kBLoads; ++j) {
         const int row = (wave * Traits::kBLoads + j) * Traits::kRowsPerLoad + lrow;
-        b_off[j] = unsigned(kEdges && n0 + row >= N ? N - 1 - n0 : row) * unsigned(K) * 2u + row_chunk(Traits::kBLoads, j) * 16;
+        b_off[j] = unsigned(kEdges && n0 + row >= N ? N - 1 - n0 : row) * unsigned(ldb) * 2u + row_chunk(Traits::kBLoads, j) * 16;
     }
     const unsigned char* a_tile = reinterpret_cast<const unsigned char*>(A + size_t(m0) * K);
-    const unsigned char* b_tile = reinterpret_cast<const unsigned char*>(Bt + size_t(n0) * K);
+    const unsigned char* b_tile = reinterpret_cast<const unsigned char*>(Bt + size_t(n0) * ldb);
     // kEdges: the k-tile that straddles K asks for pieces beyond the end of their row; those land in LDS and are
     // overwritten with zeros there (zero_k_tail), so any readable address serves: the offset is limited to the last
     // 16 bytes of the matrix, which only the last row's pieces exceed.
-    const size_t a_left = (size_t(M - m0) * K - 8) * 2, b_left = (size_t(N - n0) * K - 8) * 2;
+    const size_t a_left = (size_t(M - m0) * K - 8) * 2, b_left = (size_t(N - n0 - 1) * ldb + K - 8) * 2;
     const unsigned int a_limit = a_left < 0xfffffff0u ? unsigned(a_left) : 0xfffffff0u;
     const unsigned int b_limit = b_left < 0xfffffff0u ? unsigned(b_left) : 0xfffffff0u;
     auto a_src = [&](int j, int k0) -> const unsigned char* {

@@ -66,12 +66,14 @@ using GemmW128kTraits = GemmW128kTraitsN<8>;
 template <typename OutType, bool kEdges = false, typename T = GemmW128kTraits, bool kTail = false>
 __global__ void __launch_bounds__(T::kThreads)
     gemm_w128k(const __half* __restrict__ A, const __half* __restrict__ Bt, OutType* __restrict__ C, int M, int N, int K,
-               int lda, int ldb, int ldc) {
+               int lda, int ldb, int ldc, unsigned int* __restrict__ zero_words, int zero_count) {
     constexpr int kNT = T::kNT, kNumLoads = 8 + T::kLoadsB;
     extern __shared__ __align__(1024) unsigned char lds[];
 
     const int lane = lane_id();
     const int wave = __builtin_amdgcn_readfirstlane(wave_id());
+    if (zero_count > 0 && blockIdx.x == 0 && blockIdx.y == 0)
+        for (int i = threadIdx.x; i < zero_count; i += T::kThreads) zero_words[i] = 0u;
     int tile_m, tile_n;
     detail::xcd_tile_coords(blockIdx.x, (M + T::kBM - 1) / T::kBM, (N + T::kBN - 1) / T::kBN, tile_m, tile_n);
     const int m0 = tile_m * T::kBM, n0 = tile_n * T::kBN;

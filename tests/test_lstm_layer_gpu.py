@@ -1,0 +1,136 @@
+"""The LSTM layer whose time loop is one launch (``algo="layer"``): every instantiation, sizes where its slices, row tiles and columns
+end, more groups of rows than XCDs, and launches with fewer workgroups than slices. Against the oracle, in the tolerance of the
+layer (outputs below 1, h rounded to f16 every step: 1e-2), and against the step kernels, which differ by the order of f32 sums
+before that rounding (2^-11 per step, carried over T steps: 4e-3)."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+ABS_TOL, STEP_TOL = 1e-2, 4e-3
+
+
+def operands(tcu, device, T, B, I, H, state=True):
+    import torch
+
+    gen = torch.Generator(device=device)
+    gen.manual_seed(T * B + I + H)
+    normal = lambda *shape, std=1.0: torch.randn(*shape, generator=gen, device=device).mul_(std)
+    return (normal(T, B, I, std=0.5).half(), normal(4 * H, I + H, std=0.05).half(), normal(4 * H, std=0.1).half(),
+            normal(B, H, std=0.5).half() if state else None, normal(B, H, std=0.5) if state else None)
+
+
+def close(got, want, tol=STEP_TOL):
+    return all(float((g.float() - w.float()).abs().max()) <= tol for g, w in zip(got, want))
+
+
+@pytest.mark.parametrize("T,B,I,H", [(2, 16, 16, 16), (3, 48, 64, 112), (5, 128, 80, 128),    # 16 units, 128 columns
+                                     (4, 144, 64, 64), (3, 240, 96, 128),                     # ... 32 rows, 16 of 32 in the last group
+                                     (4, 80, 128, 144), (3, 160, 64, 256),                    # 256 columns
+                                     (3, 16, 48, 272), (3, 128, 64, 512), (3, 208, 64, 496),  # 512
+                                     (4, 80, 336, 656), (3, 144, 64, 528), (3, 256, 64, 768),  # 32 units, 768
+                                     (3, 32, 64, 784), (3, 16, 64, 1024), (3, 240, 64, 1008), (3, 256, 128, 1024),
+                                     (4, 336, 64, 112), (3, 1040, 16, 80)])                    # more groups than XCDs
+@pytest.mark.parametrize("state", [False, True])
+def test_lstm_layer_matches_the_steps(tcu, device, T, B, I, H, state):
+    import torch
+
+    print(f"lstm layer T{T} B{B} I{I} H{H} state={state}", flush=True)
+    args = operands(tcu, device, T, B, I, H, state)
+    want = tcu.lstm(*args, workspace=False)
+    h_buf = torch.full((T * B * H + 4096,), 7.0, dtype=torch.float16, device=device)
+    c_buf = torch.full((B * H + 4096,), 7.0, dtype=torch.float32, device=device)
+    need = int(tcu.lib().tcu_lstm_layer_workspace_bytes(T, B, I, H))
+    ws = torch.full((need + 256,), 0x5A, dtype=torch.uint8, device=device)
+    for _ in range(2):  # (the synchronisation words of the first call are in the workspace of the second)
+        out = (h_buf[:T * B * H].view(T, B, H), c_buf[:B * H].view(B, H))
+        assert close(tcu.lstm(*args, algo="layer", workspace=ws, out=out), want)
+    assert bool((h_buf[T * B * H:] == 7.0).all()) and bool((c_buf[B * H:] == 7.0).all()) and bool((ws[need:] == 0x5A).all())
+
+
+def test_lstm_layer_against_the_oracle(tcu, oracle, device):
+    import torch
+
+    T, B, I, H = 6, 80, 336, 656
+    x = oracle.fill_normal(T * B * I, 61, 0, 0.5).reshape(T, B, I)
+    W = oracle.fill_normal(4 * H * (I + H), 62, 0, 0.05).reshape(4 * H, I + H)
+    b = oracle.fill_normal(4 * H, 63, 0, 0.1)
+    to = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(device)
+    h_all, c_T = tcu.lstm(to(x), to(W), to(b), algo="layer")
+    h_ref, c_ref = oracle.lstm(x, W, b)
+    assert oracle.max_abs_err(h_all.float().cpu().numpy(), h_ref) <= ABS_TOL
+    assert oracle.max_abs_err(c_T.cpu().numpy(), c_ref) <= ABS_TOL
+
+
+@pytest.mark.parametrize("T,B,I,H,grid", [(5, 80, 64, 112, 1), (5, 80, 64, 112, 8), (5, 80, 64, 112, 40), (4, 144, 96, 656, 9),
+                                          (4, 256, 64, 1024, 100), (4, 336, 64, 320, 24)])
+def test_lstm_layer_with_few_workgroups(tcu, device, monkeypatch, T, B, I, H, grid):
+    """Slices without a workgroup are taken over by those that run, groups of rows by XCDs that are done; at the smallest, one
+    workgroup does everything."""
+    print(f"lstm layer T{T} B{B} I{I} H{H} grid {grid}", flush=True)
+    args = operands(tcu, device, T, B, I, H)
+    want = tcu.lstm(*args, workspace=False)
+    monkeypatch.setenv("TCU_LSTM_LAYER_GRID", str(grid))
+    assert close(tcu.lstm(*args, algo="layer"), want)
+
+
+def test_lstm_layer_two_streams_and_nan(tcu, device):
+    """Calls that overlap on two streams, each with a workspace of its own; NaN inputs stay NaNs of their rows (and end no wait
+    early or late), infinite initial states saturate."""
+    import torch
+
+    T, B, I, H = 12, 80, 96, 528
+    args = operands(tcu, device, T, B, I, H)
+    want = tcu.lstm(*args, workspace=False)
+    torch.cuda.synchronize()
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    got = []
+    for k in range(6):
+        with torch.cuda.stream(streams[k % 2]):
+            got.append(tcu.lstm(*args, algo="layer"))
+    torch.cuda.synchronize()
+    assert all(close(g, want) for g in got)
+    x, W, b, h0, c0 = (t.clone() for t in args)
+    x.view(torch.int16)[2, 17, 3] = -1  # 0xffff
+    x.view(torch.int16)[5, 40, :] = -1
+    h0[3, 5] = float("inf")
+    want, got = tcu.lstm(x, W, b, h0, c0, workspace=False), tcu.lstm(x, W, b, h0, c0, algo="layer")
+    for w, g in zip(want, got):
+        assert torch.equal(torch.isnan(w), torch.isnan(g))
+        assert close((torch.nan_to_num(g),), (torch.nan_to_num(w),))
+
+
+def test_lstm_layer_route(tcu, device):
+    """Where AUTO takes it, where not, and what it does with a caller's workspace, an h0 inside h_all and a captured stream."""
+    import torch
+
+    import tiledcuda_amd.torch_ops  # noqa: F401
+
+    uses, need = tcu.lib().tcu_lstm_uses_layer, tcu.lib().tcu_lstm_layer_workspace_bytes
+    for shape in ((16, 256, 1024, 1024), (24, 80, 336, 656), (20, 16, 416, 80), (12, 144, 80, 208)):
+        assert uses(*shape) == 1, shape
+    for shape in ((3, 16, 64, 64), (16, 256, 4096, 1024), (31, 4096, 96, 160), (16, 64, 64, 1040), (16, 24, 64, 64), (0, 1, 1, 1)):
+        assert uses(*shape) == 0, shape
+    assert need(1, 16, 64, 64) == 0 and need(2, 16, 64, 1040) == 0 and need(2, 2064, 64, 64) == 0 and need(2, 16, 64, 64) == 4096 + 2 * 16 * 256 * 4
+    T, B, I, H = 24, 48, 64, 272
+    args = operands(tcu, device, T, B, I, H)
+    steps, layer = tcu.lstm(*args, workspace=False), tcu.lstm(*args, algo="layer")
+    same = lambda a, b: torch.equal(a[0], b[0]) and torch.equal(a[1], b[1])
+    assert uses(T, B, I, H) == 1 and not same(steps, layer)
+    ws = torch.full((need(T, B, I, H),), 0x5A, dtype=torch.uint8, device=device)
+    assert same(tcu.lstm(*args), layer) and same(torch.ops.tiledcuda.lstm(*args), layer)
+    assert same(tcu.lstm(*args, workspace=ws[:-1]), steps) and bool((ws == 0x5A).all())
+    assert same(tcu.lstm(*args, workspace=ws), layer) and not bool((ws == 0x5A).all())
+    # an initial state that is a step of the output
+    out = (torch.empty(T, B, H, dtype=torch.float16, device=device), torch.empty(B, H, device=device))
+    out[0][5].copy_(args[3])
+    assert same(tcu.lstm(*args[:3], out[0][5], args[4], workspace=ws, out=out), steps)
+    # captured: the steps, or the layer in the caller's workspace, replayed with work in between
+    for workspace, want in ((None, steps), (ws, layer)):
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            tcu.lstm(*args, workspace=workspace, out=out)
+        for _ in range(3):
+            out[0].zero_(), out[1].zero_()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert same(out, want)

@@ -71,6 +71,10 @@ _SIGNATURES = {
     "tcu_lstm_uses_workspace": (ctypes.c_int, [ctypes.c_int] * 4),
     "tcu_lstm_f16_ws": (ctypes.c_int, [ctypes.c_void_p] * 7 + [ctypes.c_int] * 4 + [ctypes.c_void_p, ctypes.c_ulonglong,
                                                                                      ctypes.c_void_p]),
+    "tcu_lstm_layer_workspace_bytes": (ctypes.c_ulonglong, [ctypes.c_int] * 4),
+    "tcu_lstm_uses_layer": (ctypes.c_int, [ctypes.c_int] * 4),
+    "tcu_lstm_f16_layer": (ctypes.c_int, [ctypes.c_void_p] * 7 + [ctypes.c_int] * 4 + [ctypes.c_void_p, ctypes.c_ulonglong,
+                                                                                        ctypes.c_void_p]),
     "tcu_lstm_persistent_workspace_bytes": (ctypes.c_ulonglong, [ctypes.c_int] * 4),
     "tcu_lstm_f16_persistent": (ctypes.c_int, [ctypes.c_void_p] * 7 + [ctypes.c_int] * 4 + [ctypes.c_void_p, ctypes.c_ulonglong,
                                                                                           ctypes.c_void_p]),
@@ -330,6 +334,10 @@ def lstm(x: torch.Tensor, W: torch.Tensor, bias: torch.Tensor, h0: torch.Tensor 
     that, or a workspace of your own, under HIP graph capture: an allocation has no place in a captured stream), else one
     fused kernel per step. ``out`` = (h_all, c_T) tensors to write into instead of allocating them.
 
+    ``algo="layer"`` runs the whole time loop in one launch after the same GEMM (``tcu_lstm_f16_layer``; T >= 2, H <= 1024, B <= 2048,
+    all in multiples of 16), asking nothing of the GPU; ``algo="auto"`` takes it, with a workspace as above, where it pays (about 5
+    steps and more, up to 256 rows; not in a stream that is being captured, unless the workspace is yours).
+
     ``algo="persistent"`` runs the whole time loop in one weight-stationary launch after the same GEMM
     (``tcu_lstm_f16_persistent``: H in {256, 512, 768, 1024}, B <= 256 in multiples of 32; ``lstm_persistent_workspace_bytes``). Its
     workgroups wait for each other with a time limit; with ``check=True`` (the default) the stream is synchronised and
@@ -365,6 +373,24 @@ def lstm(x: torch.Tensor, W: torch.Tensor, bias: torch.Tensor, h0: torch.Tensor 
         if check:
             lstm_persistent_status(workspace)
         return h_all, c_out
+    if algo == "layer" or (algo == "auto" and T >= 4 and workspace is not False and x.is_cuda and lib().tcu_lstm_uses_layer(T, B, I, H)):
+        need = int(lib().tcu_lstm_layer_workspace_bytes(T, B, I, H))
+        if algo == "layer" and need == 0:
+            raise ValueError("algo='layer' needs T >= 2, B, I and H in multiples of 16, H <= 1024 and B <= 2048")
+        # (nothing is allocated in a captured stream: outside torch's own graphs the graph would keep a block that goes back to the
+        # allocator; a workspace of the caller's that is too small belongs to the plans below)
+        if workspace is None or workspace is False:
+            if algo == "layer" or not torch.cuda.is_current_stream_capturing():
+                workspace = torch.empty(need, dtype=torch.uint8, device=x.device)
+        elif not workspace.is_cuda or not workspace.is_contiguous():
+            raise ValueError("workspace must be a contiguous device tensor")
+        size = 0 if workspace is None else workspace.numel() * workspace.element_size()
+        if algo == "layer" or size >= need:
+            _check(lib().tcu_lstm_f16_layer(_dev_ptr(x, torch.float16, "x"), _dev_ptr(W, torch.float16, "W"),
+                                            _dev_ptr(bias, torch.float16, "bias"), _dev_ptr(h0, torch.float16, "h0"),
+                                            _dev_ptr(c0, torch.float32, "c0"), _dev_ptr(h_all, torch.float16, "h_all"),
+                                            _dev_ptr(c_out, torch.float32, "c_out"), T, B, I, H, workspace.data_ptr(), size, _stream()))
+            return h_all, c_out
     # (T < 4 or I < 512 never uses one; asking costs 0.5 us)
     if algo == "auto" and T >= 4 and I >= 512 and workspace is not False and x.is_cuda and lib().tcu_lstm_uses_workspace(T, B, I, H):
         algo = "hoisted"  # a long input size: its half of the gates is cheaper as one GEMM over all steps

@@ -18,6 +18,7 @@
 #include "kernels/gemm_w128k.hpp"
 #include "kernels/lstm_direct.hpp"
 #include "kernels/lstm_fwd.hpp"
+#include "kernels/lstm_layer.hpp"
 #include "kernels/lstm_ragged.hpp"
 #include "kernels/lstm_recurrent.hpp"
 #include "kernels/mod.hpp"
@@ -119,6 +120,7 @@ bool aligned16(std::initializer_list<const void*> v) {
 // array's name is only a handle for hipGetSymbolAddress, never a device address.
 constexpr unsigned long long kScratchBytes = 64ull << 20;
 constexpr unsigned long long kPersistentSyncBytes = 4096;  // synchronisation words in front of the pre-activations
+constexpr int kLstmLayerStealTicks = 3000;  // 30 us (100 MHz): long against the start of a grid, short against its steps
 static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 
 constexpr int kMaxDevices = 64;
@@ -219,11 +221,12 @@ PipePlan pipelined_plan(int M, int N, int K) {
 /// tiles.
 template <typename OutType>
 int gemm_pipelined_dispatch(const __half* A, const __half* B, OutType* C, int M, int N, int K, hipStream_t stream,
-                            int ldc = 0) {
+                            int ldc = 0, int ldb = 0, unsigned int* zero_words = nullptr, int zero_count = 0) {
     if (ldc == 0) ldc = N;
+    if (ldb == 0) ldb = K;
     if (M % 16 != 0 || N % 16 != 0 || K % 16 != 0)
         return fail(TCU_ERR_UNSUPPORTED_SHAPE, "GEMM shapes are whole 16 x 16 tiles: M, N and K must be multiples of 16");
-    if ((long)K * 512 >= (1l << 32))
+    if ((long)ldb * 512 >= (1l << 32))
         return fail(TCU_ERR_UNSUPPORTED_SHAPE, "pipelined GEMM addresses a tile's rows with 32-bit offsets: K < 2^23");
     auto go = [&](auto traits) {
         using Traits = decltype(traits);
@@ -231,9 +234,9 @@ int gemm_pipelined_dispatch(const __half* A, const __half* B, OutType* C, int M,
         if (grid > INT_MAX) return fail(TCU_ERR_UNSUPPORTED_SHAPE, "GEMM: too many tiles for one launch");
         if (M % Traits::kBM == 0 && N % Traits::kBN == 0 && K % Traits::kBK == 0)
             return launch(&gemm_pipelined<Traits, OutType, false>, dim3(unsigned(grid)), dim3(Traits::kThreads),
-                          Traits::template lds_bytes<OutType>(), stream, A, B, C, M, N, K, ldc);
+                          Traits::template lds_bytes<OutType>(), stream, A, B, C, M, N, K, ldb, ldc, zero_words, zero_count);
         return launch(&gemm_pipelined<Traits, OutType, true>, dim3(unsigned(grid)), dim3(Traits::kThreads),
-                      Traits::template lds_bytes<OutType>(), stream, A, B, C, M, N, K, ldc);
+                      Traits::template lds_bytes<OutType>(), stream, A, B, C, M, N, K, ldb, ldc, zero_words, zero_count);
     };
     switch (pipelined_plan(M, N, K).config) {
         case kPipeLarge: return go(PipeLarge{});
@@ -294,7 +297,8 @@ int launch_gemm_w128k(const __half* A, const __half* B, OutType* C, int M, int N
     // where M and N are whole tiles
     const bool whole = M % T::kBM == 0 && N % T::kBN == 0;
     auto kernel = K % T::kBK != 0 ? &gemm_w128k<OutType, true, T, true> : whole ? &gemm_w128k<OutType, false, T> : &gemm_w128k<OutType, true, T>;
-    return launch(kernel, dim3(unsigned(grid)), dim3(T::kThreads), T::kLdsBytes, stream, A, B, C, M, N, K, K, K, ldc);
+    return launch(kernel, dim3(unsigned(grid)), dim3(T::kThreads), T::kLdsBytes, stream, A, B, C, M, N, K, K, K, ldc,
+                  static_cast<unsigned int*>(nullptr), 0);
 }
 
 template <typename OutType>
@@ -590,7 +594,9 @@ bool gemm_split_is_the_choice(int M, int N, int K) {
 }
 
 template <typename OutType>
-int gemm_direct_dispatch(const __half* A, const __half* B, OutType* C, int M, int N, int K, hipStream_t stream) {
+int gemm_direct_dispatch(const __half* A, const __half* B, OutType* C, int M, int N, int K, hipStream_t stream, int ldb = 0,
+                         unsigned int* zero_words = nullptr, int zero_count = 0) {
+    if (ldb == 0) ldb = K;
     if (M % 16 != 0 || N % 16 != 0 || K % 16 != 0)
         return fail(TCU_ERR_UNSUPPORTED_SHAPE, "GEMM shapes are whole 16 x 16 tiles: M, N and K must be multiples of 16");
     const GemmDirectPlan plan = gemm_direct_plan(M, N, K);
@@ -598,7 +604,8 @@ int gemm_direct_dispatch(const __half* A, const __half* B, OutType* C, int M, in
     auto go = [&](auto traits) {
         using T = decltype(traits);
         const long grid = (long)((M + T::kBM - 1) / T::kBM) * ((N + T::kBN - 1) / T::kBN);
-        return launch(&gemm_direct<T, OutType>, dim3(unsigned(grid)), dim3(T::kThreads), T::kLdsBytes, stream, A, B, C, M, N, K);
+        return launch(&gemm_direct<T, OutType>, dim3(unsigned(grid)), dim3(T::kThreads), T::kLdsBytes, stream, A, B, C, M, N, K, ldb,
+                      zero_words, zero_count);
     };
     switch (10 * plan.ut + plan.rt) {
         case 11: return go(GemmDirectTraits<1, 1>{});
@@ -625,10 +632,10 @@ int gemm_splitk(const __half* A, const __half* B, OutType* C, int M, int N, int 
         const int tiles = ((M + Tk::kBM - 1) / Tk::kBM) * ((N + Tk::kBN - 1) / Tk::kBN);
         if (M % Tk::kBM == 0 && N % Tk::kBN == 0)
             rc = launch(&gemm_w128k<float, false, Tk>, dim3(tiles, plan.splits), dim3(Tk::kThreads), Tk::kLdsBytes, stream, A,
-                        B, partial, M, N, K / plan.splits, K, K, N);
+                        B, partial, M, N, K / plan.splits, K, K, N, static_cast<unsigned int*>(nullptr), 0);
         else  // edge tiles: rows beyond M or N loaded from the last valid row, stores guarded
             rc = launch(&gemm_w128k<float, true, Tk>, dim3(tiles, plan.splits), dim3(Tk::kThreads), Tk::kLdsBytes, stream, A,
-                        B, partial, M, N, K / plan.splits, K, K, N);
+                        B, partial, M, N, K / plan.splits, K, K, N, static_cast<unsigned int*>(nullptr), 0);
     } else {
         const int tiles = (M / T::kBM) * (N / T::kBN);
         rc = launch(&gemm_w128<float>, dim3(tiles, plan.splits), dim3(T::kThreads), T::kLdsBytes, stream, A, B, partial, M, N,
@@ -1333,7 +1340,7 @@ int launch_lstm_hoisted(const __half* x, const __half* W, const __half* bias, co
         using Tk = GemmW128kTraits;
         auto kernel = rows % Tk::kBM == 0 ? &gemm_w128k<float, false, Tk> : &gemm_w128k<float, true, Tk>;
         rc = launch(kernel, dim3(unsigned(plan.tiles128)), dim3(Tk::kThreads), Tk::kLdsBytes, stream, x, W, pre, int(rows), 4 * H, I, I,
-                    I + H, 4 * H);
+                    I + H, 4 * H, static_cast<unsigned int*>(nullptr), 0);
     } else {
         rc = gemm_w128_dispatch<float>(x, W, pre, int(rows), 4 * H, I, stream, I, I + H);
     }
@@ -1386,6 +1393,94 @@ int launch_lstm_fwd(const __half* x, const __half* W, const __half* bias, const 
         if (rc != TCU_OK) return lstm_step_failed(rc, t, T);
     }
     return TCU_OK;
+}
+
+/// The shapes that lstm_layer_xcd takes: T >= 2 (its workgroups count on a second step), H within the registers of an XCD, at most
+/// kMaxGroups groups of rows, and the 32-bit offsets of its operands and of the projection's.
+int lstm_layer_row_tiles(int B) { return B <= 128 ? 1 : 2; }
+bool lstm_layer_takes(int T, int B, int I, int H) {
+    if (T < 2 || H > 1024 || (long)T * B > INT_MAX || !lstm_direct_takes(B, I, H)) return false;
+    const int rows = 16 * lstm_layer_row_tiles(B);
+    return (B + rows - 1) / rows <= LstmLayerTraits<1, 4, 1>::kMaxGroups && (long)(I + H) * 512 < (1l << 32);
+}
+
+/// pre[T * B, 4H] = x . W[:, :I]^T in f32 with the kernel that is expected to take least, `sync` cleared on the side.
+struct LstmLayerProjection {
+    int kernel;  // 0: gemm_direct, 1: gemm_w128k, 2: gemm_w128, 3: gemm_pipelined
+    double us;
+};
+LstmLayerProjection lstm_layer_projection(long rows, int I, int H) {
+    const double mb = 16e-6 * double(rows) * H;  // of pre-activations: f32 outputs cost these kernels 0.15 to 0.6 us per MB
+    LstmLayerProjection plan{0, gemm_direct_plan(int(rows), 4 * H, I).us + 0.6 * mb};
+    const long tiles128 = ((rows + 127) / 128) * ((4l * H + 127) / 128), tiles256 = ((rows + 255) / 256) * ((4l * H + 255) / 256);
+    const double us128 = double((tiles128 + 255) / 256) * (5.0 + 0.95 * ((I + 127) / 128)) + 0.3 * mb;
+    const double us256 = gemm_w128_us(tiles256, (I + 63) / 64 * 64) + 0.15 * mb, us_pipe = pipelined_plan(int(rows), 4 * H, I).us + 0.4 * mb;
+    if (us128 < plan.us) plan = {1, us128};
+    if (us256 < plan.us) plan = {2, us256};
+    if (us_pipe < plan.us) plan = {3, us_pipe};
+    return plan;
+}
+
+/// Whether AUTO runs the layer that way: the projection, 1.5 us to the next launch, what the kernel takes before its first step (the
+/// weights arrive at 0.9 MB per us and XCD) and its steps, for every round of 8 groups of rows (measured over 90 sizes, us per step with
+/// 16 and 32 rows: H 128 0.73, 1.1; 256 0.95, 1.45; 512 1.2, 1.9; 768 1.75, 2.9; 1024 2.05, 3.9), against a launch per step. us, steps
+/// -> this: T 16, B 256, I 1024, H 1024: 149 -> 106; 24, 80, 336, 656: 109 -> 75; 20, 16, 416, 80: 60 -> 24; 8, 96, 176, 160: 25 -> 18; not taken: 8,
+/// 80, 384, 576: 34, 38; 5, 352, 144, 864: 62, 73; 31, 368, 96, 160: 111, 114. Long inputs stay with lstm_projection_pays().
+bool lstm_layer_pays(int T, int B, int I, int H) {
+    if (T < 4 || !lstm_layer_takes(T, B, I, H) || lstm_projection_pays(T, B, I, H)) return false;
+    static constexpr double kStepUs[5][2] = {{0.73, 1.1}, {0.95, 1.45}, {1.2, 1.9}, {1.75, 2.9}, {2.05, 3.9}};
+    const int size = H <= 128 ? 0 : H <= 256 ? 1 : H <= 512 ? 2 : H <= 768 ? 3 : 4, tiles = lstm_layer_row_tiles(B);
+    const int rounds = ((B + 16 * tiles - 1) / (16 * tiles) + 7) / 8;
+    const double layer = 7.5 + 9.0 * (H / 1024.0) * (H / 1024.0) + rounds * T * kStepUs[size][tiles - 1];
+    return 1.05 * (lstm_layer_projection((long)T * B, I, H).us + layer) < T * lstm_step_us(B, H, I + H);
+}
+
+template <int kTW, int kKS, int kRT>
+int launch_lstm_layer_xcd(const float* pre, const __half* W, const __half* bias, const __half* h0, const float* c0, __half* h_all,
+                          float* c_out, int T, int B, int I, int H, unsigned int* sync, int grid_limit, hipStream_t s) {
+    using Traits = LstmLayerTraits<kTW, kKS, kRT>;
+    const int peers = (H + Traits::kUnits - 1) / Traits::kUnits;
+    const int grid = grid_limit > 0 ? std::min(grid_limit, 8 * peers) : 8 * peers;
+    return launch(&lstm_layer_xcd<Traits>, dim3(unsigned(grid)), dim3(Traits::kThreads), Traits::kLdsBytes, s, pre, W, I + H, I, bias, h0,
+                  c0, h_all, c_out, T, B, H, sync, kLstmLayerStealTicks);
+}
+
+int launch_lstm_layer(const __half* x, const __half* W, const __half* bias, const __half* h0, const float* c0, __half* h_all,
+                      float* c_out, int T, int B, int I, int H, unsigned char* workspace, int grid_limit, hipStream_t s) {
+    auto sync = reinterpret_cast<unsigned int*>(workspace);
+    auto pre = reinterpret_cast<float*>(workspace + kPersistentSyncBytes);
+    constexpr int kSyncWords = LstmLayerTraits<1, 4, 1>::kSyncWords;
+    static_assert(kSyncWords * sizeof(unsigned int) <= kPersistentSyncBytes);
+    const int rows = T * B;
+    int rc;
+    switch (lstm_layer_projection(rows, I, H).kernel) {
+        case 0: rc = gemm_direct_dispatch<float>(x, W, pre, rows, 4 * H, I, s, I + H, sync, kSyncWords); break;
+        case 1: {
+            using Tk = GemmW128kTraits;
+            const long tiles = ((rows + 127l) / 128) * ((4l * H + 127) / 128);
+            auto kernel = I % Tk::kBK != 0 ? &gemm_w128k<float, true, Tk, true> : rows % Tk::kBM == 0 && 4 * H % Tk::kBN == 0
+                          ? &gemm_w128k<float, false, Tk> : &gemm_w128k<float, true, Tk>;
+            rc = launch(kernel, dim3(unsigned(tiles)), dim3(Tk::kThreads), Tk::kLdsBytes, s, x, W, pre, rows, 4 * H, I, I, I + H, 4 * H, sync,
+                        kSyncWords);
+            break;
+        }
+        case 2: rc = gemm_w128_dispatch<float>(x, W, pre, rows, 4 * H, I, s, I, I + H, 4 * H, sync, kSyncWords); break;
+        default: rc = gemm_pipelined_dispatch<float>(x, W, pre, rows, 4 * H, I, s, 4 * H, I + H, sync, kSyncWords);
+    }
+    if (rc != TCU_OK) return rc;
+    auto go = [&](auto tw, auto ks) {
+        constexpr int kTW = decltype(tw)::value, kKS = decltype(ks)::value;
+        if (lstm_layer_row_tiles(B) == 1)
+            return launch_lstm_layer_xcd<kTW, kKS, 1>(pre, W, bias, h0, c0, h_all, c_out, T, B, I, H, sync, grid_limit, s);
+        return launch_lstm_layer_xcd<kTW, kKS, 2>(pre, W, bias, h0, c0, h_all, c_out, T, B, I, H, sync, grid_limit, s);
+    };
+    using one = std::integral_constant<int, 1>;
+    using two = std::integral_constant<int, 2>;
+    if (H <= 128) return go(one{}, std::integral_constant<int, 4>{});
+    if (H <= 256) return go(one{}, std::integral_constant<int, 8>{});
+    if (H <= 512) return go(one{}, std::integral_constant<int, 16>{});
+    if (H <= 768) return go(two{}, std::integral_constant<int, 24>{});
+    return go(two{}, std::integral_constant<int, 32>{});
 }
 
 /// The weight-stationary recurrence for hidden size kH: 8 * kH / 32 workgroups, kH / 32 per XCD.
@@ -1594,6 +1689,37 @@ int tcu_lstm_f16_ws(const void* x, const void* W, const void* bias, const void* 
     auto cp = static_cast<float*>(c_out);
     auto pre = static_cast<float*>(workspace);
     return launch_lstm_hoisted(xp, wp, bp, h0p, c0p, hp, cp, T, B, I, H, pre, s);
+}
+
+unsigned long long tcu_lstm_layer_workspace_bytes(int T, int B, int I, int H) {
+    if (!positive({T, B, I, H}) || !lstm_layer_takes(T, B, I, H)) return 0;
+    return kPersistentSyncBytes + (unsigned long long)T * B * 4 * H * sizeof(float);
+}
+
+int tcu_lstm_uses_layer(int T, int B, int I, int H) { return positive({T, B, I, H}) && lstm_layer_pays(T, B, I, H) ? 1 : 0; }
+
+int tcu_lstm_f16_layer(const void* x, const void* W, const void* bias, const void* h0, const void* c0, void* h_all, void* c_out,
+                       int T, int B, int I, int H, void* workspace, unsigned long long workspace_bytes, void* stream) {
+    if (!x || !W || !bias || !h_all || !c_out || !workspace) return fail(TCU_ERR_INVALID_ARGUMENT, "tcu_lstm_f16_layer: null pointer");
+    if (!positive({T, B, I, H})) return fail(TCU_ERR_INVALID_ARGUMENT, "tcu_lstm_f16_layer: sizes must be positive");
+    if (!aligned16({x, W, bias, h0, c0, h_all, c_out, workspace}))
+        return fail(TCU_ERR_INVALID_ARGUMENT, "tcu_lstm_f16_layer: operands must be 16-byte aligned");
+    const unsigned long long need = tcu_lstm_layer_workspace_bytes(T, B, I, H);
+    if (need == 0)
+        return fail(TCU_ERR_UNSUPPORTED_SHAPE, "tcu_lstm_f16_layer: needs T >= 2, B, I and H in multiples of 16, H <= 1024 and B <= 2048");
+    if (workspace_bytes < need)
+        return fail(TCU_ERR_INVALID_ARGUMENT, "tcu_lstm_f16_layer: workspace smaller than tcu_lstm_layer_workspace_bytes()");
+    // the kernel marks all of h_all before its first step: an initial state inside it (the last step of an earlier call that
+    // wrote the same tensor) goes to the kernels that write a step at a time
+    const auto h0_first = reinterpret_cast<uintptr_t>(h0), all_first = reinterpret_cast<uintptr_t>(h_all);
+    if (h0 && h0_first < all_first + size_t(T) * B * H * 2 && all_first < h0_first + size_t(B) * H * 2)
+        return tcu_lstm_f16_algo(x, W, bias, h0, c0, h_all, c_out, T, B, I, H, TCU_LSTM_AUTO, stream);
+    int grid_limit = 0;  // fewer workgroups than the layer has slices (to exercise that they are taken over)
+    if (const char* e = std::getenv("TCU_LSTM_LAYER_GRID")) grid_limit = int(std::strtol(e, nullptr, 10));
+    return launch_lstm_layer(static_cast<const __half*>(x), static_cast<const __half*>(W), static_cast<const __half*>(bias),
+                             static_cast<const __half*>(h0), static_cast<const float*>(c0), static_cast<__half*>(h_all),
+                             static_cast<float*>(c_out), T, B, I, H, static_cast<unsigned char*>(workspace), grid_limit,
+                             static_cast<hipStream_t>(stream));
 }
 
 unsigned long long tcu_lstm_persistent_workspace_bytes(int T, int B, int I, int H) {

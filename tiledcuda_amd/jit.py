@@ -57,7 +57,8 @@ static int launch(const __half* a, const __half* b, float* c, hipStream_t stream
         if (hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess) return -3;
         raised = true;
     }}
-    hipLaunchKernelGGL(kernel, dim3(({M} / {TM}) * ({N} / {TN})), dim3(Config::kThreads), lds, stream, a, b, c, {M}, {N}, {K}, {N});
+    hipLaunchKernelGGL(kernel, dim3(({M} / {TM}) * ({N} / {TN})), dim3(Config::kThreads), lds, stream, a, b, c, {M}, {N}, {K}, {K}, {N},
+                       static_cast<unsigned int*>(nullptr), 0);
     return hipGetLastError() == hipSuccess ? 0 : -3;
 }}
 """
