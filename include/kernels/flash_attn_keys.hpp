@@ -1,10 +1,10 @@
 // FlashAttention-2 forward for launches with few query blocks, O = softmax(scale · Q·Kᵀ)·V, f16 in/out, f32 statistics:
-// the wavefronts of a workgroup share one block of 64 queries and split the keys, and several workgroups may split
+// the wavefronts of a workgroup share one block of 64 (or 32) queries and split the keys, and several workgroups may split
 // the keys once more (f32 partial outputs, added by flash_attention_combine). The other tuned kernels give a
 // wavefront its own queries: 64 queries against 8192 keys are then two wavefronts' work on one CU, and a head of 576
 // queries three workgroups'.
 //
-// Design (per workgroup: 4 wavefronts, one per SIMD at head size 128, two at 64; every wavefront owns all 64 queries):
+// Design (per workgroup: 4 wavefronts, one per SIMD at head size 128, two at 64; every wavefront owns all 64 (32) queries):
 //   * a wavefront streams blocks of 32 keys (every fourth of its workgroup's) through a ring of its own, two K and two V
 //     blocks: no barrier between the first and the last block;
 //   * Sᵀ = K·Qᵀ and Oᵀ = Vᵀ·Pᵀ with v_mfma_f32_32x32x16_f16 as in flash_attn_fwd.hpp; the rows of the K tile are read with
@@ -19,6 +19,8 @@
 // four wavefronts' 64 KiB per 32 keys, as long as the matrix instructions take; 0.67 us per block of 4 x 32 keys
 // measured), with all CUs busy the L2s (1.05 us); queries and keys arriving, and the merge, cost 6 us per workgroup at
 // head size 128, 4 us at 64.
+// Where workgroups of 64 queries leave half of the chip idle they are of 32 (kQT = 1): one 32 x 32 tile of scores per block instead of
+// two, half the fragments of Q, half the merge; 4.4 us for 64 x 64 of one head instead of 6.1, 0.5 per block instead of 0.7.
 // Measured (us, before -> now): 32 heads x 64 queries x 8192 keys, head size 128: 174 -> 31 (the keys and values take 27 at
 // the rate of a device copy); 8 x 2048^2 at 128: 50 -> 23; 1 x 2048^2: 49 -> 16; 64 x 256 of one head, column-major V: 12.0
 // -> 7.6; 32 x 1024^2 at 64: 21.4 -> 15.2.
@@ -32,12 +34,12 @@
 
 namespace tiledcuda::kernels {
 
-template <const int kD_, const bool kVColMajor_>
+template <const int kD_, const bool kVColMajor_, const int kQT_ = 2>
 struct FlashKeysTraits {
     static constexpr int kD = kD_;
     static constexpr bool kVColMajor = kVColMajor_;
     static constexpr int kWaves = 4, kThreads = kWaves * kWaveSize;
-    static constexpr int kQT = 2;             // 32-query tiles of a wavefront
+    static constexpr int kQT = kQT_;          // 32-query tiles of a wavefront: two, or one where that leaves CUs idle
     static constexpr int kBM = 32 * kQT;      // queries of a workgroup (every wavefront works on all of them)
     static constexpr int kBN = 32;            // keys of a block: one wavefront's step
     static constexpr int kRowBytes = 2 * kD;
@@ -49,7 +51,7 @@ struct FlashKeysTraits {
     static constexpr int kDSteps = kD / 16, kDTiles = kD / 32;
     static constexpr int kWaveBytes = 4 * kTileBytes;         // two K and two V slots
     static constexpr int kRingBytes = kWaves * kWaveBytes;
-    static_assert(kWaveBytes == kBM * kD * 4, "a wavefront's f32 output takes the place of its own ring");
+    static_assert(kBM * kD * 4 <= kWaveBytes, "a wavefront's f32 output takes the place of its own ring");
     static constexpr int kQOffset = kRingBytes;                          // the workgroup's queries
     static constexpr int kStatOffset = kQOffset + kBM * kRowBytes;       // (maximum, sum) per wavefront and query
     static constexpr int kFactorOffset = kStatOffset + kWaves * kBM * 8; // weight of each wavefront's output per query
@@ -57,7 +59,8 @@ struct FlashKeysTraits {
     static constexpr int kGroupsPerCu = kD == 128 ? 1 : 2;
     static constexpr bool kAgprQ = kGroupsPerCu == 1;         // Q in AGPRs: 512 registers per lane (else 256, all VGPRs)
     static_assert(kD == 128 || (kD == 64 && !kVColMajor), "head size 64 or 128");
-    static_assert(kQT * kDSteps == 2 * kLoads, "one load behind every matrix instruction of the scores");
+    static constexpr int kLoadsPerSlot = 2 * kLoads / (kQT * kDSteps);  // loads behind every matrix instruction of the scores
+    static_assert(kLoadsPerSlot * kQT * kDSteps == 2 * kLoads && (kLoadsPerSlot == 1 || kLoadsPerSlot == 2));
 
     /// XOR on the 16-byte chunk index of K row `row` (rows of 256 or 128 bytes).
     HOST_DEVICE static constexpr int k_swz(int row) { return row & (kRowBytes / 16 - 1); }
@@ -88,8 +91,8 @@ DEVICE void mfma32_score_then_load(f32x16& d, const f16x8& a, const f16x8& b, co
 }
 }  // namespace detail
 
-/// M % 64 == 0, N % 32 == 0, 1 <= splits <= N / 32, column-major V: N < 2^24 (32-bit offsets into a head's V).
-/// block = 256, dynamic LDS = Traits::kLdsBytes, grid = batch * splits * (M / 64).
+/// M % kBM == 0, N % 32 == 0, 1 <= splits <= N / 32, column-major V: N < 2^24 (32-bit offsets into a head's V).
+/// block = 256, dynamic LDS = Traits::kLdsBytes, grid = batch * splits * (M / kBM).
 /// part (null when splits == 1): f32 [splits][batch * M][kD] outputs relative to the split's own maximum, followed by
 /// [splits][batch * M] pairs (maximum in the log2 domain, sum).
 template <typename Traits>
@@ -259,7 +262,13 @@ __global__ void __launch_bounds__(Traits::kThreads, Traits::kGroupsPerCu)
         // Every score of block 0 may be -infinity (keys masked by an infinite feature; any of 4 * splits blocks of the sequence
         // is some wavefront's block 0): then the exact maximum of this wavefront's first block with another score, its keys
         // read once more, is where the query starts. A query without any starts at 0 and keeps a sum of 0.
-        if (__builtin_expect(__any(m_run[0] == -INFINITY || m_run[1] == -INFINITY), 0)) {
+        auto any_masked = [&]() {
+            bool masked = false;
+#pragma unroll
+            for (int t = 0; t < kQT; ++t) masked = masked || m_run[t] == -INFINITY;
+            return __any(masked);
+        };
+        if (__builtin_expect(any_masked(), 0)) {
             for (int j = 1; j < nb; ++j) {
                 const __half* k_row = Kh + (size_t(b_first + wave + j * Traits::kWaves) * Traits::kBN + krow) * kD + 8 * h;
 #pragma unroll
@@ -276,7 +285,7 @@ __global__ void __launch_bounds__(Traits::kThreads, Traits::kGroupsPerCu)
                     mx = fmaxf(mx, detail::exchange32(mx));
                     if (m_run[t] == -INFINITY) m_run[t] = mx;
                 }
-                if (!__any(m_run[0] == -INFINITY || m_run[1] == -INFINITY)) break;
+                if (!any_masked()) break;
             }
 #pragma unroll
             for (int t = 0; t < kQT; ++t)
@@ -306,17 +315,18 @@ __global__ void __launch_bounds__(Traits::kThreads, Traits::kGroupsPerCu)
                 kf[1] = k_frag((j + 1) & 1, 1);
             }
             constexpr int kFirst = kNext ? 0 : kQkSlots;
-            auto exp_slot = [](int n) constexpr {  // the slot that exponential n (of 32) is computed in
-                return n < 16 ? n * (kQkSlots - 1) / 16 : kQkSlots - 1 + (n - 16) * (kPvHalf - 1) / 16;
+            constexpr int kExps = 16 * kQT, kHalf = 8 * kQT;
+            auto exp_slot = [](int n) constexpr {  // the slot that exponential n (of kExps) is computed in
+                return n < kHalf ? n * (kQkSlots - 1) / kHalf : kQkSlots - 1 + (n - kHalf) * (kPvHalf - 1) / kHalf;
             };
             auto exps = [&](auto n_) {
-                constexpr int n = n_, s = n / 16, t = (n / 2) % 2, e = 8 * s + (n % 16) / 4 * 2 + n % 2;
+                constexpr int n = n_, s = n / kHalf, t = (n / 2) % kQT, e = 8 * s + (n % kHalf) / (2 * kQT) * 2 + n % 2;
                 const float p = detail::exp2_raw(s_cur[t][e]);
                 l_run[t] += p;
                 pf[t][s][e % 8] = static_cast<_Float16>(p);
             };
             if constexpr (!kNext) {
-                detail::static_for<32>([&](auto n) { exps(n); });
+                detail::static_for<kExps>([&](auto n) { exps(n); });
                 asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
                 vf[0] = v_frag(j & 1, 0, 0);
                 vf[1] = v_frag(j & 1, 1, 0);
@@ -327,12 +337,15 @@ __global__ void __launch_bounds__(Traits::kThreads, Traits::kGroupsPerCu)
                     constexpr int s = i / kQT, t = i % kQT;
                     if constexpr (t == 0 && s + 2 < Traits::kDSteps) kf[(s + 2) % 3] = k_frag((j + 1) & 1, s + 2);
                     // with K of block j + 2, then V of block j + 1 requested behind the instruction
-                    constexpr bool kOfK = i < Traits::kLoads;
-                    constexpr int l = kOfK ? i : i - Traits::kLoads;
+                    constexpr int kPer = Traits::kLoadsPerSlot;
+                    constexpr bool kOfK = i * kPer < Traits::kLoads;
+                    constexpr int l = kOfK ? i * kPer : i * kPer - Traits::kLoads;
                     const unsigned off = load_off(kOfK ? k_off : v_off, l);
                     const unsigned dst = lds0 + (kOfK ? k_slot(j & 1) : v_slot((j + 1) & 1)) + l * 1024;
                     detail::mfma32_score_then_load<s == 0, Traits::kAgprQ>(s_nxt[t], kf[s % 3], qf[t][s], m_init[t], off,
                                                                            load_base(kOfK ? k_base : v_base, l), dst);
+                    if constexpr (kPer == 2)
+                        detail::load_lds_16B_sbase(load_off(kOfK ? k_off : v_off, l + 1), load_base(kOfK ? k_base : v_base, l + 1), dst + 1024);
                 } else {
                     constexpr int f = (i - kQkSlots) / kQT, t = i % kQT, s = f / Traits::kDTiles, dt = f % Traits::kDTiles;
                     constexpr int fn = f + 2;
@@ -341,21 +354,21 @@ __global__ void __launch_bounds__(Traits::kThreads, Traits::kGroupsPerCu)
                     o_acc[t][dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[f % 3], pf[t][s], o_acc[t][dt], 0, 0, 0);
                 }
                 if constexpr (kNext) {
-                    detail::static_for<32>([&](auto n) {
+                    detail::static_for<kExps>([&](auto n) {
                         if constexpr (exp_slot(n) == i) exps(n);
                     });
                     if constexpr (i == kQkSlots - 3) {
-                        // V of block j has landed: only this step's own i + 1 loads are younger
-                        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(i + 1) : "memory");
+                        // V of block j has landed: only this step's own loads, those of i + 1 slots, are younger
+                        asm volatile("s_waitcnt vmcnt(%0)" ::"n"((i + 1) * Traits::kLoadsPerSlot) : "memory");
                         vf[0] = v_frag(j & 1, 0, 0);
                         vf[1] = v_frag(j & 1, 1, 0);
                     }
                     constexpr int r = i - kQkSlots - 2;  // maxima of the next block's scores (written by instructions three slots back or more)
                     if constexpr (r >= 0) {
-                        constexpr int kPer = (32 + (kSlots - kQkSlots - 2) - 1) / (kSlots - kQkSlots - 2);
+                        constexpr int kPer = (kExps + (kSlots - kQkSlots - 2) - 1) / (kSlots - kQkSlots - 2);
                         detail::static_for<kPer>([&](auto u) {
                             constexpr int n = r * kPer + u;
-                            if constexpr (n < 32) {
+                            if constexpr (n < kExps) {
                                 constexpr int t = n / 16, e = n % 16;
                                 mx[t] = e == 0 ? s_nxt[t][0] : fmaxf(mx[t], s_nxt[t][e]);
                             }
@@ -365,7 +378,7 @@ __global__ void __launch_bounds__(Traits::kThreads, Traits::kGroupsPerCu)
                 __builtin_amdgcn_sched_barrier(0);
             });
             if constexpr (kNext) {
-                if (__any(fmaxf(mx[0], mx[1]) > kLazy)) {
+                if (__any((kQT == 2 ? fmaxf(mx[0], mx[kQT - 1]) : mx[0]) > kLazy)) {
 #pragma unroll
                     for (int t = 0; t < kQT; ++t) {
                         const float mxq = fmaxf(mx[t], detail::exchange32(mx[t]));
@@ -417,9 +430,9 @@ __global__ void __launch_bounds__(Traits::kThreads, Traits::kGroupsPerCu)
             }
     }
     detail::lds_barrier<0>();
-    {
+    static_assert(Traits::kThreads % (Traits::kBM * Traits::kWaves) == 0 && (Traits::kBM * Traits::kWaves) % kWaveSize == 0);
+    if (threadIdx.x < Traits::kBM * Traits::kWaves) {
         const int q = threadIdx.x / 4, w = threadIdx.x % 4;
-        static_assert(Traits::kThreads == Traits::kBM * Traits::kWaves);
         const float2 ml = stat[w * Traits::kBM + q];
         float mm = fmaxf(ml.x, __shfl_xor(ml.x, 1, 4));
         mm = fmaxf(mm, __shfl_xor(mm, 2, 4));

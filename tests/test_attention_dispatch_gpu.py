@@ -270,3 +270,26 @@ def test_many_rounds_of_query_blocks(tcu, device, batch, M, N, algo):
     """More than three rounds of blocks of 256 queries that are not whole: AUTO runs the 16x16x32 kernel unless its estimate is
     far behind. Bit for bit the kernel by name."""
     _auto_is(tcu, device, batch, M, N, algo)
+
+
+@pytest.mark.parametrize("D,v_layout,batches", [(128, "row", (1, 128, 129)), (128, "col", (3, 128, 129)), (64, "row", (2, 128, 129))])
+@pytest.mark.parametrize("M,N", [(64, 64), (64, 192), (64, 320)])
+def test_keys_kernel_with_32_and_64_queries(tcu, device, D, v_layout, batches, M, N):
+    """The largest launches of workgroups of 32 queries and the smallest of 64 beyond them, with one to three blocks per wavefront
+    and wavefronts without one, against f32 (f16 probabilities and output: 2^-11 each, 1.5e-3 as everywhere)."""
+    import torch
+
+    for batch in batches:
+        print(f"attention keys rows b{batch} {M}x{N} D{D} V {v_layout}", flush=True)
+        gen = torch.Generator(device=device)
+        gen.manual_seed(batch + N)
+        q, k, v = (torch.randn(batch, n, D, generator=gen, device=device).half() for n in (M, N, N))
+        scale = 1.0 / math.sqrt(D)
+        if v_layout == "row":
+            out = tcu.flash_attention(q, k, v, algo="keys")
+        else:
+            out = torch.full_like(q, 7.0)
+            tcu.flash_attention_fwd(q.flatten(), k.flatten(), v.transpose(1, 2).contiguous().flatten(), out.view(-1), M, N, D, D,
+                                    scale=scale, batch=batch, algo="keys")
+        want = torch.matmul(torch.softmax(torch.matmul(q.float(), k.float().transpose(1, 2).contiguous()) * scale, -1), v.float())
+        assert float((out.float() - want).norm() / want.norm()) <= 1.5e-3

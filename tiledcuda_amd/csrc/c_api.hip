@@ -1020,14 +1020,24 @@ int fa_fwd_by_rows(const __half* Q, const __half* K, const __half* V, __half* O,
     }
 }
 
+/// Whether the key-splitting kernel runs workgroups of 32 queries instead of 64: where twice as many of them still have a CU each, the
+/// shorter chain of a block counts for more than keys that are fetched twice. us, 64 ->
+/// 32 queries: head size 128, one head, 64 x 64: 6.1 -> 4.4; 64 x 256: 7.5 -> 5.5; 8 x 256 x 1024: 12.1 -> 9.1; 60 x 128 x 4096: 36.0 -> 34.0; 512 x
+/// 16384 with 16 splits: 17.9 -> 15.5; beyond (2 x 2048 x 4096 with 4 splits, 512 workgroups): 20.1 -> 23.3. Head size 64, 64 x 256: 5.1 ->
+/// 4.0; 32 x 64 x 1024: 8.3 -> 6.3; 128 x 64 x 1024: 9.0 -> 7.6; two per CU: 22 x 704 x 192: 5.7 -> 6.1, 44 x 320 x 4608: 27.0 -> 29.4.
+bool attn_keys_narrow(int batch, int M, int splits) { return (long)batch * splits * (M / 32) <= 256; }
+
 template <int kD, bool kVColMajor>
 int launch_fa_keys(const __half* Q, const __half* K, const __half* V, __half* O, float* part, int batch, int M, int N,
                    int splits, float scale, hipStream_t stream) {
-    using Traits = FlashKeysTraits<kD, kVColMajor>;
-    const long grid = (long)batch * splits * (M / Traits::kBM);
-    if (grid > INT_MAX || N >= (1 << 24)) return fail(TCU_ERR_UNSUPPORTED_SHAPE, "attention: too many query blocks or keys for one launch");
-    int rc = launch(&flash_attention_keys<Traits>, dim3(unsigned(grid)), dim3(Traits::kThreads), Traits::kLdsBytes, stream, Q,
-                    K, V, O, part, batch, M, N, splits, scale);
+    auto go = [&](auto traits) {
+        using Traits = decltype(traits);
+        const long grid = (long)batch * splits * (M / Traits::kBM);
+        if (grid > INT_MAX || N >= (1 << 24)) return fail(TCU_ERR_UNSUPPORTED_SHAPE, "attention: too many query blocks or keys for one launch");
+        return launch(&flash_attention_keys<Traits>, dim3(unsigned(grid)), dim3(Traits::kThreads), Traits::kLdsBytes, stream, Q, K, V, O, part,
+                      batch, M, N, splits, scale);
+    };
+    const int rc = attn_keys_narrow(batch, M, splits) ? go(FlashKeysTraits<kD, kVColMajor, 1>{}) : go(FlashKeysTraits<kD, kVColMajor>{});
     if (rc != TCU_OK || splits == 1) return rc;
     const size_t rows = size_t(batch) * M;
     auto combine = splits <= 4 ? &flash_attention_combine<kD, 4> : splits <= 8 ? &flash_attention_combine<kD, 8> : &flash_attention_combine<kD, 16>;
@@ -1069,6 +1079,15 @@ double attn_keys_us(int batch, int M, int N, int D, int splits) {
     }
     if (D == 128 && M == 192 && splits == 1) us = std::max(us, 6.5 + double(groups) * N * 512.0 / 9e6);
     return us + (splits == 1 ? 0.0 : 2.4 + (D == 128 ? 0.011 : 0.006) * groups);
+}
+
+/// ... with workgroups of 32 queries, of which there is one round (see attn_keys_narrow()): 1.6 us less before and after the blocks (0.8 at
+/// head size 64) and two thirds of the time per block.
+double attn_keys_narrow_us(int batch, int M, int N, int D, int splits) {
+    const double heads = double(batch) * splits, blocks = double(N) / (128.0 * splits), fill = heads * (M / 32) / 256;
+    const double us = D == 128 ? 4.9 + blocks * std::max(0.62 + 0.0052 * heads, 1.05 * fill)
+                               : 4.0 + blocks * std::max(0.45 + 0.0035 * heads, 0.58 * fill);
+    return us + (splits == 1 ? 0.0 : 2.4 + (D == 128 ? 0.011 : 0.006) * heads * (M / 64));
 }
 
 /// Expected time (us) of the kernels with 64 queries per wavefront in blocks of 256 (the 16x16x32 one, and the 32x32x16 one
@@ -1139,6 +1158,8 @@ int attn_keys_plan(int batch, int M, int N, int D, int v_layout, int max_splits)
     // the first keys of a few workgroups arrive 0.5 us sooner, those of a full chip 0.3 us later: beside the other kernels
     // that counts (8 x 128 x 192 at 128: 7.5 against 7.9 us, 7 x 1600 x 128: 7.7 against 7.0)
     if (D == 128 && best == 1) best_us += 0.8 * std::min(1.0, groups / 256.0) - 0.55;
+    // (the number of splits is that of workgroups of 64 queries: those of 32 shift it by a step at most, within the model's 6 %)
+    if (attn_keys_narrow(batch, M, best)) best_us = attn_keys_narrow_us(batch, M, N, D, best) + (best > 1 ? 2.5 : 0.0);
     return best_us < attn_blocks_us(batch, M, N, D, v_layout) ? best : 0;
 }
 
