@@ -177,12 +177,14 @@ HOST_DEVICE void xcd_tile_coords(int bid, int tiles_m, int tiles_n, int& tile_m,
 /// ceil(N / kBN) tiles, rows beyond the edge are loaded from the last valid row (their products are computed and
 /// dropped) and the stores are guarded; the loop runs over ceil(K / kBK) tiles, and in the last one every lane loads
 /// the 16-byte pieces that lie beyond K from the start of its row instead and, once they have landed, overwrites them
-/// in LDS with zeros. ldb, ldc: elements between consecutive stored rows of B (K for a dense B) and rows of C (N for a dense
-/// C). zero_words / zero_count: device words that the first workgroup sets to zero on the side (null / 0: none).
-template <typename Traits, typename OutType, bool kEdges = false>
+/// in LDS with zeros. ldc: elements between consecutive rows of C (N for a dense C). kSide: B's stored rows are ldb elements apart
+/// (else K), and the first workgroup sets zero_count device words at zero_words to zero on the side (for others these would cost the
+/// smallest products 0.2 us).
+template <typename Traits, typename OutType, bool kEdges = false, bool kSide = false>
 __global__ void __launch_bounds__(Traits::kThreads)
     gemm_pipelined(const __half* __restrict__ A, const __half* __restrict__ Bt, OutType* __restrict__ C, int M, int N,
-                   int K, int ldb, int ldc, unsigned int* __restrict__ zero_words, int zero_count) {
+                   int K, int side_ldb, int ldc, unsigned int* __restrict__ zero_words, int zero_count) {
+    const int ldb = kSide ? side_ldb : K;
     constexpr int kBM = Traits::kBM, kBN = Traits::kBN, kBK = Traits::kBK;
     constexpr int kMT = Traits::kMT, kNT = Traits::kNT, kKS = Traits::kKS;
 
@@ -192,8 +194,10 @@ __global__ void __launch_bounds__(Traits::kThreads)
     const int wave = __builtin_amdgcn_readfirstlane(wave_id());
     const int wave_m = wave / Traits::kWN;
     const int wave_n = wave % Traits::kWN;
-    if (zero_count > 0 && blockIdx.x == 0)
-        for (int i = threadIdx.x; i < zero_count; i += Traits::kThreads) zero_words[i] = 0u;
+    if constexpr (kSide) {
+        if (blockIdx.x == 0)
+            for (int i = threadIdx.x; i < zero_count; i += Traits::kThreads) zero_words[i] = 0u;
+    }
 
     int tile_m, tile_n;
     detail::xcd_tile_coords(blockIdx.x, kEdges ? (M + kBM - 1) / kBM : M / kBM, kEdges ? (N + kBN - 1) / kBN : N / kBN,

@@ -185,3 +185,25 @@ def test_gemm_split_k_in_many_ranges(tcu, oracle, device, M, N, K, splits, out_d
     rows = sorted({*range(min(M, 16)), *range(M - 16, M)})
     assert oracle.max_rel_err(got[rows], oracle.gemm(A[rows], Bt)) <= REL_TOL
     assert oracle.max_rel_err(got, tcu.gemm(a, b, out_dtype=torch.float32, workspace=False).cpu().numpy()) <= REL_TOL
+
+
+@pytest.mark.parametrize("M,N,K", [(1040, 1040, 1040), (1040, 1024, 1088),   # 96 x 64 tiles: rows 80 of 96, columns 16 of 64, K 16 of 64
+                                   (1312, 784, 624), (1312, 768, 80),
+                                   (2064, 1040, 1072), (1424, 1520, 1040)])  # 96 x 96: rows 48, 80 of 96, columns 80
+@pytest.mark.parametrize("out_dtype", ["float16", "float32"])
+def test_ring_tiles_with_96_rows(tcu, device, M, N, K, out_dtype):
+    """Products that AUTO gives the ring with 96 x 64 or 96 x 96 tiles, every element of the output and what lies behind it: f32 sums
+    in another order (1e-6 of the norm), rounded to f16 (2^-11) where the output is."""
+    import torch
+
+    print(f"gemm ring 96 {M}x{N}x{K} {out_dtype}", flush=True)
+    gen = torch.Generator(device=device)
+    gen.manual_seed(M + K)
+    a, b = (torch.rand(*s, generator=gen, device=device).mul_(2).sub_(1).half() for s in ((M, K), (N, K)))
+    dtype = getattr(torch, out_dtype)
+    buf = torch.full((M * N + 4096,), 7.0, dtype=dtype, device=device)
+    tcu.gemm(a, b, out=buf[:M * N].view(M, N), workspace=False)
+    want = a.double() @ b.double().t()
+    err = float((buf[:M * N].view(M, N).double() - want).norm() / want.norm())
+    assert err <= (1e-6 if dtype == torch.float32 else 2 ** -11)
+    assert bool((buf[M * N:] == 7.0).all())

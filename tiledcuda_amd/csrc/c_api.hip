@@ -188,6 +188,8 @@ using PipeLarge = PipelinedGemmTraits<256, 256, 64, 4, 2, 2>;  // 8 wavefronts, 
 using PipeMid = PipelinedGemmTraits<128, 128, 64, 2, 2, 2>;
 using PipeSmall = PipelinedGemmTraits<64, 64, 64, 2, 2, 2>;
 using PipeSmallRing = PipelinedGemmTraits<64, 64, 64, 2, 2, 4>;  // 4-stage ring, 64 KiB of LDS: 2 workgroups per CU
+using PipeTallRing = PipelinedGemmTraits<96, 64, 64, 2, 2, 4>;   // the same, 80 KiB
+using PipeWideRing = PipelinedGemmTraits<96, 96, 64, 2, 3, 4>;   // 6 wavefronts, 96 KiB: one workgroup per CU
 
 /// Which tile the pipelined kernel takes for a shape, and what the launch is expected to cost. A launch runs
 /// ceil(tiles / capacity) rounds of workgroups, capacity = 256 CUs x the workgroups of that size a CU holds (1, 2, 4),
@@ -218,10 +220,10 @@ PipePlan pipelined_plan(int M, int N, int K) {
 
 /// The pipelined kernel for M, N, K any multiples of 16, with the tile of pipelined_plan(). Edge tiles (rows clamped,
 /// stores guarded, the K tail zeroed in LDS) are compiled in only where the shape is not a whole number of the chosen
-/// tiles.
+/// tiles. ldb other than K and words to clear: f32 results only.
 template <typename OutType>
 int gemm_pipelined_dispatch(const __half* A, const __half* B, OutType* C, int M, int N, int K, hipStream_t stream,
-                            int ldc = 0, int ldb = 0, unsigned int* zero_words = nullptr, int zero_count = 0) {
+                            int ldc = 0, int ldb = 0, unsigned int* zero_words = nullptr, int zero_count = 0, bool wide_ring = false) {
     if (ldc == 0) ldc = N;
     if (ldb == 0) ldb = K;
     if (M % 16 != 0 || N % 16 != 0 || K % 16 != 0)
@@ -232,18 +234,30 @@ int gemm_pipelined_dispatch(const __half* A, const __half* B, OutType* C, int M,
         using Traits = decltype(traits);
         const long grid = (long)((M + Traits::kBM - 1) / Traits::kBM) * ((N + Traits::kBN - 1) / Traits::kBN);
         if (grid > INT_MAX) return fail(TCU_ERR_UNSUPPORTED_SHAPE, "GEMM: too many tiles for one launch");
+        if constexpr (std::is_same_v<OutType, float>)
+            if (ldb != K || zero_count > 0)
+                return launch(&gemm_pipelined<Traits, OutType, true, true>, dim3(unsigned(grid)), dim3(Traits::kThreads),
+                              Traits::template lds_bytes<OutType>(), stream, A, B, C, M, N, K, ldb, ldc, zero_words, zero_count);
         if (M % Traits::kBM == 0 && N % Traits::kBN == 0 && K % Traits::kBK == 0)
             return launch(&gemm_pipelined<Traits, OutType, false>, dim3(unsigned(grid)), dim3(Traits::kThreads),
                           Traits::template lds_bytes<OutType>(), stream, A, B, C, M, N, K, ldb, ldc, zero_words, zero_count);
         return launch(&gemm_pipelined<Traits, OutType, true>, dim3(unsigned(grid)), dim3(Traits::kThreads),
                       Traits::template lds_bytes<OutType>(), stream, A, B, C, M, N, K, ldb, ldc, zero_words, zero_count);
     };
+    if (wide_ring) return go(PipeWideRing{});
     switch (pipelined_plan(M, N, K).config) {
         case kPipeLarge: return go(PipeLarge{});
         case kPipeMid: return go(PipeMid{});
         case kPipeSmall: return go(PipeSmall{});
-        default: return go(PipeSmallRing{});
+        default: break;
     }
+    // the ring, more than one 64 x 64 tile per CU, M not whole tiles: tiles of 96 x 64 where there is at most one of them per CU (us,
+    // f16, 64 x 64 -> 96 x 64: 1040^2 x 2064: 19.2 -> 15.1; 1312 x 784 x 2832: 24.7 -> 19.0; 624 x 2000 x 1232: 10.8, 11.1; whole tiles have
+    // no edges to lose: 832 x 1664 x 1152: 8.9, 9.4; f32 results, 32 bytes per lane and row, gain at long K only: 1184 x 1120 x 672: 8.1,
+    // 8.3)
+    const long small = (long)((M + 63) / 64) * ((N + 63) / 64), tall = (long)((M + 95) / 96) * ((N + 63) / 64);
+    if (sizeof(OutType) == 2 && M % 64 != 0 && small > 256 && small <= 512 && tall <= 256) return go(PipeTallRing{});
+    return go(PipeSmallRing{});
 }
 
 template <typename OutType>
@@ -444,6 +458,16 @@ double gemm_w128_us(long tiles, int K) {
     const double fill = last / 256.0;
     const double last_us = full == 0 ? std::max(17.0, 10.6 + 12.9 * fill) : std::min(23.5, 12.0 + 20.0 * fill);
     return 3.0 + (K / 1024.0) * (23.5 * full + last_us);
+}
+
+/// Whether a product that the K-splitting kernel would take (about one tile of 128 x 128 or 128 x 96 per CU) goes to the pipelined
+/// kernel's ring with tiles of 96 x 96 instead: with a K this short the sums over the wavefronts cost more than the fragments that they
+/// share save. One workgroup per CU, 2.5 us + per 1024 of K 6.2 us with few of them, 8.4 with 256; a K tail costs the other kernel
+/// 1 us. us, K-splitting -> this: 2064 x 1040 x 1072: 13.0 -> 12.0; longer K stays: 2048 x 1024 x 4096: 26.9, 31.0.
+bool gemm_wide_ring_is_the_choice(int M, int N, int K) {
+    const long tiles = (long)((M + 95) / 96) * ((N + 95) / 96);
+    if (tiles > 256 || (long)K * 512 >= (1l << 32)) return false;
+    return 2.5 + (6.2 + 2.2 * double(tiles) / 256.0) * K / 1024.0 < 0.97 * (gemm_w128k_us(M, N, K) + (K % 128 != 0 ? 1.0 : 0.0));
 }
 
 /// More than one round of 256 x 256 tiles, the last of them far from full (2560 x 8192: 320 tiles, the last 64 of which
@@ -693,7 +717,10 @@ int gemm_dispatch(const __half* A, const __half* B, OutType* C, int M, int N, in
             }
             // too few 256 x 256 tiles for the chip, but about one 128 x 128 tile per CU and a long enough K: the
             // kernel whose wavefronts split K (each owns the whole tile)
-            if (gemm_w128k_is_the_choice(M, N, K)) return gemm_w128k_dispatch<OutType>(A, B, C, M, N, K, stream);
+            if (gemm_w128k_is_the_choice(M, N, K)) {
+                if (gemm_wide_ring_is_the_choice(M, N, K)) return gemm_pipelined_dispatch<OutType>(A, B, C, M, N, K, stream, 0, 0, nullptr, 0, true);
+                return gemm_w128k_dispatch<OutType>(A, B, C, M, N, K, stream);
+            }
             // between the two: 256 x 128 tiles fill one round
             if (gemm_narrow_is_the_choice(M, N, K)) return gemm_w128_narrow_dispatch<OutType>(A, B, C, M, N, K, stream);
             if (M % 16 == 0 && N % 16 == 0) {
