@@ -38,20 +38,23 @@ struct GemmDirectTraits {
     static_assert(kLdsBytes <= kMaxLdsBytes);
 };
 
-/// grid = ceil(N / kBN) * ceil(M / kBM), block = 512, dynamic LDS = T::kLdsBytes. M, N, K multiples of 16, K and ldb (the
-/// distance of B's stored rows, in elements) < 2^24 (32-bit byte offsets inside a tile's rows). zero_words / zero_count: device
-/// words that the first workgroup sets to zero on the side (null / 0: none).
-template <typename T, typename OutType>
+/// grid = ceil(N / kBN) * ceil(M / kBM), block = 512, dynamic LDS = T::kLdsBytes. M, N, K multiples of 16, K < 2^24 (32-bit
+/// byte offsets inside a tile's rows). kSide: B's stored rows are side_ldb < 2^24 elements apart (else K), and the first workgroup
+/// sets zero_count device words at zero_words to zero on the side (for others these would cost up to 0.1 us of 2.4).
+template <typename T, typename OutType, bool kSide = false>
 __global__ void __launch_bounds__(T::kThreads)
-    gemm_direct(const __half* __restrict__ A, const __half* __restrict__ Bt, OutType* __restrict__ C, int M, int N, int K, int ldb,
+    gemm_direct(const __half* __restrict__ A, const __half* __restrict__ Bt, OutType* __restrict__ C, int M, int N, int K, int side_ldb,
                 unsigned int* __restrict__ zero_words, int zero_count) {
+    const int ldb = kSide ? side_ldb : K;
     constexpr int kUT = T::kUT, kRT = T::kRT, kRing = T::kRing, kBK = T::kBK, kWaves = T::kWaves;
     extern __shared__ __align__(1024) unsigned char lds[];
     const int lane = lane_id();
     const int wave = __builtin_amdgcn_readfirstlane(wave_id());
     const int line = lane & 15, group = lane >> 4;
-    if (zero_count > 0 && blockIdx.x == 0)
-        for (int i = threadIdx.x; i < zero_count; i += T::kThreads) zero_words[i] = 0u;
+    if constexpr (kSide) {
+        if (blockIdx.x == 0)
+            for (int i = threadIdx.x; i < zero_count; i += T::kThreads) zero_words[i] = 0u;
+    }
 
     // The blocks that share rows of the larger operand run on one XCD: these rows come to one L2 only. (With the row blocks of
     // one column block together whatever M and N: 4096 x 256 x 8192 41.4 us, 2048 x 256 x 8192 40.0, 8192 x 64 x 4096 21.1; in

@@ -628,8 +628,10 @@ int gemm_direct_dispatch(const __half* A, const __half* B, OutType* C, int M, in
     auto go = [&](auto traits) {
         using T = decltype(traits);
         const long grid = (long)((M + T::kBM - 1) / T::kBM) * ((N + T::kBN - 1) / T::kBN);
-        return launch(&gemm_direct<T, OutType>, dim3(unsigned(grid)), dim3(T::kThreads), T::kLdsBytes, stream, A, B, C, M, N, K, ldb,
-                      zero_words, zero_count);
+        auto kernel = &gemm_direct<T, OutType>;
+        if constexpr (std::is_same_v<OutType, float>)  // (the only results that come with a row distance of B or words to clear)
+            if (ldb != K || zero_count > 0) kernel = &gemm_direct<T, OutType, true>;
+        return launch(kernel, dim3(unsigned(grid)), dim3(T::kThreads), T::kLdsBytes, stream, A, B, C, M, N, K, ldb, zero_words, zero_count);
     };
     switch (10 * plan.ut + plan.rt) {
         case 11: return go(GemmDirectTraits<1, 1>{});
