@@ -254,9 +254,9 @@ int gemm_pipelined_dispatch(const __half* A, const __half* B, OutType* C, int M,
     // the ring, more than one 64 x 64 tile per CU, M not whole tiles: tiles of 96 x 64 where there is at most one of them per CU (us,
     // f16, 64 x 64 -> 96 x 64: 1040^2 x 2064: 19.2 -> 15.1; 1312 x 784 x 2832: 24.7 -> 19.0; 624 x 2000 x 1232: 10.8, 11.1; whole tiles have
     // no edges to lose: 832 x 1664 x 1152: 8.9, 9.4; f32 results, 32 bytes per lane and row, gain at long K only: 1184 x 1120 x 672: 8.1,
-    // 8.3)
+    // 8.3; a single step of K nowhere: 1968 x 768 x 64: 3.4, 3.5)
     const long small = (long)((M + 63) / 64) * ((N + 63) / 64), tall = (long)((M + 95) / 96) * ((N + 63) / 64);
-    if (sizeof(OutType) == 2 && M % 64 != 0 && small > 256 && small <= 512 && tall <= 256) return go(PipeTallRing{});
+    if (sizeof(OutType) == 2 && M % 64 != 0 && K >= 256 && small > 256 && small <= 512 && tall <= 256) return go(PipeTallRing{});
     return go(PipeSmallRing{});
 }
 
