@@ -375,6 +375,9 @@ __global__ void __launch_bounds__(Traits::kThreads, 1)
             } else {
                 detail::lds_barrier<0>();
                 read_pre(t);
+                // (one buffer: the next step's go where every wavefront has read this one's. Beside an h_prev the barrier of its
+                // second part lies between the two)
+                if constexpr (Traits::kPreBuffers == 1) detail::lds_barrier<63>();
                 if (next_t >= 0) load_pre(next_t, slice);
 #pragma unroll
                 for (int n = 0; n < kTW; ++n)

@@ -47,6 +47,22 @@ def test_lstm_layer_matches_the_steps(tcu, device, T, B, I, H, state):
     assert bool((h_buf[T * B * H:] == 7.0).all()) and bool((c_buf[B * H:] == 7.0).all()) and bool((ws[need:] == 0x5A).all())
 
 
+@pytest.mark.parametrize("T,B,I,H", [(2, 16, 16, 16), (3, 144, 64, 128), (2, 80, 64, 656),                         # two buffers of pre-activations
+                                     (2, 144, 48, 272), (3, 256, 64, 512), (2, 208, 48, 656), (2, 16, 64, 784),      # one: H > 768, or
+                                     (3, 80, 48, 1024), (2, 512, 48, 1008)])                                          # more than 128 rows and H > 256
+def test_lstm_layer_without_an_initial_state(tcu, device, T, B, I, H):
+    """No h0 is an h0 of zeros, bit for bit: the products of zeros add nothing to the pre-activations, whichever way step 0 takes them."""
+    import torch
+
+    print(f"lstm layer no h0 T{T} B{B} I{I} H{H}", flush=True)
+    x, W, b, h0, c0 = operands(tcu, device, T, B, I, H)
+    want = tcu.lstm(x, W, b, torch.zeros_like(h0), c0, algo="layer")
+    assert close(want, tcu.lstm(x, W, b, None, c0, workspace=False))
+    for _ in range(8):
+        got = tcu.lstm(x, W, b, None, c0, algo="layer")
+        assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+
+
 def test_lstm_layer_against_the_oracle(tcu, oracle, device):
     import torch
 
