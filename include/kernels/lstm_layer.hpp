@@ -411,6 +411,8 @@ __global__ void __launch_bounds__(Traits::kThreads, 1)
         for (;;) {
             const int slice = __builtin_amdgcn_readfirstlane(s_tile[i]);
             if (!ahead) {
+                // (what was requested for a next step, before another slice came in between, may have the same place: landed first)
+                __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
                 __syncthreads();
                 if (t == 0) fill(slice);
                 load_pre(t, slice);

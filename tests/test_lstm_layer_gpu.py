@@ -78,12 +78,13 @@ def test_lstm_layer_against_the_oracle(tcu, oracle, device):
 
 
 @pytest.mark.parametrize("T,B,I,H,grid", [(5, 80, 64, 112, 1), (5, 80, 64, 112, 8), (5, 80, 64, 112, 40), (4, 144, 96, 656, 9),
-                                          (4, 256, 64, 1024, 100), (4, 336, 64, 320, 24)])
-def test_lstm_layer_with_few_workgroups(tcu, device, monkeypatch, T, B, I, H, grid):
+                                          (4, 256, 64, 1024, 100), (4, 336, 64, 320, 24), (3, 16, 64, 784, 5), (3, 160, 64, 272, 9)])
+@pytest.mark.parametrize("state", [False, True])
+def test_lstm_layer_with_few_workgroups(tcu, device, monkeypatch, T, B, I, H, grid, state):
     """Slices without a workgroup are taken over by those that run, groups of rows by XCDs that are done; at the smallest, one
     workgroup does everything."""
-    print(f"lstm layer T{T} B{B} I{I} H{H} grid {grid}", flush=True)
-    args = operands(tcu, device, T, B, I, H)
+    print(f"lstm layer T{T} B{B} I{I} H{H} grid {grid} state={state}", flush=True)
+    args = operands(tcu, device, T, B, I, H, state)
     want = tcu.lstm(*args, workspace=False)
     monkeypatch.setenv("TCU_LSTM_LAYER_GRID", str(grid))
     assert close(tcu.lstm(*args, algo="layer"), want)
