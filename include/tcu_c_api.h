@@ -273,11 +273,12 @@ int tcu_lstm_f16_ws(const void* x, const void* W, const void* bias, const void* 
 /*
  * The LSTM layer in two launches: the input half of the gates of all steps as one GEMM into `workspace` (f32, as in
  * tcu_lstm_f16_ws), then the whole time loop as one launch that keeps the recurrent weights in registers. T >= 2, B, I and H in
- * multiples of 16, H <= 1024, B <= 2048 (tcu_lstm_layer_workspace_bytes returns 0 for shapes this path does not take). Same arguments and results (up to the order of the f32 summation) as tcu_lstm_f16; nothing is asked of
- * the GPU: workgroups that are not resident are stood in for by those that are, and every wait is for a workgroup that runs.
+ * multiples of 16, H <= 1024, B <= 2048 (tcu_lstm_layer_workspace_bytes returns 0 for shapes this path does not take). Same
+ * arguments and results (up to the order of the f32 summation) as tcu_lstm_f16; nothing is asked of the GPU: workgroups that are
+ * not resident are stood in for by those that are, and every wait is for a workgroup that runs.
  * `workspace`: device memory of at least tcu_lstm_layer_workspace_bytes(T, B, I, H) bytes, 16-byte aligned, owned by the caller
- * and free to reuse once the work enqueued here has run; its first 4 KiB are synchronisation words, cleared by the call. Calls that
- * may overlap in time need a workspace each. An h0 that lies inside h_all runs the step kernels of tcu_lstm_f16 instead. No
+ * and free to reuse once the work enqueued here has run; its first 4 KiB are synchronisation words, cleared by the call. Calls
+ * that may overlap in time need a workspace each. An h0 that lies inside h_all runs the step kernels of tcu_lstm_f16 instead. No
  * counterpart in the reference (it has no LSTM).
  */
 unsigned long long tcu_lstm_layer_workspace_bytes(int T, int B, int I, int H);
@@ -286,6 +287,11 @@ unsigned long long tcu_lstm_layer_workspace_bytes(int T, int B, int I, int H);
 int tcu_lstm_uses_layer(int T, int B, int I, int H);
 int tcu_lstm_f16_layer(const void* x, const void* W, const void* bias, const void* h0, const void* c0, void* h_all, void* c_out,
                        int T, int B, int I, int H, void* workspace, unsigned long long workspace_bytes, void* stream);
+/* The same with at most `max_workgroups` workgroups, of which those that have waited `takeover_us` stand in for the others: for
+ * tests of a layer that does not get the GPU it has room for. */
+int tcu_lstm_f16_layer_limited(const void* x, const void* W, const void* bias, const void* h0, const void* c0, void* h_all,
+                               void* c_out, int T, int B, int I, int H, void* workspace, unsigned long long workspace_bytes,
+                               int max_workgroups, int takeover_us, void* stream);
 
 /*
  * The LSTM layer with the whole time loop in ONE launch, for the large-hidden-size case where a step is bound by

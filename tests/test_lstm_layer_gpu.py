@@ -23,6 +23,22 @@ def close(got, want, tol=STEP_TOL):
     return all(float((g.float() - w.float()).abs().max()) <= tol for g, w in zip(got, want))
 
 
+def limited(tcu, args, workgroups, takeover_us=30):
+    """The layer in a launch of at most ``workgroups`` workgroups."""
+    import torch
+
+    x, W, b, h0, c0 = args
+    T, B, I = x.shape
+    H = b.numel() // 4
+    need = int(tcu.lib().tcu_lstm_layer_workspace_bytes(T, B, I, H))
+    ws = torch.full((need,), 0x5A, dtype=torch.uint8, device=x.device)
+    h_all, c_T = torch.empty(T, B, H, dtype=torch.float16, device=x.device), torch.empty(B, H, device=x.device)
+    ptr = lambda t: 0 if t is None else t.data_ptr()
+    tcu._check(tcu.lib().tcu_lstm_f16_layer_limited(*map(ptr, (x, W, b, h0, c0, h_all, c_T)), T, B, I, H, ptr(ws), need, workgroups,
+                                                    takeover_us, tcu._stream()))
+    return h_all, c_T
+
+
 @pytest.mark.parametrize("T,B,I,H", [(2, 16, 16, 16), (3, 48, 64, 112), (5, 128, 80, 128),    # 16 units, 128 columns
                                      (4, 144, 64, 64), (3, 240, 96, 128),                     # ... 32 rows, 16 of 32 in the last group
                                      (4, 80, 128, 144), (3, 160, 64, 256),                    # 256 columns
@@ -80,14 +96,25 @@ def test_lstm_layer_against_the_oracle(tcu, oracle, device):
 @pytest.mark.parametrize("T,B,I,H,grid", [(5, 80, 64, 112, 1), (5, 80, 64, 112, 8), (5, 80, 64, 112, 40), (4, 144, 96, 656, 9),
                                           (4, 256, 64, 1024, 100), (4, 336, 64, 320, 24), (3, 16, 64, 784, 5), (3, 160, 64, 272, 9)])
 @pytest.mark.parametrize("state", [False, True])
-def test_lstm_layer_with_few_workgroups(tcu, device, monkeypatch, T, B, I, H, grid, state):
+def test_lstm_layer_with_few_workgroups(tcu, device, T, B, I, H, grid, state):
     """Slices without a workgroup are taken over by those that run, groups of rows by XCDs that are done; at the smallest, one
     workgroup does everything."""
+    import torch
+
     print(f"lstm layer T{T} B{B} I{I} H{H} grid {grid} state={state}", flush=True)
     args = operands(tcu, device, T, B, I, H, state)
     want = tcu.lstm(*args, workspace=False)
-    monkeypatch.setenv("TCU_LSTM_LAYER_GRID", str(grid))
-    assert close(tcu.lstm(*args, algo="layer"), want)
+    layer = tcu.lstm(*args, algo="layer")
+    assert close(layer, want)
+    got = limited(tcu, args, grid)
+    assert torch.equal(got[0], layer[0]) and torch.equal(got[1], layer[1])
+
+
+def test_lstm_layer_limits_are_checked(tcu, device):
+    args = operands(tcu, device, 2, 16, 16, 16)
+    for limits in ((0, 30), (-1, 30), (8, -1), (8, 1000001)):
+        with pytest.raises(RuntimeError, match="workgroup"):
+            limited(tcu, args, *limits)
 
 
 def test_lstm_layer_two_streams_and_nan(tcu, device):

@@ -120,7 +120,7 @@ bool aligned16(std::initializer_list<const void*> v) {
 // array's name is only a handle for hipGetSymbolAddress, never a device address.
 constexpr unsigned long long kScratchBytes = 64ull << 20;
 constexpr unsigned long long kPersistentSyncBytes = 4096;  // synchronisation words in front of the pre-activations
-constexpr int kLstmLayerStealTicks = 3000;  // 30 us (100 MHz): long against the start of a grid, short against its steps
+constexpr int kLstmLayerTakeoverUs = 30;  // long against the start of a grid, short against its steps
 static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 
 constexpr int kMaxDevices = 64;
@@ -1485,18 +1485,25 @@ bool lstm_layer_pays(int T, int B, int I, int H) {
     return 1.05 * (lstm_layer_projection((long)T * B, I, H).us + layer) < T * lstm_step_us(B, H, I + H);
 }
 
+/// What a launch of lstm_layer_xcd may use; other values than these are for tests (tcu_lstm_f16_layer_limited).
+struct LstmLayerLimits {
+    int workgroups = INT_MAX;
+    int takeover_us = kLstmLayerTakeoverUs;
+};
+
 template <int kTW, int kKS, int kRT>
 int launch_lstm_layer_xcd(const float* pre, const __half* W, const __half* bias, const __half* h0, const float* c0, __half* h_all,
-                          float* c_out, int T, int B, int I, int H, unsigned int* sync, int grid_limit, hipStream_t s) {
+                          float* c_out, int T, int B, int I, int H, unsigned int* sync, const LstmLayerLimits& limits, hipStream_t s) {
     using Traits = LstmLayerTraits<kTW, kKS, kRT>;
     const int peers = (H + Traits::kUnits - 1) / Traits::kUnits;
-    const int grid = grid_limit > 0 ? std::min(grid_limit, 8 * peers) : 8 * peers;
+    const int grid = std::min(limits.workgroups, 8 * peers);
     return launch(&lstm_layer_xcd<Traits>, dim3(unsigned(grid)), dim3(Traits::kThreads), Traits::kLdsBytes, s, pre, W, I + H, I, bias, h0,
-                  c0, h_all, c_out, T, B, H, sync, kLstmLayerStealTicks);
+                  c0, h_all, c_out, T, B, H, sync, limits.takeover_us * 100);
 }
 
 int launch_lstm_layer(const __half* x, const __half* W, const __half* bias, const __half* h0, const float* c0, __half* h_all,
-                      float* c_out, int T, int B, int I, int H, unsigned char* workspace, int grid_limit, hipStream_t s) {
+                      float* c_out, int T, int B, int I, int H, unsigned char* workspace, const LstmLayerLimits& limits,
+                      hipStream_t s) {
     auto sync = reinterpret_cast<unsigned int*>(workspace);
     auto pre = reinterpret_cast<float*>(workspace + kPersistentSyncBytes);
     constexpr int kSyncWords = LstmLayerTraits<1, 4, 1>::kSyncWords;
@@ -1521,8 +1528,8 @@ int launch_lstm_layer(const __half* x, const __half* W, const __half* bias, cons
     auto go = [&](auto tw, auto ks) {
         constexpr int kTW = decltype(tw)::value, kKS = decltype(ks)::value;
         if (lstm_layer_row_tiles(B) == 1)
-            return launch_lstm_layer_xcd<kTW, kKS, 1>(pre, W, bias, h0, c0, h_all, c_out, T, B, I, H, sync, grid_limit, s);
-        return launch_lstm_layer_xcd<kTW, kKS, 2>(pre, W, bias, h0, c0, h_all, c_out, T, B, I, H, sync, grid_limit, s);
+            return launch_lstm_layer_xcd<kTW, kKS, 1>(pre, W, bias, h0, c0, h_all, c_out, T, B, I, H, sync, limits, s);
+        return launch_lstm_layer_xcd<kTW, kKS, 2>(pre, W, bias, h0, c0, h_all, c_out, T, B, I, H, sync, limits, s);
     };
     using one = std::integral_constant<int, 1>;
     using two = std::integral_constant<int, 2>;
@@ -1544,6 +1551,29 @@ int launch_lstm_recurrent_xcd(const __half* pre, const __half* W, const void* bi
                   W, I + kH, I, static_cast<const __half*>(bias), static_cast<const __half*>(h0),
                   static_cast<const float*>(c0), static_cast<__half*>(h_all), static_cast<float*>(c_out), T, B, sync,
                   spin_us * 100ull, peers);
+}
+
+/// tcu_lstm_f16_layer within `limits`.
+int lstm_f16_layer(const void* x, const void* W, const void* bias, const void* h0, const void* c0, void* h_all, void* c_out, int T, int B,
+                   int I, int H, void* workspace, unsigned long long workspace_bytes, const LstmLayerLimits& limits, void* stream) {
+    if (!x || !W || !bias || !h_all || !c_out || !workspace) return fail(TCU_ERR_INVALID_ARGUMENT, "tcu_lstm_f16_layer: null pointer");
+    if (!positive({T, B, I, H})) return fail(TCU_ERR_INVALID_ARGUMENT, "tcu_lstm_f16_layer: sizes must be positive");
+    if (!aligned16({x, W, bias, h0, c0, h_all, c_out, workspace}))
+        return fail(TCU_ERR_INVALID_ARGUMENT, "tcu_lstm_f16_layer: operands must be 16-byte aligned");
+    const unsigned long long need = tcu_lstm_layer_workspace_bytes(T, B, I, H);
+    if (need == 0)
+        return fail(TCU_ERR_UNSUPPORTED_SHAPE, "tcu_lstm_f16_layer: needs T >= 2, B, I and H in multiples of 16, H <= 1024 and B <= 2048");
+    if (workspace_bytes < need)
+        return fail(TCU_ERR_INVALID_ARGUMENT, "tcu_lstm_f16_layer: workspace smaller than tcu_lstm_layer_workspace_bytes()");
+    // the kernel marks all of h_all before its first step: an initial state inside it (the last step of an earlier call that
+    // wrote the same tensor) goes to the kernels that write a step at a time
+    const auto h0_first = reinterpret_cast<uintptr_t>(h0), all_first = reinterpret_cast<uintptr_t>(h_all);
+    if (h0 && h0_first < all_first + size_t(T) * B * H * 2 && all_first < h0_first + size_t(B) * H * 2)
+        return tcu_lstm_f16_algo(x, W, bias, h0, c0, h_all, c_out, T, B, I, H, TCU_LSTM_AUTO, stream);
+    return launch_lstm_layer(static_cast<const __half*>(x), static_cast<const __half*>(W), static_cast<const __half*>(bias),
+                             static_cast<const __half*>(h0), static_cast<const float*>(c0), static_cast<__half*>(h_all),
+                             static_cast<float*>(c_out), T, B, I, H, static_cast<unsigned char*>(workspace), limits,
+                             static_cast<hipStream_t>(stream));
 }
 }  // namespace
 
@@ -1750,26 +1780,15 @@ int tcu_lstm_uses_layer(int T, int B, int I, int H) { return positive({T, B, I, 
 
 int tcu_lstm_f16_layer(const void* x, const void* W, const void* bias, const void* h0, const void* c0, void* h_all, void* c_out,
                        int T, int B, int I, int H, void* workspace, unsigned long long workspace_bytes, void* stream) {
-    if (!x || !W || !bias || !h_all || !c_out || !workspace) return fail(TCU_ERR_INVALID_ARGUMENT, "tcu_lstm_f16_layer: null pointer");
-    if (!positive({T, B, I, H})) return fail(TCU_ERR_INVALID_ARGUMENT, "tcu_lstm_f16_layer: sizes must be positive");
-    if (!aligned16({x, W, bias, h0, c0, h_all, c_out, workspace}))
-        return fail(TCU_ERR_INVALID_ARGUMENT, "tcu_lstm_f16_layer: operands must be 16-byte aligned");
-    const unsigned long long need = tcu_lstm_layer_workspace_bytes(T, B, I, H);
-    if (need == 0)
-        return fail(TCU_ERR_UNSUPPORTED_SHAPE, "tcu_lstm_f16_layer: needs T >= 2, B, I and H in multiples of 16, H <= 1024 and B <= 2048");
-    if (workspace_bytes < need)
-        return fail(TCU_ERR_INVALID_ARGUMENT, "tcu_lstm_f16_layer: workspace smaller than tcu_lstm_layer_workspace_bytes()");
-    // the kernel marks all of h_all before its first step: an initial state inside it (the last step of an earlier call that
-    // wrote the same tensor) goes to the kernels that write a step at a time
-    const auto h0_first = reinterpret_cast<uintptr_t>(h0), all_first = reinterpret_cast<uintptr_t>(h_all);
-    if (h0 && h0_first < all_first + size_t(T) * B * H * 2 && all_first < h0_first + size_t(B) * H * 2)
-        return tcu_lstm_f16_algo(x, W, bias, h0, c0, h_all, c_out, T, B, I, H, TCU_LSTM_AUTO, stream);
-    int grid_limit = 0;  // fewer workgroups than the layer has slices (to exercise that they are taken over)
-    if (const char* e = std::getenv("TCU_LSTM_LAYER_GRID")) grid_limit = int(std::strtol(e, nullptr, 10));
-    return launch_lstm_layer(static_cast<const __half*>(x), static_cast<const __half*>(W), static_cast<const __half*>(bias),
-                             static_cast<const __half*>(h0), static_cast<const float*>(c0), static_cast<__half*>(h_all),
-                             static_cast<float*>(c_out), T, B, I, H, static_cast<unsigned char*>(workspace), grid_limit,
-                             static_cast<hipStream_t>(stream));
+    return lstm_f16_layer(x, W, bias, h0, c0, h_all, c_out, T, B, I, H, workspace, workspace_bytes, LstmLayerLimits{}, stream);
+}
+
+int tcu_lstm_f16_layer_limited(const void* x, const void* W, const void* bias, const void* h0, const void* c0, void* h_all, void* c_out,
+                               int T, int B, int I, int H, void* workspace, unsigned long long workspace_bytes, int max_workgroups,
+                               int takeover_us, void* stream) {
+    if (max_workgroups < 1 || takeover_us < 0 || takeover_us > 1000000)
+        return fail(TCU_ERR_INVALID_ARGUMENT, "tcu_lstm_f16_layer_limited: at least one workgroup, 0 <= takeover_us <= 1000000");
+    return lstm_f16_layer(x, W, bias, h0, c0, h_all, c_out, T, B, I, H, workspace, workspace_bytes, {max_workgroups, takeover_us}, stream);
 }
 
 unsigned long long tcu_lstm_persistent_workspace_bytes(int T, int B, int I, int H) {
