@@ -18,7 +18,8 @@
 // XCD is read from the hardware); before step 1 they wait until all slices have filled their words with ~0, and whoever has waited
 // `steal_ticks` draws another ticket and works on that slice as well, weights fetched anew per step: slow, and right with a single
 // workgroup. Groups of rows are claimed by XCD, and an XCD that is done claims another. So the layer needs no part of the GPU for
-// itself. (The waits count their tries all the same and leave h_all ~0 if one should not end.)
+// itself. (The waits count their tries all the same. A wavefront that gives one up goes on with cell states of NaN: its units are NaN
+// from that step on, and one step later so is all that is computed from them.)
 // Measured, kernel alone, us: T 24, B 80, H 656: 55 (6 us until the first workgroups know their rows, 7 for the weights, 1.75 per step:
 // 0.45 for h to come back from the L2, 0.2 to LDS, 0.6 for 48 products and their fragments, 0.3 for the cell); 16, 256, 1024: 79
 // (3.9 per step: the LDS, 64 KB of h in and 256 KB of fragments out, and h itself, 64 KB at 45 bytes per clock); 31, 80, 384: 48;
@@ -93,13 +94,13 @@ DEVICE void mfma16_weights_in_agprs(f32x4& acc, const f16x8& w, const f16x8& h) 
 /// grid = 8 * ceil(H / kUnits) (fewer work as well), block = 256, dynamic LDS = Traits::kLdsBytes; pre [T, B, 4H]; the recurrent
 /// block of W starts at column w_col0 of rows of ldw; h0 / c0 may be null (zeros), h0 must not overlap h_all; sync: kSyncWords device
 /// words, zero at the launch: per XCD (32 words apart) tickets, the group that its first workgroup found and slices filled, then
-/// whose each group of rows is. T >= 2, B <= kMaxGroups * kRows, 4H * ldw below 2^31.
+/// whose each group of rows is. max_tries: polls of a wait. T >= 2, B <= kMaxGroups * kRows, 4H * ldw below 2^31.
 template <typename Traits>
 __global__ void __launch_bounds__(Traits::kThreads, 1)
     lstm_layer_xcd(const float* __restrict__ pre, const __half* __restrict__ W, int ldw, int w_col0, const __half* __restrict__ bias,
-                   const __half* h0, const float* c0, __half* h_all, float* c_out, int T, int B, int H, unsigned int* sync, int steal_ticks) {
+                   const __half* h0, const float* c0, __half* h_all, float* c_out, int T, int B, int H, unsigned int* sync, int steal_ticks,
+                   int max_tries) {
     constexpr int kTW = Traits::kTW, kKS = Traits::kKS, kRT = Traits::kRT, kParts = Traits::kParts, kLoads = Traits::kLoads, kPitch = Traits::kPitch;
-    constexpr int kSpinLimit = 1 << 24;
     extern __shared__ __align__(1024) unsigned char lds[];
     __shared__ int s_word[2];
     __shared__ unsigned char s_tile[Traits::kMaxPeers];
@@ -140,6 +141,7 @@ __global__ void __launch_bounds__(Traits::kThreads, 1)
     if (__builtin_amdgcn_readfirstlane(s_word[0]) >= peers) return;
     int group = __builtin_amdgcn_readfirstlane(s_word[1]);
     int tiles = 1, served = 0;  // slices held; groups that the XCD has had so far
+    int limit = max_tries;      // -1: this wavefront has given up a wait
     __syncthreads();
 
     const unsigned lds0 = static_cast<unsigned>(reinterpret_cast<uintptr_t>(lds));
@@ -203,7 +205,7 @@ __global__ void __launch_bounds__(Traits::kThreads, 1)
                     __hip_atomic_store(group_word, unsigned(served + 1) << 16 | unsigned(mine), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 } else {
 #pragma unroll 1
-                    for (int n = 0; n < kSpinLimit; ++n) {
+                    for (int n = 0; n <= limit; ++n) {  // (given up: the workgroup leaves, whose slice the others of the next group miss)
                         const unsigned v = __hip_atomic_load(group_word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                         if ((v >> 16) == unsigned(served + 1)) {
                             mine = int(v & 0xffffu);
@@ -304,7 +306,7 @@ __global__ void __launch_bounds__(Traits::kThreads, 1)
             }
         };
         // One step of one slice. next_t: the step whose pre-activations are to be requested (or -1).
-        auto step = [&](int t, int slice, int next_t) __attribute__((always_inline)) -> bool {
+        auto step = [&](int t, int slice, int next_t) __attribute__((always_inline)) {
             const detail::buffer_t out = __builtin_amdgcn_make_buffer_rsrc(h_all + size_t(t) * B * H + size_t(row0) * H, 0, rows * H * 2, 0x00020000);
             const __half* h_prev = t == 0 ? h0 : h_all + size_t(t - 1) * B * H;
             f32x4 acc[kTW][kRT];
@@ -327,7 +329,11 @@ __global__ void __launch_bounds__(Traits::kThreads, 1)
                             top[0] = max(top[0], max(v[c][j][0], v[c][j][1]));
                             top[1] = max(top[1], max(v[c][j][2], v[c][j][3]));
                         }
-                        if (t == 0 || tries > kSpinLimit || !__any(max(top[0], top[1]) == ~0u)) break;
+                        if (t == 0 || !__any(max(top[0], top[1]) == ~0u)) break;
+                        if (tries >= limit) {
+                            limit = -1;
+                            break;
+                        }
                         ++tries;
                         // some of it is not there yet: read once more (a count that the optimiser can follow becomes a copy of the loop each)
                         asm volatile("" : "+s"(tries)::"memory");
@@ -371,7 +377,6 @@ __global__ void __launch_bounds__(Traits::kThreads, 1)
                 for (int n = 0; n < kTW; ++n)
 #pragma unroll
                     for (int r = 0; r < kRT; ++r) asm volatile("" : "+v"(acc[n][r]));
-                if (tries > kSpinLimit) return false;
             } else {
                 detail::lds_barrier<0>();
                 read_pre(t);
@@ -383,6 +388,12 @@ __global__ void __launch_bounds__(Traits::kThreads, 1)
                 for (int n = 0; n < kTW; ++n)
 #pragma unroll
                     for (int r = 0; r < kRT; ++r) acc[n][r] = pre_v[n][r];
+            }
+            if (__builtin_expect(limit < 0, 0)) {
+#pragma unroll
+                for (int n = 0; n < kTW; ++n)
+#pragma unroll
+                    for (int r = 0; r < kRT; ++r) c_state[n][r] = __builtin_nanf("");
             }
 #pragma unroll
             for (int n = 0; n < kTW; ++n)
@@ -400,7 +411,6 @@ __global__ void __launch_bounds__(Traits::kThreads, 1)
                     if (word == ~0u) word = 0xfffefffeu;  // two NaNs stay NaNs and are told from a word not yet written
                     __builtin_amdgcn_raw_buffer_store_b32(word, out, h_out[n][r], 0, 0);
                 }
-            return true;
         };
 
         // ---- the steps of the slices held, mostly one. Step 0 needs no other workgroup; before step 1 everyone's words have to be
@@ -427,7 +437,7 @@ __global__ void __launch_bounds__(Traits::kThreads, 1)
                 }
             }
             ahead = tiles == 1 && t + 1 < T;
-            if (!step(t, slice, ahead ? t + 1 : -1)) return;
+            step(t, slice, ahead ? t + 1 : -1);
             if (t == 0 || tiles > 1 || t + 1 == T) store_cell(slice);
             if (++i < tiles) continue;
             i = 0;
@@ -435,10 +445,13 @@ __global__ void __launch_bounds__(Traits::kThreads, 1)
                 if (threadIdx.x == 0) {
                     const unsigned target = unsigned(peers) * unsigned(served);
                     const unsigned long long start = __builtin_amdgcn_s_memrealtime();
-                    int stolen = -1;
+                    int stolen = -2;  // -1: all slices are marked; -2: given up
 #pragma unroll 1
-                    for (int n = 0; n < kSpinLimit; ++n) {
-                        if (__hip_atomic_load(ready, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= target) break;
+                    for (int n = 0;; ++n) {
+                        if (__hip_atomic_load(ready, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= target) {
+                            stolen = -1;
+                            break;
+                        }
                         if (__builtin_amdgcn_s_memrealtime() - start > (unsigned long long)steal_ticks &&
                             __hip_atomic_load(tickets, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < unsigned(peers)) {
                             const int k = int(__hip_atomic_fetch_add(tickets, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
@@ -447,6 +460,7 @@ __global__ void __launch_bounds__(Traits::kThreads, 1)
                                 break;
                             }
                         }
+                        if (n >= limit) break;
                         __builtin_amdgcn_s_sleep(1);
                     }
                     if (stolen >= 0) s_tile[tiles] = static_cast<unsigned char>(stolen);
@@ -455,6 +469,7 @@ __global__ void __launch_bounds__(Traits::kThreads, 1)
                 __syncthreads();
                 const int stolen = __builtin_amdgcn_readfirstlane(s_word[0]);
                 __syncthreads();
+                if (stolen == -2) limit = -1;
                 if (stolen >= 0) {
                     i = tiles++;
                     ahead = false;

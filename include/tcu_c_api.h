@@ -287,11 +287,12 @@ unsigned long long tcu_lstm_layer_workspace_bytes(int T, int B, int I, int H);
 int tcu_lstm_uses_layer(int T, int B, int I, int H);
 int tcu_lstm_f16_layer(const void* x, const void* W, const void* bias, const void* h0, const void* c0, void* h_all, void* c_out,
                        int T, int B, int I, int H, void* workspace, unsigned long long workspace_bytes, void* stream);
-/* The same with at most `max_workgroups` workgroups, of which those that have waited `takeover_us` stand in for the others: for
- * tests of a layer that does not get the GPU it has room for. */
+/* The same with at most `max_workgroups` workgroups, of which those that have waited `takeover_us` stand in for the others, and with
+ * waits that are given up after `max_tries` polls (outputs that depend on one are NaN from that step on): for tests of a layer that
+ * does not get the GPU it has room for. */
 int tcu_lstm_f16_layer_limited(const void* x, const void* W, const void* bias, const void* h0, const void* c0, void* h_all,
                                void* c_out, int T, int B, int I, int H, void* workspace, unsigned long long workspace_bytes,
-                               int max_workgroups, int takeover_us, void* stream);
+                               int max_workgroups, int takeover_us, int max_tries, void* stream);
 
 /*
  * The LSTM layer with the whole time loop in ONE launch, for the large-hidden-size case where a step is bound by

@@ -23,7 +23,7 @@ def close(got, want, tol=STEP_TOL):
     return all(float((g.float() - w.float()).abs().max()) <= tol for g, w in zip(got, want))
 
 
-def limited(tcu, args, workgroups, takeover_us=30):
+def limited(tcu, args, workgroups, takeover_us=30, max_tries=1 << 24):
     """The layer in a launch of at most ``workgroups`` workgroups."""
     import torch
 
@@ -32,10 +32,11 @@ def limited(tcu, args, workgroups, takeover_us=30):
     H = b.numel() // 4
     need = int(tcu.lib().tcu_lstm_layer_workspace_bytes(T, B, I, H))
     ws = torch.full((need,), 0x5A, dtype=torch.uint8, device=x.device)
-    h_all, c_T = torch.empty(T, B, H, dtype=torch.float16, device=x.device), torch.empty(B, H, device=x.device)
+    h_all = torch.full((T, B, H), 7.0, dtype=torch.float16, device=x.device)
+    c_T = torch.full((B, H), 7.0, dtype=torch.float32, device=x.device)
     ptr = lambda t: 0 if t is None else t.data_ptr()
     tcu._check(tcu.lib().tcu_lstm_f16_layer_limited(*map(ptr, (x, W, b, h0, c0, h_all, c_T)), T, B, I, H, ptr(ws), need, workgroups,
-                                                    takeover_us, tcu._stream()))
+                                                    takeover_us, max_tries, tcu._stream()))
     return h_all, c_T
 
 
@@ -112,9 +113,23 @@ def test_lstm_layer_with_few_workgroups(tcu, device, T, B, I, H, grid, state):
 
 def test_lstm_layer_limits_are_checked(tcu, device):
     args = operands(tcu, device, 2, 16, 16, 16)
-    for limits in ((0, 30), (-1, 30), (8, -1), (8, 1000001)):
+    for limits in ((0, 30), (-1, 30), (8, -1), (8, 1000001), (8, 30, -1)):
         with pytest.raises(RuntimeError, match="workgroup"):
             limited(tcu, args, *limits)
+
+
+@pytest.mark.parametrize("T,B,I,H,units", [(4, 16, 64, 656, 32), (3, 48, 64, 272, 16), (3, 160, 64, 1024, 32)])
+def test_lstm_layer_gives_up_with_nan(tcu, device, T, B, I, H, units):
+    """A wait that does not end: one workgroup, told not to take over the other slices and to poll once. The launch ends, and what the
+    workgroup computes from then on is NaN; the next call is not affected."""
+    import torch
+
+    print(f"lstm layer gives up T{T} B{B} I{I} H{H}", flush=True)
+    args = operands(tcu, device, T, B, I, H)
+    h_all, c_T = limited(tcu, args, 1, 1000000, 0)
+    assert bool(torch.isnan(h_all[1:, :, :units]).all()) and bool(torch.isnan(c_T[:, :units]).all())
+    assert bool((c_T[:, units:] == 7.0).all()) and bool((h_all[:, :, units:] == 7.0).all())
+    assert close(tcu.lstm(*args, algo="layer"), tcu.lstm(*args, workspace=False))
 
 
 def test_lstm_layer_two_streams_and_nan(tcu, device):

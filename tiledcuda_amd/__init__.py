@@ -78,7 +78,7 @@ _SIGNATURES = {
     "tcu_lstm_f16_layer": (ctypes.c_int, [ctypes.c_void_p] * 7 + [ctypes.c_int] * 4 + [ctypes.c_void_p, ctypes.c_ulonglong,
                                                                                         ctypes.c_void_p]),
     "tcu_lstm_f16_layer_limited": (ctypes.c_int, [ctypes.c_void_p] * 7 + [ctypes.c_int] * 4 + [ctypes.c_void_p, ctypes.c_ulonglong] +
-                                   [ctypes.c_int] * 2 + [ctypes.c_void_p]),
+                                   [ctypes.c_int] * 3 + [ctypes.c_void_p]),
     "tcu_lstm_persistent_workspace_bytes": (ctypes.c_ulonglong, [ctypes.c_int] * 4),
     "tcu_lstm_f16_persistent": (ctypes.c_int, [ctypes.c_void_p] * 7 + [ctypes.c_int] * 4 + [ctypes.c_void_p, ctypes.c_ulonglong,
                                                                                           ctypes.c_void_p]),

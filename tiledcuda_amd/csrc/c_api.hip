@@ -1489,6 +1489,7 @@ bool lstm_layer_pays(int T, int B, int I, int H) {
 struct LstmLayerLimits {
     int workgroups = INT_MAX;
     int takeover_us = kLstmLayerTakeoverUs;
+    int max_tries = 1 << 24;  // of 0.5 us and more each
 };
 
 template <int kTW, int kKS, int kRT>
@@ -1498,7 +1499,7 @@ int launch_lstm_layer_xcd(const float* pre, const __half* W, const __half* bias,
     const int peers = (H + Traits::kUnits - 1) / Traits::kUnits;
     const int grid = std::min(limits.workgroups, 8 * peers);
     return launch(&lstm_layer_xcd<Traits>, dim3(unsigned(grid)), dim3(Traits::kThreads), Traits::kLdsBytes, s, pre, W, I + H, I, bias, h0,
-                  c0, h_all, c_out, T, B, H, sync, limits.takeover_us * 100);
+                  c0, h_all, c_out, T, B, H, sync, limits.takeover_us * 100, limits.max_tries);
 }
 
 int launch_lstm_layer(const __half* x, const __half* W, const __half* bias, const __half* h0, const float* c0, __half* h_all,
@@ -1785,10 +1786,11 @@ int tcu_lstm_f16_layer(const void* x, const void* W, const void* bias, const voi
 
 int tcu_lstm_f16_layer_limited(const void* x, const void* W, const void* bias, const void* h0, const void* c0, void* h_all, void* c_out,
                                int T, int B, int I, int H, void* workspace, unsigned long long workspace_bytes, int max_workgroups,
-                               int takeover_us, void* stream) {
-    if (max_workgroups < 1 || takeover_us < 0 || takeover_us > 1000000)
-        return fail(TCU_ERR_INVALID_ARGUMENT, "tcu_lstm_f16_layer_limited: at least one workgroup, 0 <= takeover_us <= 1000000");
-    return lstm_f16_layer(x, W, bias, h0, c0, h_all, c_out, T, B, I, H, workspace, workspace_bytes, {max_workgroups, takeover_us}, stream);
+                               int takeover_us, int max_tries, void* stream) {
+    if (max_workgroups < 1 || takeover_us < 0 || takeover_us > 1000000 || max_tries < 0 || max_tries > 1 << 24)
+        return fail(TCU_ERR_INVALID_ARGUMENT, "tcu_lstm_f16_layer_limited: at least one workgroup, 0 <= takeover_us <= 1000000, 0 <= "
+                                              "max_tries <= 2^24");
+    return lstm_f16_layer(x, W, bias, h0, c0, h_all, c_out, T, B, I, H, workspace, workspace_bytes, {max_workgroups, takeover_us, max_tries}, stream);
 }
 
 unsigned long long tcu_lstm_persistent_workspace_bytes(int T, int B, int I, int H) {
