@@ -158,6 +158,37 @@ def test_lstm_layer_two_streams_and_nan(tcu, device):
         assert close((torch.nan_to_num(g),), (torch.nan_to_num(w),))
 
 
+def test_lstm_layers_beside_each_other(tcu, device):
+    """Two layers on two streams whose workgroups do not all fit at once: the later one waits for CUs rather than run its slices two to
+    a workgroup, which took three times as long as one layer after the other. (Both orders of streams, best of several: a third more
+    than in turn is allowed.)"""
+    import time
+
+    import torch
+
+    T, B, I, H = 64, 80, 336, 656
+    args = operands(tcu, device, T, B, I, H)
+    want = tcu.lstm(*args, algo="layer")
+    ws = [torch.empty(int(tcu.lib().tcu_lstm_layer_workspace_bytes(T, B, I, H)), dtype=torch.uint8, device=device) for _ in range(2)]
+    outs = [tuple(torch.empty_like(t) for t in want) for _ in range(2)]
+    two = [torch.cuda.Stream() for _ in range(2)]
+
+    def us(streams, calls=6):
+        torch.cuda.synchronize()
+        start = time.perf_counter()
+        for _ in range(calls):
+            for s, w, o in zip(streams, ws, outs):
+                with torch.cuda.stream(s):
+                    tcu.lstm(*args, algo="layer", workspace=w, out=o)
+        torch.cuda.synchronize()
+        return (time.perf_counter() - start) * 1e6 / calls
+
+    in_turn, together = min(us(two[:1] * 2) for _ in range(4)), min(us(two) for _ in range(4))
+    print(f"lstm layers in turn {in_turn:.0f} us, on two streams {together:.0f} us", flush=True)
+    assert all(torch.equal(a, b) for o in outs for a, b in zip(o, want))
+    assert together <= 1.33 * in_turn
+
+
 def test_lstm_layer_route(tcu, device):
     """Where AUTO takes it, where not, and what it does with a caller's workspace, an h0 inside h_all and a captured stream."""
     import torch

@@ -120,7 +120,6 @@ bool aligned16(std::initializer_list<const void*> v) {
 // array's name is only a handle for hipGetSymbolAddress, never a device address.
 constexpr unsigned long long kScratchBytes = 64ull << 20;
 constexpr unsigned long long kPersistentSyncBytes = 4096;  // synchronisation words in front of the pre-activations
-constexpr int kLstmLayerTakeoverUs = 30;  // long against the start of a grid, short against its steps
 static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 
 constexpr int kMaxDevices = 64;
@@ -1471,26 +1470,37 @@ LstmLayerProjection lstm_layer_projection(long rows, int I, int H) {
     return plan;
 }
 
+/// Expected time of the layer kernel's steps, for every round of 8 groups of rows (measured over 90 sizes, us per step with 16 and 32
+/// rows: H 128 0.73, 1.1; 256 0.95, 1.45; 512 1.2, 1.9; 768 1.75, 2.9; 1024 2.05, 3.9).
+double lstm_layer_steps_us(int T, int B, int H) {
+    static constexpr double kStepUs[5][2] = {{0.73, 1.1}, {0.95, 1.45}, {1.2, 1.9}, {1.75, 2.9}, {2.05, 3.9}};
+    const int size = H <= 128 ? 0 : H <= 256 ? 1 : H <= 512 ? 2 : H <= 768 ? 3 : 4, tiles = lstm_layer_row_tiles(B);
+    const int rounds = ((B + 16 * tiles - 1) / (16 * tiles) + 7) / 8;
+    return double(rounds) * T * kStepUs[size][tiles - 1];
+}
+
 /// Whether AUTO runs the layer that way: the projection, 1.5 us to the next launch, what the kernel takes before its first step (the
-/// weights arrive at 0.9 MB per us and XCD) and its steps, for every round of 8 groups of rows (measured over 90 sizes, us per step with
-/// 16 and 32 rows: H 128 0.73, 1.1; 256 0.95, 1.45; 512 1.2, 1.9; 768 1.75, 2.9; 1024 2.05, 3.9), against a launch per step. us, steps
+/// weights arrive at 0.9 MB per us and XCD) and its steps against a launch per step. us, steps
 /// -> this: T 16, B 256, I 1024, H 1024: 149 -> 106; 24, 80, 336, 656: 109 -> 75; 20, 16, 416, 80: 60 -> 24; 8, 96, 176, 160: 25 -> 18; not taken: 8,
 /// 80, 384, 576: 34, 38; 5, 352, 144, 864: 62, 73; 31, 368, 96, 160: 111, 114. Long inputs stay with lstm_projection_pays().
 bool lstm_layer_pays(int T, int B, int I, int H) {
     if (T < 4 || !lstm_layer_takes(T, B, I, H) || lstm_projection_pays(T, B, I, H)) return false;
-    static constexpr double kStepUs[5][2] = {{0.73, 1.1}, {0.95, 1.45}, {1.2, 1.9}, {1.75, 2.9}, {2.05, 3.9}};
-    const int size = H <= 128 ? 0 : H <= 256 ? 1 : H <= 512 ? 2 : H <= 768 ? 3 : 4, tiles = lstm_layer_row_tiles(B);
-    const int rounds = ((B + 16 * tiles - 1) / (16 * tiles) + 7) / 8;
-    const double layer = 7.5 + 9.0 * (H / 1024.0) * (H / 1024.0) + rounds * T * kStepUs[size][tiles - 1];
+    const double layer = 7.5 + 9.0 * (H / 1024.0) * (H / 1024.0) + lstm_layer_steps_us(T, B, H);
     return 1.05 * (lstm_layer_projection((long)T * B, I, H).us + layer) < T * lstm_step_us(B, H, I + H);
 }
 
 /// What a launch of lstm_layer_xcd may use; other values than these are for tests (tcu_lstm_f16_layer_limited).
 struct LstmLayerLimits {
     int workgroups = INT_MAX;
-    int takeover_us = kLstmLayerTakeoverUs;
+    int takeover_us = -1;  // lstm_layer_takeover_us()
     int max_tries = 1 << 24;  // of 0.5 us and more each
 };
+
+/// How long a workgroup waits for the others to start before it takes over the slice of one that has not: twice the time of all steps.
+/// The layer's CUs are mostly held by something as short as itself, and a workgroup with two slices fetches the weights of both again
+/// in every step, for the rest of the launch. Two layers on two streams, us for both, by the wait (30 us, 200 us; a launch per
+/// step): T 24, B 80, I 336, H 656: 149-355, 118; 165; T 64: 757, 263; 397; T 64, B 128, I 512, H 784: 1067, 357; 523.
+int lstm_layer_takeover_us(int T, int B, int H) { return int(30.0 + std::min(1e6, 2.0 * lstm_layer_steps_us(T, B, H))); }
 
 template <int kTW, int kKS, int kRT>
 int launch_lstm_layer_xcd(const float* pre, const __half* W, const __half* bias, const __half* h0, const float* c0, __half* h_all,
@@ -1499,7 +1509,8 @@ int launch_lstm_layer_xcd(const float* pre, const __half* W, const __half* bias,
     const int peers = (H + Traits::kUnits - 1) / Traits::kUnits;
     const int grid = std::min(limits.workgroups, 8 * peers);
     return launch(&lstm_layer_xcd<Traits>, dim3(unsigned(grid)), dim3(Traits::kThreads), Traits::kLdsBytes, s, pre, W, I + H, I, bias, h0,
-                  c0, h_all, c_out, T, B, H, sync, limits.takeover_us * 100, limits.max_tries);
+                  c0, h_all, c_out, T, B, H, sync,
+                  100 * (limits.takeover_us < 0 ? lstm_layer_takeover_us(T, B, H) : limits.takeover_us), limits.max_tries);
 }
 
 int launch_lstm_layer(const __half* x, const __half* W, const __half* bias, const __half* h0, const float* c0, __half* h_all,
