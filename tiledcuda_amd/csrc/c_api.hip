@@ -1470,23 +1470,34 @@ LstmLayerProjection lstm_layer_projection(long rows, int I, int H) {
     return plan;
 }
 
+int lstm_layer_rounds(int B) {  // of 8 groups of rows, one per XCD
+    const int rows = 16 * lstm_layer_row_tiles(B);
+    return ((B + rows - 1) / rows + 7) / 8;
+}
+
 /// Expected time of the layer kernel's steps, for every round of 8 groups of rows (measured over 90 sizes, us per step with 16 and 32
 /// rows: H 128 0.73, 1.1; 256 0.95, 1.45; 512 1.2, 1.9; 768 1.75, 2.9; 1024 2.05, 3.9).
 double lstm_layer_steps_us(int T, int B, int H) {
     static constexpr double kStepUs[5][2] = {{0.73, 1.1}, {0.95, 1.45}, {1.2, 1.9}, {1.75, 2.9}, {2.05, 3.9}};
-    const int size = H <= 128 ? 0 : H <= 256 ? 1 : H <= 512 ? 2 : H <= 768 ? 3 : 4, tiles = lstm_layer_row_tiles(B);
-    const int rounds = ((B + 16 * tiles - 1) / (16 * tiles) + 7) / 8;
-    return double(rounds) * T * kStepUs[size][tiles - 1];
+    const int size = H <= 128 ? 0 : H <= 256 ? 1 : H <= 512 ? 2 : H <= 768 ? 3 : 4;
+    return double(lstm_layer_rounds(B)) * T * kStepUs[size][lstm_layer_row_tiles(B) - 1];
 }
 
 /// Whether AUTO runs the layer that way: the projection, 1.5 us to the next launch, what the kernel takes before its first step (the
-/// weights arrive at 0.9 MB per us and XCD) and its steps against a launch per step. us, steps
+/// weights arrive at 0.9 MB per us and XCD) and its steps against a launch per step. The first sum is the least that was measured;
+/// where the two plans are close the second counts (fitted to 500 sizes, T 4 to 32, up to 480 rows, within 7 %): the start of many
+/// units, another round's claims. By it 3 of 600 other sizes take longer than a launch per step, at most 8 %; by the first alone 20 of 320, up to 15 %
+/// (us, steps, layer: 14 x 480 x 288 x 288: 79, 86; 5 x 368 x 144 x 768: 57, 65). Longer layers gain as much as 32 steps or more: T 1024, B 80,
+/// I 336, H 656: 4656, 2311. us, steps
 /// -> this: T 16, B 256, I 1024, H 1024: 149 -> 106; 24, 80, 336, 656: 109 -> 75; 20, 16, 416, 80: 60 -> 24; 8, 96, 176, 160: 25 -> 18; not taken: 8,
 /// 80, 384, 576: 34, 38; 5, 352, 144, 864: 62, 73; 31, 368, 96, 160: 111, 114. Long inputs stay with lstm_projection_pays().
 bool lstm_layer_pays(int T, int B, int I, int H) {
     if (T < 4 || !lstm_layer_takes(T, B, I, H) || lstm_projection_pays(T, B, I, H)) return false;
-    const double layer = 7.5 + 9.0 * (H / 1024.0) * (H / 1024.0) + lstm_layer_steps_us(T, B, H);
-    return 1.05 * (lstm_layer_projection((long)T * B, I, H).us + layer) < T * lstm_step_us(B, H, I + H);
+    const double projection = lstm_layer_projection((long)T * B, I, H).us, steps = lstm_layer_steps_us(T, B, H);
+    const double fill = (H / 1024.0) * (H / 1024.0);  // of an XCD's registers
+    const double layer = std::max(projection + 7.5 + 9.0 * fill + steps,
+                                  1.15 * projection + 5.0 + 16.0 * fill + 4.0 * (lstm_layer_rounds(B) - 1) + 1.06 * steps);
+    return 1.05 * layer < T * lstm_step_us(B, H, I + H);
 }
 
 /// What a launch of lstm_layer_xcd may use; other values than these are for tests (tcu_lstm_f16_layer_limited).
