@@ -272,7 +272,8 @@ int tcu_lstm_f16_ws(const void* x, const void* W, const void* bias, const void* 
 
 /*
  * The LSTM layer in two launches: the input half of the gates of all steps as one GEMM into `workspace` (f32, as in
- * tcu_lstm_f16_ws), then the whole time loop as one launch that keeps the recurrent weights in registers. T >= 2, B, I and H in
+ * tcu_lstm_f16_ws), then the whole time loop as one launch that keeps the recurrent weights in registers; a layer of which these
+ * pre-activations would take more than 256 MiB runs in parts of so many steps, one after the other. T >= 2, B, I and H in
  * multiples of 16, H <= 1024, B <= 2048 (tcu_lstm_layer_workspace_bytes returns 0 for shapes this path does not take). Same
  * arguments and results (up to the order of the f32 summation) as tcu_lstm_f16; nothing is asked of the GPU: workgroups that are
  * not resident are stood in for by those that are, and every wait is for a workgroup that runs.

@@ -158,6 +158,57 @@ def test_lstm_layer_two_streams_and_nan(tcu, device):
         assert close((torch.nan_to_num(g),), (torch.nan_to_num(w),))
 
 
+@pytest.mark.parametrize("T,B,I,H,parts", [(9, 2048, 16, 1024, 2), (65, 256, 64, 1024, 2), (135, 256, 16, 1008, 3), (64, 256, 64, 1024, 1)])
+def test_lstm_layer_in_parts(tcu, device, T, B, I, H, parts):
+    """Layers whose pre-activations would take more than 256 MiB: bit for bit what the parts give by themselves, in a workspace of the
+    stated size and no more, with an initial state and without."""
+    import torch
+
+    print(f"lstm layer in parts T{T} B{B} I{I} H{H}", flush=True)
+    x, W, b, h0, c0 = operands(tcu, device, T, B, I, H)
+    need = int(tcu.lib().tcu_lstm_layer_workspace_bytes(T, B, I, H))
+    assert need == 4096 + -(-T // parts) * B * H * 16 <= 4096 + 2 ** 28
+    ws = torch.full((need + 256,), 0x5A, dtype=torch.uint8, device=device)
+    for state in ((h0, c0), (None, None)):
+        got = tcu.lstm(x, W, b, *state, algo="layer", workspace=ws)
+        h, c = state
+        for k in range(parts):
+            first, last = T * k // parts, T * (k + 1) // parts
+            h_part, c = tcu.lstm(x[first:last], W, b, h, c, algo="layer")
+            assert torch.equal(got[0][first:last], h_part)
+            h = h_part[-1]
+        assert torch.equal(got[1], c)
+        assert close(got, tcu.lstm(x, W, b, *state, workspace=False), 8e-3)  # (up to 135 steps: twice the bound of the short layers)
+    assert bool((ws[need:] == 0x5A).all())
+
+
+@pytest.mark.parametrize("entry", ["python", "calls", "op"])
+def test_lstm_auto_without_memory_for_a_workspace(tcu, device, entry):
+    """AUTO needs no memory beside its outputs: where the allocator has none for the layer's workspace the steps run."""
+    import torch
+
+    import tiledcuda_amd.torch_ops  # noqa: F401
+
+    T, B, I, H = 64, 256, 64, 1024  # h_all 32 MiB, the workspace 256
+    assert tcu.lib().tcu_lstm_uses_layer(T, B, I, H) == 1
+    args = operands(tcu, device, T, B, I, H)
+    steps = tcu.lstm(*args, workspace=False)
+    out = tuple(torch.empty_like(t) for t in steps)
+    call = {"python": lambda: tcu.lstm(*args, out=out), "calls": lambda: tcu.lstm(*args), "op": lambda: torch.ops.tiledcuda.lstm(*args)}[entry]
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    total = torch.cuda.get_device_properties(device).total_memory
+    torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (128 << 20)) / total)
+    try:
+        got = call()
+        with pytest.raises(torch.OutOfMemoryError):
+            tcu.lstm(*args, algo="layer")
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    assert torch.equal(got[0], steps[0]) and torch.equal(got[1], steps[1])
+    assert not torch.equal(tcu.lstm(*args)[0], steps[0])
+
+
 def test_lstm_layers_beside_each_other(tcu, device):
     """Two layers on two streams whose workgroups do not all fit at once: the later one waits for CUs rather than run its slices two to
     a workgroup, which took three times as long as one layer after the other. (Both orders of streams, best of several: a third more

@@ -367,7 +367,8 @@ def lstm(x: torch.Tensor, W: torch.Tensor, bias: torch.Tensor, h0: torch.Tensor 
 
     ``algo="layer"`` runs the whole time loop in one launch after the same GEMM (``tcu_lstm_f16_layer``; T >= 2, H <= 1024, B <= 2048,
     all in multiples of 16), asking nothing of the GPU; ``algo="auto"`` takes it, with a workspace as above, where it pays (about 5
-    steps and more, up to 256 rows; not in a stream that is being captured, unless the workspace is yours).
+    steps and more, up to 256 rows; not in a stream that is being captured, unless the workspace is yours, nor where the memory for one,
+    at most 256 MiB, is not there).
 
     ``algo="persistent"`` runs the whole time loop in one weight-stationary launch after the same GEMM
     (``tcu_lstm_f16_persistent``: H in {256, 512, 768, 1024}, B <= 256 in multiples of 32; ``lstm_persistent_workspace_bytes``). Its
@@ -416,7 +417,11 @@ def lstm(x: torch.Tensor, W: torch.Tensor, bias: torch.Tensor, h0: torch.Tensor 
         # allocator; a workspace of the caller's that is too small belongs to the plans below)
         if workspace is None or workspace is False:
             if algo == "layer" or not torch.cuda.is_current_stream_capturing():
-                workspace = torch.empty(need, dtype=torch.uint8, device=x.device)
+                try:
+                    workspace = torch.empty(need, dtype=torch.uint8, device=x.device)
+                except torch.OutOfMemoryError:  # the steps need none
+                    if algo == "layer":
+                        raise
         elif not workspace.is_cuda or not workspace.is_contiguous():
             raise ValueError("workspace must be a contiguous device tensor")
         size = 0 if workspace is None else workspace.numel() * workspace.element_size()

@@ -1470,6 +1470,16 @@ LstmLayerProjection lstm_layer_projection(long rows, int I, int H) {
     return plan;
 }
 
+/// Launches that the layer's steps are divided into, each with its projection before it, so that the pre-activations of one take at
+/// most 256 MiB whatever T is (eight times h_all otherwise: 17 GB at T 4096, B 256, H 1024). Every part has 4 steps or more. A part
+/// costs what the layer takes before its first step once more, and its pre-activations come from nearer: us, whole -> in parts, T 1024 and
+/// B 256, I 1024, H 1024 (16 parts): 6120 -> 6280; 128, 512, 1024 (8): 3220 -> 3200; 80, 336, 656 (4): 2300 -> 2180; 256, 256, 256 (4): 1990 -> 1850.
+constexpr unsigned long long kLstmLayerPreBytes = 256ull << 20;
+int lstm_layer_parts(int T, int B, int H) {
+    const long steps = long(kLstmLayerPreBytes / (16ull * B * H));  // 8 and more: B <= 2048, H <= 1024
+    return int((T + steps - 1) / steps);
+}
+
 int lstm_layer_rounds(int B) {  // of 8 groups of rows, one per XCD
     const int rows = 16 * lstm_layer_row_tiles(B);
     return ((B + rows - 1) / rows + 7) / 8;
@@ -1493,10 +1503,11 @@ double lstm_layer_steps_us(int T, int B, int H) {
 /// 80, 384, 576: 34, 38; 5, 352, 144, 864: 62, 73; 31, 368, 96, 160: 111, 114. Long inputs stay with lstm_projection_pays().
 bool lstm_layer_pays(int T, int B, int I, int H) {
     if (T < 4 || !lstm_layer_takes(T, B, I, H) || lstm_projection_pays(T, B, I, H)) return false;
-    const double projection = lstm_layer_projection((long)T * B, I, H).us, steps = lstm_layer_steps_us(T, B, H);
+    const int parts = lstm_layer_parts(T, B, H);
+    const double projection = parts * lstm_layer_projection((long)((T + parts - 1) / parts) * B, I, H).us, steps = lstm_layer_steps_us(T, B, H);
     const double fill = (H / 1024.0) * (H / 1024.0);  // of an XCD's registers
-    const double layer = std::max(projection + 7.5 + 9.0 * fill + steps,
-                                  1.15 * projection + 5.0 + 16.0 * fill + 4.0 * (lstm_layer_rounds(B) - 1) + 1.06 * steps);
+    const double layer = std::max(projection + parts * (7.5 + 9.0 * fill) + steps,
+                                  1.15 * projection + parts * (5.0 + 16.0 * fill) + 4.0 * (lstm_layer_rounds(B) - 1) + 1.06 * steps);
     return 1.05 * layer < T * lstm_step_us(B, H, I + H);
 }
 
@@ -1524,9 +1535,9 @@ int launch_lstm_layer_xcd(const float* pre, const __half* W, const __half* bias,
                   100 * (limits.takeover_us < 0 ? lstm_layer_takeover_us(T, B, H) : limits.takeover_us), limits.max_tries);
 }
 
-int launch_lstm_layer(const __half* x, const __half* W, const __half* bias, const __half* h0, const float* c0, __half* h_all,
-                      float* c_out, int T, int B, int I, int H, unsigned char* workspace, const LstmLayerLimits& limits,
-                      hipStream_t s) {
+int launch_lstm_layer_part(const __half* x, const __half* W, const __half* bias, const __half* h0, const float* c0, __half* h_all,
+                           float* c_out, int T, int B, int I, int H, unsigned char* workspace, const LstmLayerLimits& limits,
+                           hipStream_t s) {
     auto sync = reinterpret_cast<unsigned int*>(workspace);
     auto pre = reinterpret_cast<float*>(workspace + kPersistentSyncBytes);
     constexpr int kSyncWords = LstmLayerTraits<1, 4, 1>::kSyncWords;
@@ -1561,6 +1572,20 @@ int launch_lstm_layer(const __half* x, const __half* W, const __half* bias, cons
     if (H <= 512) return go(one{}, std::integral_constant<int, 16>{});
     if (H <= 768) return go(two{}, std::integral_constant<int, 24>{});
     return go(two{}, std::integral_constant<int, 32>{});
+}
+
+/// ... in lstm_layer_parts() parts: the states that one ends with are those that the next begins with.
+int launch_lstm_layer(const __half* x, const __half* W, const __half* bias, const __half* h0, const float* c0, __half* h_all,
+                      float* c_out, int T, int B, int I, int H, unsigned char* workspace, const LstmLayerLimits& limits, hipStream_t s) {
+    const int parts = lstm_layer_parts(T, B, H);
+    for (int part = 0, t = 0; part < parts; ++part) {
+        const int end = int((long)T * (part + 1) / parts);
+        const int rc = launch_lstm_layer_part(x + size_t(t) * B * I, W, bias, t == 0 ? h0 : h_all + size_t(t - 1) * B * H, t == 0 ? c0 : c_out,
+                                              h_all + size_t(t) * B * H, c_out, end - t, B, I, H, workspace, limits, s);
+        if (rc != TCU_OK) return lstm_step_failed(rc, t, T);
+        t = end;
+    }
+    return TCU_OK;
 }
 
 /// The weight-stationary recurrence for hidden size kH: 8 * kH / 32 workgroups, kH / 32 per XCD.
@@ -1796,7 +1821,8 @@ int tcu_lstm_f16_ws(const void* x, const void* W, const void* bias, const void* 
 
 unsigned long long tcu_lstm_layer_workspace_bytes(int T, int B, int I, int H) {
     if (!positive({T, B, I, H}) || !lstm_layer_takes(T, B, I, H)) return 0;
-    return kPersistentSyncBytes + (unsigned long long)T * B * 4 * H * sizeof(float);
+    const int parts = lstm_layer_parts(T, B, H);
+    return kPersistentSyncBytes + (unsigned long long)((T + parts - 1) / parts) * B * 4 * H * sizeof(float);
 }
 
 int tcu_lstm_uses_layer(int T, int B, int I, int H) { return positive({T, B, I, H}) && lstm_layer_pays(T, B, I, H) ? 1 : 0; }

@@ -38,6 +38,14 @@ c10::DeviceIndex current_device() { return c10::hip::current_device(); }
 void* current_stream(c10::DeviceIndex device) { return c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(device).stream(); }
 bool capturing() { return c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None; }
 at::Tensor bytes(const at::Tensor& like, unsigned long long n) { return at::empty({static_cast<int64_t>(n)}, like.options().dtype(at::kByte)); }
+/// The same for a workspace that a call can do without: undefined where the memory is not there.
+at::Tensor bytes_if_free(const at::Tensor& like, unsigned long long n) {
+    try {
+        return bytes(like, n);
+    } catch (const c10::OutOfMemoryError&) {
+        return {};
+    }
+}
 
 /// The call itself, without the interpreter's lock (it may wait for a place in the stream's queue).
 template <typename F>
@@ -199,11 +207,12 @@ PyObject* lstm(PyObject*, PyObject* const* args, Py_ssize_t n) {
     const void *xp = x->data_ptr(), *wp = W->data_ptr(), *bp = bias->data_ptr();
     void *hp = h_all.data_ptr(), *cp = c_out.data_ptr();
     bool ok;
-    if (T >= 4 && tcu_lstm_uses_layer(T, B, I, H) && !capturing()) {
-        const unsigned long long need = tcu_lstm_layer_workspace_bytes(T, B, I, H);
-        const at::Tensor ws = bytes(*x, need);
-        void* const sp = ws.data_ptr();
-        ok = succeeds([&] { return tcu_lstm_f16_layer(xp, wp, bp, state[0], state[1], hp, cp, T, B, I, H, sp, need, stream); });
+    at::Tensor layer_ws;
+    const unsigned long long layer_need = T >= 4 && tcu_lstm_uses_layer(T, B, I, H) && !capturing() ? tcu_lstm_layer_workspace_bytes(T, B, I, H) : 0;
+    if (layer_need > 0) layer_ws = bytes_if_free(*x, layer_need);
+    if (layer_ws.defined()) {
+        void* const sp = layer_ws.data_ptr();
+        ok = succeeds([&] { return tcu_lstm_f16_layer(xp, wp, bp, state[0], state[1], hp, cp, T, B, I, H, sp, layer_need, stream); });
     } else if (T >= 4 && I >= 512 && tcu_lstm_uses_workspace(T, B, I, H)) {
         const unsigned long long need = tcu_lstm_workspace_bytes(T, B, I, H);
         const at::Tensor ws = bytes(*x, need);

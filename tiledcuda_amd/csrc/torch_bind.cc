@@ -161,11 +161,17 @@ std::tuple<at::Tensor, at::Tensor> lstm(const at::Tensor& x, const at::Tensor& W
     if (tcu_lstm_uses_layer(int(T), int(B), int(I), int(H)) &&
         c10::hip::currentStreamCaptureStatusMayInitCtx() == c10::hip::CaptureStatus::None) {
         const unsigned long long need = tcu_lstm_layer_workspace_bytes(int(T), int(B), int(I), int(H));
-        at::Tensor ws = at::empty({static_cast<int64_t>(need)}, x.options().dtype(at::kByte));
-        check_status(tcu_lstm_f16_layer(x.data_ptr(), W.data_ptr(), bias.data_ptr(), h0p, c0p, h_all.data_ptr(), c_out.data_ptr(),
-                                        int(T), int(B), int(I), int(H), ws.data_ptr(), need, current_stream(x)),
-                     "lstm");
-        return {h_all, c_out};
+        at::Tensor ws;
+        try {
+            ws = at::empty({static_cast<int64_t>(need)}, x.options().dtype(at::kByte));
+        } catch (const c10::OutOfMemoryError&) {  // (the steps below need none)
+        }
+        if (ws.defined()) {
+            check_status(tcu_lstm_f16_layer(x.data_ptr(), W.data_ptr(), bias.data_ptr(), h0p, c0p, h_all.data_ptr(), c_out.data_ptr(),
+                                            int(T), int(B), int(I), int(H), ws.data_ptr(), need, current_stream(x)),
+                         "lstm");
+            return {h_all, c_out};
+        }
     }
     // with a long input size the input half of the gates is cheaper as one GEMM over all steps; its [T, B, 4H] f32
     // result lives in a block from torch's caching allocator (stream-ordered, returned when `ws` dies)
