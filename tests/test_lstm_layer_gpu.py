@@ -182,6 +182,26 @@ def test_lstm_layer_in_parts(tcu, device, T, B, I, H, parts):
     assert bool((ws[need:] == 0x5A).all())
 
 
+def test_lstm_auto_with_a_workspace_the_layer_cannot_use(tcu, device):
+    """A size whose AUTO was a launch per step and never looked at the workspace: one on the host, with gaps, misaligned, too small or
+    no tensor at all is left alone, and the steps run; ``algo="layer"`` refuses it."""
+    import torch
+
+    T, B, I, H = 24, 48, 64, 272
+    args = operands(tcu, device, T, B, I, H)
+    steps = tcu.lstm(*args, workspace=False)
+    need = int(tcu.lib().tcu_lstm_layer_workspace_bytes(T, B, I, H))
+    assert tcu.lib().tcu_lstm_uses_layer(T, B, I, H) == 1 and tcu.lib().tcu_lstm_uses_workspace(T, B, I, H) == 0
+    room = torch.full((2 * need,), 0x5A, dtype=torch.uint8, device=device)
+    for ws in (torch.empty(need, dtype=torch.uint8), room[::2], room[4:need + 4], room[:need - 1]):
+        got = tcu.lstm(*args, workspace=ws)
+        assert torch.equal(got[0], steps[0]) and torch.equal(got[1], steps[1])
+        with pytest.raises((ValueError, RuntimeError)):
+            tcu.lstm(*args, algo="layer", workspace=ws)
+    got = tcu.lstm(*args, workspace=True)
+    assert torch.equal(got[0], steps[0]) and torch.equal(got[1], steps[1]) and bool((room == 0x5A).all())
+
+
 @pytest.mark.parametrize("entry", ["python", "calls", "op"])
 def test_lstm_auto_without_memory_for_a_workspace(tcu, device, entry):
     """AUTO needs no memory beside its outputs: where the allocator has none for the layer's workspace the steps run."""

@@ -414,7 +414,7 @@ def lstm(x: torch.Tensor, W: torch.Tensor, bias: torch.Tensor, h0: torch.Tensor 
         if algo == "layer" and need == 0:
             raise ValueError("algo='layer' needs T >= 2, B, I and H in multiples of 16, H <= 1024 and B <= 2048")
         # (nothing is allocated in a captured stream: outside torch's own graphs the graph would keep a block that goes back to the
-        # allocator; a workspace of the caller's that is too small belongs to the plans below)
+        # allocator; a workspace of the caller's that the layer cannot use belongs to the plans below, which may not look at it)
         if workspace is None or workspace is False:
             if algo == "layer" or not torch.cuda.is_current_stream_capturing():
                 try:
@@ -422,9 +422,10 @@ def lstm(x: torch.Tensor, W: torch.Tensor, bias: torch.Tensor, h0: torch.Tensor 
                 except torch.OutOfMemoryError:  # the steps need none
                     if algo == "layer":
                         raise
-        elif not workspace.is_cuda or not workspace.is_contiguous():
+        elif algo == "layer" and (not workspace.is_cuda or not workspace.is_contiguous()):
             raise ValueError("workspace must be a contiguous device tensor")
-        size = 0 if workspace is None else workspace.numel() * workspace.element_size()
+        usable = isinstance(workspace, torch.Tensor) and workspace.is_cuda and workspace.is_contiguous() and workspace.data_ptr() % 16 == 0
+        size = workspace.numel() * workspace.element_size() if usable or algo == "layer" else 0
         if algo == "layer" or size >= need:
             _check(lib().tcu_lstm_f16_layer(_dev_ptr(x, torch.float16, "x"), _dev_ptr(W, torch.float16, "W"),
                                             _dev_ptr(bias, torch.float16, "bias"), _dev_ptr(h0, torch.float16, "h0"),
