@@ -279,8 +279,8 @@ int tcu_lstm_f16_ws(const void* x, const void* W, const void* bias, const void* 
  * not resident are stood in for by those that are, and every wait is for a workgroup that runs.
  * `workspace`: device memory of at least tcu_lstm_layer_workspace_bytes(T, B, I, H) bytes, 16-byte aligned, owned by the caller
  * and free to reuse once the work enqueued here has run; its first 4 KiB are synchronisation words, cleared by the call. Calls
- * that may overlap in time need a workspace each. An h0 that lies inside h_all runs the step kernels of tcu_lstm_f16 instead. No
- * counterpart in the reference (it has no LSTM).
+ * that may overlap in time need a workspace each. Where x, h0 or c0 lies inside h_all the step kernels of tcu_lstm_f16 run instead.
+ * No counterpart in the reference (it has no LSTM).
  */
 unsigned long long tcu_lstm_layer_workspace_bytes(int T, int B, int I, int H);
 /* 1 where it is expected to be faster than tcu_lstm_f16 and tcu_lstm_f16_ws (about 5 steps and more, up to 256 rows), else 0: the

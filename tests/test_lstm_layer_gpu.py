@@ -182,6 +182,27 @@ def test_lstm_layer_in_parts(tcu, device, T, B, I, H, parts):
     assert bool((ws[need:] == 0x5A).all())
 
 
+def test_lstm_layer_fed_with_its_own_outputs(tcu, device):
+    """Inputs that are the outputs a step before, in the same memory: what a launch per step gives, and what feeding them one call at a
+    time gives."""
+    import torch
+
+    T, B, H = 12, 48, 272
+    assert tcu.lib().tcu_lstm_uses_layer(T, B, H, H) == 1
+    x, W, b, h0, c0 = operands(tcu, device, T, B, H, H)
+    want = [x[0]]
+    h, c = h0, c0
+    for _ in range(T):
+        h_all, c = tcu.lstm(want[-1][None], W, b, h, c)
+        h = h_all[0]
+        want.append(h)
+    for kwargs in ({}, {"algo": "layer"}, {"workspace": False}):
+        buf, c_T = torch.zeros(T + 1, B, H, dtype=torch.float16, device=device), torch.empty(B, H, device=device)
+        buf[0] = x[0]
+        tcu.lstm(buf[:-1], W, b, h0, c0, out=(buf[1:], c_T), **kwargs)
+        assert torch.equal(buf, torch.stack(want)) and torch.equal(c_T, c), kwargs
+
+
 def test_lstm_auto_with_a_workspace_the_layer_cannot_use(tcu, device):
     """A size whose AUTO was a launch per step and never looked at the workspace: one on the host, with gaps, misaligned, too small or
     no tensor at all is left alone, and the steps run; ``algo="layer"`` refuses it."""

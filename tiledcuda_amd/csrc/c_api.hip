@@ -1613,10 +1613,14 @@ int lstm_f16_layer(const void* x, const void* W, const void* bias, const void* h
         return fail(TCU_ERR_UNSUPPORTED_SHAPE, "tcu_lstm_f16_layer: needs T >= 2, B, I and H in multiples of 16, H <= 1024 and B <= 2048");
     if (workspace_bytes < need)
         return fail(TCU_ERR_INVALID_ARGUMENT, "tcu_lstm_f16_layer: workspace smaller than tcu_lstm_layer_workspace_bytes()");
-    // the kernel marks all of h_all before its first step: an initial state inside it (the last step of an earlier call that
-    // wrote the same tensor) goes to the kernels that write a step at a time
-    const auto h0_first = reinterpret_cast<uintptr_t>(h0), all_first = reinterpret_cast<uintptr_t>(h_all);
-    if (h0 && h0_first < all_first + size_t(T) * B * H * 2 && all_first < h0_first + size_t(B) * H * 2)
+    // the kernel marks all of h_all before its first step, and the projection reads all of x before any step is written: a state
+    // inside h_all (the last step of an earlier call that wrote the same tensor) or inputs that are its steps (each the output before
+    // it) go to the kernels that read and write a step at a time
+    auto inside = [&](const void* p, size_t bytes) {
+        const auto first = reinterpret_cast<uintptr_t>(p), all_first = reinterpret_cast<uintptr_t>(h_all);
+        return p && first < all_first + size_t(T) * B * H * 2 && all_first < first + bytes;
+    };
+    if (inside(h0, size_t(B) * H * 2) || inside(c0, size_t(B) * H * 4) || inside(x, size_t(T) * B * I * 2))
         return tcu_lstm_f16_algo(x, W, bias, h0, c0, h_all, c_out, T, B, I, H, TCU_LSTM_AUTO, stream);
     return launch_lstm_layer(static_cast<const __half*>(x), static_cast<const __half*>(W), static_cast<const __half*>(bias),
                              static_cast<const __half*>(h0), static_cast<const float*>(c0), static_cast<__half*>(h_all),
