@@ -79,3 +79,29 @@ def test_calls_without_a_device_leave_errors_to_python(tcu):
         tcu.gemm(torch.zeros(16, 16, dtype=torch.float16), torch.zeros(16, 16, dtype=torch.float16))
     with pytest.raises(ValueError, match="device memory"):
         tcu.scatter_nd(torch.zeros(4, 4), torch.zeros(1, 1, dtype=torch.int64), torch.zeros(1, 4))
+
+
+def test_calls_are_those_of_this_interpreter(tcu, monkeypatch):
+    """The module's name is one that other interpreters do not load; without it, or with one compiled for another torch, the Python code
+    makes the calls and says so once."""
+    import os
+    import subprocess
+    import sys
+    import sysconfig
+    import warnings
+
+    assert module(tcu).__file__.endswith("_calls" + sysconfig.get_config_var("EXT_SUFFIX"))
+    other = subprocess.run([sys.executable, "-c", "import torch; torch.__version__ = '0.0.1'; import tiledcuda_amd._calls"], text=True,
+                           cwd=os.path.dirname(os.path.dirname(tcu.__file__)), capture_output=True)
+    assert other.returncode != 0 and "ImportError: compiled for torch" in other.stderr
+    monkeypatch.setattr(tcu, "_ready_calls", None)
+    monkeypatch.delattr(tcu, "_calls", raising=False)
+    monkeypatch.setitem(sys.modules, "tiledcuda_amd._calls", None)
+    with pytest.warns(RuntimeWarning, match="_calls"):
+        absent = tcu._native()
+    assert absent.gemm(1, 2, 3) is None and absent.lstm() is None
+    with warnings.catch_warnings():
+        warnings.simplefilter("error")
+        assert tcu._native() is absent
+    with pytest.raises(ValueError, match="device memory"):
+        tcu.gemm(torch.zeros(16, 16, dtype=torch.float16), torch.zeros(16, 16, dtype=torch.float16))

@@ -13,6 +13,7 @@ from __future__ import annotations
 import ctypes
 import math
 import os
+import warnings
 
 import torch
 
@@ -24,7 +25,6 @@ __all__ = [
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 _LIB_PATH = os.path.join(_HERE, "lib", "libtiledcuda_amd.so")
-_CALLS_PATH = os.path.join(_HERE, "_calls.so")
 _lib = None
 _ready_calls = None
 
@@ -120,15 +120,26 @@ def lib() -> ctypes.CDLL:
     return _lib
 
 
+class _NoCalls:
+    """Stands in for ``_calls`` where there is none for this interpreter: no call is an ordinary one."""
+
+    def __getattr__(self, name):
+        return lambda *args: None
+
+
 def _native():
     """The ordinary calls without Python in between (csrc/py_calls.cc): functions that return None for every call that is anything
-    else, which the code below then makes."""
+    else, which the code below then makes. The module is built for one Python and one torch; with another the code below makes all
+    calls, with the same kernels."""
     global _ready_calls
     if _ready_calls is None:
         lib()
-        if not os.path.exists(_CALLS_PATH):
-            raise ImportError(f"{_CALLS_PATH} is missing: build it with `python -c 'import __graft_entry__ as g; g.build()'`.")
-        from . import _calls as module
+        try:
+            from . import _calls as module
+        except ImportError as e:
+            warnings.warn(f"tiledcuda_amd._calls is not there for this Python and torch ({e}): calls take 3 us longer. Build it with "
+                          "`python -c 'import __graft_entry__ as g; g.build()'`.", RuntimeWarning, stacklevel=3)
+            module = _NoCalls()
         _ready_calls = module
     return _ready_calls
 

@@ -17,6 +17,7 @@
 
 #include <climits>
 #include <cmath>
+#include <cstring>
 
 #include "tcu_c_api.h"
 
@@ -271,4 +272,13 @@ PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_calls", nullptr, -1, kMethods, n
 
 }  // namespace
 
-extern "C" __attribute__((visibility("default"))) PyObject* PyInit__calls() { return PyModule_Create(&kModule); }
+extern "C" __attribute__((visibility("default"))) PyObject* PyInit__calls() {
+    // torch's C++ classes are those of the release that this was compiled against
+    THPObjectPtr torch(PyImport_ImportModule("torch")), version(torch ? PyObject_GetAttrString(torch.get(), "__version__") : nullptr);
+    THPObjectPtr text(version ? PyObject_Str(version.get()) : nullptr);
+    const char* const running = text ? PyUnicode_AsUTF8(text.get()) : nullptr;
+    if (!running) return nullptr;
+    if (std::strcmp(running, TCU_TORCH_VERSION) != 0)
+        return PyErr_Format(PyExc_ImportError, "compiled for torch %s, this is %s", TCU_TORCH_VERSION, running);
+    return PyModule_Create(&kModule);
+}
