@@ -159,6 +159,10 @@ int tcu_version(void);
 /* Message of the last error raised on the calling thread ("" if none). */
 const char* tcu_last_error(void);
 
+/* Name (as compiled) of the kernel that the calling thread's last launch through this library ran, or of the one `back` launches
+ * before it; "" beyond the last four. What a call that leaves the choice to the library has run. */
+const char* tcu_recent_kernel(int back);
+
 /* Number of HIP devices visible, or a negative tcu_status. */
 int tcu_device_count(void);
 

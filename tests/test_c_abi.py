@@ -38,6 +38,17 @@ def test_version_and_error_string(tcu):
     assert isinstance(tcu.last_error(), str)
 
 
+def test_recent_kernel_without_a_launch(tcu):
+    """A thread that has launched nothing has no last kernel, whichever is asked for."""
+    import threading
+
+    names = []
+    thread = threading.Thread(target=lambda: names.extend(tcu.lib().tcu_recent_kernel(k) for k in (-1, 0, 3, 4, 1 << 30)))
+    thread.start()
+    thread.join()
+    assert names == [b""] * 5
+
+
 @pytest.mark.parametrize("call", [
     lambda l: l.tcu_gemm_f16(0, 0, 0, 128, 64, 256, 0, 0, 0),
     lambda l: l.tcu_b2b_gemm_f16(0, 0, 0, 0, 64, 64, 64, 64, 1, 0, 0),

@@ -80,6 +80,41 @@ def test_lstm_layer_without_an_initial_state(tcu, device, T, B, I, H):
         assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
 
 
+def ran(tcu, name, back=0):
+    """Whether the kernel of the last launch but ``back`` is ``name`` (an instantiation of the template)."""
+    return f"{len(name)}{name}I" in tcu.lib().tcu_recent_kernel(back).decode()
+
+
+@pytest.mark.parametrize("T,B,I,H,projection", [(7, 16, 16, 16, "gemm_direct"),
+                                                # K-splitting: rows and gates partial, rows whole, both whole; K tails with the same
+                                                (23, 208, 384, 112, "gemm_w128k"), (19, 256, 384, 112, "gemm_w128k"), (17, 128, 384, 256, "gemm_w128k"),
+                                                (23, 208, 704, 112, "gemm_w128k"), (17, 128, 704, 256, "gemm_w128k"), (9, 224, 704, 464, "gemm_w128k"),
+                                                # 256 x 256 tiles: partial, whole; K tails; the layer with odd multiples of 16
+                                                (23, 208, 64, 64, "gemm_w128"), (19, 256, 64, 64, "gemm_w128"), (24, 240, 16, 64, "gemm_w128"),
+                                                (23, 256, 16, 64, "gemm_w128"), (24, 80, 336, 656, "gemm_w128"),
+                                                # the pipelined kernel's ring and its 64 x 64 tiles, with K tails and without
+                                                (9, 96, 16, 16, "gemm_pipelined"), (8, 48, 64, 64, "gemm_pipelined"),
+                                                (10, 208, 336, 256, "gemm_pipelined"), (12, 112, 1024, 768, "gemm_pipelined")])
+def test_lstm_layer_projections(tcu, device, T, B, I, H, projection):
+    """Every kernel that computes the input half of the gates, with W's row distance and the synchronisation words to clear: twice in one
+    workspace whose words hold something else before each call. AUTO takes the same."""
+    import torch
+
+    print(f"lstm layer projection T{T} B{B} I{I} H{H} {projection}", flush=True)
+    args = operands(tcu, device, T, B, I, H)
+    want = tcu.lstm(*args, workspace=False)
+    need = int(tcu.lib().tcu_lstm_layer_workspace_bytes(T, B, I, H))
+    ws = torch.full((need + 256,), 0x5A, dtype=torch.uint8, device=device)
+    for _ in range(2):
+        got = tcu.lstm(*args, algo="layer", workspace=ws)
+        assert ran(tcu, "lstm_layer_xcd") and ran(tcu, projection, 1)
+        assert close(got, want)
+        ws[:4096] = 0x5A
+    assert bool((ws[need:] == 0x5A).all()) and tcu.lib().tcu_lstm_uses_layer(T, B, I, H) == 1
+    auto = tcu.lstm(*args)
+    assert ran(tcu, "lstm_layer_xcd") and ran(tcu, projection, 1) and torch.equal(auto[0], got[0]) and torch.equal(auto[1], got[1])
+
+
 def test_lstm_layer_against_the_oracle(tcu, oracle, device):
     import torch
 

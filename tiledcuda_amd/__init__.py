@@ -51,6 +51,7 @@ SCATTER_MODES = {"assign": 0, "add": 1}
 # every exported symbol with its ctypes signature (also what the symbol test checks)
 _SIGNATURES = {
     "tcu_version": (ctypes.c_int, []),
+    "tcu_recent_kernel": (ctypes.c_char_p, [ctypes.c_int]),
     "tcu_last_error": (ctypes.c_char_p, []),
     "tcu_device_count": (ctypes.c_int, []),
     "tcu_gemm_f16": (ctypes.c_int, [ctypes.c_void_p] * 3 + [ctypes.c_int] * 5 + [ctypes.c_void_p]),

@@ -57,6 +57,11 @@ int hip_fail(hipError_t e, const char* what) {
 /// Launch with dynamic LDS; raises the limit when the kernel needs more than the default. The kernel's parameter types
 /// are taken from the kernel pointer and every argument is converted to its parameter's type before its address goes
 /// into the argument array: an argument of another width or a wrong count is a compile error, not a garbled launch.
+/// The kernels that the thread's last launches ran (host functions; tcu_recent_kernel names them).
+constexpr unsigned kRecentKernels = 4;
+thread_local const void* g_recent_kernels[kRecentKernels];
+thread_local unsigned g_launches = 0;
+
 template <typename... Params, typename... Args>
 int launch(void (*kernel)(Params...), dim3 grid, dim3 block, int lds_bytes, hipStream_t stream, Args&&... args) {
     static_assert(sizeof...(Params) == sizeof...(Args), "launch: argument count differs from the kernel's parameter count");
@@ -91,6 +96,7 @@ int launch(void (*kernel)(Params...), dim3 grid, dim3 block, int lds_bytes, hipS
     }(std::index_sequence_for<Params...>{});
     hipError_t e = hipLaunchKernel(reinterpret_cast<const void*>(kernel), grid, block, argv, size_t(lds_bytes), stream);
     if (e != hipSuccess) return hip_fail(e, "kernel launch");
+    g_recent_kernels[g_launches++ % kRecentKernels] = reinterpret_cast<const void*>(kernel);
     return TCU_OK;
 }
 
@@ -1632,6 +1638,12 @@ int lstm_f16_layer(const void* x, const void* W, const void* bias, const void* h
 extern "C" {
 
 int tcu_version(void) { return 100; }
+
+const char* tcu_recent_kernel(int back) {
+    if (back < 0 || unsigned(back) >= kRecentKernels || unsigned(back) >= g_launches) return "";
+    const char* name = hipKernelNameRefByPtr(g_recent_kernels[(g_launches - 1 - back) % kRecentKernels], nullptr);
+    return name ? name : "";
+}
 
 const char* tcu_last_error(void) { return g_last_error.c_str(); }
 
