@@ -187,13 +187,16 @@ def test_gemm_split_k_in_many_ranges(tcu, oracle, device, M, N, K, splits, out_d
     assert oracle.max_rel_err(got, tcu.gemm(a, b, out_dtype=torch.float32, workspace=False).cpu().numpy()) <= REL_TOL
 
 
-@pytest.mark.parametrize("M,N,K", [(1040, 1040, 1040), (1040, 1024, 1088),   # 96 x 64 tiles: rows 80 of 96, columns 16 of 64, K 16 of 64
-                                   (1312, 784, 624), (1312, 768, 272),
-                                   (2064, 1040, 1072), (1424, 1520, 1040)])  # 96 x 96: rows 48, 80 of 96, columns 80
+@pytest.mark.parametrize("M,N,K,tile,whole", [(1040, 1040, 1040, (96, 64), False),   # rows 80 of 96, columns 16 of 64, K 16 of 64
+                                              (1040, 1024, 1088, (96, 64), False), (1312, 784, 624, (96, 64), False),
+                                              (1312, 832, 272, (96, 64), False), (288, 3328, 256, (96, 64), True),
+                                              (2064, 1040, 1072, (96, 96), False),   # rows 48 of 96, columns 80, K 48 of 64
+                                              (1424, 1552, 1040, (96, 96), False), (1056, 1824, 1600, (96, 96), True)])
 @pytest.mark.parametrize("out_dtype", ["float16", "float32"])
-def test_ring_tiles_with_96_rows(tcu, device, M, N, K, out_dtype):
-    """Products that AUTO gives the ring with 96 x 64 or 96 x 96 tiles, every element of the output and what lies behind it: f32 sums
-    in another order (1e-6 of the norm), rounded to f16 (2^-11) where the output is."""
+def test_ring_tiles_with_96_rows(tcu, device, M, N, K, tile, whole, out_dtype):
+    """Products that AUTO gives the ring with 96 x 64 or 96 x 96 tiles where the results are f16, and other tiles where they are f32:
+    every element of the output and what lies behind it, f32 sums in another order (1e-6 of the norm), rounded to f16 (2^-11) where
+    the output is."""
     import torch
 
     print(f"gemm ring 96 {M}x{N}x{K} {out_dtype}", flush=True)
@@ -203,6 +206,9 @@ def test_ring_tiles_with_96_rows(tcu, device, M, N, K, out_dtype):
     dtype = getattr(torch, out_dtype)
     buf = torch.full((M * N + 4096,), 7.0, dtype=dtype, device=device)
     tcu.gemm(a, b, out=buf[:M * N].view(M, N), workspace=False)
+    kernel = tcu.lib().tcu_recent_kernel(0).decode()
+    assert (f"PipelinedGemmTraitsILi{tile[0]}ELi{tile[1]}E" in kernel) == (out_dtype == "float16"), kernel
+    assert out_dtype == "float32" or (f"__halfLb{int(not whole)}E" in kernel), kernel  # (with edges or without)
     want = a.double() @ b.double().t()
     err = float((buf[:M * N].view(M, N).double() - want).norm() / want.norm())
     assert err <= (1e-6 if dtype == torch.float32 else 2 ** -11)

@@ -465,10 +465,12 @@ double gemm_w128_us(long tiles, int K) {
     return 3.0 + (K / 1024.0) * (23.5 * full + last_us);
 }
 
-/// Whether a product that the K-splitting kernel would take (about one tile of 128 x 128 or 128 x 96 per CU) goes to the pipelined
-/// kernel's ring with tiles of 96 x 96 instead: with a K this short the sums over the wavefronts cost more than the fragments that they
-/// share save. One workgroup per CU, 2.5 us + per 1024 of K 6.2 us with few of them, 8.4 with 256; a K tail costs the other kernel
-/// 1 us. us, K-splitting -> this: 2064 x 1040 x 1072: 13.0 -> 12.0; longer K stays: 2048 x 1024 x 4096: 26.9, 31.0.
+/// Whether a product with f16 results that the K-splitting kernel would take (about one tile of 128 x 128 or 128 x 96 per CU) goes to the
+/// pipelined kernel's ring with tiles of 96 x 96 instead: with a K this short the sums over the wavefronts cost more than the fragments
+/// that they share save. One workgroup per CU, 2.5 us + per 1024 of K 6.2 us with few of them, 8.4 with 256; a K tail costs the other
+/// kernel 1 us. us, K-splitting -> this: 2064 x 1040 x 1072: 13.6 -> 11.4; 576 x 3776 x 1264: 14.2 -> 12.3; 992 x 1952 x 1680: 14.8 -> 15.2 (of
+/// 36 such sizes 33 are shorter, on average by 8 %). f32 results take this kernel 1.3 us more and stay (34 sizes, on average as long:
+/// 2096 x 1040 x 1424: 16.0, 14.8; 976 x 1936 x 1552: 14.9, 15.9), and so does a longer K (2048 x 1024 x 4096: 26.9, 31.0).
 bool gemm_wide_ring_is_the_choice(int M, int N, int K) {
     const long tiles = (long)((M + 95) / 96) * ((N + 95) / 96);
     if (tiles > 256 || (long)K * 512 >= (1l << 32)) return false;
@@ -725,7 +727,8 @@ int gemm_dispatch(const __half* A, const __half* B, OutType* C, int M, int N, in
             // too few 256 x 256 tiles for the chip, but about one 128 x 128 tile per CU and a long enough K: the
             // kernel whose wavefronts split K (each owns the whole tile)
             if (gemm_w128k_is_the_choice(M, N, K)) {
-                if (gemm_wide_ring_is_the_choice(M, N, K)) return gemm_pipelined_dispatch<OutType>(A, B, C, M, N, K, stream, 0, 0, nullptr, 0, true);
+                if (sizeof(OutType) == 2 && gemm_wide_ring_is_the_choice(M, N, K))
+                    return gemm_pipelined_dispatch<OutType>(A, B, C, M, N, K, stream, 0, 0, nullptr, 0, true);
                 return gemm_w128k_dispatch<OutType>(A, B, C, M, N, K, stream);
             }
             // between the two: 256 x 128 tiles fill one round
