@@ -1558,8 +1558,8 @@ int launch_lstm_layer_part(const __half* x, const __half* W, const __half* bias,
         case 1: {
             using Tk = GemmW128kTraits;
             const long tiles = ((rows + 127l) / 128) * ((4l * H + 127) / 128);
-            auto kernel = I % Tk::kBK != 0 ? &gemm_w128k<float, true, Tk, true> : rows % Tk::kBM == 0 && 4 * H % Tk::kBN == 0
-                          ? &gemm_w128k<float, false, Tk> : &gemm_w128k<float, true, Tk>;
+            auto kernel = I % Tk::kBK != 0 ? &gemm_w128k<float, true, Tk, true, true> : rows % Tk::kBM == 0 && 4 * H % Tk::kBN == 0
+                          ? &gemm_w128k<float, false, Tk, false, true> : &gemm_w128k<float, true, Tk, false, true>;
             rc = launch(kernel, dim3(unsigned(tiles)), dim3(Tk::kThreads), Tk::kLdsBytes, s, x, W, pre, rows, 4 * H, I, I, I + H, 4 * H, sync,
                         kSyncWords);
             break;
