@@ -54,14 +54,14 @@ int hip_fail(hipError_t e, const char* what) {
     return fail(TCU_ERR_HIP, std::string(what) + ": " + hipGetErrorString(e));
 }
 
-/// Launch with dynamic LDS; raises the limit when the kernel needs more than the default. The kernel's parameter types
-/// are taken from the kernel pointer and every argument is converted to its parameter's type before its address goes
-/// into the argument array: an argument of another width or a wrong count is a compile error, not a garbled launch.
 /// The kernels that the thread's last launches ran (host functions; tcu_recent_kernel names them).
 constexpr unsigned kRecentKernels = 4;
 thread_local const void* g_recent_kernels[kRecentKernels];
 thread_local unsigned g_launches = 0;
 
+/// Launch with dynamic LDS; raises the limit when the kernel needs more than the default. The kernel's parameter types
+/// are taken from the kernel pointer and every argument is converted to its parameter's type before its address goes
+/// into the argument array: an argument of another width or a wrong count is a compile error, not a garbled launch.
 template <typename... Params, typename... Args>
 int launch(void (*kernel)(Params...), dim3 grid, dim3 block, int lds_bytes, hipStream_t stream, Args&&... args) {
     static_assert(sizeof...(Params) == sizeof...(Args), "launch: argument count differs from the kernel's parameter count");
@@ -225,7 +225,7 @@ PipePlan pipelined_plan(int M, int N, int K) {
 
 /// The pipelined kernel for M, N, K any multiples of 16, with the tile of pipelined_plan(). Edge tiles (rows clamped,
 /// stores guarded, the K tail zeroed in LDS) are compiled in only where the shape is not a whole number of the chosen
-/// tiles. ldb other than K and words to clear: f32 results only.
+/// tiles. ldb other than K and words to clear: f32 results only; wide_ring: f16 results only.
 template <typename OutType>
 int gemm_pipelined_dispatch(const __half* A, const __half* B, OutType* C, int M, int N, int K, hipStream_t stream,
                             int ldc = 0, int ldb = 0, unsigned int* zero_words = nullptr, int zero_count = 0, bool wide_ring = false) {
@@ -249,19 +249,23 @@ int gemm_pipelined_dispatch(const __half* A, const __half* B, OutType* C, int M,
         return launch(&gemm_pipelined<Traits, OutType, true>, dim3(unsigned(grid)), dim3(Traits::kThreads),
                       Traits::template lds_bytes<OutType>(), stream, A, B, C, M, N, K, ldb, ldc, zero_words, zero_count);
     };
-    if (wide_ring) return go(PipeWideRing{});
+    if constexpr (std::is_same_v<OutType, __half>)
+        if (wide_ring) return go(PipeWideRing{});
     switch (pipelined_plan(M, N, K).config) {
         case kPipeLarge: return go(PipeLarge{});
         case kPipeMid: return go(PipeMid{});
         case kPipeSmall: return go(PipeSmall{});
         default: break;
     }
-    // the ring, more than one 64 x 64 tile per CU, M not whole tiles: tiles of 96 x 64 where there is at most one of them per CU (us,
-    // f16, 64 x 64 -> 96 x 64: 1040^2 x 2064: 19.2 -> 15.1; 1312 x 784 x 2832: 24.7 -> 19.0; 624 x 2000 x 1232: 10.8, 11.1; whole tiles have
-    // no edges to lose: 832 x 1664 x 1152: 8.9, 9.4; f32 results, 32 bytes per lane and row, gain at long K only: 1184 x 1120 x 672: 8.1,
-    // 8.3; a single step of K nowhere: 1968 x 768 x 64: 3.4, 3.5)
-    const long small = (long)((M + 63) / 64) * ((N + 63) / 64), tall = (long)((M + 95) / 96) * ((N + 63) / 64);
-    if (sizeof(OutType) == 2 && M % 64 != 0 && K >= 256 && small > 256 && small <= 512 && tall <= 256) return go(PipeTallRing{});
+    // the ring, f16 results, more than one 64 x 64 tile per CU, M not whole tiles: tiles of 96 x 64 where there is at most one of them
+    // per CU. us, 64 x 64 -> 96 x 64: 1040^2 x 2064: 19.2 -> 15.1; 1312 x 784 x 2832: 24.7 -> 19.0; 624 x 1984 x 1344: 10.0, 10.1 (of 60 such
+    // sizes 57 are as short or shorter, on average by 11 %, and 3 longer, at most by 2.5 %: 2544 x 448 x 3936: 23.7, 24.3). Whole tiles
+    // have no edges to lose (832 x 1664 x 1152: 8.9, 9.4), f32 results, 32 bytes per lane and row, gain at long K only (1184 x 1120 x
+    // 672: 8.1, 8.3), a single step of K nothing (1968 x 768 x 64: 3.4, 3.5).
+    if constexpr (std::is_same_v<OutType, __half>) {
+        const long small = (long)((M + 63) / 64) * ((N + 63) / 64), tall = (long)((M + 95) / 96) * ((N + 63) / 64);
+        if (M % 64 != 0 && K >= 256 && small > 256 && small <= 512 && tall <= 256) return go(PipeTallRing{});
+    }
     return go(PipeSmallRing{});
 }
 
@@ -727,7 +731,7 @@ int gemm_dispatch(const __half* A, const __half* B, OutType* C, int M, int N, in
             // too few 256 x 256 tiles for the chip, but about one 128 x 128 tile per CU and a long enough K: the
             // kernel whose wavefronts split K (each owns the whole tile)
             if (gemm_w128k_is_the_choice(M, N, K)) {
-                if (sizeof(OutType) == 2 && gemm_wide_ring_is_the_choice(M, N, K))
+                if (std::is_same_v<OutType, __half> && gemm_wide_ring_is_the_choice(M, N, K))
                     return gemm_pipelined_dispatch<OutType>(A, B, C, M, N, K, stream, 0, 0, nullptr, 0, true);
                 return gemm_w128k_dispatch<OutType>(A, B, C, M, N, K, stream);
             }
