@@ -105,3 +105,31 @@ def test_calls_are_those_of_this_interpreter(tcu, monkeypatch):
         assert tcu._native() is absent
     with pytest.raises(ValueError, match="device memory"):
         tcu.gemm(torch.zeros(16, 16, dtype=torch.float16), torch.zeros(16, 16, dtype=torch.float16))
+
+
+@pytest.mark.gpu
+def test_entries_inside_torch_compile(tcu, device):
+    """Functions that torch.compile traces call the entries, every one of them, without a warning about a function it does not know."""
+    import warnings
+
+    half = lambda *shape: (torch.randn(*shape, device=device) * 0.3).half()
+    a, q = half(64, 64), half(2, 64, 64)
+    x, W, bias = half(5, 32, 64), half(4 * 48, 64 + 48), half(4 * 48)
+    flat, idx = half(64 * 128), torch.tensor([[3], [1]], device=device)
+
+    def op(t):
+        o = torch.empty_like(t)
+        tcu.flash_attention_fwd(t, flat, flat, o, 64, 64, 128, 128, scale=0.1)
+        return o
+
+    def scatter(t):
+        d = torch.ones(8, 64, device=device).half()
+        tcu.scatter_nd(d, idx, t[:2].contiguous(), mode="add")
+        return d
+
+    for f, t in ((lambda t: tcu.gemm(t * 2, a), a), (lambda t: tcu.b2b_gemm(t * 2, a, a), a), (lambda t: tcu.flash_attention(t * 2, q, q), q),
+                 (lambda t: op(t * 2), flat), (lambda t: tcu.lstm(t * 2, W, bias)[0], x), (lambda t: scatter(t * 2), a)):
+        want = f(t) + 1
+        with warnings.catch_warnings():
+            warnings.filterwarnings("error", message=".*does not know how to trace")
+            assert torch.equal(torch.compile(lambda t: f(t) + 1, backend="eager")(t), want)

@@ -27,6 +27,8 @@ _HERE = os.path.dirname(os.path.abspath(__file__))
 _LIB_PATH = os.path.join(_HERE, "lib", "libtiledcuda_amd.so")
 _lib = None
 _ready_calls = None
+# torch.compile, reading these entries, stops at a C function that it does not know with a warning; at the ctypes calls it stops without
+_tracing = torch.compiler.is_dynamo_compiling
 
 TCU_OK = 0
 TCU_ERR_INVALID_ARGUMENT = -1
@@ -191,7 +193,7 @@ def gemm(a: torch.Tensor, b_t: torch.Tensor, out: torch.Tensor | None = None,
     torch's caching allocator for the call; ``workspace=False`` never splits (use it, or a workspace of your own, when
     the call is being captured into a HIP graph: an allocation has no place in a captured stream).
     """
-    if out is None and workspace is None and algo == "auto":
+    if out is None and workspace is None and algo == "auto" and not _tracing():
         out = (_ready_calls or _native()).gemm(a, b_t, out_dtype)
         if out is not None:
             return out
@@ -233,7 +235,7 @@ def b2b_gemm(a: torch.Tensor, b_t: torch.Tensor, c_t: torch.Tensor, out: torch.T
              out_dtype: torch.dtype = torch.float16, algo: str = "auto") -> torch.Tensor:
     """D = (A · B) · C per batch item; ``b_t`` [.., N, K] and ``c_t`` [.., P, N] are the
     column-major operands of the reference's fused two-GEMM example stored as arrays."""
-    if out is None and algo == "auto":
+    if out is None and algo == "auto" and not _tracing():
         out = (_ready_calls or _native()).b2b_gemm(a, b_t, c_t, out_dtype)
         if out is not None:
             return out
@@ -285,7 +287,8 @@ def flash_attention_fwd(Q: torch.Tensor, K: torch.Tensor, V: torch.Tensor, O: to
     device tensors; K as [n, k], V as [p, n]; O written in place; ``scale`` defaults to the
     reference's 1; ``algo`` picks a kernel and ``workspace`` is as in ``flash_attention``).  Unsupported shapes raise
     ``RuntimeError`` like the reference op."""
-    if workspace is None and algo == "auto" and (_ready_calls or _native()).flash_attention_fwd(Q, K, V, O, m, n, k, p, scale, batch):
+    if workspace is None and algo == "auto" and not _tracing() and \
+            (_ready_calls or _native()).flash_attention_fwd(Q, K, V, O, m, n, k, p, scale, batch):
         return
     if min(m, n, k, p, batch) <= 0:
         raise ValueError("m, n, k, p and batch must be positive")
@@ -310,7 +313,7 @@ def flash_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scale: fl
     when none is given, through one taken from torch's caching allocator for the call; ``workspace=False`` never splits. A call
     that is being captured into a HIP graph splits through a workspace of yours only (it has to live as long as the graph)
     and without one runs unsplit: an allocation has no place in a captured stream."""
-    if out is None and workspace is None and algo == "auto":
+    if out is None and workspace is None and algo == "auto" and not _tracing():
         out = (_ready_calls or _native()).flash_attention(q, k, v, scale)
         if out is not None:
             return out
@@ -386,7 +389,7 @@ def lstm(x: torch.Tensor, W: torch.Tensor, bias: torch.Tensor, h0: torch.Tensor 
     (``tcu_lstm_f16_persistent``: H in {256, 512, 768, 1024}, B <= 256 in multiples of 32; ``lstm_persistent_workspace_bytes``). Its
     workgroups wait for each other with a time limit; with ``check=True`` (the default) the stream is synchronised and
     a RuntimeError raised if a wait expired, ``check=False`` leaves that to a later ``lstm_persistent_status(workspace)``."""
-    if out is None and workspace is None and algo == "auto":
+    if out is None and workspace is None and algo == "auto" and not _tracing():
         pair = (_ready_calls or _native()).lstm(x, W, bias, h0, c0)
         if pair is not None:
             return pair
@@ -492,7 +495,7 @@ def scatter_nd(scatter_data: torch.Tensor, scatter_indices: torch.Tensor, scatte
     [..., d_k, ..., d_{r-1}]. (The reference wrapper is handed flattened tensors, which loses the shapes its op
     reads them from; pass the shaped tensors here.) Rows with an out-of-range index are skipped; if
     ``skipped_rows`` (uint32/int32 device tensor of one element, zeroed by the caller) is given it counts them."""
-    if skipped_rows is None and mode in SCATTER_MODES and \
+    if skipped_rows is None and mode in SCATTER_MODES and not _tracing() and \
             (_ready_calls or _native()).scatter_nd(scatter_data, scatter_indices, scatter_updates, SCATTER_MODES[mode]):
         return
     k = scatter_indices.shape[-1]
