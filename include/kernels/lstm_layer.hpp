@@ -22,8 +22,8 @@
 // from that step on, and one step later so is all that is computed from them.)
 // Measured, kernel alone, us: T 24, B 80, H 656: 55 (6 us until the first workgroups know their rows, 7 for the weights, 1.75 per step:
 // 0.45 for h to come back from the L2, 0.2 to LDS, 0.6 for 48 products and their fragments, 0.3 for the cell); 16, 256, 1024: 79
-// (3.9 per step: the LDS, 64 KB of h in and 256 KB of fragments out, and h itself, 64 KB at 45 bytes per clock); 31, 80, 384: 48;
-// 20, 32, 96: 20.
+// (20 before the first step, 3.7 per step: the LDS, 64 KB of h in and 256 KB of fragments out, and h itself, 64 KB at 45 bytes per
+// clock); 31, 80, 384: 48; 20, 32, 96: 20.
 #pragma once
 
 #include <type_traits>

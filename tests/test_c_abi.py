@@ -49,6 +49,22 @@ def test_recent_kernel_without_a_launch(tcu):
     assert names == [b""] * 5
 
 
+def test_workspaces_that_the_entries_do_not_ask_for(tcu):
+    """What the Python entries know without asking, a ctypes call saved, is what the library answers: 512 keys or fewer are never split,
+    fewer than 4 steps or 512 inputs never have a projection of their own, fewer than 4 steps never run as a layer."""
+    l = tcu.lib()
+    for D, v in ((64, 0), (128, 0), (128, 1)):
+        for batch in (1, 7, 32, 256):
+            for M in (64, 192, 576, 4096):
+                assert [n for n in range(64, 1153, 64) if l.tcu_flash_attn_workspace_bytes(batch, M, n, D, D, v) and n <= 512] == []
+    assert l.tcu_flash_attn_workspace_bytes(1, 64, 8192, 128, 128, 0) > 0
+    for T, I in ((1, 4096), (3, 4096), (3, 64), (16, 384)):
+        for B, H in ((64, 128), (256, 1024), (2048, 256)):
+            assert l.tcu_lstm_uses_workspace(T, B, I, H) == 0
+            assert T >= 4 or l.tcu_lstm_uses_layer(T, B, I, H) == 0
+    assert l.tcu_lstm_uses_workspace(8, 64, 8192, 4096) == 1
+
+
 @pytest.mark.parametrize("call", [
     lambda l: l.tcu_gemm_f16(0, 0, 0, 128, 64, 256, 0, 0, 0),
     lambda l: l.tcu_b2b_gemm_f16(0, 0, 0, 0, 64, 64, 64, 64, 1, 0, 0),

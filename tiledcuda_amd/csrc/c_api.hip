@@ -1385,7 +1385,7 @@ double lstm_step_us(int B, int H, int columns) {
 /// 512, H 1024: 118, 138. Of 115 more sizes the chosen plan is within 3 % of the shorter for 108, at most 14 % above it
 /// (T 4, B 1472, I 1280, H 128: 41, 36).
 bool lstm_projection_pays(int T, int B, int I, int H) {
-    if (tcu_lstm_workspace_bytes(T, B, I, H) == 0 || I < 512 || T < 4 || (long)T * B > INT_MAX) return false;
+    if (I < 512 || T < 4 || tcu_lstm_workspace_bytes(T, B, I, H) == 0 || (long)T * B > INT_MAX) return false;
     if (!lstm_direct_takes(B, I, H)) return true;  // (the streaming step kernel: half of its bytes are W[:, :I])
     const double projection = 3.5 + 0.83 * lstm_projection_plan((long)T * B, I, H).us + 0.37 * 16e-6 * T * double(B) * H;
     return 1.02 * (projection + T * lstm_step_us(B, H, H)) < T * lstm_step_us(B, H, I + H);
@@ -1743,6 +1743,7 @@ int tcu_flash_attn_fwd_f16(const void* Q, const void* K, const void* V, void* O,
 unsigned long long tcu_flash_attn_workspace_bytes(int batch, int M, int N, int Kdim, int P, int v_layout) {
     if (!positive({batch, M, N, Kdim, P}) || Kdim != P || M % 64 != 0 || N % 64 != 0) return 0;
     if (v_layout != TCU_V_ROW_MAJOR && v_layout != TCU_V_COL_MAJOR) return 0;
+    if (N <= 512) return 0;  // (never split: not worth a plan)
     const int splits = attn_keys_plan(batch, M, N, Kdim, v_layout, 16);
     return splits > 1 ? (unsigned long long)splits * batch * M * (Kdim + 2) * sizeof(float) : 0;
 }

@@ -121,8 +121,8 @@ PyObject* b2b_gemm(PyObject*, PyObject* const* args, Py_ssize_t n) {
 bool attention(const void* q, const void* k, const void* v, void* o, int batch, int M, int N, int D, int P, float scale, int v_layout,
                const at::Tensor& like, c10::DeviceIndex device) {
     void* const stream = current_stream(device);
-    // (fewer keys are never split; in a captured stream nothing is allocated)
-    const unsigned long long need = N > 512 ? tcu_flash_attn_workspace_bytes(batch, M, N, D, P, v_layout) : 0;
+    // (in a captured stream nothing is allocated)
+    const unsigned long long need = tcu_flash_attn_workspace_bytes(batch, M, N, D, P, v_layout);
     if (need > 0 && !capturing()) {
         const at::Tensor ws = bytes(like, need);
         void* const wp = ws.data_ptr();
@@ -209,12 +209,12 @@ PyObject* lstm(PyObject*, PyObject* const* args, Py_ssize_t n) {
     void *hp = h_all.data_ptr(), *cp = c_out.data_ptr();
     bool ok;
     at::Tensor layer_ws;
-    const unsigned long long layer_need = T >= 4 && tcu_lstm_uses_layer(T, B, I, H) && !capturing() ? tcu_lstm_layer_workspace_bytes(T, B, I, H) : 0;
+    const unsigned long long layer_need = tcu_lstm_uses_layer(T, B, I, H) && !capturing() ? tcu_lstm_layer_workspace_bytes(T, B, I, H) : 0;
     if (layer_need > 0) layer_ws = bytes_if_free(*x, layer_need);
     if (layer_ws.defined()) {
         void* const sp = layer_ws.data_ptr();
         ok = succeeds([&] { return tcu_lstm_f16_layer(xp, wp, bp, state[0], state[1], hp, cp, T, B, I, H, sp, layer_need, stream); });
-    } else if (T >= 4 && I >= 512 && tcu_lstm_uses_workspace(T, B, I, H)) {
+    } else if (tcu_lstm_uses_workspace(T, B, I, H)) {
         const unsigned long long need = tcu_lstm_workspace_bytes(T, B, I, H);
         const at::Tensor ws = bytes(*x, need);
         void* const sp = ws.data_ptr();
